@@ -1116,17 +1116,31 @@ int attention_core(int dtype, const void* Q, const void* K, const void* V, void*
     return ATN_OK;
 }
 
-int pe_apply_core(int dtype, const void* in, void* out, long n_rows, int seq_len, int D,
-                  const atn_pe_desc* pe, hipStream_t stream) {
+// One or two pre-pass tensors of the same head_d, dtype and encoding.
+struct PeIo {
+    const void* in;
+    void* out;
+    long n_rows;
+    int seq_len;
+};
+
+int pe_apply_core(int dtype, const PeIo* io, int n, int D, const atn_pe_desc* pe,
+                  hipStream_t stream) {
     if (dtype != ATN_DTYPE_F32 && dtype != ATN_DTYPE_BF16) return ATN_ERR_BAD_ARGUMENT;
-    if (!in || !out || !pe) return ATN_ERR_NULL_POINTER;
-    if (n_rows < 1 || seq_len < 1 || D < 1) return ATN_ERR_BAD_DIMENSION;
-    int64_t n;
-    if (!mul_ok(n_rows, D, &n) || n > INT64_MAX / 8) return ATN_ERR_SIZE_OVERFLOW;
     const size_t es = elem_size(dtype);
-    if (!aligned(in, es) || !aligned(out, es)) return ATN_ERR_MISALIGNED;
-    if (in != out && overlaps(in, n * (int64_t)es, out, n * (int64_t)es))
-        return ATN_ERR_ALIASING;
+    const size_t va = dtype == ATN_DTYPE_F32 ? 16 : 8;
+    int vec = D % 4 == 0, npos = 0;
+    for (int i = 0; i < n; ++i) {
+        if (!io[i].in || !io[i].out || !pe) return ATN_ERR_NULL_POINTER;
+        if (io[i].n_rows < 1 || io[i].seq_len < 1 || D < 1) return ATN_ERR_BAD_DIMENSION;
+        int64_t e;
+        if (!mul_ok(io[i].n_rows, D, &e) || e > INT64_MAX / 8) return ATN_ERR_SIZE_OVERFLOW;
+        if (!aligned(io[i].in, es) || !aligned(io[i].out, es)) return ATN_ERR_MISALIGNED;
+        if (io[i].in != io[i].out && overlaps(io[i].in, e * (int64_t)es, io[i].out, e * (int64_t)es))
+            return ATN_ERR_ALIASING;
+        vec = vec && aligned(io[i].in, va) && aligned(io[i].out, va);
+        npos = std::max(npos, io[i].seq_len);
+    }
     atn_pe_desc d = *pe;
     d.apply_q = d.apply_k = 1;
     PePlan plan;
@@ -1136,13 +1150,26 @@ int pe_apply_core(int dtype, const void* in, void* out, long n_rows, int seq_len
     int dev;
     st = current_device(&dev);
     if (st != ATN_OK) return st;
-    st = bind_tables(&d, plan, D, seq_len, stream);
+    st = bind_tables(&d, plan, D, npos, stream);
     if (st != ATN_OK) return st;
-    const size_t va = dtype == ATN_DTYPE_F32 ? 16 : 8;
-    const int vec = (D % 4 == 0) && aligned(in, va) && aligned(out, va);
-    ATN_HIP(atn::launch_pe_apply(dtype, plan.pek, in, out, n_rows, seq_len, D, plan.q, vec,
-                                 stream));
+    atn::PeTensor t[2];
+    for (int i = 0; i < n; ++i)
+        t[i] = atn::PeTensor{io[i].in, io[i].out, io[i].n_rows, io[i].seq_len, plan.q};
+    ATN_HIP(atn::launch_pe_apply(dtype, plan.pek, t, n, D, vec, stream));
     return ATN_OK;
+}
+
+// Q -> Qe and K -> Ke of the fp32 "separate" pipelines: one launch, or one
+// after the other where a buffer of the one overlaps one of the other (a
+// caller may reuse Q's memory for K's result).
+int pe_apply_qk(const Shape& s, const float* Q, float* Qe, const float* K, float* Ke,
+                const atn_pe_desc* pe) {
+    const PeIo io[2] = {{Q, Qe, (long)(s.BH * s.Lq), s.Lq}, {K, Ke, (long)(s.BH * s.Lk), s.Lk}};
+    const int64_t qb = s.nq * 4, kb = s.nk * 4;
+    if (!overlaps(Qe, qb, K, kb) && !overlaps(Ke, kb, Q, qb) && !overlaps(Qe, qb, Ke, kb))
+        return pe_apply_core(ATN_DTYPE_F32, io, 2, s.D, pe, nullptr);
+    const int st = pe_apply_core(ATN_DTYPE_F32, &io[0], 1, s.D, pe, nullptr);
+    return st != ATN_OK ? st : pe_apply_core(ATN_DTYPE_F32, &io[1], 1, s.D, pe, nullptr);
 }
 
 // ---------------------------------------------------------------- drop-in helpers
@@ -1434,7 +1461,8 @@ size_t atn_attention_workspace_bytes(int dtype, int batch, int heads, int len_q,
 
 int atn_pe_apply_ex(int dtype, const void* in, void* out, long n_rows, int seq_len, int head_d,
                     const atn_pe_desc* pe, void* stream) {
-    return pe_apply_core(dtype, in, out, n_rows, seq_len, head_d, pe, (hipStream_t)stream);
+    const PeIo io{in, out, n_rows, seq_len};
+    return pe_apply_core(dtype, &io, 1, head_d, pe, (hipStream_t)stream);
 }
 
 int atn_attention_path_ex(int dtype, int batch, int heads, int len_q, int len_k, int head_d,
@@ -1528,9 +1556,7 @@ void attention_forward_separate_rope(const float* Q, const float* K, const float
     Shape s;
     int st = check_shape(batch_sz, num_heads, len_q, len_k, head_d, &s);
     if (st != ATN_OK) die(st, w);
-    st = pe_apply_core(ATN_DTYPE_F32, Q, Q_rope, (long)(s.BH * len_q), len_q, head_d, &d, nullptr);
-    if (st != ATN_OK) die(st, w);
-    st = pe_apply_core(ATN_DTYPE_F32, K, K_rope, (long)(s.BH * len_k), len_k, head_d, &d, nullptr);
+    st = pe_apply_qk(s, Q, Q_rope, K, K_rope, &d);
     if (st != ATN_OK) die(st, w);
     dropin_attention(w, ATN_DTYPE_F32, Q_rope, K_rope, V, out,
                      batch_sz, num_heads, len_q, len_k, head_d, nullptr);
@@ -1542,9 +1568,8 @@ void rope_forward(const float* input, float* output, const float* cos_cache,
     if (!cos_cache || !sin_cache) die(ATN_ERR_NULL_POINTER, "rope_forward");
     if (rotary_dim == 0) die(ATN_ERR_BAD_ROTARY, "rope_forward");
     const atn_pe_desc d = rope_desc(rotary_dim, ATN_ROPE_INTERLEAVED, true, true, cos_cache, sin_cache);
-    sync_or_die(pe_apply_core(ATN_DTYPE_F32, input, output, total_tokens, seq_len, hdim, &d,
-                              nullptr),
-                "rope_forward");
+    const PeIo io{input, output, total_tokens, seq_len};
+    sync_or_die(pe_apply_core(ATN_DTYPE_F32, &io, 1, hdim, &d, nullptr), "rope_forward");
 }
 
 void apply_sinusoidal_embeddings(const float* input, const float* sin_table,
@@ -1552,8 +1577,8 @@ void apply_sinusoidal_embeddings(const float* input, const float* sin_table,
                                  int hdim, int seqlen) {
     if (!sin_table || !cos_table) die(ATN_ERR_NULL_POINTER, "apply_sinusoidal_embeddings");
     const atn_pe_desc d = sin_desc(true, true, sin_table, cos_table);
-    sync_or_die(pe_apply_core(ATN_DTYPE_F32, input, output, total_tokens, seqlen, hdim, &d,
-                              nullptr),
+    const PeIo io{input, output, total_tokens, seqlen};
+    sync_or_die(pe_apply_core(ATN_DTYPE_F32, &io, 1, hdim, &d, nullptr),
                 "apply_sinusoidal_embeddings");
 }
 
@@ -1575,7 +1600,8 @@ void attention_forward_sinusoidal_hybrid(const float* Q, const float* K, const f
     int st = check_shape(batch_sz, num_heads, len_q, len_k, head_d, &s);
     if (st != ATN_OK) die(st, w);
     const atn_pe_desc dk = sin_desc(true, true, sin_table, cos_table);
-    st = pe_apply_core(ATN_DTYPE_F32, K, K_emb, (long)(s.BH * len_k), len_k, head_d, &dk, nullptr);
+    const PeIo io{K, K_emb, (long)(s.BH * len_k), len_k};
+    st = pe_apply_core(ATN_DTYPE_F32, &io, 1, head_d, &dk, nullptr);
     if (st != ATN_OK) die(st, w);
     const atn_pe_desc dq = sin_desc(true, false, sin_table, cos_table);
     dropin_attention(w, ATN_DTYPE_F32, Q, K_emb, V, out,
@@ -1592,9 +1618,7 @@ void attention_forward_sinusoidal_separate(const float* Q, const float* K, const
     int st = check_shape(batch_sz, num_heads, len_q, len_k, head_d, &s);
     if (st != ATN_OK) die(st, w);
     const atn_pe_desc d = sin_desc(true, true, sin_table, cos_table);
-    st = pe_apply_core(ATN_DTYPE_F32, Q, Q_emb, (long)(s.BH * len_q), len_q, head_d, &d, nullptr);
-    if (st != ATN_OK) die(st, w);
-    st = pe_apply_core(ATN_DTYPE_F32, K, K_emb, (long)(s.BH * len_k), len_k, head_d, &d, nullptr);
+    st = pe_apply_qk(s, Q, Q_emb, K, K_emb, &d);
     if (st != ATN_OK) die(st, w);
     dropin_attention(w, ATN_DTYPE_F32, Q_emb, K_emb, V, out,
                      batch_sz, num_heads, len_q, len_k, head_d, nullptr);

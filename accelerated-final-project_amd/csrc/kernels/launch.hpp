@@ -108,7 +108,17 @@ constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;  // ATN_NOALLOC_SCRATC
 bool noalloc_ready(int dev);
 hipError_t noalloc_scratch(int dev, size_t sync_bytes, hipStream_t st, void** ptr);
 
-hipError_t launch_pe_apply(int dtype, int pek, const void* in, void* out, long n_rows,
-                           int seq_len, int D, const PeSide& pe, int vec_ok, hipStream_t st);
+// Positional-encoding pre-pass (pe.hip) over one or two tensors of rows of
+// head_d D (position = row % seq_len; in == out allowed): both of the two
+// share the tables, layout and rotary width of their PeSide.
+struct PeTensor {
+    const void* in;
+    void* out;
+    long n_rows;
+    int seq_len;
+    PeSide pe;
+};
+hipError_t launch_pe_apply(int dtype, int pek, const PeTensor* t, int n, int D, int vec_ok,
+                           hipStream_t st);
 
 }  // namespace atn

@@ -1,0 +1,296 @@
+// Positional-encoding pre-pass (gfx950): out[row] = PE(in[row]) with position
+// row % seq_len, over one tensor (atn_pe_apply_ex) or two at once (Q and K of
+// the "separate" pipelines).
+//
+// Pure copy traffic, so bytes in flight and idle lanes decide.  k_pe_rows
+// numbers the 4-dim groups of all rows through and gives every thread U of
+// them, 256 apart, with the loads of all U issued before any arithmetic:
+// every lane works whatever head_d is (a workgroup per row, as k_pe_apply
+// below, uses 32 of 256 lanes at head_d 128).  fp32 (4,32,512,128) with the
+// caller's duplicated caches, Q and K (67 MB in, 67 MB out): two launches of
+// 41.7 us -> one of 30.9 us (1.6 -> 4.35 TB/s; a large copy reaches 4.7), and
+// the "separate" RoPE call at that shape 152 -> 102 us.
+#include <algorithm>
+
+#include "common.hpp"
+#include "launch.hpp"
+
+namespace atn {
+
+namespace {
+
+// x / d and x % d for x < 2^16 + d by a host-made multiplier (d < 2^15), or,
+// for d >= 2^15, by one compare (there x < 2 d)
+struct SmallDiv {
+    unsigned d, mul;  // mul = ceil(2^32 / d), 0: the compare form
+    __device__ __forceinline__ unsigned div(unsigned x) const {
+        return mul ? __umulhi(x, mul) : (x >= d ? 1u : 0u);
+    }
+};
+SmallDiv small_div(long d) {
+    SmallDiv s;
+    s.d = (unsigned)d;
+    // ceil(2^32 / d) times x, >> 32, is x / d while x d < 2^32; d = 1 has no
+    // 32-bit multiplier and is taken apart by the kernel
+    s.mul = d < (1 << 15) ? (unsigned)((((uint64_t)1 << 32) + d - 1) / d) : 0u;
+    return s;
+}
+
+struct PeSeg {
+    const void* in;
+    void* out;
+    long units;    // groups in all rows
+    int seq_len;
+    SmallDiv pos;  // by seq_len
+    PeSide pe;
+};
+
+struct PeRowsArgs {
+    PeSeg seg[2];
+    unsigned blocks0;  // workgroups of seg[0]
+    int D;
+    int upr;           // units per row
+    SmallDiv row;      // by upr
+};
+
+// A unit: 4 dims of a row (8 for rotate-half: a group below half the rotary
+// width and its partner group, so that the two are read once and an in-place
+// call reads both before it writes either).  Rotate-half rows hold rotary / 8
+// pair units, then (D - rotary) / 4 plain ones.
+template <typename T, int PEK, bool DUP, int U>
+__global__ __launch_bounds__(256) void k_pe_rows(PeRowsArgs a) {
+    const bool second = blockIdx.x >= a.blocks0;
+    const PeSeg& g = a.seg[second ? 1 : 0];
+    const long base = (long)(blockIdx.x - (second ? a.blocks0 : 0)) * (256 * U);
+    const long row0 = base / a.upr;
+    const unsigned c0 = (unsigned)(base - row0 * a.upr), p0 = (unsigned)(row0 % g.seq_len);
+    const T* in = static_cast<const T*>(g.in);
+    T* out = static_cast<T*>(g.out);
+    const int D = a.D, rot = g.pe.rotary, h = rot >> 1, ld = g.pe.ld;
+    constexpr bool kHalf = PEK == kPeRopeHalf;
+
+    float4 x[U], y[U], c[U], s[U];
+    const T* src[U];
+    int d[U];
+    bool on[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const unsigned i = threadIdx.x + 256u * u;
+        on[u] = base + i < g.units;
+        const unsigned k = on[u] ? c0 + i : c0;
+        const unsigned dr = a.upr == 1 ? k : a.row.div(k);
+        const unsigned unit = k - dr * (unsigned)a.upr;
+        const unsigned p = p0 + dr;
+        const int pos = g.seq_len == 1 ? 0 : (int)(p - g.pos.div(p) * g.pos.d);
+        src[u] = in + (size_t)(row0 + dr) * D;
+        bool enc = true;
+        if constexpr (kHalf) {
+            enc = (int)unit < (rot >> 3);
+            d[u] = enc ? (int)unit * 4 : rot + ((int)unit - (rot >> 3)) * 4;
+            x[u] = Elem<T>::ld4(src[u], d[u]);
+            y[u] = Elem<T>::ld4(src[u], enc ? d[u] + h : d[u]);
+        } else {
+            d[u] = (int)unit * 4;
+            enc = PEK == kPeSinusoidal || d[u] < rot;
+            x[u] = Elem<T>::ld4(src[u], d[u]);
+        }
+        // the angles (groups past the rotary width read a valid, unused one)
+        const int e = enc ? d[u] : 0;
+        if constexpr (PEK == kPeSinusoidal) {
+            if constexpr (DUP) {
+                const float4 sn = *reinterpret_cast<const float4*>(g.pe.a + (size_t)pos * ld + e);
+                const float4 cs = *reinterpret_cast<const float4*>(g.pe.b + (size_t)pos * ld + e);
+                c[u] = make_float4(sn.x, cs.y, sn.z, cs.w);
+            } else {
+                const size_t t = (size_t)pos * ld + (e >> 1);
+                const float2 sn = *reinterpret_cast<const float2*>(g.pe.a + t);
+                const float2 cs = *reinterpret_cast<const float2*>(g.pe.b + t);
+                c[u] = make_float4(sn.x, cs.x, sn.y, cs.y);
+            }
+        } else if constexpr (kHalf) {
+            if constexpr (DUP) {
+                const float* pc = g.pe.a + (size_t)pos * ld + 2 * e;
+                const float* ps = g.pe.b + (size_t)pos * ld + 2 * e;
+                const float4 ca = *reinterpret_cast<const float4*>(pc);
+                const float4 cb = *reinterpret_cast<const float4*>(pc + 4);
+                const float4 sa = *reinterpret_cast<const float4*>(ps);
+                const float4 sb = *reinterpret_cast<const float4*>(ps + 4);
+                c[u] = make_float4(ca.x, ca.z, cb.x, cb.z);
+                s[u] = make_float4(sa.x, sa.z, sb.x, sb.z);
+            } else {
+                c[u] = *reinterpret_cast<const float4*>(g.pe.a + (size_t)pos * ld + e);
+                s[u] = *reinterpret_cast<const float4*>(g.pe.b + (size_t)pos * ld + e);
+            }
+        } else {
+            if constexpr (DUP) {
+                const float4 cs = *reinterpret_cast<const float4*>(g.pe.a + (size_t)pos * ld + e);
+                const float4 sn = *reinterpret_cast<const float4*>(g.pe.b + (size_t)pos * ld + e);
+                c[u] = make_float4(cs.x, sn.x, cs.z, sn.z);
+            } else {
+                const size_t t = (size_t)pos * ld + (e >> 1);
+                const float2 cs = *reinterpret_cast<const float2*>(g.pe.a + t);
+                const float2 sn = *reinterpret_cast<const float2*>(g.pe.b + t);
+                c[u] = make_float4(cs.x, sn.x, cs.y, sn.y);
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (!on[u]) continue;
+        T* dst = out + (src[u] - in);
+        const float4 v = x[u];
+        if constexpr (PEK == kPeSinusoidal) {
+            Elem<T>::st4(dst, d[u], make_float4(v.x + c[u].x, v.y + c[u].y, v.z + c[u].z,
+                                                v.w + c[u].w));
+        } else if constexpr (kHalf) {
+            if (d[u] < h) {
+                const float4 w = y[u];
+                Elem<T>::st4(dst, d[u],
+                             make_float4(rot_first(v.x, w.x, c[u].x, s[u].x),
+                                         rot_first(v.y, w.y, c[u].y, s[u].y),
+                                         rot_first(v.z, w.z, c[u].z, s[u].z),
+                                         rot_first(v.w, w.w, c[u].w, s[u].w)));
+                Elem<T>::st4(dst, d[u] + h,
+                             make_float4(rot_second(v.x, w.x, c[u].x, s[u].x),
+                                         rot_second(v.y, w.y, c[u].y, s[u].y),
+                                         rot_second(v.z, w.z, c[u].z, s[u].z),
+                                         rot_second(v.w, w.w, c[u].w, s[u].w)));
+            } else {
+                Elem<T>::st4(dst, d[u], v);
+            }
+        } else {
+            Elem<T>::st4(dst, d[u],
+                         d[u] < rot ? make_float4(rot_first(v.x, v.y, c[u].x, c[u].y),
+                                                  rot_second(v.x, v.y, c[u].x, c[u].y),
+                                                  rot_first(v.z, v.w, c[u].z, c[u].w),
+                                                  rot_second(v.z, v.w, c[u].z, c[u].w))
+                                    : v);
+        }
+    }
+}
+
+// Any head_d, rotary width, alignment and table: a workgroup per row.
+template <typename T, int PEK>
+__global__ __launch_bounds__(256) void k_pe_apply(const T* __restrict__ in, T* __restrict__ out,
+                                                   long n_rows, int seq_len, int D, PeSide pe,
+                                                   int vec_ok) {
+    const bool vec = vec_ok != 0;
+    for (long row = blockIdx.x; row < n_rows; row += gridDim.x) {
+        const int pos = (int)(row % seq_len);
+        const T* xr = in + (size_t)row * D;
+        T* yr = out + (size_t)row * D;
+        for (int d = threadIdx.x * 4; d < D; d += 256 * 4) {
+            const float4 v = load_row4_pe<T, PEK>(xr, pos, d, D, pe, vec);
+            if (vec && d + 3 < D) {
+                Elem<T>::st4(yr, d, v);
+            } else {
+                const float vv[4] = {v.x, v.y, v.z, v.w};
+                for (int c = 0; c < 4 && d + c < D; ++c) Elem<T>::st(yr, d + c, vv[c]);
+            }
+        }
+    }
+}
+
+// Whether k_pe_rows takes this call: whole 4-dim groups whose angles are
+// whole vectors of the tables (16-byte aligned tables and rows where the
+// caller brings them), and unit counts that a grid holds.
+bool rows_ok(int pek, int D, const PeSide& pe, int vec_ok) {
+    if (!vec_ok || D % 4 != 0 || D >= (1 << 30)) return false;
+    const bool a16 = ((uintptr_t)pe.a % 16) == 0 && ((uintptr_t)pe.b % 16) == 0;
+    if (!a16) return false;
+    if (pek == kPeRopeInterleaved) return pe.rotary % 4 == 0 && pe.ld % (pe.dup ? 4 : 2) == 0;
+    if (pek == kPeRopeHalf) return pe.rotary % 8 == 0 && pe.ld % 4 == 0;
+    return pe.ld % (pe.dup ? 4 : 2) == 0;
+}
+
+template <typename T, int PEK, bool DUP>
+void run_rows(const PeRowsArgs& a, unsigned blocks, hipStream_t st) {
+    hipLaunchKernelGGL((k_pe_rows<T, PEK, DUP, PEK == kPeRopeHalf ? 2 : 4>), dim3(blocks),
+                       dim3(256), 0, st, a);
+}
+
+template <typename T>
+hipError_t pe_rows_t(int pek, const PeTensor* t, int n, int D, hipStream_t st) {
+    const int U = pek == kPeRopeHalf ? 2 : 4;
+    PeRowsArgs a{};
+    a.D = D;
+    a.upr = pek == kPeRopeHalf ? t[0].pe.rotary / 8 + (D - t[0].pe.rotary) / 4 : D / 4;
+    a.row = small_div(a.upr);
+    long blocks[2] = {0, 0};
+    for (int i = 0; i < n; ++i) {
+        PeSeg& g = a.seg[i];
+        g.in = t[i].in;
+        g.out = t[i].out;
+        g.units = t[i].n_rows * a.upr;
+        g.seq_len = t[i].seq_len;
+        g.pos = small_div(t[i].seq_len);
+        g.pe = t[i].pe;
+        blocks[i] = (g.units + 256 * U - 1) / (256 * U);
+    }
+    if (blocks[0] + blocks[1] > INT32_MAX / 2) return hipErrorInvalidConfiguration;
+    a.blocks0 = (unsigned)blocks[0];
+    const unsigned grid = (unsigned)(blocks[0] + blocks[1]);
+    const bool dup = t[0].pe.dup != 0;
+    switch (pek) {
+        case kPeRopeInterleaved:
+            dup ? run_rows<T, kPeRopeInterleaved, true>(a, grid, st)
+                : run_rows<T, kPeRopeInterleaved, false>(a, grid, st);
+            break;
+        case kPeRopeHalf:
+            dup ? run_rows<T, kPeRopeHalf, true>(a, grid, st)
+                : run_rows<T, kPeRopeHalf, false>(a, grid, st);
+            break;
+        case kPeSinusoidal:
+            dup ? run_rows<T, kPeSinusoidal, true>(a, grid, st)
+                : run_rows<T, kPeSinusoidal, false>(a, grid, st);
+            break;
+        default:
+            return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t pe_apply_t(int pek, const PeTensor& t, int D, int vec_ok, hipStream_t st) {
+    const dim3 grid((unsigned)std::min<long>(t.n_rows, 65536)), block(256);
+    const T* x = static_cast<const T*>(t.in);
+    T* y = static_cast<T*>(t.out);
+    switch (pek) {
+        case kPeRopeInterleaved:
+            hipLaunchKernelGGL((k_pe_apply<T, kPeRopeInterleaved>), grid, block, 0, st, x, y,
+                               t.n_rows, t.seq_len, D, t.pe, vec_ok);
+            break;
+        case kPeRopeHalf:
+            hipLaunchKernelGGL((k_pe_apply<T, kPeRopeHalf>), grid, block, 0, st, x, y, t.n_rows,
+                               t.seq_len, D, t.pe, vec_ok);
+            break;
+        case kPeSinusoidal:
+            hipLaunchKernelGGL((k_pe_apply<T, kPeSinusoidal>), grid, block, 0, st, x, y, t.n_rows,
+                               t.seq_len, D, t.pe, vec_ok);
+            break;
+        default:
+            return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_pe_apply(int dtype, int pek, const PeTensor* t, int n, int D, int vec_ok,
+                           hipStream_t st) {
+    bool rows = true;
+    for (int i = 0; i < n; ++i)
+        rows = rows && rows_ok(pek, D, t[i].pe, vec_ok) &&
+               t[i].n_rows <= ((long)1 << 40) / std::max(1, D / 4);
+    if (rows)
+        return dtype == kDtypeF32 ? pe_rows_t<float>(pek, t, n, D, st)
+                                  : pe_rows_t<uint16_t>(pek, t, n, D, st);
+    for (int i = 0; i < n; ++i) {
+        const hipError_t e = dtype == kDtypeF32 ? pe_apply_t<float>(pek, t[i], D, vec_ok, st)
+                                                : pe_apply_t<uint16_t>(pek, t[i], D, vec_ok, st);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+}  // namespace atn

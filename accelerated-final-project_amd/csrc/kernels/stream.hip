@@ -299,29 +299,6 @@ __global__ __launch_bounds__(256) void k_pv(const float* __restrict__ P, const T
     }
 }
 
-// Positional-encoding pre-pass: out[row] = PE(in[row]) with position
-// row % seq_len (the "separate"/"hybrid" pipelines' pre-pass).
-template <typename T, int PEK>
-__global__ __launch_bounds__(256) void k_pe_apply(const T* __restrict__ in, T* __restrict__ out,
-                                                   long n_rows, int seq_len, int D, PeSide pe,
-                                                   int vec_ok) {
-    const bool vec = vec_ok != 0;
-    for (long row = blockIdx.x; row < n_rows; row += gridDim.x) {
-        const int pos = (int)(row % seq_len);
-        const T* xr = in + (size_t)row * D;
-        T* yr = out + (size_t)row * D;
-        for (int d = threadIdx.x * 4; d < D; d += 256 * 4) {
-            const float4 v = load_row4_pe<T, PEK>(xr, pos, d, D, pe, vec);
-            if (vec && d + 3 < D) {
-                Elem<T>::st4(yr, d, v);
-            } else {
-                const float vv[4] = {v.x, v.y, v.z, v.w};
-                for (int c = 0; c < 4 && d + c < D; ++c) Elem<T>::st(yr, d + c, vv[c]);
-            }
-        }
-    }
-}
-
 template <typename T>
 hipError_t qk_partial_t(int pek, const void* Q, const void* K, float* S, int BH, int Lq, int Lk,
                         int D, int dchunk, int nsplit, const PeSide& pq, const PeSide& pk,
@@ -347,32 +324,6 @@ hipError_t qk_partial_t(int pek, const void* Q, const void* K, float* S, int BH,
         case kPeSinusoidal:
             hipLaunchKernelGGL((k_qk_partial<T, kPeSinusoidal>), grid, block, 0, st, q, k, S, BH,
                                Lq, Lk, D, dchunk, nsplit, tiles_q, tiles_k, pq, pk, vec_ok);
-            break;
-        default:
-            return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-template <typename T>
-hipError_t pe_apply_t(int pek, const void* in, void* out, long n_rows, int seq_len, int D,
-                      const PeSide& pe, int vec_ok, hipStream_t st) {
-    const long nwg = n_rows < 65536 ? n_rows : 65536;
-    const T* x = static_cast<const T*>(in);
-    T* y = static_cast<T*>(out);
-    const dim3 grid((unsigned)nwg), block(256);
-    switch (pek) {
-        case kPeRopeInterleaved:
-            hipLaunchKernelGGL((k_pe_apply<T, kPeRopeInterleaved>), grid, block, 0, st, x, y,
-                               n_rows, seq_len, D, pe, vec_ok);
-            break;
-        case kPeRopeHalf:
-            hipLaunchKernelGGL((k_pe_apply<T, kPeRopeHalf>), grid, block, 0, st, x, y, n_rows,
-                               seq_len, D, pe, vec_ok);
-            break;
-        case kPeSinusoidal:
-            hipLaunchKernelGGL((k_pe_apply<T, kPeSinusoidal>), grid, block, 0, st, x, y, n_rows,
-                               seq_len, D, pe, vec_ok);
             break;
         default:
             return hipErrorInvalidValue;
@@ -446,13 +397,6 @@ hipError_t launch_pv(int dtype, const float* P, const void* V, void* O, int BH, 
                            tiles_q, tiles_d, vec_ok);
     }
     return hipGetLastError();
-}
-
-hipError_t launch_pe_apply(int dtype, int pek, const void* in, void* out, long n_rows,
-                           int seq_len, int D, const PeSide& pe, int vec_ok, hipStream_t st) {
-    if (dtype == kDtypeF32)
-        return pe_apply_t<float>(pek, in, out, n_rows, seq_len, D, pe, vec_ok, st);
-    return pe_apply_t<uint16_t>(pek, in, out, n_rows, seq_len, D, pe, vec_ok, st);
 }
 
 }  // namespace atn
