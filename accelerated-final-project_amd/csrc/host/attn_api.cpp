@@ -100,6 +100,9 @@ struct PePlan {
     // second attempt after that kernel's exchange timed out)
     bool no_fused = false;
     bool no_flash = false;  // nor the flash kernel (atn_tuning.no_flash)
+    // the scratch holds no copies (encoded Q and K): the split-D pipeline that
+    // encodes inside its QK^T kernel
+    bool lean = false;
 };
 
 int check_pe(const atn_pe_desc* pe, int D, PePlan* plan) {
@@ -733,6 +736,94 @@ GemmPlan gemm_plan(int dtype, const Shape& s, const PePlan& plan) {
     return p;
 }
 
+// ---------------------------------------------------------------- tile plan
+// The split-D pipeline on pipelined 16-bit tiles (tile16.hip).  Workspace
+// after the sync region: partial scores [nsplit][BH][Lq][ldS] (fp32), P's two
+// 16-bit parts [BH][Lq][ldP] each, and, with a positional encoding, the
+// encoded Q and K (fp32): encoding them once in a pass of its own costs a
+// read and a write of each, encoding them inside the QK^T tiles a table read
+// and the arithmetic in every tile that shares a row (and the loads of a
+// stage wait for them: (1,4,512,512,2048) rotate-half 92.9 us inside, 10 + 23
+// us apart).
+struct TilePlan {
+    bool ok = false;
+    int tile_qk = 0, tile_pv = 0, nsplit = 0, dchunk = 0, ldS = 0, ldP = 0;
+    size_t ph_off = 0, pl_off = 0, q_off = 0, k_off = 0, bytes = 0;
+};
+
+// Estimated time (us) of a tile kernel: wgs workgroups of `stages` 32-deep
+// stages on 256 CUs.  Measured over 26 fp32 shapes, every tile and 8 D-chunk
+// counts (B H 2-32, sides 16-3144, D 264-6096): a CU spends 0.36 us per
+// stage of each 64 x 64 workgroup it holds (0.40 with one alone) and 1.12 us
+// per stage of a 128 x 128 one (0.8 us where few CUs run, 1.25 with one
+// workgroup on every CU), so 128 x 128 is the faster wherever its grid fills
+// the chip and 64 x 64 below.  Taking the least estimate loses 3 % on average
+// over the best measured choice of those shapes.
+double tile_us(int tile, int64_t wgs, int64_t stages) {
+    const double w = (double)wgs / 256.0;
+    const double per = tile == 64 ? std::max(0.40, 0.36 * w)
+                                  : std::max(0.80 + 0.45 * std::min(w, 1.0), 1.12 * w);
+    return per * (double)stages;
+}
+
+TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan) {
+    TilePlan p;
+    if (plan.lean || dtype != ATN_DTYPE_F32) return p;
+    p.ldS = (int)((s.Lk + 3) / 4 * 4);
+    p.ldP = (int)((s.Lk + 7) / 8 * 8);
+    const int64_t es = 4, lim = atn::kTileMaxBytes;
+    if ((int64_t)s.Lq * s.D * es >= lim || (int64_t)s.Lk * s.D * es >= lim ||
+        (int64_t)s.Lq * p.ldP * 2 >= lim)
+        return p;
+    auto tiles = [](int64_t a, int64_t b, int t) { return ((a + t - 1) / t) * ((b + t - 1) / t); };
+    // a forced tile (atn_tuning.splitd_tile): 128 only where both sides reach it
+    const int force = tune().splitd_tile;
+    auto allowed = [&](int t, int a, int b) {
+        if (force == 128) return a >= 128 && b >= 128 ? t == 128 : t == 64;
+        return force == 64 ? t == 64 : true;
+    };
+    // D-chunks: each more is one more partial of every score, written at
+    // 3.7 TB/s and read back at 6
+    double best = 0;
+    const double part = (double)s.BH * s.Lq * p.ldS * 4.0 * (1 / 3.7e6 + 1 / 6.0e6);
+    const int maxs = std::max(1, std::min(s.D / 64, 32));
+    for (int t : {128, 64}) {
+        if (!allowed(t, s.Lq, s.Lk)) continue;
+        const int64_t n = s.BH * tiles(s.Lq, s.Lk, t);
+        for (int want = 1; want <= maxs; ++want) {
+            const int dchunk = ((s.D + want - 1) / want + 31) / 32 * 32;
+            const int ns = (s.D + dchunk - 1) / dchunk;
+            if (ns != want) continue;
+            const double us = tile_us(t, n * ns, dchunk / 32) + part * ns;
+            if (p.nsplit == 0 || us < best) {
+                best = us;
+                p.tile_qk = t;
+                p.nsplit = ns;
+                p.dchunk = dchunk;
+            }
+        }
+    }
+    const int kst = (s.Lk + 31) / 32;
+    p.tile_pv = !allowed(64, s.Lq, s.D) ||
+                        (allowed(128, s.Lq, s.D) &&
+                         tile_us(128, s.BH * tiles(s.Lq, s.D, 128), kst) <
+                             tile_us(64, s.BH * tiles(s.Lq, s.D, 64), kst))
+                    ? 128
+                    : 64;
+    size_t off = kSyncBytes;
+    auto take = [&](size_t b) { size_t o = off; off += round256(b); return o; };
+    take((size_t)p.nsplit * s.BH * s.Lq * p.ldS * 4);
+    p.ph_off = take((size_t)s.BH * s.Lq * p.ldP * 2);
+    p.pl_off = take((size_t)s.BH * s.Lq * p.ldP * 2);
+    if (plan.pek != atn::kPeNone) {
+        if (plan.q.on) p.q_off = take((size_t)s.nq * 4);
+        if (plan.k.on) p.k_off = take((size_t)s.nk * 4);
+    }
+    p.bytes = off;
+    p.ok = true;
+    return p;
+}
+
 // ---------------------------------------------------------------- core
 // Scratch the library may use for one call before splitting it: the
 // caller's workspace size, the allocation-free array, or this cap for the
@@ -850,7 +941,8 @@ size_t path_need(int dtype, const Shape& s, const PePlan& plan, bool query_devic
                  int a16) {
     const FusedPlan fp = plan.no_fused ? FusedPlan{} : fused_plan(dtype, plan.pek, s, query_device);
     const GemmPlan gp = gemm_plan(dtype, s, plan);
-    const size_t split = kSyncBytes + stream_plan(s).bytes;
+    const TilePlan tp = tile_plan(dtype, s, plan);
+    const size_t split = tp.ok ? tp.bytes : kSyncBytes + stream_plan(s).bytes;
     if (vec < 0 || a16 < 0)
         return std::max({fp.ok ? fp.bytes : (size_t)0, gp.ok ? gp.bytes : (size_t)0, split,
                          flash_ok(dtype, s, plan) ? kSyncBytes + flash_split_bound(s)
@@ -925,12 +1017,15 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
     const bool use_flash = !use_fused && a16 && flash_ok(dtype, s, plan);
     const bool use_gemm = !use_fused && !use_flash && gp.ok && aligned(Q, 16) && aligned(K, 16) &&
                           aligned(V, 16) && aligned(out, 16);
+    const TilePlan tp = tile_plan(dtype, s, plan);
+    const bool use_tile = !use_fused && !use_flash && !use_gemm && tp.ok;
     const int fform = use_flash ? flash_form(s, dev) : 0;
     const FlashSplit fs = use_flash ? flash_split(s, flash_rows(fform, D)) : FlashSplit{};
     const size_t need =
         use_fused ? fd.bytes
                   : (use_flash ? kSyncBytes + fs.bytes
-                               : (use_gemm ? gp.bytes : kSyncBytes + sp.bytes));
+                               : (use_gemm ? gp.bytes
+                                           : (use_tile ? tp.bytes : kSyncBytes + sp.bytes)));
     void* ws = workspace;
     if (no_alloc) {
         if (need > atn::kNoAllocScratchBytes) return ATN_ERR_SCRATCH_LIMIT;
@@ -1021,6 +1116,29 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
                                   scale, plan.q, plan.k, fs.nsplit, fs.kchunk, scratch, stream));
         return ATN_OK;
     }
+    if (use_tile) {
+        char* w = static_cast<char*>(ws);
+        uint16_t* ph = reinterpret_cast<uint16_t*>(w + tp.ph_off);
+        uint16_t* pl = reinterpret_cast<uint16_t*>(w + tp.pl_off);
+        const void *qt = Q, *kt = K;
+        if (tp.q_off || tp.k_off) {
+            atn::PeTensor t[2];
+            int n = 0;
+            if (tp.q_off) t[n++] = {Q, w + tp.q_off, (long)(s.BH * Lq), Lq, plan.q};
+            if (tp.k_off) t[n++] = {K, w + tp.k_off, (long)(s.BH * Lk), Lk, plan.k};
+            ATN_HIP(atn::launch_pe_apply(dtype, plan.pek, t, n, D, vec_qk, stream));
+            if (tp.q_off) qt = w + tp.q_off;
+            if (tp.k_off) kt = w + tp.k_off;
+        }
+        atn::QkTileArgs qa{qt, kt, scratch, (int)s.BH, Lq, Lk, D, tp.dchunk, tp.nsplit, tp.ldS, 0, 0};
+        ATN_HIP(atn::launch_qk_tile(dtype, tp.tile_qk, qa, stream));
+        ATN_HIP(atn::launch_softmax_split(dtype, scratch, ph, pl, (long)(s.BH * Lq), Lk, tp.ldS,
+                                          tp.ldP, tp.nsplit, (size_t)s.BH * Lq * tp.ldS, scale,
+                                          stream));
+        atn::PvTileArgs pa{ph, pl, V, out, (int)s.BH, Lq, Lk, D, D, tp.ldP, aligned(out, 16), 0, 0};
+        ATN_HIP(atn::launch_pv_tile(dtype, tp.tile_pv, pa, stream));
+        return ATN_OK;
+    }
     float* S = scratch;
     float* P = sp.nsplit > 1 ? S + sp.s_elems : S;
     ATN_HIP(atn::launch_qk_partial(dtype, plan.pek, Q, K, S, (int)s.BH, Lq, Lk, D, sp.dchunk,
@@ -1088,7 +1206,14 @@ int attention_core(int dtype, const void* Q, const void* K, const void* V, void*
     if (path_need(dtype, s, plan, true, vec, a16) <= cap)
         return attention_run(dtype, Q, K, V, out, s, plan, dev, workspace, workspace_bytes,
                              stream, no_alloc);
-    const Chunking ch = plan_chunks(dtype, s, plan, cap, true, vec, a16);
+    Chunking ch = plan_chunks(dtype, s, plan, cap, true, vec, a16);
+    if (ch.heads == 0) {  // not even a row beside the copies of K: without them
+        plan.lean = true;
+        if (path_need(dtype, s, plan, true, vec, a16) <= cap)
+            return attention_run(dtype, Q, K, V, out, s, plan, dev, workspace, workspace_bytes,
+                                 stream, no_alloc);
+        ch = plan_chunks(dtype, s, plan, cap, true, vec, a16);
+    }
     if (ch.heads == 0) return no_alloc ? ATN_ERR_SCRATCH_LIMIT : ATN_ERR_WORKSPACE;
     const char* q8 = static_cast<const char*>(Q);
     const char* k8 = static_cast<const char*>(K);
@@ -1455,8 +1580,13 @@ size_t atn_attention_workspace_bytes(int dtype, int batch, int heads, int len_q,
     // exceeds the library's cap, of the chunks the call then runs in
     const size_t full = path_need(dtype, s, plan, false, -1, -1);
     if (full <= library_cap()) return full;
-    const Chunking ch = plan_chunks(dtype, s, plan, library_cap(), false, -1, -1);
-    return ch.heads > 0 ? ch.need : full;
+    Chunking ch = plan_chunks(dtype, s, plan, library_cap(), false, -1, -1);
+    if (ch.heads > 0) return ch.need;
+    plan.lean = true;
+    const size_t lean = path_need(dtype, s, plan, false, -1, -1);
+    if (lean <= library_cap()) return lean;
+    ch = plan_chunks(dtype, s, plan, library_cap(), false, -1, -1);
+    return ch.heads > 0 ? ch.need : lean;
 }
 
 int atn_pe_apply_ex(int dtype, const void* in, void* out, long n_rows, int seq_len, int head_d,

@@ -42,6 +42,37 @@ hipError_t launch_qk_s16(int pek, const float* Q, const float* K, float* S, int 
                          hipStream_t st);
 hipError_t launch_pv_s16(const float* P, const float* V, float* O, int BH, int Lq, int Lk, int D,
                          hipStream_t st);
+// The same three steps on pipelined 16-bit MFMA tiles (tile16.hip): output
+// tiles of tile x tile (64 or 128), rows of S ldS (a multiple of 4) and of
+// P's two 16-bit parts ldP (a multiple of 8) elements apart.  fp32 takes any
+// head_d and element-aligned bases, bf16 head_d % 8 == 0 and 16-byte aligned
+// Q, K and V; every head's tensors and P parts under kTileMaxBytes.
+constexpr long kTileMaxBytes = (1L << 31) - 65536;
+struct QkTileArgs {
+    const void* Q;
+    const void* K;
+    float* S;  // [nsplit][BH][Lq][ldS]
+    int BH, Lq, Lk, D, dchunk, nsplit, ldS;
+    int tiles_q, tiles_k;  // (filled by the launcher)
+};
+struct PvTileArgs {
+    const uint16_t* ph;  // 2^15 P, hi and lo parts [BH][Lq][ldP]
+    const uint16_t* pl;
+    const void* V;
+    void* O;
+    int BH, Lq, Lk;
+    int D;        // row stride of V and its valid dims
+    int ldO;      // row stride of O and its valid dims (<= D)
+    int ldP;
+    int o_align;  // O may be stored 4 elements at a time
+    int tiles_q, tiles_d;  // (filled by the launcher)
+};
+hipError_t launch_qk_tile(int dtype, int tile, QkTileArgs a, hipStream_t st);
+hipError_t launch_softmax_split(int dtype, float* S, uint16_t* ph, uint16_t* pl, long rows, int Lk,
+                                int ldS, int ldP, int nsplit, size_t split_stride, float scale,
+                                hipStream_t st);
+hipError_t launch_pv_tile(int dtype, int tile, PvTileArgs a, hipStream_t st);
+
 // Single-launch split-D kernel for len_q <= 64, len_k <= 128 (fused_small.hip):
 // row groups of MB query rows, D slices of dc dims; gather1 selects the
 // one-gather exchange (each thread polls (MB*NK/256) * nchunk <= 64 words)

@@ -1,0 +1,811 @@
+// The split-D pipeline on pipelined 16-bit MFMA tiles (gfx950): k_qk_tile
+// (partial scores over a D-chunk), k_softmax_split (exact row softmax, P as
+// two 16-bit parts) and k_pv_tile (O = P V).
+//
+// Operands (KIND): fp32 as hi + lo fp16 parts (split16.hpp, three exact
+// products per product), or raw bf16 (one exact product; P as hi + lo bf16
+// parts).  P leaves the softmax already split (times 2^15, so that small
+// probabilities keep their bits), so the PV kernel converts V alone.
+//
+// What bounds these kernels is VALU issue (the fp16 split: 4 instructions per
+// value pair) beside the MFMAs where the grid fills the chip, and the latency
+// of a stage where it leaves a CU one workgroup.  So a stage's 16-byte loads
+// go out one stage (128 x 128 tiles) or two (64 x 64: two register sets)
+// before their LDS writes, LDS is double-buffered with one barrier per stage,
+// and two stages run through one MFMA chain before their sum is added to the
+// tile's (half the additions of a sum per stage; the rounding against exact
+// 64-bit results stays below that of a sum per stage and of one chain: 4.3e-7
+// normwise at (1,4,512,512,2048), 6.7e-7 with one chain).  Register use stays
+// clear of spills: a spill's reload waits (vmcnt) for the loads in flight.  A
+// value beyond fp16's range is found in passing (one v_max3 per pair); its
+// workgroup then computes the tile again, every stage scaled by powers of two
+// from its largest finite magnitudes.
+//
+// Tiles of 128 x 128 (4 waves of 64 x 64) or 64 x 64 (4 waves of 32 x 32) on
+// 32 x 32 x 16 MFMA.  LDS rows of 32 elements (64 bytes) per part, their
+// 16-byte chunks permuted by tile_swz(row) so that fragment reads hit
+// distinct banks unpadded (SQ_LDS_BANK_CONFLICT 0): 64 KiB for both stages of
+// a 128 x 128 tile, two workgroups per CU.  Rows of S and P are padded to
+// whole vectors, so ragged key counts store and load 16 bytes as well.
+//
+// fp32 calls, before (stream16.hip's kernels) -> these: (1,4,512,512,2048)
+// 57.4 -> 48.8 us, (2,2,422,422,2360) 81 -> 49, (2,2,128,1415,1520) 98 -> 40,
+// (1,2,517,517,1272) 58 -> 31; at (1,4,1453,1453,1024) Q K^T runs at 215
+// TFLOP/s of fp32 work (650 of fp16 products).
+#include <algorithm>
+#include <type_traits>
+
+#include "common.hpp"
+#include "launch.hpp"
+#include "split16.hpp"
+
+namespace atn {
+
+namespace {
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef short bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+
+constexpr int kKindF32 = 0, kKindBF16 = 1;
+
+// Depth of a QK stage: 128 bytes of a row either way (fp32: 32 elements as
+// two parts; bf16: 64 elements, the two 32-deep halves in the parts' places).
+template <int KIND>
+struct Tile {
+    using T = typename std::conditional<KIND == kKindF32, float, uint16_t>::type;
+    static constexpr int ES = KIND == kKindF32 ? 4 : 2;
+    static constexpr int DEPTH = 128 / ES;
+    static constexpr int PER16 = 16 / ES;  // elements per 16-byte load
+};
+
+__device__ __forceinline__ int tile_swz(int row) { return ((row >> 1) & 3) ^ ((row >> 3) & 1); }
+// 16-bit element offset of chunk c (8 elements) of a 32-element LDS row
+__device__ __forceinline__ int tile_at(int row, int c) { return row * 32 + ((c ^ tile_swz(row)) << 3); }
+
+template <int KIND>
+__device__ __forceinline__ v16f mfma32(const uint4& a, const uint4& b, const v16f& c) {
+    if constexpr (KIND == kKindF32)
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
+                                                      __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a),
+                                                       __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ uint4 ld_buf_u4(__amdgpu_buffer_rsrc_t r, unsigned off) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ float4 as_f4(const uint4& u) {
+    return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z),
+                       __uint_as_float(u.w));
+}
+
+// 4 values times s as hi and lo fp16 parts
+__device__ __forceinline__ void split4(const uint4& u, float one, uint2& hi, uint2& lo) {
+    const float4 v = as_f4(u);
+    split2_f16_one(v.x, v.y, one, hi.x, lo.x);
+    split2_f16_one(v.z, v.w, one, hi.y, lo.y);
+}
+__device__ __forceinline__ void split4_scaled(const uint4& u, float s, uint2& hi, uint2& lo) {
+    const float4 v = as_f4(u);
+    split2_f16(v.x * s, v.y * s, hi.x, lo.x);
+    split2_f16(v.z * s, v.w * s, hi.y, lo.y);
+}
+
+// Consecutive tiles on one XCD: workgroup ids are dealt to the 8 XCDs in
+// turn, each XCD takes a contiguous share of the n tiles.
+__device__ __forceinline__ unsigned xcd_tile(unsigned id, unsigned n) {
+    const unsigned x = id & 7, i = id >> 3, per = n >> 3, rem = n & 7;
+    return x * per + min(x, rem) + i;
+}
+
+// Workgroup maximum of two per-thread values; every thread must call it.
+__device__ __forceinline__ void wg_max2(float& a, float& b, float* sh) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    a = wave_max(a);
+    b = wave_max(b);
+    if (lane == 0) {
+        sh[wave] = a;
+        sh[4 + wave] = b;
+    }
+    __syncthreads();
+    a = fmaxf(fmaxf(sh[0], sh[1]), fmaxf(sh[2], sh[3]));
+    b = fmaxf(fmaxf(sh[4], sh[5]), fmaxf(sh[6], sh[7]));
+}
+
+__device__ __forceinline__ float max4abs(float m, const uint4& u) {
+    const float4 v = as_f4(u);
+    return vmax3abs(vmax3abs(m, v.x, v.y), v.z, v.w);
+}
+
+// Whether any thread of the workgroup saw a value outside fp16's range
+__device__ __forceinline__ bool wg_over(float big, int* flag) {
+    const bool over = __ballot(!(big < kF16Range)) != 0;
+    if ((threadIdx.x & 63) == 0) flag[threadIdx.x >> 6] = over;
+    __syncthreads();
+    return (flag[0] | flag[1] | flag[2] | flag[3]) != 0;
+}
+
+// Partial scores S_split[bh][i][j] = sum over the chunk's dims of q_id k_jd
+// for one TL x TL tile.  Wave w computes S^T for its TL/2 keys x TL/2
+// queries: a lane holds 4 consecutive keys of one query per 16-byte store
+// (rows of S are ldS, a multiple of 4, apart).  RAG: head_d is no multiple of
+// 4 (fp32; rows then start at 4-byte boundaries and the last group of a row
+// is read element by element).
+template <int KIND, int TL, bool RAG>
+__global__ __launch_bounds__(256, 2) void k_qk_tile(QkTileArgs a) {
+    using G = Tile<KIND>;
+    constexpr int ROUNDS = TL / 32;     // loader rounds of 32 rows per operand
+    constexpr int NI = TL / 64;         // 32 x 32 MFMA tiles per wave and side
+    constexpr int PART = TL * 32;       // elements of one part of one operand
+    constexpr int AHEAD = TL == 64 ? 2 : 1;  // stages a load is issued before its LDS write
+    __shared__ __align__(16) uint16_t sq[2][2 * PART];  // [stage][part][row][32]
+    __shared__ __align__(16) uint16_t sk[2][2 * PART];
+    __shared__ float slot[8];
+    __shared__ int flag[4];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+    const int tk = (int)(t % a.tiles_k);
+    t /= a.tiles_k;
+    const int tq = (int)(t % a.tiles_q);
+    t /= a.tiles_q;
+    const int split = (int)(t % a.nsplit), bh = (int)(t / a.nsplit);
+    const int q0 = tq * TL, k0 = tk * TL;
+    const int dbeg = split * a.dchunk, dend = min(a.D, dbeg + a.dchunk);
+
+    const char* Qh = static_cast<const char*>(a.Q) + (size_t)bh * a.Lq * a.D * G::ES;
+    const char* Kh = static_cast<const char*>(a.K) + (size_t)bh * a.Lk * a.D * G::ES;
+    const int qbytes = a.Lq * a.D * G::ES, kbytes = a.Lk * a.D * G::ES;
+    // loader: row lrow + 32 i, the 16 bytes lc of the stage's 128
+    const int lrow = tid >> 3, lc = tid & 7;
+    unsigned qoff[ROUNDS], koff[ROUNDS];  // (a row outside the tensor stays past its end)
+#pragma unroll
+    for (int i = 0; i < ROUNDS; ++i) {
+        const int qi = q0 + lrow + 32 * i, kj = k0 + lrow + 32 * i;
+        qoff[i] = qi < a.Lq ? (unsigned)(qi * a.D * G::ES + lc * 16) : (unsigned)kBufOob;
+        koff[i] = kj < a.Lk ? (unsigned)(kj * a.D * G::ES + lc * 16) : (unsigned)kBufOob;
+    }
+    struct Regs {
+        uint4 q[ROUNDS], k[ROUNDS];
+    };
+    auto issue = [&](Regs& r, int d0) {
+        // the stage's depth goes into the (scalar) buffer base
+        const int d = d0 + lc * G::PER16, sh = min(d0, a.D) * G::ES;
+        const bool in = d < dend;
+        const __amdgpu_buffer_rsrc_t rq = buf_rsrc(Qh + sh, qbytes - sh);
+        const __amdgpu_buffer_rsrc_t rk = buf_rsrc(Kh + sh, kbytes - sh);
+        if (RAG && d0 + G::DEPTH > a.D) {
+            // the row's last stage, element by element
+#pragma unroll
+            for (int i = 0; i < ROUNDS; ++i) {
+                uint32_t w[8];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const bool ok = d + c < dend;
+                    w[c] = __builtin_amdgcn_raw_buffer_load_b32(
+                        rq, ok ? (int)qoff[i] + 4 * c : kBufOob, 0, 0);
+                    w[4 + c] = __builtin_amdgcn_raw_buffer_load_b32(
+                        rk, ok ? (int)koff[i] + 4 * c : kBufOob, 0, 0);
+                }
+                r.q[i] = make_uint4(w[0], w[1], w[2], w[3]);
+                r.k[i] = make_uint4(w[4], w[5], w[6], w[7]);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < ROUNDS; ++i) {
+                r.q[i] = ld_buf_u4(rq, in ? qoff[i] : (unsigned)kBufOob);
+                r.k[i] = ld_buf_u4(rk, in ? koff[i] : (unsigned)kBufOob);
+            }
+        }
+    };
+    float big = 0.f;
+    const float one = unit_opaque();
+    // LDS place of this thread's 16 bytes: fp32 half a chunk of both parts,
+    // bf16 a chunk of one part
+    auto place = [&](int i) {
+        const int row = lrow + 32 * i;
+        return KIND == kKindF32 ? tile_at(row, lc >> 1) + 4 * (lc & 1)
+                                : (lc >> 2) * PART + tile_at(row, lc & 3);
+    };
+    auto store = [&](const Regs& r, uint16_t* q, uint16_t* k) {
+#pragma unroll
+        for (int i = 0; i < ROUNDS; ++i) {
+            const int o = place(i);
+            if constexpr (KIND == kKindF32) {
+                uint2 hi, lo;
+                split4(r.q[i], one, hi, lo);
+                *reinterpret_cast<uint2*>(q + o) = hi;
+                *reinterpret_cast<uint2*>(q + PART + o) = lo;
+                split4(r.k[i], one, hi, lo);
+                *reinterpret_cast<uint2*>(k + o) = hi;
+                *reinterpret_cast<uint2*>(k + PART + o) = lo;
+                big = max4abs(max4abs(big, r.q[i]), r.k[i]);
+            } else {
+                *reinterpret_cast<uint4*>(q + o) = r.q[i];
+                *reinterpret_cast<uint4*>(k + o) = r.k[i];
+            }
+        }
+    };
+
+    const int wq = (wave & 1) * (TL / 2), wk = (wave >> 1) * (TL / 2);  // wave's queries, keys
+    const int fr = lane & 31, fc = lane >> 5;
+    v16f acc[NI][NI], sum[NI][NI];  // [key tile][query tile]
+    auto each = [&](auto f) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int j = 0; j < NI; ++j) f(acc[i][j], sum[i][j]);
+    };
+    auto zero = [&]() { each([](v16f&, v16f& y) { y = v16f{}; }); };
+    // the pair of stages just summed, into the tile's sum
+    auto flush = [&]() { each([](v16f& x, v16f& y) { y += x; }); };
+    auto compute = [&](const uint16_t* q, const uint16_t* k, auto fresh) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            uint4 ka[2][NI], qa[2][NI];
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    ka[p][i] = *reinterpret_cast<const uint4*>(
+                        k + p * PART + tile_at(wk + 32 * i + fr, 2 * ks + fc));
+                    qa[p][i] = *reinterpret_cast<const uint4*>(
+                        q + p * PART + tile_at(wq + 32 * i + fr, 2 * ks + fc));
+                }
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    v16f c = decltype(fresh)::value && ks == 0 ? v16f{} : acc[i][j];
+                    if constexpr (KIND == kKindF32) {
+                        c = mfma32<KIND>(ka[1][i], qa[0][j], c);
+                        c = mfma32<KIND>(ka[0][i], qa[1][j], c);
+                        c = mfma32<KIND>(ka[0][i], qa[0][j], c);
+                    } else {
+                        c = mfma32<KIND>(ka[0][i], qa[0][j], c);
+                        c = mfma32<KIND>(ka[1][i], qa[1][j], c);
+                    }
+                    acc[i][j] = c;
+                }
+        }
+    };
+
+    Regs r0, r1;
+    Regs& rb = AHEAD == 2 ? r1 : r0;
+    issue(r0, dbeg);
+    if (AHEAD == 2) issue(r1, dbeg + G::DEPTH);
+    zero();
+    store(r0, sq[0], sk[0]);
+    issue(r0, dbeg + AHEAD * G::DEPTH);
+    __syncthreads();
+    const int stages = (dend - dbeg + G::DEPTH - 1) / G::DEPTH;
+    for (int n = 0, d0 = dbeg; n < stages >> 1; ++n, d0 += 2 * G::DEPTH) {
+        compute(sq[0], sk[0], std::true_type{});
+        store(rb, sq[1], sk[1]);
+        issue(rb, d0 + (AHEAD + 1) * G::DEPTH);
+        __syncthreads();
+        compute(sq[1], sk[1], std::false_type{});
+        flush();
+        store(r0, sq[0], sk[0]);
+        issue(r0, d0 + (AHEAD + 2) * G::DEPTH);
+        __syncthreads();
+    }
+    if (stages & 1) {
+        compute(sq[0], sk[0], std::true_type{});
+        flush();
+    }
+    if constexpr (KIND == kKindF32) {
+        if (wg_over(big, flag)) {
+            zero();
+            for (int d0 = dbeg; d0 < dend; d0 += G::DEPTH) {
+                issue(r0, d0);
+                float mq = 0.f, mk = 0.f;
+#pragma unroll
+                for (int i = 0; i < ROUNDS; ++i) {
+                    mq = max_finite4(mq, as_f4(r0.q[i]));
+                    mk = max_finite4(mk, as_f4(r0.k[i]));
+                }
+                __syncthreads();  // the last stage's reads (and the slots') are done
+                wg_max2(mq, mk, slot);
+                const float s1 = pow2_scale(mq), s2 = pow2_scale(mk);
+#pragma unroll
+                for (int i = 0; i < ROUNDS; ++i) {
+                    const int o = place(i);
+                    uint2 hi, lo;
+                    split4_scaled(r0.q[i], s1, hi, lo);
+                    *reinterpret_cast<uint2*>(sq[0] + o) = hi;
+                    *reinterpret_cast<uint2*>(sq[0] + PART + o) = lo;
+                    split4_scaled(r0.k[i], s2, hi, lo);
+                    *reinterpret_cast<uint2*>(sk[0] + o) = hi;
+                    *reinterpret_cast<uint2*>(sk[0] + PART + o) = lo;
+                }
+                __syncthreads();
+                const float u = pow2_unit(mq) * pow2_unit(mk);
+                compute(sq[0], sk[0], std::true_type{});
+                each([u](v16f& x, v16f& y) { y += x * u; });
+            }
+        }
+    }
+
+    // register r of a tile: key 8 (r / 4) + 4 (lane / 32) + r % 4 of query lane % 32
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+        const int qi = q0 + wq + 32 * j + fr;
+        if (qi >= a.Lq) continue;
+        float* srow = a.S + (((size_t)split * a.BH + bh) * a.Lq + qi) * a.ldS;
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int kj = k0 + wk + 32 * i + 8 * b + 4 * fc;
+                const float4 v = make_float4(sum[i][j][4 * b], sum[i][j][4 * b + 1],
+                                             sum[i][j][4 * b + 2], sum[i][j][4 * b + 3]);
+                if (kj < a.ldS) *reinterpret_cast<float4*>(srow + kj) = v;
+            }
+    }
+}
+
+// 2^15 p as hi + lo parts: fp16 (fp32 calls) or bf16
+template <int KIND>
+__device__ __forceinline__ void split_p(float4 p, uint2& hi, uint2& lo) {
+    if constexpr (KIND == kKindF32) {
+        split2_f16(p.x, p.y, hi.x, lo.x);
+        split2_f16(p.z, p.w, hi.y, lo.y);
+    } else {
+        const float v[4] = {p.x, p.y, p.z, p.w};
+        uint32_t h[4], l[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            h[c] = f32_to_bf16_bits(v[c]);
+            l[c] = f32_to_bf16_bits(v[c] - bf16_bits_to_f32(h[c]));
+        }
+        hi = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+        lo = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+    }
+}
+
+// Row softmax of the summed partial scores, exact (max, exp, sum, divide),
+// written as two 16-bit parts of 2^15 P (rows ldP apart, zeros from Lk on).
+// TPR threads per row hold it in registers (thread t the 4 keys from
+// 4 (t + TPR u) on), so S is read once; every partial's load is independent.
+template <int KIND, int TPR, int NV>
+__global__ __launch_bounds__(256) void k_softmax_split(const float* __restrict__ S,
+                                                       uint16_t* __restrict__ ph,
+                                                       uint16_t* __restrict__ pl, long rows,
+                                                       int Lk, int ldS, int ldP, int nsplit,
+                                                       size_t split_stride, float scale) {
+    __shared__ float red[8];
+    const int tid = threadIdx.x, t = tid % TPR;
+    const long row = (long)blockIdx.x * (256 / TPR) + tid / TPR;
+    if (TPR == 64 && row >= rows) return;
+    const float* s = S + (size_t)row * ldS;
+    float4 v[NV];
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int c = 4 * (t + TPR * u);
+        v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (c < Lk) v[u] = *reinterpret_cast<const float4*>(s + c);
+    }
+#pragma unroll 4
+    for (int sp = 1; sp < nsplit; ++sp) {
+        const float* q = s + (size_t)sp * split_stride;
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+            const int c = 4 * (t + TPR * u);
+            if (c < Lk) {
+                const float4 w = *reinterpret_cast<const float4*>(q + c);
+                v[u].x += w.x;
+                v[u].y += w.y;
+                v[u].z += w.z;
+                v[u].w += w.w;
+            }
+        }
+    }
+    float m = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int c = 4 * (t + TPR * u);
+        v[u].x = c < Lk ? v[u].x * scale : -INFINITY;
+        v[u].y = c + 1 < Lk ? v[u].y * scale : -INFINITY;
+        v[u].z = c + 2 < Lk ? v[u].z * scale : -INFINITY;
+        v[u].w = c + 3 < Lk ? v[u].w * scale : -INFINITY;
+        m = fmaxf(m, fmaxf(fmaxf(v[u].x, v[u].y), fmaxf(v[u].z, v[u].w)));
+    }
+    m = wave_max(m);
+    if constexpr (TPR == 256) {
+        if ((tid & 63) == 0) red[tid >> 6] = m;
+        __syncthreads();
+        m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    }
+    float l = 0.f;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int c = 4 * (t + TPR * u);
+        v[u].x = c < Lk ? expf(v[u].x - m) : 0.f;
+        v[u].y = c + 1 < Lk ? expf(v[u].y - m) : 0.f;
+        v[u].z = c + 2 < Lk ? expf(v[u].z - m) : 0.f;
+        v[u].w = c + 3 < Lk ? expf(v[u].w - m) : 0.f;
+        l += (v[u].x + v[u].y) + (v[u].z + v[u].w);
+    }
+    l = wave_sum(l);
+    if constexpr (TPR == 256) {
+        if ((tid & 63) == 0) red[4 + (tid >> 6)] = l;
+        __syncthreads();
+        l = (red[4] + red[5]) + (red[6] + red[7]);
+    }
+    l *= 1.0f / 32768.0f;  // P written times 2^15 (exact)
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int c = 4 * (t + TPR * u);
+        if (c < ldP) {
+            uint2 hi, lo;
+            split_p<KIND>(make_float4(v[u].x / l, v[u].y / l, v[u].z / l, v[u].w / l), hi, lo);
+            *reinterpret_cast<uint2*>(ph + (size_t)row * ldP + c) = hi;
+            *reinterpret_cast<uint2*>(pl + (size_t)row * ldP + c) = lo;
+        }
+    }
+}
+
+// Rows longer than the registers hold: the sums go back to the first
+// partial's place, and the row is read three times.
+template <int KIND>
+__global__ __launch_bounds__(256) void k_softmax_long(float* S, uint16_t* __restrict__ ph,
+                                                      uint16_t* __restrict__ pl, long rows, int Lk,
+                                                      int ldS, int ldP, int nsplit,
+                                                      size_t split_stride, float scale) {
+    __shared__ float red[8];
+    const int tid = threadIdx.x;
+    for (long row = blockIdx.x; row < rows; row += gridDim.x) {
+        float* s = S + (size_t)row * ldS;
+        float m = -INFINITY;
+        for (int c = tid; c < Lk; c += 256) {
+            float x = s[c];
+            for (int sp = 1; sp < nsplit; ++sp) x += s[(size_t)sp * split_stride + c];
+            x *= scale;
+            s[c] = x;
+            m = fmaxf(m, x);
+        }
+        m = wave_max(m);
+        if ((tid & 63) == 0) red[tid >> 6] = m;
+        __syncthreads();
+        m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+        float l = 0.f;
+        for (int c = tid; c < Lk; c += 256) {
+            const float e = expf(s[c] - m);
+            s[c] = e;
+            l += e;
+        }
+        l = wave_sum(l);
+        if ((tid & 63) == 0) red[4 + (tid >> 6)] = l;
+        __syncthreads();
+        l = ((red[4] + red[5]) + (red[6] + red[7])) * (1.0f / 32768.0f);
+        for (int c = 4 * tid; c < ldP; c += 1024) {
+            float p[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) p[k] = c + k < Lk ? s[c + k] / l : 0.f;
+            uint2 hi, lo;
+            split_p<KIND>(make_float4(p[0], p[1], p[2], p[3]), hi, lo);
+            *reinterpret_cast<uint2*>(ph + (size_t)row * ldP + c) = hi;
+            *reinterpret_cast<uint2*>(pl + (size_t)row * ldP + c) = lo;
+        }
+        __syncthreads();  // red reused by the next row
+    }
+}
+
+// O[bh][i][d] = sum_j P_ij V_jd for one tile of TL queries x TL dims, 32 keys
+// a stage.  Wave w computes O^T for its TL/2 dims x TL/2 queries: a lane
+// holds 4 consecutive dims of one query.  P rows go to LDS as they are; V
+// stays [key][dim] there and reaches the MFMA by the transposing LDS read
+// (rows of TL + 32 elements: the four rows of a read on distinct banks).
+template <int KIND, int TL, bool RAG>
+__global__ __launch_bounds__(256, 2) void k_pv_tile(PvTileArgs a) {
+    using G = Tile<KIND>;
+    constexpr int NI = TL / 64, PART = TL * 32;
+    constexpr int AHEAD = TL == 64 ? 2 : 1;
+    constexpr int VSTR = TL + 32, VPARTS = KIND == kKindF32 ? 2 : 1, VPART = 32 * VSTR;
+    constexpr int VL = TL / G::PER16;             // V loader: lanes per row
+    constexpr int VROWS = 256 / VL, VROUNDS = 32 / VROWS > 0 ? 32 / VROWS : 1;
+    static_assert(VROWS <= 32, "a round of V rows within a stage");
+    __shared__ __align__(16) uint16_t sp[2][2 * PART];
+    __shared__ __align__(16) uint16_t sv[2][VPARTS * VPART];
+    __shared__ float slot[8];
+    __shared__ int flag[4];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+    const int tq = (int)(t % a.tiles_q);
+    t /= a.tiles_q;
+    const int td = (int)(t % a.tiles_d), bh = (int)(t / a.tiles_d);
+    const int q0 = tq * TL, d0 = td * TL;
+
+    const char* ph = reinterpret_cast<const char*>(a.ph + (size_t)bh * a.Lq * a.ldP);
+    const char* pl = reinterpret_cast<const char*>(a.pl + (size_t)bh * a.Lq * a.ldP);
+    const int pbytes = a.Lq * a.ldP * 2, vbytes = a.Lk * a.D * G::ES;
+    const char* Vh = static_cast<const char*>(a.V) + (size_t)bh * a.Lk * a.D * G::ES;
+    // P loader: row lrow + 64 i, chunk lc of both parts
+    constexpr int PR = TL / 64;
+    const int lrow = tid >> 2, lc = tid & 3;
+    unsigned poff[PR];
+#pragma unroll
+    for (int i = 0; i < PR; ++i) {
+        const int row = q0 + lrow + 64 * i;
+        poff[i] = row < a.Lq ? (unsigned)((row * a.ldP + 8 * lc) * 2) : (unsigned)kBufOob;
+    }
+    const int vrow = tid / VL, vcol = (tid % VL) * G::PER16;
+    unsigned voff[VROUNDS];  // (past the head's end from key Lk on)
+#pragma unroll
+    for (int i = 0; i < VROUNDS; ++i)
+        voff[i] = d0 + vcol < a.D
+                      ? (unsigned)(((vrow + VROWS * i) * a.D + d0 + vcol) * G::ES)
+                      : (unsigned)kBufOob;
+    struct Regs {
+        uint4 h[PR], l[PR], v[VROUNDS];
+    };
+    auto issue = [&](Regs& r, int kk) {
+const int psh = min(kk, a.ldP) * 2;
+        const __amdgpu_buffer_rsrc_t rh = buf_rsrc(ph + psh, pbytes - psh);
+        const __amdgpu_buffer_rsrc_t rl = buf_rsrc(pl + psh, pbytes - psh);
+#pragma unroll
+        for (int i = 0; i < PR; ++i) {
+            const unsigned o = kk + 8 * lc < a.ldP ? poff[i] : (unsigned)kBufOob;
+            r.h[i] = ld_buf_u4(rh, o);
+            r.l[i] = ld_buf_u4(rl, o);
+        }
+        const size_t vsh = (size_t)min(kk, a.Lk) * a.D * G::ES;
+        const __amdgpu_buffer_rsrc_t rv = buf_rsrc(Vh + vsh, vbytes - (int)vsh);
+#pragma unroll
+        for (int i = 0; i < VROUNDS; ++i) {
+            if (RAG && KIND == kKindF32 && d0 + TL > a.D) {
+                uint32_t w[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    w[c] = __builtin_amdgcn_raw_buffer_load_b32(
+                        rv, d0 + vcol + c < a.D ? (int)voff[i] + 4 * c : kBufOob, 0, 0);
+                r.v[i] = make_uint4(w[0], w[1], w[2], w[3]);
+            } else {
+                r.v[i] = ld_buf_u4(rv, voff[i]);
+            }
+        }
+    };
+    float big = 0.f;
+    const float one = unit_opaque();
+    auto store_p = [&](const Regs& r, uint16_t* p) {
+#pragma unroll
+        for (int i = 0; i < PR; ++i) {
+            const int o = tile_at(lrow + 64 * i, lc);
+            *reinterpret_cast<uint4*>(p + o) = r.h[i];
+            *reinterpret_cast<uint4*>(p + PART + o) = r.l[i];
+        }
+    };
+    auto store = [&](const Regs& r, uint16_t* p, uint16_t* v) {
+        store_p(r, p);
+#pragma unroll
+        for (int i = 0; i < VROUNDS; ++i) {
+            const int o = (vrow + VROWS * i) * VSTR + vcol;
+            if constexpr (KIND == kKindF32) {
+                uint2 hi, lo;
+                split4(r.v[i], one, hi, lo);
+                *reinterpret_cast<uint2*>(v + o) = hi;
+                *reinterpret_cast<uint2*>(v + VPART + o) = lo;
+                big = max4abs(big, r.v[i]);
+            } else {
+                *reinterpret_cast<uint4*>(v + o) = r.v[i];
+            }
+        }
+    };
+
+    const int wq = (wave & 1) * (TL / 2), wd = (wave >> 1) * (TL / 2);
+    const int fr = lane & 31, fc = lane >> 5;
+    // V^T fragment: dims 16 (lane / 16 % 2) + lane % 16, keys 8 (lane / 32) + 0..7
+    const int va = (8 * fc + ((lane & 15) >> 2)) * VSTR + wd + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    v16f acc[NI][NI], sum[NI][NI];  // [dim tile][query tile]
+    auto each = [&](auto f) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int j = 0; j < NI; ++j) f(acc[i][j], sum[i][j]);
+    };
+    auto zero = [&]() { each([](v16f&, v16f& y) { y = v16f{}; }); };
+    // the pair of stages just summed, into the tile's sum
+    auto flush = [&]() { each([](v16f& x, v16f& y) { y += x; }); };
+    auto compute = [&](const uint16_t* p, const uint16_t* v, auto fresh) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            uint4 pa[2][NI], vv[VPARTS][NI];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+#pragma unroll
+                for (int w = 0; w < VPARTS; ++w) {
+                    const uint16_t* at = v + w * VPART + va + 16 * ks * VSTR + 32 * i;
+                    const uint2 x = lds_tr16(at), y = lds_tr16(at + 4 * VSTR);
+                    vv[w][i] = make_uint4(x.x, x.y, y.x, y.y);
+                }
+#pragma unroll
+                for (int w = 0; w < 2; ++w)
+                    pa[w][i] = *reinterpret_cast<const uint4*>(
+                        p + w * PART + tile_at(wq + 32 * i + fr, 2 * ks + fc));
+            }
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    v16f c = decltype(fresh)::value && ks == 0 ? v16f{} : acc[i][j];
+                    if constexpr (KIND == kKindF32)
+                        c = mfma32<KIND>(vv[VPARTS - 1][i], pa[0][j], c);
+                    c = mfma32<KIND>(vv[0][i], pa[1][j], c);
+                    c = mfma32<KIND>(vv[0][i], pa[0][j], c);
+                    acc[i][j] = c;
+                }
+        }
+    };
+
+    Regs r0, r1;
+    Regs& rb = AHEAD == 2 ? r1 : r0;
+    issue(r0, 0);
+    if (AHEAD == 2) issue(r1, 32);
+    zero();
+    store(r0, sp[0], sv[0]);
+    issue(r0, 32 * AHEAD);
+    __syncthreads();
+    const int stages = (a.Lk + 31) / 32;
+    for (int n = 0, kk = 0; n < stages >> 1; ++n, kk += 64) {
+        compute(sp[0], sv[0], std::true_type{});
+        store(rb, sp[1], sv[1]);
+        issue(rb, kk + 32 * (AHEAD + 1));
+        __syncthreads();
+        compute(sp[1], sv[1], std::false_type{});
+        flush();
+        store(r0, sp[0], sv[0]);
+        issue(r0, kk + 32 * (AHEAD + 2));
+        __syncthreads();
+    }
+    if (stages & 1) {
+        compute(sp[0], sv[0], std::true_type{});
+        flush();
+    }
+    if constexpr (KIND == kKindF32) {
+        if (wg_over(big, flag)) {
+            zero();
+            for (int kk = 0; kk < a.Lk; kk += 32) {
+                issue(r0, kk);
+                float mv = 0.f, none = 0.f;
+#pragma unroll
+                for (int i = 0; i < VROUNDS; ++i) mv = max_finite4(mv, as_f4(r0.v[i]));
+                __syncthreads();
+                wg_max2(mv, none, slot);
+                const float s1 = pow2_scale(mv), u = pow2_unit(mv);
+                store_p(r0, sp[0]);
+#pragma unroll
+                for (int i = 0; i < VROUNDS; ++i) {
+                    const int o = (vrow + VROWS * i) * VSTR + vcol;
+                    uint2 hi, lo;
+                    split4_scaled(r0.v[i], s1, hi, lo);
+                    *reinterpret_cast<uint2*>(sv[0] + o) = hi;
+                    *reinterpret_cast<uint2*>(sv[0] + (VPARTS - 1) * VPART + o) = lo;
+                }
+                __syncthreads();
+                compute(sp[0], sv[0], std::true_type{});
+                each([u](v16f& x, v16f& y) { y += x * u; });
+            }
+        }
+    }
+
+    constexpr float kPInv = 1.0f / 32768.0f;  // P's 2^15
+    using T = typename G::T;
+    T* Oh = static_cast<T*>(a.O) + (size_t)bh * a.Lq * a.ldO;
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+        const int qi = q0 + wq + 32 * j + fr;
+        if (qi >= a.Lq) continue;
+        T* orow = Oh + (size_t)qi * a.ldO;
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int d = d0 + wd + 32 * i + 8 * b + 4 * fc;
+                float v[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    v[c] = sum[i][j][4 * b + c] * kPInv;
+                if (!RAG) {
+                    if (d < a.ldO) Elem<T>::st4(orow, d, make_float4(v[0], v[1], v[2], v[3]));
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (d + c < a.ldO) Elem<T>::st(orow, d + c, v[c]);
+                }
+            }
+    }
+}
+
+template <int KIND, int TL>
+void run_qk(const QkTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
+    if (KIND == kKindF32 && rag)
+        hipLaunchKernelGGL((k_qk_tile<KIND, TL, KIND == kKindF32>), dim3(grid), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((k_qk_tile<KIND, TL, false>), dim3(grid), dim3(256), 0, st, a);
+}
+
+template <int KIND, int TL>
+void run_pv(const PvTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
+    if (rag)
+        hipLaunchKernelGGL((k_pv_tile<KIND, TL, true>), dim3(grid), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((k_pv_tile<KIND, TL, false>), dim3(grid), dim3(256), 0, st, a);
+}
+
+template <int KIND>
+hipError_t softmax_k(float* S, uint16_t* ph, uint16_t* pl, long rows, int Lk, int ldS, int ldP,
+                     int nsplit, size_t stride, float scale, hipStream_t st) {
+    // a wave per row while that gives every CU several waves; a workgroup
+    // per row for few rows and for rows longer than a wave's registers hold
+    const bool wave = Lk <= 2048 && (rows >= 4096 || Lk <= 256);
+#define ATN_SOFTMAX(TPR, NV)                                                                    \
+    hipLaunchKernelGGL((k_softmax_split<KIND, TPR, NV>),                                        \
+                       dim3((unsigned)((rows + 256 / TPR - 1) / (256 / TPR))), dim3(256), 0, st, \
+                       S, ph, pl, rows, Lk, ldS, ldP, nsplit, stride, scale)
+    if (Lk > 8192 || rows > INT32_MAX)
+        hipLaunchKernelGGL(k_softmax_long<KIND>, dim3((unsigned)std::min<long>(rows, 65536)),
+                           dim3(256), 0, st, S, ph, pl, rows, Lk, ldS, ldP, nsplit, stride, scale);
+    else if (wave && Lk <= 256)
+        ATN_SOFTMAX(64, 1);
+    else if (wave && Lk <= 512)
+        ATN_SOFTMAX(64, 2);
+    else if (wave && Lk <= 1024)
+        ATN_SOFTMAX(64, 4);
+    else if (wave)
+        ATN_SOFTMAX(64, 8);
+    else if (Lk <= 1024)
+        ATN_SOFTMAX(256, 1);
+    else if (Lk <= 2048)
+        ATN_SOFTMAX(256, 2);
+    else if (Lk <= 4096)
+        ATN_SOFTMAX(256, 4);
+    else
+        ATN_SOFTMAX(256, 8);
+#undef ATN_SOFTMAX
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_qk_tile(int dtype, int tile, QkTileArgs a, hipStream_t st) {
+    a.tiles_q = (a.Lq + tile - 1) / tile;
+    a.tiles_k = (a.Lk + tile - 1) / tile;
+    const unsigned grid = (unsigned)((long)a.BH * a.tiles_q * a.tiles_k * a.nsplit);
+    const bool rag = a.D % 4 != 0;
+    if (dtype == kDtypeF32)
+        tile == 128 ? run_qk<kKindF32, 128>(a, rag, grid, st) : run_qk<kKindF32, 64>(a, rag, grid, st);
+    else
+        tile == 128 ? run_qk<kKindBF16, 128>(a, false, grid, st)
+                    : run_qk<kKindBF16, 64>(a, false, grid, st);
+    return hipGetLastError();
+}
+
+hipError_t launch_softmax_split(int dtype, float* S, uint16_t* ph, uint16_t* pl, long rows, int Lk,
+                                int ldS, int ldP, int nsplit, size_t split_stride, float scale,
+                                hipStream_t st) {
+    return dtype == kDtypeF32
+               ? softmax_k<kKindF32>(S, ph, pl, rows, Lk, ldS, ldP, nsplit, split_stride, scale, st)
+               : softmax_k<kKindBF16>(S, ph, pl, rows, Lk, ldS, ldP, nsplit, split_stride, scale, st);
+}
+
+hipError_t launch_pv_tile(int dtype, int tile, PvTileArgs a, hipStream_t st) {
+    a.tiles_q = (a.Lq + tile - 1) / tile;
+    a.tiles_d = (a.D + tile - 1) / tile;
+    const unsigned grid = (unsigned)((long)a.BH * a.tiles_q * a.tiles_d);
+    const bool rag = a.ldO % 4 != 0 || a.o_align == 0;
+    if (dtype == kDtypeF32)
+        tile == 128 ? run_pv<kKindF32, 128>(a, rag, grid, st) : run_pv<kKindF32, 64>(a, rag, grid, st);
+    else
+        tile == 128 ? run_pv<kKindBF16, 128>(a, rag, grid, st)
+                    : run_pv<kKindBF16, 64>(a, rag, grid, st);
+    return hipGetLastError();
+}
+
+}  // namespace atn
