@@ -103,6 +103,11 @@ struct PePlan {
     // the scratch holds no copies (encoded Q and K): the split-D pipeline that
     // encodes inside its QK^T kernel
     bool lean = false;
+    // bf16 calls that the GEMM path would take run on the split-D tiles
+    // (decided on the whole call, so that its chunks all do the same), and the
+    // whole call's D-chunk there
+    bool tiles = false;
+    int dchunk = 0;
 };
 
 int check_pe(const atn_pe_desc* pe, int D, PePlan* plan) {
@@ -748,33 +753,44 @@ GemmPlan gemm_plan(int dtype, const Shape& s, const PePlan& plan) {
 struct TilePlan {
     bool ok = false;
     int tile_qk = 0, tile_pv = 0, nsplit = 0, dchunk = 0, ldS = 0, ldP = 0;
-    size_t ph_off = 0, pl_off = 0, q_off = 0, k_off = 0, bytes = 0;
+    int Dp = 0;              // bf16: row stride of the copies (0: none)
+    bool qk_f32 = false;     // Q K^T on fp32 (encoded or fp32 inputs)
+    double us = 0;           // estimated time of the call
+    size_t ph_off = 0, pl_off = 0, q_off = 0, k_off = 0, v_off = 0, bytes = 0;
 };
 
-// Estimated time (us) of a tile kernel: wgs workgroups of `stages` 32-deep
-// stages on 256 CUs.  Measured over 26 fp32 shapes, every tile and 8 D-chunk
-// counts (B H 2-32, sides 16-3144, D 264-6096): a CU spends 0.36 us per
-// stage of each 64 x 64 workgroup it holds (0.40 with one alone) and 1.12 us
-// per stage of a 128 x 128 one (0.8 us where few CUs run, 1.25 with one
-// workgroup on every CU), so 128 x 128 is the faster wherever its grid fills
-// the chip and 64 x 64 below.  Taking the least estimate loses 3 % on average
-// over the best measured choice of those shapes.
-double tile_us(int tile, int64_t wgs, int64_t stages) {
+// Estimated time (us) of a tile kernel: wgs workgroups of `stages` stages on
+// 256 CUs.  Measured over 26 fp32 and 24 bf16 shapes with every tile and 8
+// D-chunk counts (B H 2-64, sides 16-4096, D 264-8192): a CU spends
+// `each` us per stage of every workgroup it holds, `alone` with one on few
+// CUs, `busy` more with one on each.  fp32 (and Q K^T of encoded bf16), 32
+// deep: 64 x 64 0.40 alone, 0.36 each; 128 x 128 0.80 (+ 0.45), 1.12 each.
+// bf16 Q K^T, 64 deep: 0.31, 0.31; 0.72 (+ 0.15), 0.85.  bf16 P V, 32 keys:
+// 0.36, 0.28; 0.65 (+ 0.10), 0.72.  So 128 x 128 is the faster wherever its
+// grid fills the chip, 64 x 64 below.
+enum { kTileF32 = 0, kTileQkBf16 = 1, kTilePvBf16 = 2 };
+double tile_us(int kind, int tile, int64_t wgs, int64_t stages) {
+    static const double c[3][2][3] = {{{0.40, 0.00, 0.36}, {0.80, 0.45, 1.12}},
+                                      {{0.31, 0.00, 0.31}, {0.72, 0.15, 0.85}},
+                                      {{0.36, 0.00, 0.28}, {0.65, 0.10, 0.72}}};
+    const double* k = c[kind][tile == 128];
     const double w = (double)wgs / 256.0;
-    const double per = tile == 64 ? std::max(0.40, 0.36 * w)
-                                  : std::max(0.80 + 0.45 * std::min(w, 1.0), 1.12 * w);
-    return per * (double)stages;
+    return std::max(k[0] + k[1] * std::min(w, 1.0), k[2] * w) * (double)stages;
 }
 
-TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan) {
+TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
     TilePlan p;
-    if (plan.lean || dtype != ATN_DTYPE_F32) return p;
+    if (plan.lean) return p;
     p.ldS = (int)((s.Lk + 3) / 4 * 4);
     p.ldP = (int)((s.Lk + 7) / 8 * 8);
-    const int64_t es = 4, lim = atn::kTileMaxBytes;
-    if ((int64_t)s.Lq * s.D * es >= lim || (int64_t)s.Lk * s.D * es >= lim ||
+    const bool bf = dtype == ATN_DTYPE_BF16;
+    p.qk_f32 = !bf || plan.pek != atn::kPeNone;
+    if (bf && (s.D % 8 != 0 || !a16)) p.Dp = (s.D + 7) / 8 * 8;
+    const int64_t es = p.qk_f32 ? 4 : 2, lim = atn::kTileMaxBytes, W = std::max(s.D, p.Dp);
+    if ((int64_t)s.Lq * W * es >= lim || (int64_t)s.Lk * W * es >= lim ||
         (int64_t)s.Lq * p.ldP * 2 >= lim)
         return p;
+    const int depth = p.qk_f32 ? 32 : 64;  // of a Q K^T stage
     auto tiles = [](int64_t a, int64_t b, int t) { return ((a + t - 1) / t) * ((b + t - 1) / t); };
     // a forced tile (atn_tuning.splitd_tile): 128 only where both sides reach it
     const int force = tune().splitd_tile;
@@ -783,18 +799,20 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan) {
         return force == 64 ? t == 64 : true;
     };
     // D-chunks: each more is one more partial of every score, written at
-    // 3.7 TB/s and read back at 6
+    // 3.7 TB/s and read back at 6.  A chunked call keeps the whole call's.
     double best = 0;
+    const int kq = p.qk_f32 ? kTileF32 : kTileQkBf16, kv = bf ? kTilePvBf16 : kTileF32;
     const double part = (double)s.BH * s.Lq * p.ldS * 4.0 * (1 / 3.7e6 + 1 / 6.0e6);
     const int maxs = std::max(1, std::min(s.D / 64, 32));
     for (int t : {128, 64}) {
         if (!allowed(t, s.Lq, s.Lk)) continue;
         const int64_t n = s.BH * tiles(s.Lq, s.Lk, t);
-        for (int want = 1; want <= maxs; ++want) {
-            const int dchunk = ((s.D + want - 1) / want + 31) / 32 * 32;
+        const int fixed = plan.dchunk > 0 ? (s.D + plan.dchunk - 1) / plan.dchunk : 0;
+        for (int want = fixed ? fixed : 1; want <= (fixed ? fixed : maxs); ++want) {
+            const int dchunk = fixed ? plan.dchunk : ((s.D + want - 1) / want + 31) / 32 * 32;
             const int ns = (s.D + dchunk - 1) / dchunk;
             if (ns != want) continue;
-            const double us = tile_us(t, n * ns, dchunk / 32) + part * ns;
+            const double us = tile_us(kq, t, n * ns, (dchunk + depth - 1) / depth) + part * ns;
             if (p.nsplit == 0 || us < best) {
                 best = us;
                 p.tile_qk = t;
@@ -804,24 +822,56 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan) {
         }
     }
     const int kst = (s.Lk + 31) / 32;
-    p.tile_pv = !allowed(64, s.Lq, s.D) ||
-                        (allowed(128, s.Lq, s.D) &&
-                         tile_us(128, s.BH * tiles(s.Lq, s.D, 128), kst) <
-                             tile_us(64, s.BH * tiles(s.Lq, s.D, 64), kst))
-                    ? 128
-                    : 64;
+    const double pv64 = tile_us(kv, 64, s.BH * tiles(s.Lq, s.D, 64), kst),
+                 pv128 = tile_us(kv, 128, s.BH * tiles(s.Lq, s.D, 128), kst);
+    p.tile_pv = !allowed(64, s.Lq, s.D) || (allowed(128, s.Lq, s.D) && pv128 < pv64) ? 128 : 64;
+    // + launches, the softmax's own traffic, the encoding pass (2 bytes read
+    // and 4 written per element of Q and K; 4 and 4 for fp32)
+    p.us = best + std::min(pv64, pv128) + 9.0 + (double)s.BH * s.Lq * p.ldS * 4.0 / 5.5e6;
+    if (plan.pek != atn::kPeNone) p.us += 3.0 + (double)(s.nq + s.nk) * (bf ? 6.0 : 8.0) / 4.5e6;
     size_t off = kSyncBytes;
     auto take = [&](size_t b) { size_t o = off; off += round256(b); return o; };
     take((size_t)p.nsplit * s.BH * s.Lq * p.ldS * 4);
     p.ph_off = take((size_t)s.BH * s.Lq * p.ldP * 2);
     p.pl_off = take((size_t)s.BH * s.Lq * p.ldP * 2);
     if (plan.pek != atn::kPeNone) {
-        if (plan.q.on) p.q_off = take((size_t)s.nq * 4);
-        if (plan.k.on) p.k_off = take((size_t)s.nk * 4);
+        if (plan.q.on || bf) p.q_off = take((size_t)s.nq * 4);
+        if (plan.k.on || bf) p.k_off = take((size_t)s.nk * 4);
+    } else if (p.Dp) {
+        p.q_off = take((size_t)s.BH * s.Lq * p.Dp * 2);
+        p.k_off = take((size_t)s.BH * s.Lk * p.Dp * 2);
     }
+    if (p.Dp) p.v_off = take((size_t)s.BH * s.Lk * p.Dp * 2);
     p.bytes = off;
     p.ok = true;
     return p;
+}
+
+// Whether a bf16 call of the GEMM path runs on the split-D tiles instead.  The
+// GEMMs' 256 x 256 tiles leave most CUs idle on a small grid, and each
+// workgroup then walks all of D (or all keys) alone: about 1.4 us per 64-deep
+// step of Q K^T, 2.2 per 64 keys of P V and 15 us besides, per round of 256
+// workgroups (wall times of 29 shapes; K's encoding inside the GEMM makes a
+// step 2.2 us, an encoding pass costs its traffic).  The tiles cut D as well
+// and win there: (1,2,68,68,624) 37.3 -> 11.6 us, (2,4,82,82,2392) 72.5 ->
+// 15.8, (1,4,512,512,2048) 62.5 -> 31, (1,8,64,4096,2048) 195 -> 91; from
+// about 128 GEMM tiles on the GEMMs lead ((4,8,444,444,1008) 66 against 93
+// us, (4,16,508,508,1888) 201 against 315).
+void choose_tiles(int dtype, const Shape& s, PePlan& plan) {
+    const TilePlan tp = tile_plan(dtype, s, plan, true);
+    if (!tp.ok) return;
+    plan.dchunk = tp.dchunk;
+    if (dtype != ATN_DTYPE_BF16 || plan.no_flash || tune().gemm_fused_k != 0) return;
+    const GemmPlan gp = gemm_plan(dtype, s, plan);
+    if (!gp.ok) return;
+    auto wgs = [&](int a, int b) {
+        return (double)(s.BH * ((a + 255) / 256) * ((b + 255) / 256)) / 256.0;
+    };
+    double us = 15.0 + std::ceil(wgs(s.Lq, s.Lk)) * ((s.D + 63) / 64) * (gp.benc ? 2.2 : 1.4) +
+                std::ceil(wgs(s.Lq, s.D)) * ((s.Lk + 63) / 64) * 2.2;
+    if (gp.encoded) us += 4.0 + (double)s.nq * 4.0 / 4.5e6;
+    if (gp.encoded && gp.benc == 0) us += 4.0 + (double)s.nk * 4.0 / 4.5e6;
+    plan.tiles = tp.us < 0.95 * us;
 }
 
 // ---------------------------------------------------------------- core
@@ -941,16 +991,16 @@ size_t path_need(int dtype, const Shape& s, const PePlan& plan, bool query_devic
                  int a16) {
     const FusedPlan fp = plan.no_fused ? FusedPlan{} : fused_plan(dtype, plan.pek, s, query_device);
     const GemmPlan gp = gemm_plan(dtype, s, plan);
-    const TilePlan tp = tile_plan(dtype, s, plan);
+    if (fp.ok && vec > 0) return fp.bytes;
+    if (a16 > 0 && vec >= 0 && flash_ok(dtype, s, plan))  // the flash kernel: only its key splits' parts
+        return kSyncBytes + flash_split_bound(s);
+    const TilePlan tp = tile_plan(dtype, s, plan, a16 > 0);
     const size_t split = tp.ok ? tp.bytes : kSyncBytes + stream_plan(s).bytes;
     if (vec < 0 || a16 < 0)
         return std::max({fp.ok ? fp.bytes : (size_t)0, gp.ok ? gp.bytes : (size_t)0, split,
                          flash_ok(dtype, s, plan) ? kSyncBytes + flash_split_bound(s)
                                                   : (size_t)0});
-    if (fp.ok && vec) return fp.bytes;
-    if (a16 && flash_ok(dtype, s, plan))  // the flash kernel: only its key splits' parts
-        return kSyncBytes + flash_split_bound(s);
-    if (gp.ok && a16) return gp.bytes;
+    if (gp.ok && a16 && !(plan.tiles && tp.ok)) return gp.bytes;
     return split;
 }
 
@@ -1015,10 +1065,11 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
     const bool use_fused = fd.ok && vec_qk && vec_vo;
     const bool a16 = aligned(Q, 16) && aligned(K, 16) && aligned(V, 16) && aligned(out, 16);
     const bool use_flash = !use_fused && a16 && flash_ok(dtype, s, plan);
-    const bool use_gemm = !use_fused && !use_flash && gp.ok && aligned(Q, 16) && aligned(K, 16) &&
-                          aligned(V, 16) && aligned(out, 16);
-    const TilePlan tp = tile_plan(dtype, s, plan);
-    const bool use_tile = !use_fused && !use_flash && !use_gemm && tp.ok;
+    const bool use_gemm =
+        !use_fused && !use_flash && gp.ok && a16 && !(plan.tiles && !plan.lean);
+    const TilePlan tp = use_fused || use_flash || use_gemm ? TilePlan{}
+                                                           : tile_plan(dtype, s, plan, a16);
+    const bool use_tile = tp.ok;
     const int fform = use_flash ? flash_form(s, dev) : 0;
     const FlashSplit fs = use_flash ? flash_split(s, flash_rows(fform, D)) : FlashSplit{};
     const size_t need =
@@ -1120,22 +1171,31 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
         char* w = static_cast<char*>(ws);
         uint16_t* ph = reinterpret_cast<uint16_t*>(w + tp.ph_off);
         uint16_t* pl = reinterpret_cast<uint16_t*>(w + tp.pl_off);
-        const void *qt = Q, *kt = K;
-        if (tp.q_off || tp.k_off) {
+        const void *qt = tp.q_off ? w + tp.q_off : Q, *kt = tp.k_off ? w + tp.k_off : K;
+        const void* vt = tp.v_off ? w + tp.v_off : V;
+        const long nq = (long)(s.BH * Lq), nk = (long)(s.BH * Lk);
+        int Dqk = D;
+        if (plan.pek != atn::kPeNone) {
+            // (a side without the encoding is only widened; its PeSide is off)
             atn::PeTensor t[2];
             int n = 0;
-            if (tp.q_off) t[n++] = {Q, w + tp.q_off, (long)(s.BH * Lq), Lq, plan.q};
-            if (tp.k_off) t[n++] = {K, w + tp.k_off, (long)(s.BH * Lk), Lk, plan.k};
-            ATN_HIP(atn::launch_pe_apply(dtype, plan.pek, t, n, D, vec_qk, stream));
-            if (tp.q_off) qt = w + tp.q_off;
-            if (tp.k_off) kt = w + tp.k_off;
+            if (tp.q_off) t[n++] = {Q, w + tp.q_off, nq, Lq, plan.q};
+            if (tp.k_off) t[n++] = {K, w + tp.k_off, nk, Lk, plan.k};
+            if (n > 0)
+                ATN_HIP(atn::launch_pe_apply(dtype, ATN_DTYPE_F32, plan.pek, t, n, D, vec_qk, stream));
+        } else if (tp.Dp) {
+            Dqk = tp.Dp;
         }
-        atn::QkTileArgs qa{qt, kt, scratch, (int)s.BH, Lq, Lk, D, tp.dchunk, tp.nsplit, tp.ldS, 0, 0};
-        ATN_HIP(atn::launch_qk_tile(dtype, tp.tile_qk, qa, stream));
-        ATN_HIP(atn::launch_softmax_split(dtype, scratch, ph, pl, (long)(s.BH * Lq), Lk, tp.ldS,
-                                          tp.ldP, tp.nsplit, (size_t)s.BH * Lq * tp.ldS, scale,
-                                          stream));
-        atn::PvTileArgs pa{ph, pl, V, out, (int)s.BH, Lq, Lk, D, D, tp.ldP, aligned(out, 16), 0, 0};
+        if (tp.Dp) {
+            atn::PadTensor t[3] = {{V, w + tp.v_off, nk}, {Q, w + tp.q_off, nq}, {K, w + tp.k_off, nk}};
+            ATN_HIP(atn::launch_pad_rows(t, plan.pek == atn::kPeNone ? 3 : 1, D, tp.Dp, stream));
+        }
+        const atn::QkTileArgs qa{qt, kt, scratch, (int)s.BH, Lq, Lk, Dqk, tp.dchunk, tp.nsplit, tp.ldS, 0, 0};
+        ATN_HIP(atn::launch_qk_tile(tp.qk_f32 ? ATN_DTYPE_F32 : ATN_DTYPE_BF16, tp.tile_qk, qa, stream));
+        ATN_HIP(atn::launch_softmax_split(dtype, scratch, ph, pl, nq, Lk, tp.ldS, tp.ldP, tp.nsplit,
+                                          (size_t)s.BH * Lq * tp.ldS, scale, stream));
+        const atn::PvTileArgs pa{ph, pl, vt, out, (int)s.BH, Lq, Lk, tp.Dp ? tp.Dp : D, D, tp.ldP,
+                                 aligned(out, dtype == ATN_DTYPE_F32 ? 16 : 8), 0, 0};
         ATN_HIP(atn::launch_pv_tile(dtype, tp.tile_pv, pa, stream));
         return ATN_OK;
     }
@@ -1190,6 +1250,10 @@ int attention_core(int dtype, const void* Q, const void* K, const void* V, void*
     if (st != ATN_OK) return st;
     st = bind_tables(pe, plan, D, Lq > Lk ? Lq : Lk, stream, no_alloc);
     if (st != ATN_OK) return st;
+
+    if (!flash_ok(dtype, s, plan) &&
+        (plan.no_fused || !fused_plan(dtype, plan.pek, s, true).ok))
+        choose_tiles(dtype, s, plan);
 
     const size_t cap = no_alloc ? atn::kNoAllocScratchBytes
                                 : (workspace != nullptr ? workspace_bytes : library_cap());
@@ -1280,7 +1344,7 @@ int pe_apply_core(int dtype, const PeIo* io, int n, int D, const atn_pe_desc* pe
     atn::PeTensor t[2];
     for (int i = 0; i < n; ++i)
         t[i] = atn::PeTensor{io[i].in, io[i].out, io[i].n_rows, io[i].seq_len, plan.q};
-    ATN_HIP(atn::launch_pe_apply(dtype, plan.pek, t, n, D, vec, stream));
+    ATN_HIP(atn::launch_pe_apply(dtype, dtype, plan.pek, t, n, D, vec, stream));
     return ATN_OK;
 }
 
@@ -1576,6 +1640,7 @@ size_t atn_attention_workspace_bytes(int dtype, int batch, int heads, int len_q,
     if (check_shape(batch, heads, len_q, len_k, head_d, &s) != ATN_OK) return 0;
     PePlan plan;
     if (check_pe(pe, head_d, &plan) != ATN_OK) return 0;
+    choose_tiles(dtype, s, plan);
     // the largest workspace of every plan the call could take, or, when that
     // exceeds the library's cap, of the chunks the call then runs in
     const size_t full = path_need(dtype, s, plan, false, -1, -1);

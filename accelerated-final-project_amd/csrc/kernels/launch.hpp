@@ -141,7 +141,8 @@ hipError_t noalloc_scratch(int dev, size_t sync_bytes, hipStream_t st, void** pt
 
 // Positional-encoding pre-pass (pe.hip) over one or two tensors of rows of
 // head_d D (position = row % seq_len; in == out allowed): both of the two
-// share the tables, layout and rotary width of their PeSide.
+// share the tables, layout and rotary width of their PeSide.  out_dtype: the
+// input's, or fp32 for bf16 inputs.
 struct PeTensor {
     const void* in;
     void* out;
@@ -149,7 +150,15 @@ struct PeTensor {
     int seq_len;
     PeSide pe;
 };
-hipError_t launch_pe_apply(int dtype, int pek, const PeTensor* t, int n, int D, int vec_ok,
-                           hipStream_t st);
+hipError_t launch_pe_apply(int dtype, int out_dtype, int pek, const PeTensor* t, int n, int D,
+                           int vec_ok, hipStream_t st);
+// bf16 rows of D copied into 16-byte aligned rows of Dp (D rounded up to a
+// multiple of 8), zeros past D: up to three tensors, any element alignment.
+struct PadTensor {
+    const void* in;
+    void* out;
+    long n_rows;
+};
+hipError_t launch_pad_rows(const PadTensor* t, int n, int D, int Dp, hipStream_t st);
 
 }  // namespace atn

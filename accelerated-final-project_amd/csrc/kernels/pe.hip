@@ -57,7 +57,7 @@ struct PeRowsArgs {
 // width and its partner group, so that the two are read once and an in-place
 // call reads both before it writes either).  Rotate-half rows hold rotary / 8
 // pair units, then (D - rotary) / 4 plain ones.
-template <typename T, int PEK, bool DUP, int U>
+template <typename T, typename TO, int PEK, bool DUP, int U>
 __global__ __launch_bounds__(256) void k_pe_rows(PeRowsArgs a) {
     const bool second = blockIdx.x >= a.blocks0;
     const PeSeg& g = a.seg[second ? 1 : 0];
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256) void k_pe_rows(PeRowsArgs a) {
     const long row0 = base / a.upr;
     const unsigned c0 = (unsigned)(base - row0 * a.upr), p0 = (unsigned)(row0 % g.seq_len);
     const T* in = static_cast<const T*>(g.in);
-    T* out = static_cast<T*>(g.out);
+    TO* out = static_cast<TO*>(g.out);
     const int D = a.D, rot = g.pe.rotary, h = rot >> 1, ld = g.pe.ld;
     constexpr bool kHalf = PEK == kPeRopeHalf;
 
@@ -137,29 +137,32 @@ __global__ __launch_bounds__(256) void k_pe_rows(PeRowsArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         if (!on[u]) continue;
-        T* dst = out + (src[u] - in);
+        TO* dst = out + (src[u] - in);
         const float4 v = x[u];
-        if constexpr (PEK == kPeSinusoidal) {
-            Elem<T>::st4(dst, d[u], make_float4(v.x + c[u].x, v.y + c[u].y, v.z + c[u].z,
+        if (!g.pe.on) {  // widened or copied only
+            Elem<TO>::st4(dst, d[u], v);
+            if (kHalf && d[u] < h) Elem<TO>::st4(dst, d[u] + h, y[u]);
+        } else if constexpr (PEK == kPeSinusoidal) {
+            Elem<TO>::st4(dst, d[u], make_float4(v.x + c[u].x, v.y + c[u].y, v.z + c[u].z,
                                                 v.w + c[u].w));
         } else if constexpr (kHalf) {
             if (d[u] < h) {
                 const float4 w = y[u];
-                Elem<T>::st4(dst, d[u],
+                Elem<TO>::st4(dst, d[u],
                              make_float4(rot_first(v.x, w.x, c[u].x, s[u].x),
                                          rot_first(v.y, w.y, c[u].y, s[u].y),
                                          rot_first(v.z, w.z, c[u].z, s[u].z),
                                          rot_first(v.w, w.w, c[u].w, s[u].w)));
-                Elem<T>::st4(dst, d[u] + h,
+                Elem<TO>::st4(dst, d[u] + h,
                              make_float4(rot_second(v.x, w.x, c[u].x, s[u].x),
                                          rot_second(v.y, w.y, c[u].y, s[u].y),
                                          rot_second(v.z, w.z, c[u].z, s[u].z),
                                          rot_second(v.w, w.w, c[u].w, s[u].w)));
             } else {
-                Elem<T>::st4(dst, d[u], v);
+                Elem<TO>::st4(dst, d[u], v);
             }
         } else {
-            Elem<T>::st4(dst, d[u],
+            Elem<TO>::st4(dst, d[u],
                          d[u] < rot ? make_float4(rot_first(v.x, v.y, c[u].x, c[u].y),
                                                   rot_second(v.x, v.y, c[u].x, c[u].y),
                                                   rot_first(v.z, v.w, c[u].z, c[u].w),
@@ -170,22 +173,22 @@ __global__ __launch_bounds__(256) void k_pe_rows(PeRowsArgs a) {
 }
 
 // Any head_d, rotary width, alignment and table: a workgroup per row.
-template <typename T, int PEK>
-__global__ __launch_bounds__(256) void k_pe_apply(const T* __restrict__ in, T* __restrict__ out,
+template <typename T, typename TO, int PEK>
+__global__ __launch_bounds__(256) void k_pe_apply(const T* __restrict__ in, TO* __restrict__ out,
                                                    long n_rows, int seq_len, int D, PeSide pe,
                                                    int vec_ok) {
     const bool vec = vec_ok != 0;
     for (long row = blockIdx.x; row < n_rows; row += gridDim.x) {
         const int pos = (int)(row % seq_len);
         const T* xr = in + (size_t)row * D;
-        T* yr = out + (size_t)row * D;
+        TO* yr = out + (size_t)row * D;
         for (int d = threadIdx.x * 4; d < D; d += 256 * 4) {
             const float4 v = load_row4_pe<T, PEK>(xr, pos, d, D, pe, vec);
             if (vec && d + 3 < D) {
-                Elem<T>::st4(yr, d, v);
+                Elem<TO>::st4(yr, d, v);
             } else {
                 const float vv[4] = {v.x, v.y, v.z, v.w};
-                for (int c = 0; c < 4 && d + c < D; ++c) Elem<T>::st(yr, d + c, vv[c]);
+                for (int c = 0; c < 4 && d + c < D; ++c) Elem<TO>::st(yr, d + c, vv[c]);
             }
         }
     }
@@ -203,13 +206,13 @@ bool rows_ok(int pek, int D, const PeSide& pe, int vec_ok) {
     return pe.ld % (pe.dup ? 4 : 2) == 0;
 }
 
-template <typename T, int PEK, bool DUP>
+template <typename T, typename TO, int PEK, bool DUP>
 void run_rows(const PeRowsArgs& a, unsigned blocks, hipStream_t st) {
-    hipLaunchKernelGGL((k_pe_rows<T, PEK, DUP, PEK == kPeRopeHalf ? 2 : 4>), dim3(blocks),
+    hipLaunchKernelGGL((k_pe_rows<T, TO, PEK, DUP, PEK == kPeRopeHalf ? 2 : 4>), dim3(blocks),
                        dim3(256), 0, st, a);
 }
 
-template <typename T>
+template <typename T, typename TO>
 hipError_t pe_rows_t(int pek, const PeTensor* t, int n, int D, hipStream_t st) {
     const int U = pek == kPeRopeHalf ? 2 : 4;
     PeRowsArgs a{};
@@ -233,16 +236,16 @@ hipError_t pe_rows_t(int pek, const PeTensor* t, int n, int D, hipStream_t st) {
     const bool dup = t[0].pe.dup != 0;
     switch (pek) {
         case kPeRopeInterleaved:
-            dup ? run_rows<T, kPeRopeInterleaved, true>(a, grid, st)
-                : run_rows<T, kPeRopeInterleaved, false>(a, grid, st);
+            dup ? run_rows<T, TO, kPeRopeInterleaved, true>(a, grid, st)
+                : run_rows<T, TO, kPeRopeInterleaved, false>(a, grid, st);
             break;
         case kPeRopeHalf:
-            dup ? run_rows<T, kPeRopeHalf, true>(a, grid, st)
-                : run_rows<T, kPeRopeHalf, false>(a, grid, st);
+            dup ? run_rows<T, TO, kPeRopeHalf, true>(a, grid, st)
+                : run_rows<T, TO, kPeRopeHalf, false>(a, grid, st);
             break;
         case kPeSinusoidal:
-            dup ? run_rows<T, kPeSinusoidal, true>(a, grid, st)
-                : run_rows<T, kPeSinusoidal, false>(a, grid, st);
+            dup ? run_rows<T, TO, kPeSinusoidal, true>(a, grid, st)
+                : run_rows<T, TO, kPeSinusoidal, false>(a, grid, st);
             break;
         default:
             return hipErrorInvalidValue;
@@ -250,22 +253,22 @@ hipError_t pe_rows_t(int pek, const PeTensor* t, int n, int D, hipStream_t st) {
     return hipGetLastError();
 }
 
-template <typename T>
+template <typename T, typename TO>
 hipError_t pe_apply_t(int pek, const PeTensor& t, int D, int vec_ok, hipStream_t st) {
     const dim3 grid((unsigned)std::min<long>(t.n_rows, 65536)), block(256);
     const T* x = static_cast<const T*>(t.in);
-    T* y = static_cast<T*>(t.out);
+    TO* y = static_cast<TO*>(t.out);
     switch (pek) {
         case kPeRopeInterleaved:
-            hipLaunchKernelGGL((k_pe_apply<T, kPeRopeInterleaved>), grid, block, 0, st, x, y,
+            hipLaunchKernelGGL((k_pe_apply<T, TO, kPeRopeInterleaved>), grid, block, 0, st, x, y,
                                t.n_rows, t.seq_len, D, t.pe, vec_ok);
             break;
         case kPeRopeHalf:
-            hipLaunchKernelGGL((k_pe_apply<T, kPeRopeHalf>), grid, block, 0, st, x, y, t.n_rows,
+            hipLaunchKernelGGL((k_pe_apply<T, TO, kPeRopeHalf>), grid, block, 0, st, x, y, t.n_rows,
                                t.seq_len, D, t.pe, vec_ok);
             break;
         case kPeSinusoidal:
-            hipLaunchKernelGGL((k_pe_apply<T, kPeSinusoidal>), grid, block, 0, st, x, y, t.n_rows,
+            hipLaunchKernelGGL((k_pe_apply<T, TO, kPeSinusoidal>), grid, block, 0, st, x, y, t.n_rows,
                                t.seq_len, D, t.pe, vec_ok);
             break;
         default:
@@ -274,23 +277,76 @@ hipError_t pe_apply_t(int pek, const PeTensor& t, int D, int vec_ok, hipStream_t
     return hipGetLastError();
 }
 
-}  // namespace
-
-hipError_t launch_pe_apply(int dtype, int pek, const PeTensor* t, int n, int D, int vec_ok,
-                           hipStream_t st) {
+template <typename T, typename TO>
+hipError_t pe_any(int pek, const PeTensor* t, int n, int D, int vec_ok, hipStream_t st) {
     bool rows = true;
     for (int i = 0; i < n; ++i)
         rows = rows && rows_ok(pek, D, t[i].pe, vec_ok) &&
                t[i].n_rows <= ((long)1 << 40) / std::max(1, D / 4);
-    if (rows)
-        return dtype == kDtypeF32 ? pe_rows_t<float>(pek, t, n, D, st)
-                                  : pe_rows_t<uint16_t>(pek, t, n, D, st);
+    if (rows) return pe_rows_t<T, TO>(pek, t, n, D, st);
     for (int i = 0; i < n; ++i) {
-        const hipError_t e = dtype == kDtypeF32 ? pe_apply_t<float>(pek, t[i], D, vec_ok, st)
-                                                : pe_apply_t<uint16_t>(pek, t[i], D, vec_ok, st);
+        const hipError_t e = pe_apply_t<T, TO>(pek, t[i], D, vec_ok, st);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+}  // namespace
+
+hipError_t launch_pe_apply(int dtype, int out_dtype, int pek, const PeTensor* t, int n, int D,
+                           int vec_ok, hipStream_t st) {
+    if (dtype == kDtypeF32) return pe_any<float, float>(pek, t, n, D, vec_ok, st);
+    return out_dtype == kDtypeF32 ? pe_any<uint16_t, float>(pek, t, n, D, vec_ok, st)
+                                  : pe_any<uint16_t, uint16_t>(pek, t, n, D, vec_ok, st);
+}
+
+// Rows of D bf16 into rows of Dp (a multiple of 8), zeros past D: up to three
+// tensors, 8 elements of a row per thread.  Source rows start anywhere, so
+// they are read two bytes at a time; the copies' tiles are then read 16.
+namespace {
+struct PadArgs {
+    const uint16_t* in[3];
+    uint16_t* out[3];
+    long units[3];
+    unsigned first[3];  // the tensor's first workgroup
+    int D, Dp;
+};
+__global__ __launch_bounds__(256) void k_pad_rows(PadArgs a) {
+    const int s = blockIdx.x >= a.first[2] ? 2 : (blockIdx.x >= a.first[1] ? 1 : 0);
+    const long u = (long)(blockIdx.x - a.first[s]) * 256 + threadIdx.x;
+    if (u >= a.units[s]) return;
+    const int per = a.Dp >> 3;
+    const long row = u / per;
+    const int d = (int)(u - row * per) * 8;
+    const uint16_t* x = a.in[s] + (size_t)row * a.D;
+    uint32_t w[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const uint32_t lo = d + 2 * c < a.D ? x[d + 2 * c] : 0u;
+        const uint32_t hi = d + 2 * c + 1 < a.D ? x[d + 2 * c + 1] : 0u;
+        w[c] = lo | (hi << 16);
+    }
+    *reinterpret_cast<uint4*>(a.out[s] + (size_t)row * a.Dp + d) = make_uint4(w[0], w[1], w[2], w[3]);
+}
+}  // namespace
+
+hipError_t launch_pad_rows(const PadTensor* t, int n, int D, int Dp, hipStream_t st) {
+    PadArgs a{};
+    a.D = D;
+    a.Dp = Dp;
+    long blocks = 0;
+    for (int i = 0; i < 3; ++i) {
+        a.first[i] = (unsigned)blocks;
+        if (i >= n) continue;
+        a.in[i] = static_cast<const uint16_t*>(t[i].in);
+        a.out[i] = static_cast<uint16_t*>(t[i].out);
+        a.units[i] = t[i].n_rows * (Dp / 8);
+        blocks += (a.units[i] + 255) / 256;
+        if (blocks > INT32_MAX / 2) return hipErrorInvalidConfiguration;
+    }
+    for (int i = n; i < 3; ++i) a.first[i] = ~0u;
+    hipLaunchKernelGGL(k_pad_rows, dim3((unsigned)blocks), dim3(256), 0, st, a);
+    return hipGetLastError();
 }
 
 }  // namespace atn

@@ -31,7 +31,9 @@
 // fp32 calls, before (stream16.hip's kernels) -> these: (1,4,512,512,2048)
 // 57.4 -> 48.8 us, (2,2,422,422,2360) 81 -> 49, (2,2,128,1415,1520) 98 -> 40,
 // (1,2,517,517,1272) 58 -> 31; at (1,4,1453,1453,1024) Q K^T runs at 215
-// TFLOP/s of fp32 work (650 of fp16 products).
+// TFLOP/s of fp32 work (650 of fp16 products).  bf16: (1,2,273,757,3081)
+// 184 -> 48 us (before: fp32 MFMA on two-byte loads), and the GEMM path's
+// small grids ((1,2,68,68,624) 37.3 -> 11.5 us, see the host's rule).
 #include <algorithm>
 #include <type_traits>
 

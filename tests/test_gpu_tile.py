@@ -105,3 +105,84 @@ def test_scratch_without_encoded_copies(am, dev, tuner, pe):
     am.attention_ex(q, k, v, out, pe=desc, workspace=ws)
     hip_rt.synchronize()
     _check(out.numpy(), Q, K, V, pe)
+
+
+@pytest.mark.parametrize("tile", [0, 64, 128])
+@pytest.mark.parametrize("shape,pe", [
+    ((1, 2, 68, 68, 624), "none"),       # a small grid of the GEMM path's
+    ((1, 1, 129, 200, 264), "none"),     # 4 full 64-deep stages and one of 8 dims
+    ((1, 2, 130, 140, 328), "half"),
+    ((1, 1, 65, 257, 1000), "rope_q"),   # K only widened
+    ((2, 1, 200, 70, 512), "half_k"),
+    ((1, 1, 70, 65, 2056), "sin"),
+    ((1, 1, 131, 129, 261), "none"),     # head_d % 8 == 1: padded copies
+    ((1, 2, 66, 200, 262), "none"),
+    ((1, 1, 128, 128, 516), "rope"),
+    ((1, 1, 90, 150, 269), "sin"),
+    ((1, 1, 150, 90, 18), "half"),
+], ids=str)
+def test_tile_edges_bf16(am, dev, tuner, tile, shape, pe):
+    import hip_rt
+    B, Hh, Lq, Lk, D = shape
+    print(f"[case] bf16 tile {tile} {shape} {pe}", flush=True)
+    if tile:
+        tuner.set(splitd_tile=tile)
+    sigma = 0.5 if pe == "sin" else 1.0
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 800 + Lq + D, "bf16", sigma)
+    out = H.empty(Q.shape, "bf16")
+    am.attention_ex(q, k, v, out, pe=_desc(am, pe))
+    hip_rt.synchronize()
+    n, nrel, mabs = H.check_bf16(out.numpy(), _ref(pe, Q, K, V))
+    assert n == 0, (nrel, mabs)
+    # one rounding of the output (2^-9 at most), P to 16 bits, exact products
+    assert nrel < 2.0 ** -9
+
+
+@pytest.mark.parametrize("D", [264, 267, 40], ids=str)
+def test_misaligned_bases_bf16(am, dev, D):
+    """bf16 tensors 2 bytes off: copied into aligned rows first."""
+    import hip_rt
+    B, Hh, Lq, Lk = 1, 2, 100, 140
+    print(f"[case] misaligned bf16 {D}", flush=True)
+    Q, K, V = (oracle.bf16_bits_to_f32(oracle.f32_to_bf16_bits(x))
+               for x in H.rng_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), seed=961))
+    dev_t = [H.upload(np.concatenate([[0.0], x.ravel()]).astype(np.float32), "bf16")
+             for x in (Q, K, V)]
+    out = H.empty((Q.size + 1,), "bf16")
+    st = am.lib().atn_attention_fwd_ex(1, *[t.ptr + 2 for t in dev_t], out.ptr + 2, B, Hh, Lq, Lk, D,
+                                       None, None, 0, None)
+    assert st == 0
+    hip_rt.synchronize()
+    n, nrel, mabs = H.check_bf16(out.numpy()[1:].reshape(Q.shape), _ref("none", Q, K, V))
+    assert n == 0, (nrel, mabs)
+
+
+@pytest.mark.parametrize("scale", [2.0 ** 40, 2.0 ** -40], ids=str)
+def test_bf16_range(am, dev, scale):
+    """bf16 keeps fp32's exponents: V far outside fp16's range."""
+    import hip_rt
+    B, Hh, Lq, Lk, D = 1, 1, 70, 90, 272
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 811, "bf16")
+    v = H.upload(V * np.float32(scale), "bf16")
+    out = H.empty(Q.shape, "bf16")
+    am.attention_ex(q, k, v, out)
+    hip_rt.synchronize()
+    n, nrel, mabs = H.check_bf16(out.numpy() / np.float32(scale), _ref("none", Q, K, V))
+    assert n == 0, (nrel, mabs)
+
+
+def test_chunked_tiles(am, dev, tuner):
+    """A bf16 call of the tiles in chunks of heads and rows: the same bits."""
+    import hip_rt
+    B, Hh, Lq, Lk, D = 1, 3, 300, 260, 1000
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 812, "bf16")
+    full, out = H.empty(Q.shape, "bf16"), H.empty(Q.shape, "bf16")
+    am.attention_ex(q, k, v, full)
+    hip_rt.synchronize()
+    tuner.set(workspace_cap_mib=1)
+    ws = hip_rt.DeviceArray(((1 << 20) // 4,), "f32", fill=0)
+    am.attention_ex(q, k, v, out, workspace=ws)
+    hip_rt.synchronize()
+    assert np.array_equal(out.bits(), full.bits())
+    n, nrel, mabs = H.check_bf16(out.numpy(), _ref("none", Q, K, V))
+    assert n == 0, (nrel, mabs)
