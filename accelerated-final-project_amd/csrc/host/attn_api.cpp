@@ -108,6 +108,8 @@ struct PePlan {
     // whole call's D-chunk there
     bool tiles = false;
     int dchunk = 0;
+    // flash kernel, bf16 with an encoding: K encoded once by a pass of its own
+    bool kpre = false;
 };
 
 int check_pe(const atn_pe_desc* pe, int D, PePlan* plan) {
@@ -983,6 +985,34 @@ size_t flash_split_bound(const Shape& s) {
     return b;
 }
 
+// K~ (fp16) and its tiles' units, behind the key splits' parts.
+size_t flash_kpre_bytes(const Shape& s) {
+    return 256 + round256((size_t)s.nk * 2) + round256((size_t)s.BH * ((s.Lk + 63) / 64) * 4);
+}
+
+// Whether a bf16 flash call that encodes K does so once, to fp16 in scratch,
+// instead of in every query block's workgroup as it loads each tile.  In the
+// kernel the encoding lies on every tile's critical path, about 0.9 us per
+// 64-key tile a workgroup walks; the pass costs a launch and its traffic.  So
+// it pays for long walks over few bytes: same box, (4,8,1107,1107,128) RoPE
+// 99 -> 72 us, (1,16,3000,3000,64) rotate-half 169 -> 85, (4,16,300,1500,128)
+// 71 -> 52, (1,8,4096,4096,128) 118 -> 97; not at (4,32,512,512,128) (39.4 ->
+// 42.7), (8,16,300,300,64) (17.8 -> 20.7) or under key splits of few tiles
+// ((1,4,200,4000,128) 29.7 -> 31.4).  fp32 calls, whose products take three
+// times as long beside the same encoding, gained 3-5 % at most and lost up to
+// 20 % (their copies are twice the bytes): they encode in the kernel.
+bool flash_kpre(int dtype, const Shape& s, const PePlan& plan, int rows, size_t cap) {
+    if (dtype != ATN_DTYPE_BF16 || plan.pek == atn::kPeNone || !plan.k.on || s.Lq <= 64 ||
+        tune().flash_form != 0 ||
+        kSyncBytes + flash_split_bound(s) + flash_kpre_bytes(s) > cap)
+        return false;
+    const FlashSplit f = flash_split(s, rows);
+    const int64_t wgs = s.BH * ((s.Lq + rows - 1) / rows) * f.nsplit;
+    const double tiles =
+        ((f.nsplit > 1 ? f.kchunk : s.Lk) + 63) / 64 * std::ceil((double)wgs / 256.0);
+    return tiles * 0.9 > 1.2 * (4.0 + (double)s.nk * 4.0 / 4.5e6);
+}
+
 // Scratch bytes of the path a call of shape s takes: fused (when planned and
 // vector-aligned), else GEMM (when planned and 16-byte aligned), else the
 // split-D pipeline.  vec / a16: the alignment of the call's pointers; pass
@@ -993,13 +1023,15 @@ size_t path_need(int dtype, const Shape& s, const PePlan& plan, bool query_devic
     const GemmPlan gp = gemm_plan(dtype, s, plan);
     if (fp.ok && vec > 0) return fp.bytes;
     if (a16 > 0 && vec >= 0 && flash_ok(dtype, s, plan))  // the flash kernel: only its key splits' parts
-        return kSyncBytes + flash_split_bound(s);
+        return kSyncBytes + flash_split_bound(s) + (plan.kpre ? flash_kpre_bytes(s) : 0);
     const TilePlan tp = tile_plan(dtype, s, plan, a16 > 0);
     const size_t split = tp.ok ? tp.bytes : kSyncBytes + stream_plan(s).bytes;
     if (vec < 0 || a16 < 0)
         return std::max({fp.ok ? fp.bytes : (size_t)0, gp.ok ? gp.bytes : (size_t)0, split,
-                         flash_ok(dtype, s, plan) ? kSyncBytes + flash_split_bound(s)
-                                                  : (size_t)0});
+                         flash_ok(dtype, s, plan)
+                             ? kSyncBytes + flash_split_bound(s) +
+                                   (plan.kpre ? flash_kpre_bytes(s) : 0)
+                             : (size_t)0});
     if (gp.ok && a16 && !(plan.tiles && tp.ok)) return gp.bytes;
     return split;
 }
@@ -1074,7 +1106,7 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
     const FlashSplit fs = use_flash ? flash_split(s, flash_rows(fform, D)) : FlashSplit{};
     const size_t need =
         use_fused ? fd.bytes
-                  : (use_flash ? kSyncBytes + fs.bytes
+                  : (use_flash ? kSyncBytes + fs.bytes + (plan.kpre ? flash_kpre_bytes(s) : 0)
                                : (use_gemm ? gp.bytes
                                            : (use_tile ? tp.bytes : kSyncBytes + sp.bytes)));
     void* ws = workspace;
@@ -1163,8 +1195,20 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
         return ATN_OK;
     }
     if (use_flash) {
-        ATN_HIP(atn::launch_flash(dtype, plan.pek, fform, Q, K, V, out, (int)s.BH, Lq, Lk, D,
-                                  scale, plan.q, plan.k, fs.nsplit, fs.kchunk, scratch, stream));
+        const void* kt = K;
+        const float* kunit = nullptr;
+        if (plan.kpre) {
+            char* w = reinterpret_cast<char*>(scratch) + round256(fs.bytes);
+            uint16_t* ke = reinterpret_cast<uint16_t*>(w);
+            float* u = reinterpret_cast<float*>(w + round256((size_t)s.nk * 2));
+            ATN_HIP(atn::launch_encode_key_tiles(plan.pek, static_cast<const uint16_t*>(K), ke, u,
+                                                 (int)s.BH, Lk, D, plan.k, stream));
+            kt = ke;
+            kunit = u;
+        }
+        ATN_HIP(atn::launch_flash(dtype, plan.pek, fform, Q, kt, V, out, (int)s.BH, Lq, Lk, D,
+                                  scale, plan.q, plan.k, fs.nsplit, fs.kchunk, scratch, kunit,
+                                  stream));
         return ATN_OK;
     }
     if (use_tile) {
@@ -1257,6 +1301,8 @@ int attention_core(int dtype, const void* Q, const void* K, const void* V, void*
 
     const size_t cap = no_alloc ? atn::kNoAllocScratchBytes
                                 : (workspace != nullptr ? workspace_bytes : library_cap());
+    if (plan.pek != atn::kPeNone && flash_ok(dtype, s, plan))
+        plan.kpre = flash_kpre(dtype, s, plan, flash_rows(flash_form(s, dev), D), cap);
     // chunk pointers keep the base alignment when a row is a multiple of 16
     // bytes; otherwise plan for the largest path
     const size_t va = dtype == ATN_DTYPE_F32 ? 16 : 8;
@@ -1641,6 +1687,11 @@ size_t atn_attention_workspace_bytes(int dtype, int batch, int heads, int len_q,
     PePlan plan;
     if (check_pe(pe, head_d, &plan) != ATN_OK) return 0;
     choose_tiles(dtype, s, plan);
+    // (the form, which decides for K's encoded copy, is the device's: with it
+    // wherever it fits)
+    plan.kpre = dtype == ATN_DTYPE_BF16 && plan.pek != atn::kPeNone && s.Lq > 64 &&
+                flash_ok(dtype, s, plan) &&
+                kSyncBytes + flash_split_bound(s) + flash_kpre_bytes(s) <= library_cap();
     // the largest workspace of every plan the call could take, or, when that
     // exceeds the library's cap, of the chunks the call then runs in
     const size_t full = path_need(dtype, s, plan, false, -1, -1);

@@ -201,7 +201,12 @@ constexpr int flash_waves_per_simd() {
     return sizeof(T) == 2 && PEK == kPeNone && NW == 8 && RW == 16 && DP <= 128 ? 4 : 8 / NW;
 }
 
-template <typename T, int DP, int PEK, int NW, int RW>
+// KPRE (bf16 with an encoding): Kg holds K~, encoded to fp16 by a pass of its
+// own (launch_encode_key_tiles), kunit the unit of each of its 64-key tiles;
+// the kernel then encodes its query rows only and stages K~ as it is, the
+// bits that it would have staged itself.  (The host's rule and what it
+// measured: flash_kpre in attn_api.cpp.)
+template <typename T, int DP, int PEK, int NW, int RW, bool KPRE>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     flash_waves_per_simd<T, DP, PEK, NW, RW>()))) void k_flash(const T* __restrict__ Qg,
                                                              const T* __restrict__ Kg,
@@ -210,9 +215,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
                                                              int D, int qblocks, float scale,
                                                              PeSide pq, PeSide pk, int nsplit,
                                                              int kchunk, float* __restrict__ part,
-                                                             float4* __restrict__ stats) {
+                                                             float4* __restrict__ stats,
+                                                             const float* __restrict__ kunit) {
     constexpr bool kBf = sizeof(T) == 2;
     constexpr bool kRaw = kBf && PEK == kPeNone;
+    constexpr bool kBits = kRaw || KPRE;  // K goes to LDS as loaded
+    static_assert(!KPRE || (kBf && !kRaw), "pre-encoded keys");
     constexpr int es = (int)sizeof(T);
     // MFMA operands: Q K^T (op_t) and P V (pv_t).  bf16 V is never encoded,
     // so it always goes in as loaded, with P as bf16.
@@ -378,13 +386,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     const __amdgpu_buffer_rsrc_t rk = buf_rsrc(Kh, Lk * D * es);
     const __amdgpu_buffer_rsrc_t rv = buf_rsrc(Vh, Lk * D * es);
     float4 kr[G::NLD], vr[G::NLD];
-    uint2 kw[G::NLD], vw[G::NLD];  // raw bf16: the loaded bits
+    uint2 kw[G::NLD], vw[G::NLD];  // the loaded bits (raw bf16, K~, bf16 V)
+    float ku = 1.f;                // unit of the loaded K~ tile
+    static_assert(!KPRE || G::KT == 64, "a unit per 64 keys");
     auto issue = [&](int k0) {
+        if constexpr (KPRE) ku = kunit[(size_t)bh * ((LkAll + 63) / 64) + ((kbeg + k0) >> 6)];
 #pragma unroll
         for (int i = 0; i < G::NLD; ++i) {
             const int key = k0 + lrow + G::RSTEP * i;
             const int off = key < Lk && lcol < D ? (key * D + lcol) * es : kOob;
-            if constexpr (kRaw) {
+            if constexpr (kBits) {
                 const auto a = __builtin_amdgcn_raw_buffer_load_b64(rk, off, 0, 0);
                 kw[i] = make_uint2(a[0], a[1]);
             } else {
@@ -404,7 +415,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     // stay so through a scaling and must not set the scale of the finite
     // values beside them.
     auto maxima = [&](int k0, int par) {
-        if constexpr (kRaw) return;  // no scales
+        if constexpr (kBits) return;  // no scales to find
         if constexpr (PEK != kPeNone) {
             if (pk.on && pe4_batch_ok(PEK, pk)) {
                 // every group's loads at once (rows past Lk clamped, their
@@ -488,8 +499,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     // (fp32) or hi (encoded bf16 K) fp16 parts into LDS buffer par; bf16 V
     // goes in as loaded
     auto stage = [&](int par, float& uk, float& sv, float& uv) {
-        if constexpr (kRaw) {
-            uk = sv = uv = 1.f;
+        if constexpr (kBits) {
+            uk = ku;
+            sv = uv = 1.f;
             uint16_t* buf = smem + par * G::TILE;
 #pragma unroll
             for (int i = 0; i < G::NLD; ++i) {
@@ -855,25 +867,26 @@ struct FlashArgs {
     int nsplit, kchunk;
     float* part;
     float4* stats;
+    const float* kunit;  // not null: K is encoded fp16 (KPRE)
 };
 
-template <typename T, int DP, int PEK, int NW, int RW>
+template <typename T, int DP, int PEK, int NW, int RW, bool KPRE = false>
 hipError_t launch_t(const FlashArgs& a, hipStream_t st) {
     using G = FlashGeo<DP, PEK != kPeNone, NW, RW, sizeof(T) == 4>;
     static bool attr = false;
     if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_flash<T, DP, PEK, NW, RW>,
+        hipError_t e = hipFuncSetAttribute((const void*)k_flash<T, DP, PEK, NW, RW, KPRE>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, G::BYTES);
         if (e != hipSuccess) return e;
         attr = true;
     }
     const int qblocks = (a.Lq + G::ROWS - 1) / G::ROWS;
     const int kchunk = a.nsplit > 1 ? a.kchunk : a.Lk;
-    hipLaunchKernelGGL((k_flash<T, DP, PEK, NW, RW>), dim3((unsigned)(a.BH * qblocks * a.nsplit)),
+    hipLaunchKernelGGL((k_flash<T, DP, PEK, NW, RW, KPRE>), dim3((unsigned)(a.BH * qblocks * a.nsplit)),
                        dim3(G::THREADS), G::BYTES, st, static_cast<const T*>(a.Q),
                        static_cast<const T*>(a.K), static_cast<const T*>(a.V), static_cast<T*>(a.O),
                        a.Lq, a.Lk, a.D, qblocks, a.scale, a.pq, a.pk, a.nsplit, kchunk, a.part,
-                       a.stats);
+                       a.stats, a.kunit);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.nsplit == 1) return e;
     const int rows = a.BH * a.Lq;
@@ -886,6 +899,14 @@ hipError_t launch_t(const FlashArgs& a, hipStream_t st) {
 // an encoding)
 template <typename T, int PEK, int NW, int RW>
 hipError_t launch_pe(const FlashArgs& a, hipStream_t st) {
+    if constexpr (sizeof(T) == 2 && PEK != kPeNone && NW == 8) {
+        if (a.kunit != nullptr) {
+            if (a.D <= 32) return launch_t<T, 32, PEK, NW, RW, true>(a, st);
+            if (a.D <= 64) return launch_t<T, 64, PEK, NW, RW, true>(a, st);
+            if (a.D <= 128) return launch_t<T, 128, PEK, NW, RW, true>(a, st);
+        }
+    }
+    if (a.kunit != nullptr) return hipErrorInvalidValue;
     if (a.D <= 32) return launch_t<T, 32, PEK, NW, RW>(a, st);
     if (a.D <= 64) return launch_t<T, 64, PEK, NW, RW>(a, st);
     if (a.D <= 128) return launch_t<T, 128, PEK, NW, RW>(a, st);
@@ -928,12 +949,13 @@ bool flash_supported(int dtype, int pek, int D) {
 
 hipError_t launch_flash(int dtype, int pek, int form, const void* Q, const void* K, const void* V,
                         void* O, int BH, int Lq, int Lk, int D, float scale, const PeSide& pq,
-                        const PeSide& pk, int nsplit, int kchunk, float* part, hipStream_t st) {
+                        const PeSide& pk, int nsplit, int kchunk, float* part, const float* kunit,
+                        hipStream_t st) {
     if (nsplit < 1 || (nsplit > 1 && (part == nullptr || kchunk < 1 ||
                                       (long long)kchunk * (nsplit - 1) >= Lk)))
         return hipErrorInvalidValue;
     FlashArgs a{Q, K, V, O, BH, Lq, Lk, D, scale, pq, pk, nsplit, kchunk, part,
-                reinterpret_cast<float4*>(part + (size_t)nsplit * BH * Lq * D)};
+                reinterpret_cast<float4*>(part + (size_t)nsplit * BH * Lq * D), kunit};
     if (dtype == kDtypeF32) return launch_typed<float>(pek, form, a, st);
     if (dtype == kDtypeBF16) return launch_typed<uint16_t>(pek, form, a, st);
     return hipErrorInvalidValue;

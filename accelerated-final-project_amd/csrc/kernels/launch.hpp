@@ -128,7 +128,15 @@ constexpr int kFlashForm4x16 = 1, kFlashForm8x16 = 2, kFlashForm4x32 = 3, kFlash
 bool flash_supported(int dtype, int pek, int D);
 hipError_t launch_flash(int dtype, int pek, int form, const void* Q, const void* K, const void* V,
                         void* O, int BH, int Lq, int Lk, int D, float scale, const PeSide& pq,
-                        const PeSide& pk, int nsplit, int kchunk, float* part, hipStream_t st);
+                        const PeSide& pk, int nsplit, int kchunk, float* part, const float* kunit,
+                        hipStream_t st);
+// kunit (bf16 with an encoding, the forms of 8 waves): K is then K~ and kunit
+// its units, both from launch_encode_key_tiles: the rows of BH heads of Lk
+// keys encoded to fp16 (same strides), each tile of 64 keys times a power of
+// two where its largest magnitude lies outside [2^-3, 65504), the inverse in
+// unit[BH][ceil(Lk / 64)].  head_d % 4 == 0, <= kFlashMaxDEncoded.
+hipError_t launch_encode_key_tiles(int pek, const uint16_t* K, uint16_t* out, float* unit, int BH,
+                                   int Lk, int D, const PeSide& pe, hipStream_t st);
 
 // Allocation-free entry point: the per-device scratch array (noalloc.hip),
 // kNoAllocScratchBytes long.  noalloc_scratch() returns its device address

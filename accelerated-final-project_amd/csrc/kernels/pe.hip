@@ -14,6 +14,7 @@
 
 #include "common.hpp"
 #include "launch.hpp"
+#include "split16.hpp"
 
 namespace atn {
 
@@ -298,6 +299,90 @@ hipError_t launch_pe_apply(int dtype, int out_dtype, int pek, const PeTensor* t,
     if (dtype == kDtypeF32) return pe_any<float, float>(pek, t, n, D, vec_ok, st);
     return out_dtype == kDtypeF32 ? pe_any<uint16_t, float>(pek, t, n, D, vec_ok, st)
                                   : pe_any<uint16_t, uint16_t>(pek, t, n, D, vec_ok, st);
+}
+
+// K~ of the flash kernel, bf16 to fp16: one workgroup per tile of 64 keys
+// (the flash kernel's), NG groups of 4 dims per thread, all loads first.  The
+// tile's largest finite magnitude is known before anything is written, so
+// the values and units are those of the flash kernel's own staging.
+namespace {
+template <int PEK, int NG>
+__global__ __launch_bounds__(256) void k_encode_key_tiles(const uint16_t* __restrict__ K,
+                                                          uint16_t* __restrict__ out,
+                                                          float* __restrict__ unit, int tiles,
+                                                          int Lk, int D, PeSide pe) {
+    __shared__ float slot[4];
+    const int tid = threadIdx.x, vpr = D >> 2;
+    const int bh = blockIdx.x / tiles, k0 = (blockIdx.x % tiles) * 64;
+    const int groups = min(64, Lk - k0) * vpr;  // the tile's rows are consecutive
+    const uint16_t* src = K + ((size_t)bh * Lk + k0) * D;
+    uint16_t* dst = out + ((size_t)bh * Lk + k0) * D;
+    float4 x[NG];
+    int d[NG], pos[NG];
+    const uint16_t* row[NG];
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+        const int g = min(tid + 256 * i, groups - 1), r = g / vpr;
+        d[i] = (g - r * vpr) * 4;
+        pos[i] = k0 + r;
+        row[i] = src + (size_t)r * D;
+        x[i] = Elem<uint16_t>::ld4(row[i], d[i]);
+    }
+    if (pe.on) {
+        if (pe4_batch_ok(PEK, pe)) {
+            pe4_batch<uint16_t, PEK, NG>(x, d, row, pos, D, pe);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NG; ++i)
+                x[i] = apply_pe4<uint16_t, PEK>(x[i], row[i], pos[i], d[i], D, pe, true);
+        }
+    }
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < NG; ++i) m = max_finite4(m, x[i]);
+    m = wave_max(m);
+    if ((tid & 63) == 0) slot[tid >> 6] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(slot[0], slot[1]), fmaxf(slot[2], slot[3]));
+    const bool plain = m >= 0.125f && m < kF16Range;
+    const float s = plain ? 1.f : pow2_scale(m);
+    if (tid == 0) unit[blockIdx.x] = plain ? 1.f : pow2_unit(m);
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+        const f16x2 a = {(_Float16)(x[i].x * s), (_Float16)(x[i].y * s)};
+        const f16x2 b = {(_Float16)(x[i].z * s), (_Float16)(x[i].w * s)};
+        if (tid + 256 * i < groups)
+            *reinterpret_cast<uint2*>(dst + 4 * (size_t)(tid + 256 * i)) =
+                make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
+    }
+}
+
+template <int PEK>
+void run_key_tiles(const uint16_t* K, uint16_t* out, float* unit, int BH, int Lk, int D,
+                   const PeSide& pe, hipStream_t st) {
+    const int tiles = (Lk + 63) / 64;
+    const dim3 grid((unsigned)(BH * tiles)), block(256);
+    if (D <= 64)
+        hipLaunchKernelGGL((k_encode_key_tiles<PEK, 4>), grid, block, 0, st, K, out, unit, tiles, Lk,
+                           D, pe);
+    else
+        hipLaunchKernelGGL((k_encode_key_tiles<PEK, 8>), grid, block, 0, st, K, out, unit, tiles, Lk,
+                           D, pe);
+}
+}  // namespace
+
+hipError_t launch_encode_key_tiles(int pek, const uint16_t* K, uint16_t* out, float* unit, int BH,
+                                   int Lk, int D, const PeSide& pe, hipStream_t st) {
+    if (D > kFlashMaxDEncoded || D % 4 != 0) return hipErrorInvalidValue;
+    switch (pek) {
+        case kPeRopeInterleaved:
+            run_key_tiles<kPeRopeInterleaved>(K, out, unit, BH, Lk, D, pe, st);
+            break;
+        case kPeRopeHalf: run_key_tiles<kPeRopeHalf>(K, out, unit, BH, Lk, D, pe, st); break;
+        case kPeSinusoidal: run_key_tiles<kPeSinusoidal>(K, out, unit, BH, Lk, D, pe, st); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 // Rows of D bf16 into rows of Dp (a multiple of 8), zeros past D: up to three

@@ -649,3 +649,47 @@ def test_flash_split_graph_replays(am, dev):
     n, nrel, mabs = H.check_bf16(eager.numpy(), oracle.attention(Q, K, V, nthreads=16))
     assert n == 0, (nrel, mabs)
     st.destroy()
+
+
+@pytest.mark.parametrize("pe", ["rope", "half", "rope_part", "sin"])
+@pytest.mark.parametrize("shape,form,scale", [
+    ((4, 8, 1107, 1107, 96), "8x16", 1.0),        # ragged rows, head_d padded
+    ((4, 16, 300, 1500, 128), "8x16", 1.0),
+    ((8, 32, 512, 520, 64), "8x32", 1.0),
+    ((1, 4, 4200, 4160, 40), "8x32", 1.0),        # key splits
+    ((1, 16, 1100, 1100, 100), "8x16", 2.0 ** 30),  # K tiles scaled by a power of two
+    ((1, 16, 1100, 1100, 100), "8x16", 2.0 ** -20),
+], ids=str)
+def test_flash_keys_encoded_once(am, dev, tuner, shape, form, scale, pe):
+    """bf16 calls that encode K by a pass of its own, bit for bit as with K
+    encoded in the kernel (a forced form), and sampled rows of the oracle."""
+    import hip_rt
+    B, Hh, Lq, Lk, D = shape
+    print(f"[case] keys encoded once {shape} {pe} x{scale}", flush=True)
+    desc = {"rope": am.make_pe("rope"), "half": am.make_pe("rope", "half"),
+            "rope_part": am.make_pe("rope", "half", D // 2 // 4 * 4), "sin": am.make_pe("sinusoidal")}[pe]
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 700 + Lq, "bf16",
+                                           0.5 if pe == "sin" else 1.0)
+    if scale != 1.0:
+        K = K * np.float32(scale)
+        Q = Q * np.float32(1 / scale)
+        k, q = H.upload(K, "bf16"), H.upload(Q, "bf16")
+    out, forced = H.empty(Q.shape, "bf16"), H.empty(Q.shape, "bf16")
+    am.attention_ex(q, k, v, out, pe=desc)
+    hip_rt.synchronize()
+    tuner.set(flash_form=form)
+    am.attention_ex(q, k, v, forced, pe=desc)
+    hip_rt.synchronize()
+    assert np.array_equal(out.bits(), forced.bits())
+    if scale == 1.0:
+        rot = D if pe != "rope_part" else D // 2 // 4 * 4
+        r0, r1 = (B * Hh - 1) * Lq + Lq - 20, B * Hh * Lq  # the last head's last rows
+        if pe == "sin":
+            ref = oracle.attention_sinusoidal(Q, K, V, *oracle.sinusoidal_table(max(Lq, Lk), D),
+                                              rows=(r0, r1), nthreads=16)
+        else:
+            c, s = oracle.rope_cache(max(Lq, Lk), rot)
+            ref = oracle.attention_rope(Q, K, V, c, s, rotary_dim=rot, rows=(r0, r1), nthreads=16,
+                                        pairing="interleaved" if pe == "rope" else "half")
+        n, nrel, mabs = H.check_bf16(out.numpy().reshape(-1, D)[r0:r1], ref.reshape(-1, D)[r0:r1])
+        assert n == 0, (nrel, mabs)
