@@ -88,6 +88,13 @@ size_t elem_size(int dtype) { return dtype == ATN_DTYPE_F32 ? 4 : 2; }
 
 bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
+// The flash kernel's plan (flash_plan): form, key parts of kchunk keys, and
+// whether K's encoding is a pass of its own.
+struct FlashPlan {
+    int form = 0, nsplit = 1, kchunk = 0;
+    bool kpre = false;
+};
+
 // ---------------------------------------------------------------- resolved encoding
 struct PePlan {
     int pek = atn::kPeNone;   // kernel template selector
@@ -108,8 +115,7 @@ struct PePlan {
     // whole call's D-chunk there
     bool tiles = false;
     int dchunk = 0;
-    // flash kernel, bf16 with an encoding: K encoded once by a pass of its own
-    bool kpre = false;
+    FlashPlan flash;  // a call of the flash kernel: its plan
 };
 
 int check_pe(const atn_pe_desc* pe, int D, PePlan* plan) {
@@ -900,117 +906,116 @@ bool flash_ok(int dtype, const Shape& s, const PePlan& plan) {
            (int64_t)s.Lq * s.D * es < lim && (int64_t)s.Lk * s.D * es < lim;
 }
 
-// The flash kernel's workgroup form (atn_tuning.flash_form forces one).
-// 8 waves of 32 query rows (32 x 32 MFMA tiles: each wave reads a K/V tile
-// from LDS once per 32 rows, and each tile is converted once per 256 rows)
-// when head_d <= 128 and the grid of 256-row blocks gives every CU a
-// workgroup; else 8 waves of 16 rows (twice the workgroups).  Measured
-// with interleaved rounds on 14 shapes: the reference's (4,32,512,512,128)
-// 70.6 -> 62.9 us, RoPE there 108 -> 86 us; below a workgroup per CU the
-// 32-row form loses (up to 1.6x at (1,4,2048,2048,128)).  Up to 64 query
-// rows, 4 waves of 16 rows (64-row blocks: no wave of padding rows; with key
-// splits, same box: (1,32,16,4096,128) bf16 33.2 -> 29.6 us, (1,8,64,4096,
-// 128) fp32 35.7 -> 33.8 us).  From 4096 keys on, the 32-row form even below
-// a workgroup per CU (its key splits then fill the grid): each K/V tile read
-// and encoded once per 256 rows outweighs the splits' merge there (same box:
-// bf16 (1,8,4096,4096,128) 102 -> 91 us, (1,2,16384,16384,128) 346 -> 280 us,
-// RoPE rotate-half 173 -> 128 us, sinusoidal (1,4,8192,8192,128) 338 -> 216
-// us, fp32 (1,4,8192,8192,128) 432 -> 395 us, fp32 (1,8,4096,4096,64) 131
-// -> 123 us; at 1024 keys the 16-row form stays ahead: 33 against 43 us at
-// (2,16,1024,1024,128)).
-int flash_form(const Shape& s, int dev) {
-    const int forced = tune().flash_form;
-    if (forced >= atn::kFlashForm4x16 && forced <= atn::kFlashForm8x32) return forced;
-    if (s.D > 128) return atn::kFlashForm8x16;
-    if (s.Lq <= 64) return atn::kFlashForm4x16;
-    int cus = 0;
-    {
-        std::lock_guard<std::mutex> lk(g_mu);
-        DeviceState& ds = g_dev[dev];
-        if (ds.cus == 0 &&
-            hipDeviceGetAttribute(&ds.cus, hipDeviceAttributeMultiprocessorCount, dev) !=
-                hipSuccess)
-            ds.cus = 0;
-        cus = ds.cus > 0 ? ds.cus : 256;
-    }
-    if (s.BH * ((s.Lq + 255) / 256) >= (int64_t)cus) return atn::kFlashForm8x32;
-    return s.Lk >= 4096 ? atn::kFlashForm8x32 : atn::kFlashForm8x16;
-}
-
 // Query rows per workgroup of a flash form.
 int flash_rows(int form, int D) {
     if (D > 128) form = atn::kFlashForm8x16;
     return form == atn::kFlashForm4x16 ? 64 : (form == atn::kFlashForm8x32 ? 256 : 128);
 }
 
-// Key splits of the flash kernel.  A workgroup walks all keys of its query
-// block, so a grid of few (head, query block) pairs leaves CUs idle (64
-// workgroups at (1,4,2048,2048,128), 32 for 16 queries against 4096 keys at
-// 32 heads).  Such calls split the keys into parts of whole 64-key chunks,
-// two at least, so that the grid reaches about kFlashSplitTarget workgroups;
-// each part writes its normalized output and statistics (fp32) and a second
-// kernel merges them.  Decided from the shape alone (plus
-// atn_tuning.flash_split), so the workspace queries need no device.
-struct FlashSplit {
-    int nsplit = 1, kchunk = 0;
-    size_t bytes = 0;  // scratch of the parts
-};
-constexpr int kFlashSplitTarget = 256, kFlashSplitBelow = 128, kFlashSplitMax = 32;
+// Scratch of a flash plan: the key splits' parts (normalized outputs and
+// statistics), then K~ (fp16) and its tiles' units.
+size_t flash_parts_bytes(const Shape& s, int nsplit) {
+    return nsplit > 1 ? round256((size_t)nsplit * s.BH * s.Lq * (s.D + 4) * 4) : 0;
+}
+size_t flash_bytes(const Shape& s, const FlashPlan& f) {
+    return flash_parts_bytes(s, f.nsplit) +
+           (f.kpre ? round256((size_t)s.nk * 2) + round256((size_t)s.BH * ((s.Lk + 63) / 64) * 4)
+                   : 0);
+}
 
-FlashSplit flash_split(const Shape& s, int rows) {
-    FlashSplit f;
-    const int forced = tune().flash_split;
-    if (forced == 1) return f;
-    const int64_t grid = s.BH * ((s.Lq + rows - 1) / rows);
+// The flash kernel's workgroup form, its key splits (parts of whole 64-key
+// chunks, merged by a second kernel) and, for bf16 calls that encode K,
+// whether K is encoded once into scratch (kpre) instead of in every query
+// block's workgroup: the least estimated time of all that fit `cap`.
+//
+// A workgroup walks its keys tile by tile at a nearly constant rate and most
+// forms fill a CU, so a call takes whole rounds of 256 workgroups: 288 of them
+// take two rounds, which 160 of twice the rows, or three times as many with
+// a third of the keys, undercut ((4,8,1107,1107,128) fp32: 8 waves of 16 rows
+// 123 us, of 32 rows 91).  Per 64-key tile and round, measured at 1-2 rounds
+// (us, head_d <= 64 / <= 128 / <= 256): see t below; forms whose workgroups fit
+// two to a CU take `pair` times that for both.  A merge costs 5 us and its
+// parts 0.5 us per MB.  Over 122 calls (fp32 and bf16, plain and RoPE, B H
+// 1-256, lengths 1-8192) with every form and 14 split counts timed, the
+// choice loses 0.6 % on average over the best of them; the rule before
+// (splits only below 128 workgroups, towards 256) lost 8 %.  K once:
+// (4,8,1107,1107,128) bf16 RoPE 99 -> 63 us, (1,16,3000,3000,64) rotate-half
+// 169 -> 85; not worth its launch and traffic at (4,32,512,512,128) (39.4 us
+// against 42.7).  fp32 calls, whose products take three times as long beside
+// the same encoding, gained 3-5 % at most and lost up to 20 %.
+FlashPlan flash_plan_uncached(int dtype, const Shape& s, const PePlan& plan, size_t cap) {
+    // [fp32 plain, fp32 encoded, bf16 plain, bf16 encoded, bf16 K once][form][head_d class]
+    static const double t[5][3][3] = {
+        {{1.6, 2.6, 0}, {2.0, 3.2, 5.8}, {2.75, 4.75, 0}},
+        {{2.3, 3.8, 0}, {2.45, 3.95, 0}, {3.35, 5.85, 0}},
+        {{0.8, 1.2, 0}, {0.9, 1.4, 2.75}, {1.3, 1.85, 0}},
+        {{1.5, 2.4, 0}, {1.6, 2.6, 0}, {2.05, 3.2, 0}},
+        {{0, 0, 0}, {0.8, 1.65, 0}, {1.5, 1.95, 0}},
+    };
+    const atn_tuning& tn = tune();
+    const int dc = s.D <= 64 ? 0 : (s.D <= 128 ? 1 : 2);
+    const bool bf = dtype == ATN_DTYPE_BF16, enc = plan.pek != atn::kPeNone;
     const int chunks = (s.Lk + 63) / 64;
-    int64_t n;
-    if (forced >= 2) {
-        n = std::min<int64_t>(forced, chunks);
-    } else {
-        if (grid > kFlashSplitBelow) return f;
-        n = std::min<int64_t>({(kFlashSplitTarget + grid - 1) / grid, chunks / 2, kFlashSplitMax});
+    FlashPlan best;
+    double best_us = 0;
+    static const int forms[3] = {atn::kFlashForm4x16, atn::kFlashForm8x16, atn::kFlashForm8x32};
+    const int forced = tn.flash_form;
+    for (int once = 0; once < 2; ++once) {
+        if (once && !(bf && enc && plan.k.on && s.Lq > 64 && forced == 0)) break;
+        for (int fi = 0; fi < 3; ++fi) {
+            int form = forms[fi];
+            if (forced == atn::kFlashForm4x32) {  // (a tuning override only; as 8 waves of 16)
+                if (fi != 1) continue;
+                form = forced;
+            } else if (forced != 0 && s.D <= 128 ? form != forced
+                       : s.D > 128 || s.Lq > 64  ? (form == atn::kFlashForm4x16 ||
+                                                   (s.D > 128 && form != atn::kFlashForm8x16))
+                                                 : form != atn::kFlashForm4x16) {
+                continue;
+            }
+            const int rows = flash_rows(form, s.D);
+            const int64_t grid = s.BH * ((s.Lq + rows - 1) / rows);
+            const double tile = t[bf ? (once ? 4 : 2 + enc) : enc][fi][dc];
+            const bool two = fi == 0 || (bf && !enc && fi == 1 && dc < 2);
+            const double pair = fi == 0 ? 1.5 : 1.78;
+            int last = 0;
+            for (int n = 1; n <= std::min(chunks, 32); ++n) {
+                if (tn.flash_split >= 1 && n != std::min(tn.flash_split, chunks)) continue;
+                const int per = (chunks + n - 1) / n, ns = (chunks + per - 1) / per;
+                if (ns == last) continue;
+                last = ns;
+                const FlashPlan f{form, ns, per * 64, once != 0};
+                if (n > 1 && tn.flash_split < 2 && kSyncBytes + flash_bytes(s, f) > cap) break;
+                if (once && kSyncBytes + flash_bytes(s, f) > cap) break;
+                const int64_t w = grid * ns, slots = two ? 512 : 256;
+                double us = std::ceil((double)w / (double)slots);
+                const int64_t rem = w % 512;
+                us += per * tile *
+                      (two ? (double)(w / 512) * pair + (rem == 0 ? 0.0 : rem <= 256 ? 1.0 : pair)
+                           : us);
+                if (ns > 1) us += 5.0 + (double)ns * s.BH * s.Lq * s.D * 4.0 * 0.5e-6;
+                if (once) us += 4.0 + (double)s.nk * 4.0 / 4.5e6;
+                if (best.form == 0 || us < best_us) {
+                    best = f;
+                    best_us = us;
+                }
+            }
+        }
     }
-    if (n < 2) return f;
-    f.kchunk = (int)((chunks + n - 1) / n) * 64;
-    f.nsplit = (s.Lk + f.kchunk - 1) / f.kchunk;
-    if (f.nsplit < 2) return FlashSplit{};
-    f.bytes = (size_t)f.nsplit * s.BH * s.Lq * (s.D + 4) * 4;
-    return f;
+    return best;
 }
 
-// The most scratch any flash form's split of this shape takes.
-size_t flash_split_bound(const Shape& s) {
-    size_t b = 0;
-    for (int rows : {64, 128, 256}) b = std::max(b, flash_split(s, rows).bytes);
-    return b;
-}
-
-// K~ (fp16) and its tiles' units, behind the key splits' parts.
-size_t flash_kpre_bytes(const Shape& s) {
-    return 256 + round256((size_t)s.nk * 2) + round256((size_t)s.BH * ((s.Lk + 63) / 64) * 4);
-}
-
-// Whether a bf16 flash call that encodes K does so once, to fp16 in scratch,
-// instead of in every query block's workgroup as it loads each tile.  In the
-// kernel the encoding lies on every tile's critical path, about 0.9 us per
-// 64-key tile a workgroup walks; the pass costs a launch and its traffic.  So
-// it pays for long walks over few bytes: same box, (4,8,1107,1107,128) RoPE
-// 99 -> 72 us, (1,16,3000,3000,64) rotate-half 169 -> 85, (4,16,300,1500,128)
-// 71 -> 52, (1,8,4096,4096,128) 118 -> 97; not at (4,32,512,512,128) (39.4 ->
-// 42.7), (8,16,300,300,64) (17.8 -> 20.7) or under key splits of few tiles
-// ((1,4,200,4000,128) 29.7 -> 31.4).  fp32 calls, whose products take three
-// times as long beside the same encoding, gained 3-5 % at most and lost up to
-// 20 % (their copies are twice the bytes): they encode in the kernel.
-bool flash_kpre(int dtype, const Shape& s, const PePlan& plan, int rows, size_t cap) {
-    if (dtype != ATN_DTYPE_BF16 || plan.pek == atn::kPeNone || !plan.k.on || s.Lq <= 64 ||
-        tune().flash_form != 0 ||
-        kSyncBytes + flash_split_bound(s) + flash_kpre_bytes(s) > cap)
-        return false;
-    const FlashSplit f = flash_split(s, rows);
-    const int64_t wgs = s.BH * ((s.Lq + rows - 1) / rows) * f.nsplit;
-    const double tiles =
-        ((f.nsplit > 1 ? f.kchunk : s.Lk) + 63) / 64 * std::ceil((double)wgs / 256.0);
-    return tiles * 0.9 > 1.2 * (4.0 + (double)s.nk * 4.0 / 4.5e6);
+// The thread's last plan is kept (repeated calls of one shape).
+FlashPlan flash_plan(int dtype, const Shape& s, const PePlan& plan, size_t cap) {
+    const auto key = std::make_tuple(dtype, plan.pek, plan.k.on, s.BH, s.Lq, s.Lk, s.D, cap,
+                                     g_tune.load(std::memory_order_acquire));
+    thread_local std::remove_const_t<decltype(key)> last{};
+    thread_local FlashPlan kept;
+    if (kept.form == 0 || key != last) {
+        kept = flash_plan_uncached(dtype, s, plan, cap);
+        last = key;
+    }
+    return kept;
 }
 
 // Scratch bytes of the path a call of shape s takes: fused (when planned and
@@ -1023,15 +1028,13 @@ size_t path_need(int dtype, const Shape& s, const PePlan& plan, bool query_devic
     const GemmPlan gp = gemm_plan(dtype, s, plan);
     if (fp.ok && vec > 0) return fp.bytes;
     if (a16 > 0 && vec >= 0 && flash_ok(dtype, s, plan))  // the flash kernel: only its key splits' parts
-        return kSyncBytes + flash_split_bound(s) + (plan.kpre ? flash_kpre_bytes(s) : 0);
+        return kSyncBytes + flash_bytes(s, plan.flash);
     const TilePlan tp = tile_plan(dtype, s, plan, a16 > 0);
     const size_t split = tp.ok ? tp.bytes : kSyncBytes + stream_plan(s).bytes;
     if (vec < 0 || a16 < 0)
         return std::max({fp.ok ? fp.bytes : (size_t)0, gp.ok ? gp.bytes : (size_t)0, split,
-                         flash_ok(dtype, s, plan)
-                             ? kSyncBytes + flash_split_bound(s) +
-                                   (plan.kpre ? flash_kpre_bytes(s) : 0)
-                             : (size_t)0});
+                         flash_ok(dtype, s, plan) ? kSyncBytes + flash_bytes(s, plan.flash)
+                                                  : (size_t)0});
     if (gp.ok && a16 && !(plan.tiles && tp.ok)) return gp.bytes;
     return split;
 }
@@ -1102,11 +1105,9 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
     const TilePlan tp = use_fused || use_flash || use_gemm ? TilePlan{}
                                                            : tile_plan(dtype, s, plan, a16);
     const bool use_tile = tp.ok;
-    const int fform = use_flash ? flash_form(s, dev) : 0;
-    const FlashSplit fs = use_flash ? flash_split(s, flash_rows(fform, D)) : FlashSplit{};
     const size_t need =
         use_fused ? fd.bytes
-                  : (use_flash ? kSyncBytes + fs.bytes + (plan.kpre ? flash_kpre_bytes(s) : 0)
+                  : (use_flash ? kSyncBytes + flash_bytes(s, plan.flash)
                                : (use_gemm ? gp.bytes
                                            : (use_tile ? tp.bytes : kSyncBytes + sp.bytes)));
     void* ws = workspace;
@@ -1197,8 +1198,9 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
     if (use_flash) {
         const void* kt = K;
         const float* kunit = nullptr;
-        if (plan.kpre) {
-            char* w = reinterpret_cast<char*>(scratch) + round256(fs.bytes);
+        const FlashPlan& f = plan.flash;
+        if (f.kpre) {
+            char* w = reinterpret_cast<char*>(scratch) + flash_parts_bytes(s, f.nsplit);
             uint16_t* ke = reinterpret_cast<uint16_t*>(w);
             float* u = reinterpret_cast<float*>(w + round256((size_t)s.nk * 2));
             ATN_HIP(atn::launch_encode_key_tiles(plan.pek, static_cast<const uint16_t*>(K), ke, u,
@@ -1206,8 +1208,8 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
             kt = ke;
             kunit = u;
         }
-        ATN_HIP(atn::launch_flash(dtype, plan.pek, fform, Q, kt, V, out, (int)s.BH, Lq, Lk, D,
-                                  scale, plan.q, plan.k, fs.nsplit, fs.kchunk, scratch, kunit,
+        ATN_HIP(atn::launch_flash(dtype, plan.pek, f.form, Q, kt, V, out, (int)s.BH, Lq, Lk, D,
+                                  scale, plan.q, plan.k, f.nsplit, f.kchunk, scratch, kunit,
                                   stream));
         return ATN_OK;
     }
@@ -1301,8 +1303,7 @@ int attention_core(int dtype, const void* Q, const void* K, const void* V, void*
 
     const size_t cap = no_alloc ? atn::kNoAllocScratchBytes
                                 : (workspace != nullptr ? workspace_bytes : library_cap());
-    if (plan.pek != atn::kPeNone && flash_ok(dtype, s, plan))
-        plan.kpre = flash_kpre(dtype, s, plan, flash_rows(flash_form(s, dev), D), cap);
+    if (flash_ok(dtype, s, plan)) plan.flash = flash_plan(dtype, s, plan, cap);
     // chunk pointers keep the base alignment when a row is a multiple of 16
     // bytes; otherwise plan for the largest path
     const size_t va = dtype == ATN_DTYPE_F32 ? 16 : 8;
@@ -1687,11 +1688,7 @@ size_t atn_attention_workspace_bytes(int dtype, int batch, int heads, int len_q,
     PePlan plan;
     if (check_pe(pe, head_d, &plan) != ATN_OK) return 0;
     choose_tiles(dtype, s, plan);
-    // (the form, which decides for K's encoded copy, is the device's: with it
-    // wherever it fits)
-    plan.kpre = dtype == ATN_DTYPE_BF16 && plan.pek != atn::kPeNone && s.Lq > 64 &&
-                flash_ok(dtype, s, plan) &&
-                kSyncBytes + flash_split_bound(s) + flash_kpre_bytes(s) <= library_cap();
+    if (flash_ok(dtype, s, plan)) plan.flash = flash_plan(dtype, s, plan, library_cap());
     // the largest workspace of every plan the call could take, or, when that
     // exceeds the library's cap, of the chunks the call then runs in
     const size_t full = path_need(dtype, s, plan, false, -1, -1);

@@ -205,7 +205,7 @@ constexpr int flash_waves_per_simd() {
 // own (launch_encode_key_tiles), kunit the unit of each of its 64-key tiles;
 // the kernel then encodes its query rows only and stages K~ as it is, the
 // bits that it would have staged itself.  (The host's rule and what it
-// measured: flash_kpre in attn_api.cpp.)
+// measured: flash_plan in attn_api.cpp.)
 template <typename T, int DP, int PEK, int NW, int RW, bool KPRE>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     flash_waves_per_simd<T, DP, PEK, NW, RW>()))) void k_flash(const T* __restrict__ Qg,
@@ -825,27 +825,33 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
 // log2 of its weight sum = c0 m_s + g_s (c0 is the same for every split of
 // a row: the query's scale does not depend on the keys).  O = sum w_s O_s /
 // sum w_s with w_s = 2^((m_s - M) c0 + g_s), M = max m_s (differences of the
-// maxima first, so that huge logits stay exact).  One thread per 4 dims,
-// 4 rows per workgroup.
+// maxima first, so that huge logits stay exact).  One thread per 4 dims, the
+// groups of all rows numbered through (every lane works whatever head_d is),
+// the loads of up to 4 splits at once: pure traffic, (1,8,4096,4096,128) with
+// two splits (42 MB) 11.6 -> 10.0 us.
 template <typename T>
 __global__ __launch_bounds__(256) void k_flash_combine(const float* __restrict__ part,
                                                        const float4* __restrict__ stats,
                                                        T* __restrict__ Og, int Lq, int D,
-                                                       int nsplit, int rows) {
-    const int t = threadIdx.x;
-    const int row = blockIdx.x * 4 + (t >> 6), d = 4 * (t & 63);
-    if (row >= rows || d >= D) return;
-    const int bh = row / Lq, q = row - bh * Lq;
-    const size_t base = (size_t)bh * nsplit * Lq + q;
+                                                       int nsplit, long groups) {
+    const unsigned vpr = (unsigned)D >> 2;
+    const long g0 = (long)blockIdx.x * 256, row0 = g0 / vpr;
+    const unsigned c = (unsigned)(g0 - row0 * vpr) + threadIdx.x, dr = c / vpr;
+    if (g0 + threadIdx.x >= groups) return;
+    const long row = row0 + dr, bh = row / Lq;
+    const int d = 4 * (int)(c - dr * vpr);
+    const size_t base = (size_t)bh * nsplit * Lq + (size_t)(row - bh * Lq);
     float M = -INFINITY;
+#pragma unroll 4
     for (int s = 0; s < nsplit; ++s) M = fmaxf(M, stats[base + (size_t)s * Lq].x);
     float wsum = 0.f;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
     for (int s = 0; s < nsplit; ++s) {
         const size_t pr = base + (size_t)s * Lq;
         const float4 st = stats[pr];
-        const float w = __builtin_amdgcn_exp2f(fmaf(st.x - M, st.y, st.z));
         const float4 v = *reinterpret_cast<const float4*>(part + pr * D + d);
+        const float w = __builtin_amdgcn_exp2f(fmaf(st.x - M, st.y, st.z));
         wsum += w;
         acc.x = fmaf(w, v.x, acc.x);
         acc.y = fmaf(w, v.y, acc.y);
@@ -855,6 +861,72 @@ __global__ __launch_bounds__(256) void k_flash_combine(const float* __restrict__
     const float inv = 1.f / wsum;
     Elem<T>::st4(Og + (size_t)row * D, d,
                  make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv));
+}
+
+// The same for few rows of many splits (decoding), where a thread per group
+// would walk the splits one latency after another on a handful of CUs: each of
+// a workgroup's 4 waves takes every fourth split of 64 groups, up to 8 loads
+// at once, and the waves' sums meet in LDS, weighed by their own maxima.
+template <typename T>
+__global__ __launch_bounds__(256) void k_flash_combine_few(const float* __restrict__ part,
+                                                           const float4* __restrict__ stats,
+                                                           T* __restrict__ Og, int Lq, int D,
+                                                           int nsplit, long groups) {
+    __shared__ float4 sum[4][64];
+    __shared__ float2 mw[4][64];  // a wave's maximum and weight sum
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const unsigned vpr = (unsigned)D >> 2;
+    const long g = min((long)blockIdx.x * 64 + lane, groups - 1);
+    const long row = g / vpr, bh = row / Lq;
+    const int d = 4 * (int)(g - row * vpr);
+    const size_t base = (size_t)bh * nsplit * Lq + (size_t)(row - bh * Lq);
+    float c0 = 0.f, m = -INFINITY, wsum = 0.f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    // nsplit <= 32: at most 8 per wave
+    float4 st[8], v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int s = wave + 4 * i;
+        const size_t pr = base + (size_t)(s < nsplit ? s : 0) * Lq;
+        st[i] = stats[pr];
+        v[i] = *reinterpret_cast<const float4*>(part + pr * D + d);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if (wave + 4 * i < nsplit) m = fmaxf(m, st[i].x);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        if (wave + 4 * i >= nsplit) continue;
+        c0 = st[i].y;
+        const float w = __builtin_amdgcn_exp2f(fmaf(st[i].x - m, c0, st[i].z));
+        wsum += w;
+        acc.x = fmaf(w, v[i].x, acc.x);
+        acc.y = fmaf(w, v[i].y, acc.y);
+        acc.z = fmaf(w, v[i].z, acc.z);
+        acc.w = fmaf(w, v[i].w, acc.w);
+    }
+    sum[wave][lane] = acc;
+    mw[wave][lane] = make_float2(m, wsum);
+    __syncthreads();
+    if (wave != 0 || (long)blockIdx.x * 64 + lane >= groups) return;
+    float M = m;  // (wave 0 always has a split; a wave without one weighs 2^-inf)
+#pragma unroll
+    for (int w = 1; w < 4; ++w) M = fmaxf(M, mw[w][lane].x);
+    float ws = 0.f;
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        if (w >= nsplit) continue;
+        const float f = __builtin_amdgcn_exp2f((mw[w][lane].x - M) * c0);
+        const float4 x = sum[w][lane];
+        ws = fmaf(f, mw[w][lane].y, ws);
+        o.x = fmaf(f, x.x, o.x);
+        o.y = fmaf(f, x.y, o.y);
+        o.z = fmaf(f, x.z, o.z);
+        o.w = fmaf(f, x.w, o.w);
+    }
+    const float inv = 1.f / ws;
+    Elem<T>::st4(Og + (size_t)row * D, d, make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv));
 }
 
 // the arguments of one flash call (pointers typed by the launch)
@@ -889,9 +961,15 @@ hipError_t launch_t(const FlashArgs& a, hipStream_t st) {
                        a.stats, a.kunit);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.nsplit == 1) return e;
-    const int rows = a.BH * a.Lq;
-    hipLaunchKernelGGL((k_flash_combine<T>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st,
-                       a.part, a.stats, static_cast<T*>(a.O), a.Lq, a.D, a.nsplit, rows);
+    const long groups = (long)a.BH * a.Lq * (a.D / 4);
+    if (groups < (1 << 15) && a.nsplit >= 4 && a.nsplit <= 32) {
+        hipLaunchKernelGGL((k_flash_combine_few<T>), dim3((unsigned)((groups + 63) / 64)),
+                           dim3(256), 0, st, a.part, a.stats, static_cast<T*>(a.O), a.Lq, a.D,
+                           a.nsplit, groups);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL((k_flash_combine<T>), dim3((unsigned)((groups + 255) / 256)), dim3(256), 0,
+                       st, a.part, a.stats, static_cast<T*>(a.O), a.Lq, a.D, a.nsplit, groups);
     return hipGetLastError();
 }
 

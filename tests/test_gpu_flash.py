@@ -652,17 +652,19 @@ def test_flash_split_graph_replays(am, dev):
 
 
 @pytest.mark.parametrize("pe", ["rope", "half", "rope_part", "sin"])
-@pytest.mark.parametrize("shape,form,scale", [
-    ((4, 8, 1107, 1107, 96), "8x16", 1.0),        # ragged rows, head_d padded
-    ((4, 16, 300, 1500, 128), "8x16", 1.0),
-    ((8, 32, 512, 520, 64), "8x32", 1.0),
-    ((1, 4, 4200, 4160, 40), "8x32", 1.0),        # key splits
-    ((1, 16, 1100, 1100, 100), "8x16", 2.0 ** 30),  # K tiles scaled by a power of two
-    ((1, 16, 1100, 1100, 100), "8x16", 2.0 ** -20),
+@pytest.mark.parametrize("shape,scale", [
+    ((4, 8, 1107, 1107, 96), 1.0),        # ragged rows, head_d padded
+    ((4, 16, 300, 1500, 128), 1.0),
+    ((8, 32, 512, 520, 64), 1.0),
+    ((1, 4, 4200, 4160, 40), 1.0),        # key splits
+    ((1, 16, 1100, 1100, 100), 2.0 ** 30),  # K tiles scaled by a power of two
+    ((1, 16, 1100, 1100, 100), 2.0 ** -20),
 ], ids=str)
-def test_flash_keys_encoded_once(am, dev, tuner, shape, form, scale, pe):
-    """bf16 calls that encode K by a pass of its own, bit for bit as with K
-    encoded in the kernel (a forced form), and sampled rows of the oracle."""
+def test_flash_keys_encoded_once(am, dev, tuner, shape, scale, pe):
+    """bf16 calls that encode K by a pass of its own: bit for bit the result of
+    one of the forms with K encoded in the kernel (a forced form and split
+    count: the library's own choice of the two is not forced), and sampled rows
+    of the oracle."""
     import hip_rt
     B, Hh, Lq, Lk, D = shape
     print(f"[case] keys encoded once {shape} {pe} x{scale}", flush=True)
@@ -674,13 +676,17 @@ def test_flash_keys_encoded_once(am, dev, tuner, shape, form, scale, pe):
         K = K * np.float32(scale)
         Q = Q * np.float32(1 / scale)
         k, q = H.upload(K, "bf16"), H.upload(Q, "bf16")
-    out, forced = H.empty(Q.shape, "bf16"), H.empty(Q.shape, "bf16")
+    out = H.empty(Q.shape, "bf16")
     am.attention_ex(q, k, v, out, pe=desc)
     hip_rt.synchronize()
-    tuner.set(flash_form=form)
-    am.attention_ex(q, k, v, forced, pe=desc)
-    hip_rt.synchronize()
-    assert np.array_equal(out.bits(), forced.bits())
+    same, forced = [], H.empty(Q.shape, "bf16")
+    for form in ("8x16", "8x32"):
+        for split in range(1, 9):
+            tuner.set(flash_form=form, flash_split=split)
+            am.attention_ex(q, k, v, forced, pe=desc)
+            hip_rt.synchronize()
+            same.append(np.array_equal(out.bits(), forced.bits()))
+    assert any(same)
     if scale == 1.0:
         rot = D if pe != "rope_part" else D // 2 // 4 * 4
         r0, r1 = (B * Hh - 1) * Lq + Lq - 20, B * Hh * Lq  # the last head's last rows
@@ -693,3 +699,20 @@ def test_flash_keys_encoded_once(am, dev, tuner, shape, form, scale, pe):
                                         pairing="interleaved" if pe == "rope" else "half")
         n, nrel, mabs = H.check_bf16(out.numpy().reshape(-1, D)[r0:r1], ref.reshape(-1, D)[r0:r1])
         assert n == 0, (nrel, mabs)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("parts", [3, 4, 5, 8, 9, 31, 32])
+@pytest.mark.parametrize("Lq", [3, 700], ids=str)
+def test_flash_merge_forms(am, dev, tuner, dt, parts, Lq):
+    """Both merge kernels (few rows of 4 to 32 parts; the rest), with parts
+    that some of a workgroup's waves have none of."""
+    B, Hh, Lk, D = 1, 3, 2100, 68
+    print(f"[case] merge {dt} {Lq} rows, {parts} parts", flush=True)
+    Q, K, V = H.rng_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), seed=620 + parts)
+    tuner.set(flash_split=parts)
+    ref = oracle.attention(*((Q, K, V) if dt == "f32" else
+                             [oracle.bf16_bits_to_f32(oracle.f32_to_bf16_bits(x)) for x in (Q, K, V)]),
+                           nthreads=16)
+    n, err = _check(dt, _call(am, dt, Q, K, V), ref)
+    assert n == 0, err
