@@ -768,22 +768,21 @@ struct TilePlan {
 };
 
 // Estimated time (us) of a tile kernel: wgs workgroups of `stages` stages on
-// 256 CUs.  Measured over 26 fp32 and 24 bf16 shapes with every tile and 8
-// D-chunk counts (B H 2-64, sides 16-4096, D 264-8192): a CU spends
-// `each` us per stage of every workgroup it holds, `alone` with one on few
-// CUs, `busy` more with one on each.  fp32 (and Q K^T of encoded bf16), 32
-// deep: 64 x 64 0.40 alone, 0.36 each; 128 x 128 0.80 (+ 0.45), 1.12 each.
-// bf16 Q K^T, 64 deep: 0.31, 0.31; 0.72 (+ 0.15), 0.85.  bf16 P V, 32 keys:
-// 0.36, 0.28; 0.65 (+ 0.10), 0.72.  So 128 x 128 is the faster wherever its
-// grid fills the chip, 64 x 64 below.
+// 256 CUs, w workgroups a CU.  A stage takes c0 + c1 w with at most one
+// workgroup on a CU, at least c2 from the first CU that holds two, c3 w beyond
+// (measured over 20 fp32 and 11 bf16 shapes, every tile and 5 D-chunk counts:
+// B H 2-32, sides 64-4096, D 264-6096, launch and score writes taken off).
+// 128 x 128 does four times the work of 64 x 64 in two to three times the
+// time, so it is the faster wherever its grid fills the chip.  Stages: fp32
+// (and Q K^T of encoded bf16) 32 deep, bf16 Q K^T 64 deep, bf16 P V 32 keys.
 enum { kTileF32 = 0, kTileQkBf16 = 1, kTilePvBf16 = 2 };
 double tile_us(int kind, int tile, int64_t wgs, int64_t stages) {
-    static const double c[3][2][3] = {{{0.40, 0.00, 0.36}, {0.80, 0.45, 1.12}},
-                                      {{0.31, 0.00, 0.31}, {0.72, 0.15, 0.85}},
-                                      {{0.36, 0.00, 0.28}, {0.65, 0.10, 0.72}}};
+    static const double c[3][2][4] = {{{0.36, 0.09, 0.45, 0.28}, {0.58, 0.36, 1.50, 0.75}},
+                                      {{0.30, 0.08, 0.40, 0.23}, {0.58, 0.17, 1.30, 0.60}},
+                                      {{0.30, 0.10, 0.42, 0.26}, {0.45, 0.42, 1.50, 0.68}}};
     const double* k = c[kind][tile == 128];
     const double w = (double)wgs / 256.0;
-    return std::max(k[0] + k[1] * std::min(w, 1.0), k[2] * w) * (double)stages;
+    return (w <= 1.0 ? k[0] + k[1] * w : std::max(k[2], k[3] * w)) * (double)stages;
 }
 
 TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
@@ -861,8 +860,8 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
 // step of Q K^T, 2.2 per 64 keys of P V and 15 us besides, per round of 256
 // workgroups (wall times of 29 shapes; K's encoding inside the GEMM makes a
 // step 2.2 us, an encoding pass costs its traffic).  The tiles cut D as well
-// and win there: (1,2,68,68,624) 37.3 -> 11.6 us, (2,4,82,82,2392) 72.5 ->
-// 15.8, (1,4,512,512,2048) 62.5 -> 31, (1,8,64,4096,2048) 195 -> 91; from
+// and win there: (1,2,68,68,624) 37.3 -> 10.6 us, (2,4,82,82,2392) 72.5 ->
+// 16.3, (1,4,512,512,2048) 62.5 -> 31, (1,8,64,4096,2048) 195 -> 91; from
 // about 128 GEMM tiles on the GEMMs lead ((4,8,444,444,1008) 66 against 93
 // us, (4,16,508,508,1888) 201 against 315).
 void choose_tiles(int dtype, const Shape& s, PePlan& plan) {

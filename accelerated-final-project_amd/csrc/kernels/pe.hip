@@ -386,8 +386,10 @@ hipError_t launch_encode_key_tiles(int pek, const uint16_t* K, uint16_t* out, fl
 }
 
 // Rows of D bf16 into rows of Dp (a multiple of 8), zeros past D: up to three
-// tensors, 8 elements of a row per thread.  Source rows start anywhere, so
-// they are read two bytes at a time; the copies' tiles are then read 16.
+// tensors, 8 elements of a row per thread: 16 bytes at whatever alignment the
+// source row has (the device runs in unaligned-access mode).  Pure traffic:
+// (2,8,400,400,1500), Q, K and V (58 MB in, 58 out), 36 us with two-byte
+// loads, 19 so.
 namespace {
 struct PadArgs {
     const uint16_t* in[3];
@@ -398,18 +400,23 @@ struct PadArgs {
 };
 __global__ __launch_bounds__(256) void k_pad_rows(PadArgs a) {
     const int s = blockIdx.x >= a.first[2] ? 2 : (blockIdx.x >= a.first[1] ? 1 : 0);
-    const long u = (long)(blockIdx.x - a.first[s]) * 256 + threadIdx.x;
-    if (u >= a.units[s]) return;
-    const int per = a.Dp >> 3;
-    const long row = u / per;
-    const int d = (int)(u - row * per) * 8;
-    const uint16_t* x = a.in[s] + (size_t)row * a.D;
+    const unsigned per = (unsigned)a.Dp >> 3;
+    const long u0 = (long)(blockIdx.x - a.first[s]) * 256, row0 = u0 / per;
+    if (u0 + threadIdx.x >= a.units[s]) return;
+    const unsigned k = (unsigned)(u0 - row0 * per) + threadIdx.x, dr = k / per;
+    const long row = row0 + dr;
+    const int d = (int)(k - dr * per) * 8;
+    const uint16_t* x = a.in[s] + (size_t)row * a.D + d;
     uint32_t w[4];
+    if (d + 8 <= a.D) {
+        __builtin_memcpy(w, x, 16);
+    } else {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const uint32_t lo = d + 2 * c < a.D ? x[d + 2 * c] : 0u;
-        const uint32_t hi = d + 2 * c + 1 < a.D ? x[d + 2 * c + 1] : 0u;
-        w[c] = lo | (hi << 16);
+        for (int c = 0; c < 4; ++c) {
+            const uint32_t lo = d + 2 * c < a.D ? x[2 * c] : 0u;
+            const uint32_t hi = d + 2 * c + 1 < a.D ? x[2 * c + 1] : 0u;
+            w[c] = lo | (hi << 16);
+        }
     }
     *reinterpret_cast<uint4*>(a.out[s] + (size_t)row * a.Dp + d) = make_uint4(w[0], w[1], w[2], w[3]);
 }

@@ -21,19 +21,27 @@
 // workgroup then computes the tile again, every stage scaled by powers of two
 // from its largest finite magnitudes.
 //
-// Tiles of 128 x 128 (4 waves of 64 x 64) or 64 x 64 (4 waves of 32 x 32) on
-// 32 x 32 x 16 MFMA.  LDS rows of 32 elements (64 bytes) per part, their
+// Tiles of 128 x 128 or 64 x 64 (4 waves) on 32 x 32 x 16 MFMA.  A grid of at
+// most one 128 x 128 workgroup a CU runs it as 8 waves of 64 x 32, two to a
+// SIMD: half the sums per wave leave registers for loads two stages ahead,
+// and one wave's fp16 split runs beside the other's MFMAs.  (1,4,512,512,2048)
+// Q K^T 22.8 -> 20.9 us, P V 22.4 -> 20.3; (2,4,1024,1024,512) P V 45.7 ->
+// 36.7.  With two workgroups on a CU 4 waves of 64 x 64 are the better: they
+// read a third fewer fragments per product ((2,2,504,1387,4424) Q K^T 124.7
+// us against 136.9).  LDS rows of 32 elements (64 bytes) per part, their
 // 16-byte chunks permuted by tile_swz(row) so that fragment reads hit
 // distinct banks unpadded (SQ_LDS_BANK_CONFLICT 0): 64 KiB for both stages of
 // a 128 x 128 tile, two workgroups per CU.  Rows of S and P are padded to
-// whole vectors, so ragged key counts store and load 16 bytes as well.
+// whole vectors, so ragged key counts store and load 16 bytes as well; rows
+// of O whose D is odd are stored 4 elements at a time at any alignment
+// ((2,8,400,400,1501) P V of bf16 56 -> 33 us).
 //
 // fp32 calls, before (stream16.hip's kernels) -> these: (1,4,512,512,2048)
-// 57.4 -> 48.8 us, (2,2,422,422,2360) 81 -> 49, (2,2,128,1415,1520) 98 -> 40,
+// 57.9 -> 45.9 us, (2,2,422,422,2360) 81 -> 49, (2,2,128,1415,1520) 98 -> 40,
 // (1,2,517,517,1272) 58 -> 31; at (1,4,1453,1453,1024) Q K^T runs at 215
 // TFLOP/s of fp32 work (650 of fp16 products).  bf16: (1,2,273,757,3081)
-// 184 -> 48 us (before: fp32 MFMA on two-byte loads), and the GEMM path's
-// small grids ((1,2,68,68,624) 37.3 -> 11.5 us, see the host's rule).
+// 184 -> 35 us (before: fp32 MFMA on two-byte loads), and the GEMM path's
+// small grids ((1,2,68,68,624) 37.3 -> 10.6 us, see the host's rule).
 #include <algorithm>
 #include <type_traits>
 
@@ -104,17 +112,23 @@ __device__ __forceinline__ unsigned xcd_tile(unsigned id, unsigned n) {
 }
 
 // Workgroup maximum of two per-thread values; every thread must call it.
+template <int NW>
 __device__ __forceinline__ void wg_max2(float& a, float& b, float* sh) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     a = wave_max(a);
     b = wave_max(b);
     if (lane == 0) {
         sh[wave] = a;
-        sh[4 + wave] = b;
+        sh[NW + wave] = b;
     }
     __syncthreads();
-    a = fmaxf(fmaxf(sh[0], sh[1]), fmaxf(sh[2], sh[3]));
-    b = fmaxf(fmaxf(sh[4], sh[5]), fmaxf(sh[6], sh[7]));
+    a = sh[0];
+    b = sh[NW];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) {
+        a = fmaxf(a, sh[w]);
+        b = fmaxf(b, sh[NW + w]);
+    }
 }
 
 __device__ __forceinline__ float max4abs(float m, const uint4& u) {
@@ -123,11 +137,15 @@ __device__ __forceinline__ float max4abs(float m, const uint4& u) {
 }
 
 // Whether any thread of the workgroup saw a value outside fp16's range
+template <int NW>
 __device__ __forceinline__ bool wg_over(float big, int* flag) {
     const bool over = __ballot(!(big < kF16Range)) != 0;
     if ((threadIdx.x & 63) == 0) flag[threadIdx.x >> 6] = over;
     __syncthreads();
-    return (flag[0] | flag[1] | flag[2] | flag[3]) != 0;
+    int any = flag[0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) any |= flag[w];
+    return any != 0;
 }
 
 // Partial scores S_split[bh][i][j] = sum over the chunk's dims of q_id k_jd
@@ -136,17 +154,18 @@ __device__ __forceinline__ bool wg_over(float big, int* flag) {
 // (rows of S are ldS, a multiple of 4, apart).  RAG: head_d is no multiple of
 // 4 (fp32; rows then start at 4-byte boundaries and the last group of a row
 // is read element by element).
-template <int KIND, int TL, bool RAG>
-__global__ __launch_bounds__(256, 2) void k_qk_tile(QkTileArgs a) {
+template <int KIND, int TL, int NW, bool RAG>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs a) {
     using G = Tile<KIND>;
-    constexpr int ROUNDS = TL / 32;     // loader rounds of 32 rows per operand
-    constexpr int NI = TL / 64;         // 32 x 32 MFMA tiles per wave and side
+    constexpr int LROWS = 8 * NW, ROUNDS = TL / LROWS;  // loader: rows per round, rounds
+    constexpr int WK = NW / 2;                          // waves along the keys (2 along the queries)
+    constexpr int NK = TL / WK / 32, NQ = TL / 64;      // 32 x 32 MFMA tiles per wave
     constexpr int PART = TL * 32;       // elements of one part of one operand
-    constexpr int AHEAD = TL == 64 ? 2 : 1;  // stages a load is issued before its LDS write
+    constexpr int AHEAD = TL == 64 || NW == 8 ? 2 : 1;  // stages a load is issued before its LDS write
     __shared__ __align__(16) uint16_t sq[2][2 * PART];  // [stage][part][row][32]
     __shared__ __align__(16) uint16_t sk[2][2 * PART];
-    __shared__ float slot[8];
-    __shared__ int flag[4];
+    __shared__ float slot[2 * NW];
+    __shared__ int flag[NW];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -167,7 +186,7 @@ __global__ __launch_bounds__(256, 2) void k_qk_tile(QkTileArgs a) {
     unsigned qoff[ROUNDS], koff[ROUNDS];  // (a row outside the tensor stays past its end)
 #pragma unroll
     for (int i = 0; i < ROUNDS; ++i) {
-        const int qi = q0 + lrow + 32 * i, kj = k0 + lrow + 32 * i;
+        const int qi = q0 + lrow + LROWS * i, kj = k0 + lrow + LROWS * i;
         qoff[i] = qi < a.Lq ? (unsigned)(qi * a.D * G::ES + lc * 16) : (unsigned)kBufOob;
         koff[i] = kj < a.Lk ? (unsigned)(kj * a.D * G::ES + lc * 16) : (unsigned)kBufOob;
     }
@@ -209,7 +228,7 @@ __global__ __launch_bounds__(256, 2) void k_qk_tile(QkTileArgs a) {
     // LDS place of this thread's 16 bytes: fp32 half a chunk of both parts,
     // bf16 a chunk of one part
     auto place = [&](int i) {
-        const int row = lrow + 32 * i;
+        const int row = lrow + LROWS * i;
         return KIND == kKindF32 ? tile_at(row, lc >> 1) + 4 * (lc & 1)
                                 : (lc >> 2) * PART + tile_at(row, lc & 3);
     };
@@ -233,14 +252,14 @@ __global__ __launch_bounds__(256, 2) void k_qk_tile(QkTileArgs a) {
         }
     };
 
-    const int wq = (wave & 1) * (TL / 2), wk = (wave >> 1) * (TL / 2);  // wave's queries, keys
+    const int wq = (wave & 1) * (TL / 2), wk = (wave >> 1) * (TL / WK);  // wave's queries, keys
     const int fr = lane & 31, fc = lane >> 5;
-    v16f acc[NI][NI], sum[NI][NI];  // [key tile][query tile]
+    v16f acc[NK][NQ], sum[NK][NQ];  // [key tile][query tile]
     auto each = [&](auto f) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
+        for (int i = 0; i < NK; ++i)
 #pragma unroll
-            for (int j = 0; j < NI; ++j) f(acc[i][j], sum[i][j]);
+            for (int j = 0; j < NQ; ++j) f(acc[i][j], sum[i][j]);
     };
     auto zero = [&]() { each([](v16f&, v16f& y) { y = v16f{}; }); };
     // the pair of stages just summed, into the tile's sum
@@ -248,20 +267,22 @@ __global__ __launch_bounds__(256, 2) void k_qk_tile(QkTileArgs a) {
     auto compute = [&](const uint16_t* q, const uint16_t* k, auto fresh) {
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            uint4 ka[2][NI], qa[2][NI];
+            uint4 ka[2][NK], qa[2][NQ];
 #pragma unroll
-            for (int p = 0; p < 2; ++p)
+            for (int p = 0; p < 2; ++p) {
 #pragma unroll
-                for (int i = 0; i < NI; ++i) {
+                for (int i = 0; i < NK; ++i)
                     ka[p][i] = *reinterpret_cast<const uint4*>(
                         k + p * PART + tile_at(wk + 32 * i + fr, 2 * ks + fc));
-                    qa[p][i] = *reinterpret_cast<const uint4*>(
-                        q + p * PART + tile_at(wq + 32 * i + fr, 2 * ks + fc));
-                }
 #pragma unroll
-            for (int i = 0; i < NI; ++i)
+                for (int j = 0; j < NQ; ++j)
+                    qa[p][j] = *reinterpret_cast<const uint4*>(
+                        q + p * PART + tile_at(wq + 32 * j + fr, 2 * ks + fc));
+            }
 #pragma unroll
-                for (int j = 0; j < NI; ++j) {
+            for (int i = 0; i < NK; ++i)
+#pragma unroll
+                for (int j = 0; j < NQ; ++j) {
                     v16f c = decltype(fresh)::value && ks == 0 ? v16f{} : acc[i][j];
                     if constexpr (KIND == kKindF32) {
                         c = mfma32<KIND>(ka[1][i], qa[0][j], c);
@@ -301,7 +322,7 @@ __global__ __launch_bounds__(256, 2) void k_qk_tile(QkTileArgs a) {
         flush();
     }
     if constexpr (KIND == kKindF32) {
-        if (wg_over(big, flag)) {
+        if (wg_over<NW>(big, flag)) {
             zero();
             for (int d0 = dbeg; d0 < dend; d0 += G::DEPTH) {
                 issue(r0, d0);
@@ -312,7 +333,7 @@ __global__ __launch_bounds__(256, 2) void k_qk_tile(QkTileArgs a) {
                     mk = max_finite4(mk, as_f4(r0.k[i]));
                 }
                 __syncthreads();  // the last stage's reads (and the slots') are done
-                wg_max2(mq, mk, slot);
+                wg_max2<NW>(mq, mk, slot);
                 const float s1 = pow2_scale(mq), s2 = pow2_scale(mk);
 #pragma unroll
                 for (int i = 0; i < ROUNDS; ++i) {
@@ -335,12 +356,12 @@ __global__ __launch_bounds__(256, 2) void k_qk_tile(QkTileArgs a) {
 
     // register r of a tile: key 8 (r / 4) + 4 (lane / 32) + r % 4 of query lane % 32
 #pragma unroll
-    for (int j = 0; j < NI; ++j) {
+    for (int j = 0; j < NQ; ++j) {
         const int qi = q0 + wq + 32 * j + fr;
         if (qi >= a.Lq) continue;
         float* srow = a.S + (((size_t)split * a.BH + bh) * a.Lq + qi) * a.ldS;
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
+        for (int i = 0; i < NK; ++i)
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
                 const int kj = k0 + wk + 32 * i + 8 * b + 4 * fc;
@@ -498,24 +519,35 @@ __global__ __launch_bounds__(256) void k_softmax_long(float* S, uint16_t* __rest
     }
 }
 
+// 4 consecutive elements to an address of element alignment only: one store
+// (the device runs in unaligned-access mode)
+__device__ __forceinline__ void st4_any(float* p, float4 v) { __builtin_memcpy(p, &v, 16); }
+__device__ __forceinline__ void st4_any(uint16_t* p, float4 v) {
+    uint2 w;
+    w.x = (uint32_t)f32_to_bf16_bits(v.x) | ((uint32_t)f32_to_bf16_bits(v.y) << 16);
+    w.y = (uint32_t)f32_to_bf16_bits(v.z) | ((uint32_t)f32_to_bf16_bits(v.w) << 16);
+    __builtin_memcpy(p, &w, 8);
+}
+
 // O[bh][i][d] = sum_j P_ij V_jd for one tile of TL queries x TL dims, 32 keys
 // a stage.  Wave w computes O^T for its TL/2 dims x TL/2 queries: a lane
 // holds 4 consecutive dims of one query.  P rows go to LDS as they are; V
 // stays [key][dim] there and reaches the MFMA by the transposing LDS read
 // (rows of TL + 32 elements: the four rows of a read on distinct banks).
-template <int KIND, int TL, bool RAG>
-__global__ __launch_bounds__(256, 2) void k_pv_tile(PvTileArgs a) {
+template <int KIND, int TL, int NW, bool RAG>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_pv_tile(PvTileArgs a) {
     using G = Tile<KIND>;
-    constexpr int NI = TL / 64, PART = TL * 32;
-    constexpr int AHEAD = TL == 64 ? 2 : 1;
+    constexpr int PART = TL * 32, WD = NW / 2;          // waves along the dims (2 along the queries)
+    constexpr int ND = TL / WD / 32, NQ = TL / 64;      // 32 x 32 MFMA tiles per wave
+    constexpr int AHEAD = TL == 64 || NW == 8 ? 2 : 1;
     constexpr int VSTR = TL + 32, VPARTS = KIND == kKindF32 ? 2 : 1, VPART = 32 * VSTR;
     constexpr int VL = TL / G::PER16;             // V loader: lanes per row
-    constexpr int VROWS = 256 / VL, VROUNDS = 32 / VROWS > 0 ? 32 / VROWS : 1;
+    constexpr int VROWS = 64 * NW / VL, VROUNDS = 32 / VROWS > 0 ? 32 / VROWS : 1;
     static_assert(VROWS <= 32, "a round of V rows within a stage");
     __shared__ __align__(16) uint16_t sp[2][2 * PART];
     __shared__ __align__(16) uint16_t sv[2][VPARTS * VPART];
-    __shared__ float slot[8];
-    __shared__ int flag[4];
+    __shared__ float slot[2 * NW];
+    __shared__ int flag[NW];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -529,13 +561,13 @@ __global__ __launch_bounds__(256, 2) void k_pv_tile(PvTileArgs a) {
     const char* pl = reinterpret_cast<const char*>(a.pl + (size_t)bh * a.Lq * a.ldP);
     const int pbytes = a.Lq * a.ldP * 2, vbytes = a.Lk * a.D * G::ES;
     const char* Vh = static_cast<const char*>(a.V) + (size_t)bh * a.Lk * a.D * G::ES;
-    // P loader: row lrow + 64 i, chunk lc of both parts
-    constexpr int PR = TL / 64;
+    // P loader: row lrow + PROWS i, chunk lc of both parts
+    constexpr int PROWS = 16 * NW, PR = TL / PROWS;
     const int lrow = tid >> 2, lc = tid & 3;
     unsigned poff[PR];
 #pragma unroll
     for (int i = 0; i < PR; ++i) {
-        const int row = q0 + lrow + 64 * i;
+        const int row = q0 + lrow + PROWS * i;
         poff[i] = row < a.Lq ? (unsigned)((row * a.ldP + 8 * lc) * 2) : (unsigned)kBufOob;
     }
     const int vrow = tid / VL, vcol = (tid % VL) * G::PER16;
@@ -579,7 +611,7 @@ const int psh = min(kk, a.ldP) * 2;
     auto store_p = [&](const Regs& r, uint16_t* p) {
 #pragma unroll
         for (int i = 0; i < PR; ++i) {
-            const int o = tile_at(lrow + 64 * i, lc);
+            const int o = tile_at(lrow + PROWS * i, lc);
             *reinterpret_cast<uint4*>(p + o) = r.h[i];
             *reinterpret_cast<uint4*>(p + PART + o) = r.l[i];
         }
@@ -601,16 +633,16 @@ const int psh = min(kk, a.ldP) * 2;
         }
     };
 
-    const int wq = (wave & 1) * (TL / 2), wd = (wave >> 1) * (TL / 2);
+    const int wq = (wave & 1) * (TL / 2), wd = (wave >> 1) * (TL / WD);
     const int fr = lane & 31, fc = lane >> 5;
     // V^T fragment: dims 16 (lane / 16 % 2) + lane % 16, keys 8 (lane / 32) + 0..7
     const int va = (8 * fc + ((lane & 15) >> 2)) * VSTR + wd + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-    v16f acc[NI][NI], sum[NI][NI];  // [dim tile][query tile]
+    v16f acc[ND][NQ], sum[ND][NQ];  // [dim tile][query tile]
     auto each = [&](auto f) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
+        for (int i = 0; i < ND; ++i)
 #pragma unroll
-            for (int j = 0; j < NI; ++j) f(acc[i][j], sum[i][j]);
+            for (int j = 0; j < NQ; ++j) f(acc[i][j], sum[i][j]);
     };
     auto zero = [&]() { each([](v16f&, v16f& y) { y = v16f{}; }); };
     // the pair of stages just summed, into the tile's sum
@@ -618,9 +650,9 @@ const int psh = min(kk, a.ldP) * 2;
     auto compute = [&](const uint16_t* p, const uint16_t* v, auto fresh) {
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            uint4 pa[2][NI], vv[VPARTS][NI];
+            uint4 pa[2][NQ], vv[VPARTS][ND];
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
+            for (int i = 0; i < ND; ++i)
 #pragma unroll
                 for (int w = 0; w < VPARTS; ++w) {
                     const uint16_t* at = v + w * VPART + va + 16 * ks * VSTR + 32 * i;
@@ -628,14 +660,15 @@ const int psh = min(kk, a.ldP) * 2;
                     vv[w][i] = make_uint4(x.x, x.y, y.x, y.y);
                 }
 #pragma unroll
+            for (int j = 0; j < NQ; ++j)
+#pragma unroll
                 for (int w = 0; w < 2; ++w)
-                    pa[w][i] = *reinterpret_cast<const uint4*>(
-                        p + w * PART + tile_at(wq + 32 * i + fr, 2 * ks + fc));
-            }
+                    pa[w][j] = *reinterpret_cast<const uint4*>(
+                        p + w * PART + tile_at(wq + 32 * j + fr, 2 * ks + fc));
 #pragma unroll
-            for (int i = 0; i < NI; ++i)
+            for (int i = 0; i < ND; ++i)
 #pragma unroll
-                for (int j = 0; j < NI; ++j) {
+                for (int j = 0; j < NQ; ++j) {
                     v16f c = decltype(fresh)::value && ks == 0 ? v16f{} : acc[i][j];
                     if constexpr (KIND == kKindF32)
                         c = mfma32<KIND>(vv[VPARTS - 1][i], pa[0][j], c);
@@ -671,7 +704,7 @@ const int psh = min(kk, a.ldP) * 2;
         flush();
     }
     if constexpr (KIND == kKindF32) {
-        if (wg_over(big, flag)) {
+        if (wg_over<NW>(big, flag)) {
             zero();
             for (int kk = 0; kk < a.Lk; kk += 32) {
                 issue(r0, kk);
@@ -679,7 +712,7 @@ const int psh = min(kk, a.ldP) * 2;
 #pragma unroll
                 for (int i = 0; i < VROUNDS; ++i) mv = max_finite4(mv, as_f4(r0.v[i]));
                 __syncthreads();
-                wg_max2(mv, none, slot);
+                wg_max2<NW>(mv, none, slot);
                 const float s1 = pow2_scale(mv), u = pow2_unit(mv);
                 store_p(r0, sp[0]);
 #pragma unroll
@@ -701,12 +734,12 @@ const int psh = min(kk, a.ldP) * 2;
     using T = typename G::T;
     T* Oh = static_cast<T*>(a.O) + (size_t)bh * a.Lq * a.ldO;
 #pragma unroll
-    for (int j = 0; j < NI; ++j) {
+    for (int j = 0; j < NQ; ++j) {
         const int qi = q0 + wq + 32 * j + fr;
         if (qi >= a.Lq) continue;
         T* orow = Oh + (size_t)qi * a.ldO;
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
+        for (int i = 0; i < ND; ++i)
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
                 const int d = d0 + wd + 32 * i + 8 * b + 4 * fc;
@@ -714,31 +747,62 @@ const int psh = min(kk, a.ldP) * 2;
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
                     v[c] = sum[i][j][4 * b + c] * kPInv;
-                if (!RAG) {
-                    if (d < a.ldO) Elem<T>::st4(orow, d, make_float4(v[0], v[1], v[2], v[3]));
-                } else {
+                if (d + 3 < a.ldO) {
+                    // (rows of any alignment: 8 or 16 bytes at once all the same)
+                    if (!RAG)
+                        Elem<T>::st4(orow, d, make_float4(v[0], v[1], v[2], v[3]));
+                    else
+                        st4_any(orow + d, make_float4(v[0], v[1], v[2], v[3]));
+                } else if (RAG) {
 #pragma unroll
-                    for (int c = 0; c < 4; ++c)
+                    for (int c = 0; c < 3; ++c)
                         if (d + c < a.ldO) Elem<T>::st(orow, d + c, v[c]);
                 }
             }
     }
 }
 
-template <int KIND, int TL>
+// 128 x 128 tiles take 8 waves (64 x 32 each) while no CU gets a second
+// workgroup: two waves per SIMD then, and loads two stages ahead (fp32
+// (1,4,512,512,2048): Q K^T 22.8 -> 20.9 us, P V 22.4 -> 20.3; (2,4,1024,1024,
+// 512) P V 45.7 -> 36.7).  Beyond that 4 waves of 64 x 64, two workgroups per
+// CU, read a third less from LDS ((2,2,504,1387,4424) Q K^T 124.7 us against
+// 136.9).
+constexpr unsigned kOnePerCu = 256;
+
+template <int KIND, int TL, int NW>
 void run_qk(const QkTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
     if (KIND == kKindF32 && rag)
-        hipLaunchKernelGGL((k_qk_tile<KIND, TL, KIND == kKindF32>), dim3(grid), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, KIND == kKindF32>), dim3(grid), dim3(64 * NW), 0,
+                           st, a);
     else
-        hipLaunchKernelGGL((k_qk_tile<KIND, TL, false>), dim3(grid), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, false>), dim3(grid), dim3(64 * NW), 0, st, a);
+}
+template <int KIND>
+void run_qk_tile(int tile, const QkTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
+    if (tile == 64)
+        run_qk<KIND, 64, 4>(a, rag, grid, st);
+    else if (grid <= kOnePerCu)
+        run_qk<KIND, 128, 8>(a, rag, grid, st);
+    else
+        run_qk<KIND, 128, 4>(a, rag, grid, st);
 }
 
-template <int KIND, int TL>
+template <int KIND, int TL, int NW>
 void run_pv(const PvTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
     if (rag)
-        hipLaunchKernelGGL((k_pv_tile<KIND, TL, true>), dim3(grid), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((k_pv_tile<KIND, TL, NW, true>), dim3(grid), dim3(64 * NW), 0, st, a);
     else
-        hipLaunchKernelGGL((k_pv_tile<KIND, TL, false>), dim3(grid), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((k_pv_tile<KIND, TL, NW, false>), dim3(grid), dim3(64 * NW), 0, st, a);
+}
+template <int KIND>
+void run_pv_tile(int tile, const PvTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
+    if (tile == 64)
+        run_pv<KIND, 64, 4>(a, rag, grid, st);
+    else if (grid <= kOnePerCu)
+        run_pv<KIND, 128, 8>(a, rag, grid, st);
+    else
+        run_pv<KIND, 128, 4>(a, rag, grid, st);
 }
 
 template <int KIND>
@@ -782,10 +846,9 @@ hipError_t launch_qk_tile(int dtype, int tile, QkTileArgs a, hipStream_t st) {
     const unsigned grid = (unsigned)((long)a.BH * a.tiles_q * a.tiles_k * a.nsplit);
     const bool rag = a.D % 4 != 0;
     if (dtype == kDtypeF32)
-        tile == 128 ? run_qk<kKindF32, 128>(a, rag, grid, st) : run_qk<kKindF32, 64>(a, rag, grid, st);
+        run_qk_tile<kKindF32>(tile, a, rag, grid, st);
     else
-        tile == 128 ? run_qk<kKindBF16, 128>(a, false, grid, st)
-                    : run_qk<kKindBF16, 64>(a, false, grid, st);
+        run_qk_tile<kKindBF16>(tile, a, false, grid, st);
     return hipGetLastError();
 }
 
@@ -803,10 +866,9 @@ hipError_t launch_pv_tile(int dtype, int tile, PvTileArgs a, hipStream_t st) {
     const unsigned grid = (unsigned)((long)a.BH * a.tiles_q * a.tiles_d);
     const bool rag = a.ldO % 4 != 0 || a.o_align == 0;
     if (dtype == kDtypeF32)
-        tile == 128 ? run_pv<kKindF32, 128>(a, rag, grid, st) : run_pv<kKindF32, 64>(a, rag, grid, st);
+        run_pv_tile<kKindF32>(tile, a, rag, grid, st);
     else
-        tile == 128 ? run_pv<kKindBF16, 128>(a, rag, grid, st)
-                    : run_pv<kKindBF16, 64>(a, rag, grid, st);
+        run_pv_tile<kKindBF16>(tile, a, rag, grid, st);
     return hipGetLastError();
 }
 
