@@ -93,6 +93,7 @@ bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
 struct FlashPlan {
     int form = 0, nsplit = 1, kchunk = 0;
     bool kpre = false;
+    double us = 0;  // estimated time
 };
 
 // ---------------------------------------------------------------- resolved encoding
@@ -110,9 +111,9 @@ struct PePlan {
     // the scratch holds no copies (encoded Q and K): the split-D pipeline that
     // encodes inside its QK^T kernel
     bool lean = false;
-    // bf16 calls that the GEMM path would take run on the split-D tiles
-    // (decided on the whole call, so that its chunks all do the same), and the
-    // whole call's D-chunk there
+    // calls that the GEMM path (bf16) or the flash kernel would take run on the
+    // split-D tiles (decided on the whole call, so that its chunks all do the
+    // same), and the whole call's D-chunk there
     bool tiles = false;
     int dchunk = 0;
     FlashPlan flash;  // a call of the flash kernel: its plan
@@ -901,7 +902,7 @@ size_t library_cap() {
 bool flash_ok(int dtype, const Shape& s, const PePlan& plan) {
     const int64_t lim = (int64_t)1 << 31;
     const int64_t es = dtype == ATN_DTYPE_F32 ? 4 : 2;
-    return !plan.no_flash && atn::flash_supported(dtype, plan.pek, s.D) &&
+    return !plan.no_flash && !(plan.tiles && !plan.lean) && atn::flash_supported(dtype, plan.pek, s.D) &&
            (int64_t)s.Lq * s.D * es < lim && (int64_t)s.Lk * s.D * es < lim;
 }
 
@@ -956,7 +957,6 @@ FlashPlan flash_plan_uncached(int dtype, const Shape& s, const PePlan& plan, siz
     const bool bf = dtype == ATN_DTYPE_BF16, enc = plan.pek != atn::kPeNone;
     const int chunks = (s.Lk + 63) / 64;
     FlashPlan best;
-    double best_us = 0;
     static const int forms[3] = {atn::kFlashForm4x16, atn::kFlashForm8x16, atn::kFlashForm8x32};
     const int forced = tn.flash_form;
     for (int once = 0; once < 2; ++once) {
@@ -983,7 +983,7 @@ FlashPlan flash_plan_uncached(int dtype, const Shape& s, const PePlan& plan, siz
                 const int per = (chunks + n - 1) / n, ns = (chunks + per - 1) / per;
                 if (ns == last) continue;
                 last = ns;
-                const FlashPlan f{form, ns, per * 64, once != 0};
+                const FlashPlan f{form, ns, per * 64, once != 0, 0};
                 if (n > 1 && tn.flash_split < 2 && kSyncBytes + flash_bytes(s, f) > cap) break;
                 if (once && kSyncBytes + flash_bytes(s, f) > cap) break;
                 const int64_t w = grid * ns, slots = two ? 512 : 256;
@@ -994,9 +994,9 @@ FlashPlan flash_plan_uncached(int dtype, const Shape& s, const PePlan& plan, siz
                            : us);
                 if (ns > 1) us += 5.0 + (double)ns * s.BH * s.Lq * s.D * 4.0 * 0.5e-6;
                 if (once) us += 4.0 + (double)s.nk * 4.0 / 4.5e6;
-                if (best.form == 0 || us < best_us) {
+                if (best.form == 0 || us < best.us) {
                     best = f;
-                    best_us = us;
+                    best.us = us;
                 }
             }
         }
@@ -1015,6 +1015,25 @@ FlashPlan flash_plan(int dtype, const Shape& s, const PePlan& plan, size_t cap) 
         last = key;
     }
     return kept;
+}
+
+// A flash call's plan, or its move to the split-D tiles (plan.tiles) where
+// those are the faster: head_d 129-256 on a grid so small that the flash
+// kernel's workgroups, which hold 256 dims of output each and take about 7 us
+// beside their tiles (first loads, last stores), leave CUs idle and its key
+// splits need a merge.  (1,4,417,417,256) fp32 27.4 -> 21.0 us, bf16 22.8 ->
+// 17.2; (2,16,142,142,256) fp32 25.4 -> 18.7; (1,8,130,130,200) 17.6 -> 12.4 and
+// 14.9 -> 11.2.  Of 42 calls timed both ways the line at 0.8 takes 10 over,
+// each faster, and leaves 6 that would gain 6-12 %; (1,8,600,600,256) is past
+// it (34.7 us against 36.2, bf16 29.2 against 34.2).  At head_d <= 128 the
+// flash kernel led at 50 of 52.  Only where the whole call's scratch fits.
+void plan_flash(int dtype, const Shape& s, PePlan& plan, size_t cap) {
+    plan.flash = flash_plan(dtype, s, plan, cap);
+    if (s.D <= 128 || tune().flash_form != 0 || tune().flash_split != 0) return;
+    const TilePlan tp = tile_plan(dtype, s, plan, true);
+    if (!tp.ok || tp.Dp != 0 || tp.bytes > cap || tp.us >= 0.8 * (plan.flash.us + 7.0)) return;
+    plan.tiles = true;
+    plan.dchunk = tp.dchunk;
 }
 
 // Scratch bytes of the path a call of shape s takes: fused (when planned and
@@ -1302,7 +1321,7 @@ int attention_core(int dtype, const void* Q, const void* K, const void* V, void*
 
     const size_t cap = no_alloc ? atn::kNoAllocScratchBytes
                                 : (workspace != nullptr ? workspace_bytes : library_cap());
-    if (flash_ok(dtype, s, plan)) plan.flash = flash_plan(dtype, s, plan, cap);
+    if (flash_ok(dtype, s, plan)) plan_flash(dtype, s, plan, cap);
     // chunk pointers keep the base alignment when a row is a multiple of 16
     // bytes; otherwise plan for the largest path
     const size_t va = dtype == ATN_DTYPE_F32 ? 16 : 8;
@@ -1687,7 +1706,7 @@ size_t atn_attention_workspace_bytes(int dtype, int batch, int heads, int len_q,
     PePlan plan;
     if (check_pe(pe, head_d, &plan) != ATN_OK) return 0;
     choose_tiles(dtype, s, plan);
-    if (flash_ok(dtype, s, plan)) plan.flash = flash_plan(dtype, s, plan, library_cap());
+    if (flash_ok(dtype, s, plan)) plan_flash(dtype, s, plan, library_cap());
     // the largest workspace of every plan the call could take, or, when that
     // exceeds the library's cap, of the chunks the call then runs in
     const size_t full = path_need(dtype, s, plan, false, -1, -1);

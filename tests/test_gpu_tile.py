@@ -186,3 +186,31 @@ def test_chunked_tiles(am, dev, tuner):
     assert np.array_equal(out.bits(), full.bits())
     n, nrel, mabs = H.check_bf16(out.numpy(), _ref("none", Q, K, V))
     assert n == 0, (nrel, mabs)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("shape", [(1, 4, 417, 417, 256), (1, 8, 130, 130, 200), (1, 1, 300, 290, 136),
+                                   (2, 3, 65, 129, 248)], ids=str)
+def test_small_grids_of_the_flash_kernel(am, dev, tuner, dt, shape):
+    """head_d 129-256 on small grids runs on the tiles, and on the flash kernel
+    where the scratch is too small for them: both against the oracle, and a
+    forced flash form agrees with the small-scratch call bit for bit."""
+    import hip_rt
+    B, Hh, Lq, Lk, D = shape
+    code = {"f32": 0, "bf16": 1}[dt]
+    print(f"[case] flash or tiles {dt} {shape}", flush=True)
+    assert am.path(code, B, Hh, Lq, Lk, D) == am.ATN_PATH_FLASH
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 820 + Lq, dt)
+    out, small, flash = (H.empty(Q.shape, dt) for _ in range(3))
+    am.attention_ex(q, k, v, out)
+    ws = hip_rt.DeviceArray(((64 << 10) // 4,), "f32", fill=0)
+    am.attention_ex(q, k, v, small, workspace=ws)
+    tuner.set(flash_split=1)
+    am.attention_ex(q, k, v, flash)
+    hip_rt.synchronize()
+    ref = _ref("none", Q, K, V)
+    for got in (out, small):
+        n, nrel, mabs = H.check_f32(got.numpy(), ref) if dt == "f32" else H.check_bf16(got.numpy(), ref)
+        assert n == 0, (nrel, mabs)
+    assert np.array_equal(small.numpy(), flash.numpy())
+    assert not np.array_equal(out.numpy(), flash.numpy())  # the tiles' sums
