@@ -117,6 +117,9 @@ struct PePlan {
     bool tiles = false;
     int dchunk = 0;
     FlashPlan flash;  // a call of the flash kernel: its plan
+    // set when a kernel that can end its wait unfinished was launched (the
+    // single-launch kernel with an exchange between workgroups)
+    bool* waits = nullptr;
 };
 
 int check_pe(const atn_pe_desc* pe, int D, PePlan* plan) {
@@ -187,9 +190,9 @@ struct DeviceState {
     int cus = 0;
     int xccs = 0;  // XCDs the device reports (8 on a whole MI355X)
     std::map<std::pair<int, int>, int> fused_per_cu;  // (dtype, LDS bytes) -> workgroups per CU
-    // Two pinned host words that receive the status words of the null
-    // stream's library workspace and of the allocation-free scratch behind
-    // each synchronous drop-in call (allocated once, kept).
+    // Pinned host memory that receives the status word of the null stream's
+    // library workspace behind a synchronous drop-in call whose kernel waits
+    // on other workgroups (allocated once, kept).
     int* status_host = nullptr;
 };
 
@@ -1207,6 +1210,7 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
             if (is_capturing(stream)) return ATN_ERR_CAPTURE;
             ATN_HIP(hipMemsetAsync(status, 0x01, 1, stream));
         }
+        if (plan.waits != nullptr && fd.nchunk > 1) *plan.waits = true;
         ATN_HIP(atn::launch_fused_small(dtype, plan.pek, Q, K, V, out, part, red, epochs, done,
                                         status, xctr, (int)s.BH, Lq, Lk, D, fd.MB, fd.dc,
                                         fd.nchunk, fd.gather1, fd.xcd, scale, plan.q, plan.k,
@@ -1282,7 +1286,7 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
 int attention_core(int dtype, const void* Q, const void* K, const void* V, void* out, int B,
                    int H, int Lq, int Lk, int D, const atn_pe_desc* pe, void* workspace,
                    size_t workspace_bytes, hipStream_t stream, bool no_alloc = false,
-                   bool no_fused = false) {
+                   bool no_fused = false, bool* waits = nullptr) {
     if (dtype != ATN_DTYPE_F32 && dtype != ATN_DTYPE_BF16) return ATN_ERR_BAD_ARGUMENT;
     if (!Q || !K || !V || !out) return ATN_ERR_NULL_POINTER;
     Shape s;
@@ -1298,6 +1302,7 @@ int attention_core(int dtype, const void* Q, const void* K, const void* V, void*
     st = check_pe(pe, D, &plan);
     if (st != ATN_OK) return st;
     plan.no_fused = no_fused || tune().no_fused != 0;
+    plan.waits = waits;
     plan.no_flash = tune().no_flash != 0;
     // every path needs at least the sync region; the path-specific size is
     // checked once the device has chosen the path
@@ -1478,28 +1483,32 @@ int workspace_status(void* ws, hipStream_t stream) {
     return ATN_ERR_DEVICE_TIMEOUT;
 }
 
-// Completion of a synchronous drop-in call (enqueued on the null stream):
-// the status word of the null stream's library workspace, the only
-// workspace a drop-in uses, is copied into a pinned host word behind the
-// call, so the one device synchronization covers the call and its status
-// check.  A set word runs the recovery of workspace_status() and returns
-// ATN_ERR_DEVICE_TIMEOUT; any other failure ends the process (the
-// reference's CUDA_CHECK, final/attention.cu:12-21).  The allocation-free
-// scratch is not looked at: its status belongs to the noalloc callers, who
-// query it with atn_sync_status_ex.
-int finish_sync(int status, const char* where) {
+// Completion of a synchronous drop-in call (enqueued on the null stream).
+// `waits`: one of its kernels waits on other workgroups and may have given up;
+// the status word of the null stream's library workspace, the only workspace
+// a drop-in uses, is then copied into a pinned host word behind the call, so
+// the one device synchronization covers the call and its status check.  Other
+// calls cannot fail so, and skip the copy, about 2 us of a call bound by its
+// launch ((1,1,4,4,8) 16.9 -> 14.6 us); a word that an earlier call left set
+// stays for atn_sync_status_ex and for the next call that waits.  A set word
+// runs the recovery of workspace_status() and returns ATN_ERR_DEVICE_TIMEOUT;
+// any other failure ends the process (the reference's CUDA_CHECK,
+// final/attention.cu:12-21).  The allocation-free scratch is not looked at:
+// its status belongs to the noalloc callers, who query it with
+// atn_sync_status_ex.
+int finish_sync(int status, const char* where, bool waits) {
     if (status != ATN_OK) die(status, where);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         g_last_hip_error = (int)e;
         die(ATN_ERR_HIP, where);
     }
-    int dev;
-    int st = current_device(&dev);
-    if (st != ATN_OK) die(st, where);
     void* lib_ws = nullptr;
     int* host = nullptr;
-    {
+    if (waits) {
+        int dev;
+        const int st = current_device(&dev);
+        if (st != ATN_OK) die(st, where);
         std::lock_guard<std::mutex> lk(g_mu);
         DeviceState& ds = g_dev[dev];
         auto it = ds.ws.find(nullptr);
@@ -1530,7 +1539,7 @@ int finish_sync(int status, const char* where) {
 }
 
 void sync_or_die(int status, const char* where) {
-    const int st = finish_sync(status, where);
+    const int st = finish_sync(status, where, false);
     if (st != ATN_OK) die(st, where);
 }
 
@@ -1541,9 +1550,10 @@ void sync_or_die(int status, const char* where) {
 // that wait on no other workgroup; a second failure ends the process.
 void dropin_attention(const char* where, int dtype, const void* Q, const void* K, const void* V,
                       void* out, int B, int H, int Lq, int Lk, int D, const atn_pe_desc* pe) {
-    if (finish_sync(attention_core(dtype, Q, K, V, out, B, H, Lq, Lk, D, pe, nullptr, 0, nullptr),
-                    where) == ATN_OK)
-        return;
+    bool waits = false;
+    const int st = attention_core(dtype, Q, K, V, out, B, H, Lq, Lk, D, pe, nullptr, 0, nullptr,
+                                  false, false, &waits);
+    if (finish_sync(st, where, waits) == ATN_OK) return;
     g_reruns.fetch_add(1, std::memory_order_relaxed);
     std::fprintf(stderr,
                  "attn_mi355x: %s: the single-launch kernel's wait timed out; running the call "
