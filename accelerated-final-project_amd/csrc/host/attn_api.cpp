@@ -977,7 +977,9 @@ FlashPlan flash_plan_uncached(int dtype, const Shape& s, const PePlan& plan, siz
             }
             const int rows = flash_rows(form, s.D);
             const int64_t grid = s.BH * ((s.Lq + rows - 1) / rows);
-            const double tile = t[bf ? (once ? 4 : 2 + enc) : enc][fi][dc];
+            // (heads of 65-96 and 129-192 dims: products over three quarters)
+            const bool quarters = fi > 0 && ((s.D > 64 && s.D <= 96) || (s.D > 128 && s.D <= 192));
+            const double tile = (quarters ? 0.9 : 1.0) * t[bf ? (once ? 4 : 2 + enc) : enc][fi][dc];
             const bool two = fi == 0 || (bf && !enc && fi == 1 && dc < 2);
             const double pair = fi == 0 ? 1.5 : 1.78;
             int last = 0;

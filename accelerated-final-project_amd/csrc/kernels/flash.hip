@@ -61,7 +61,13 @@ namespace {
 // and 4 waves of 16 rows at DP <= 64 (two workgroups per CU still fit in
 // LDS), else 32 (two LDS buffers of it then leave room for two 4-wave
 // workgroups per CU), and at least one load round of the workgroup.
-template <int DP, bool PE, int NW, int RW, bool HL = true>
+// DE <= DP: the dims the products run over, a multiple of 32.  The padding past
+// them is zeros, so leaving its products out changes no bit.  Three quarters
+// of DP for head dims 65-96 and 129-192: (8,16,604,604,96) fp32 107 -> 93.5 us,
+// bf16 45.9 -> 42.4, (1,8,2048,2048,96) fp32 RoPE 69 -> 65, (2,16,684,684,80)
+// rotate-half 53.7 -> 49.2, (1,16,3749,640,160) 137.5 -> 117.3, bf16 61.5 ->
+// 55.1.  Seven eighths (head dims 97-112) gave 0-3 %: not worth the variants.
+template <int DP, bool PE, int NW, int RW, bool HL = true, int DE = DP>
 struct FlashGeo {
     static_assert(RW == 16 || (RW == 32 && DP <= 128), "forms");
     static constexpr int THREADS = 64 * NW, ROWS = RW * NW;
@@ -72,10 +78,10 @@ struct FlashGeo {
     static constexpr int KT = KT0 > THREADS / (DP / 4) ? KT0 : THREADS / (DP / 4);
     static constexpr int MT = RW;                   // MFMA tile edge
     static constexpr int KD = RW == 16 ? 32 : 16;   // MFMA depth: dims of Q K^T, keys of P V
-    static constexpr int KS = DP / KD;              // KD-deep steps of Q K^T
+    static constexpr int KS = (DE + KD - 1) / KD;   // KD-deep steps of Q K^T
     static constexpr int NJ = KT / MT;              // MT-key tiles of S^T
     static constexpr int NB = KT / KD;              // KD-key blocks of P V
-    static constexpr int NDT = DP / MT;             // MT-dim tiles of O^T
+    static constexpr int NDT = (DE + MT - 1) / MT;  // MT-dim tiles of O^T
     static constexpr int SPT = MT * MT / 64;        // accumulator floats per lane and tile
     static constexpr int VPR = DP / 4;              // 16-byte vectors per row
     static constexpr int RSTEP = THREADS / VPR;     // rows per load round
@@ -206,7 +212,7 @@ constexpr int flash_waves_per_simd() {
 // the kernel then encodes its query rows only and stages K~ as it is, the
 // bits that it would have staged itself.  (The host's rule and what it
 // measured: flash_plan in attn_api.cpp.)
-template <typename T, int DP, int PEK, int NW, int RW, bool KPRE>
+template <typename T, int DP, int PEK, int NW, int RW, bool KPRE, int DE>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     flash_waves_per_simd<T, DP, PEK, NW, RW>()))) void k_flash(const T* __restrict__ Qg,
                                                              const T* __restrict__ Kg,
@@ -226,7 +232,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     // so it always goes in as loaded, with P as bf16.
     typedef std::conditional_t<kRaw, bf16x8_t, f16x8> op_t;
     typedef std::conditional_t<kBf, bf16x8_t, f16x8> pv_t;
-    using G = FlashGeo<DP, PEK != kPeNone, NW, RW, !kBf>;
+    using G = FlashGeo<DP, PEK != kPeNone, NW, RW, !kBf, DE>;
     typedef std::conditional_t<RW == 16, v4f, v16f> acc_t;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     uint16_t* smem = reinterpret_cast<uint16_t*>(smem_raw);
@@ -942,19 +948,19 @@ struct FlashArgs {
     const float* kunit;  // not null: K is encoded fp16 (KPRE)
 };
 
-template <typename T, int DP, int PEK, int NW, int RW, bool KPRE = false>
+template <typename T, int DP, int PEK, int NW, int RW, bool KPRE = false, int DE = DP>
 hipError_t launch_t(const FlashArgs& a, hipStream_t st) {
     using G = FlashGeo<DP, PEK != kPeNone, NW, RW, sizeof(T) == 4>;
     static bool attr = false;
     if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_flash<T, DP, PEK, NW, RW, KPRE>,
+        hipError_t e = hipFuncSetAttribute((const void*)k_flash<T, DP, PEK, NW, RW, KPRE, DE>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, G::BYTES);
         if (e != hipSuccess) return e;
         attr = true;
     }
     const int qblocks = (a.Lq + G::ROWS - 1) / G::ROWS;
     const int kchunk = a.nsplit > 1 ? a.kchunk : a.Lk;
-    hipLaunchKernelGGL((k_flash<T, DP, PEK, NW, RW, KPRE>), dim3((unsigned)(a.BH * qblocks * a.nsplit)),
+    hipLaunchKernelGGL((k_flash<T, DP, PEK, NW, RW, KPRE, DE>), dim3((unsigned)(a.BH * qblocks * a.nsplit)),
                        dim3(G::THREADS), G::BYTES, st, static_cast<const T*>(a.Q),
                        static_cast<const T*>(a.K), static_cast<const T*>(a.V), static_cast<T*>(a.O),
                        a.Lq, a.Lk, a.D, qblocks, a.scale, a.pq, a.pk, a.nsplit, kchunk, a.part,
@@ -974,20 +980,27 @@ hipError_t launch_t(const FlashArgs& a, hipStream_t st) {
 }
 
 // head dims padded to 32, 64, 128 (and 256 for 8 waves of 16 rows without
-// an encoding)
+// an encoding), in the forms of 8 waves with products over 96 and 192 dims
+// where those hold the head (FlashGeo's DE)
 template <typename T, int PEK, int NW, int RW>
 hipError_t launch_pe(const FlashArgs& a, hipStream_t st) {
     if constexpr (sizeof(T) == 2 && PEK != kPeNone && NW == 8) {
         if (a.kunit != nullptr) {
             if (a.D <= 32) return launch_t<T, 32, PEK, NW, RW, true>(a, st);
             if (a.D <= 64) return launch_t<T, 64, PEK, NW, RW, true>(a, st);
+            if (a.D <= 96) return launch_t<T, 128, PEK, NW, RW, true, 96>(a, st);
             if (a.D <= 128) return launch_t<T, 128, PEK, NW, RW, true>(a, st);
         }
     }
     if (a.kunit != nullptr) return hipErrorInvalidValue;
     if (a.D <= 32) return launch_t<T, 32, PEK, NW, RW>(a, st);
     if (a.D <= 64) return launch_t<T, 64, PEK, NW, RW>(a, st);
+    if constexpr (NW == 8) {
+        if (a.D <= 96) return launch_t<T, 128, PEK, NW, RW, false, 96>(a, st);
+    }
     if (a.D <= 128) return launch_t<T, 128, PEK, NW, RW>(a, st);
+    if constexpr (PEK == kPeNone && NW == 8 && RW == 16)
+        if (a.D <= 192) return launch_t<T, 256, PEK, NW, RW, false, 192>(a, st);
     if constexpr (PEK == kPeNone && NW == 8 && RW == 16) return launch_t<T, 256, PEK, NW, RW>(a, st);
     return hipErrorInvalidValue;
 }

@@ -716,3 +716,28 @@ def test_flash_merge_forms(am, dev, tuner, dt, parts, Lq):
                            nthreads=16)
     n, err = _check(dt, _call(am, dt, Q, K, V), ref)
     assert n == 0, err
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("D,pe,form", [(68, "none", "8x16"), (92, "half", "8x32"), (96, "rope", "8x16"),
+                                       (96, "none", "8x32"), (100, "none", "8x16"), (132, "none", "8x16"),
+                                       (192, "none", "8x16"), (196, "none", "8x16")], ids=str)
+def test_flash_three_quarter_heads(am, dev, tuner, dt, D, pe, form):
+    """Heads whose products run over 96 or 192 dims, and the first past them."""
+    import hip_rt
+    B, Hh, Lq, Lk = 1, 2, 140, 200
+    print(f"[case] three quarters {dt} {D} {pe} {form}", flush=True)
+    tuner.set(flash_form=form, flash_split=1)
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 740 + D, dt)
+    out = H.empty(Q.shape, dt)
+    desc = {"none": None, "rope": am.make_pe("rope"), "half": am.make_pe("rope", "half")}[pe]
+    am.attention_ex(q, k, v, out, pe=desc)
+    hip_rt.synchronize()
+    if pe == "none":
+        ref = oracle.attention(Q, K, V, nthreads=16)
+    else:
+        c, s = oracle.rope_cache(Lk, D)
+        ref = oracle.attention_rope(Q, K, V, c, s, pairing="half" if pe == "half" else "interleaved",
+                                    nthreads=16)
+    n, a, b = H.check_f32(out.numpy(), ref) if dt == "f32" else H.check_bf16(out.numpy(), ref)
+    assert n == 0, (a, b)
