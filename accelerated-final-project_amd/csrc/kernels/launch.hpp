@@ -13,7 +13,8 @@ namespace atn {
 constexpr int kDtypeF32 = 0;
 constexpr int kDtypeBF16 = 1;
 
-// Split-D streaming pipeline (stream.hip).
+// Split-D pipeline without copies of its inputs (stream.hip): calls whose
+// scratch is too small for the tiles below.
 hipError_t launch_qk_partial(int dtype, int pek, const void* Q, const void* K, float* S, int BH,
                              int Lq, int Lk, int D, int dchunk, int nsplit, const PeSide& pq,
                              const PeSide& pk, int vec_ok, hipStream_t st);

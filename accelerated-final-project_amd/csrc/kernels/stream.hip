@@ -21,9 +21,14 @@
 // All math is fp32; bf16 storage is widened at load and rounded (RNE) once
 // at the final store.  Workgroups are 256 threads (4 waves) computing 64x64
 // tiles, a 32x32 quadrant per wave on fp32 MFMA, from LDS-staged 32-deep
-// slices.  fp32 calls with head_d % 4 == 0 and 16-byte aligned bases run
-// stages 1 and 3 on 16-bit MFMA instead (stream16.hip); these kernels serve
-// bf16 (head_d % 8 != 0 or misaligned), odd head dims and misaligned fp32.
+// slices.
+//
+// What comes here: calls whose scratch cannot hold what the pipelined tiles
+// need beside the scores (tile16.hip: encoded or padded copies of Q, K and V,
+// P in two parts), and heads of 2 GiB and more.  Encodings are applied at
+// load, so the only scratch is the scores'.  Of those calls fp32 with head_d
+// % 4 == 0 and 16-byte aligned bases runs stages 1 and 3 on 16-bit MFMA
+// (stream16.hip), the rest on the kernels below.
 #include <algorithm>
 
 #include "common.hpp"

@@ -1,12 +1,13 @@
-// The split-D pipeline's two contractions for fp32 inputs on 16-bit MFMA
-// (gfx950): k_qk_s16 (partial scores over a D-chunk) and k_pv_s16 (O = P V).
+// The scratch-lean split-D pipeline's two contractions for fp32 inputs on
+// 16-bit MFMA (gfx950): k_qk_s16 (partial scores over a D-chunk) and k_pv_s16
+// (O = P V).  Calls with the scratch for it run tile16.hip instead.
 //
 // Same decomposition and memory layout as stream.hip's k_qk_partial / k_pv
 // (S and P in the workspace, split along D for the scores), with the
 // operands held as hi + lo fp16 parts (split16.hpp: 22 significant bits,
 // three exact products per product on v_mfma_f32_16x16x32_f16) instead of
-// fp32 MFMA operands.  These kernels take fp32 calls with head_d % 4 == 0
-// and 16-byte aligned bases; the others stay on stream.hip's.
+// fp32 MFMA operands.  These kernels take the fp32 calls among stream.hip's
+// with head_d % 4 == 0 and 16-byte aligned bases.
 //
 // Two tile sizes (TL): 64 x 64 output tiles in 64-deep stages (each of the 4
 // waves 16 rows x 64 columns) for short sides, and 128 x 128 in 32-deep

@@ -292,15 +292,18 @@ int atn_prepare_pe_ex(const atn_pe_desc *pe, int head_d, int max_positions);
  * split-D pipeline runs).  Without a device the answer assumes 256 compute
  * units. */
 #define ATN_PATH_FUSED_SMALL 1 /* one launch: split-D slices + device-side S all-reduce */
-#define ATN_PATH_SPLIT_D 2     /* three launches: partial QK^T, softmax, PV */
+#define ATN_PATH_SPLIT_D 2     /* partial QK^T over D-chunks, softmax, PV (before them a pass
+                                  that encodes Q and K, or pads bf16 rows) */
 #define ATN_PATH_FLASH 4       /* outside the single-launch window, head_d % 4 == 0, fp32 and
                                   bf16: head_d <= 256 (128 with an encoding): one launch,
-                                  online softmax over key tiles, no scratch; grids that would
-                                  leave CUs idle split the keys (parts in the workspace, a
-                                  second launch merges them) */
+                                  online softmax over key tiles; grids that would leave CUs
+                                  idle split the keys (parts in the workspace, a second launch
+                                  merges them), long bf16 calls encode K once into the
+                                  workspace, small grids of head_d > 128 run the split-D
+                                  kernels; all need no scratch where none is given */
 #define ATN_PATH_GEMM 3        /* bf16, D % 8 == 0, head_d > 256 (> 128 with an encoding),
                                   outside the single-launch window: MFMA QK^T GEMM, row
-                                  softmax, MFMA PV GEMM */
+                                  softmax, MFMA PV GEMM; small grids run the split-D kernels */
 int atn_attention_path_ex(int dtype, int batch, int heads, int len_q, int len_k, int head_d,
                           const atn_pe_desc *pe);
 
@@ -338,14 +341,13 @@ typedef struct atn_tuning {
                               2 = 8 waves of 16, 3 = 4 waves of 32, 4 = 8 waves of 32
                               (3 and 4: head_d <= 128; head_d > 128 always runs 2);
                               0: the library's choice */
-    int splitd_tile;       /* split-D pipeline, fp32 16-bit kernels: 64 or 128 forces
-                              that output tile (128 where both of its sides reach
-                              128); 0: 128 x 128 where that grid gives every CU two
-                              workgroups, else 64 x 64 */
+    int splitd_tile;       /* split-D pipeline's 16-bit kernels: 64 or 128 forces that
+                              output tile (128 where both of its sides reach 128); 0:
+                              the smaller estimated time */
     int flash_split;       /* flash kernel key splits: 1 never split, n >= 2 split the keys
-                              into n parts (fewer for short key lengths: two 64-key chunks
-                              at least per part); 0: the library's choice (splits where
-                              the grid would leave CUs idle) */
+                              into n parts (fewer for short key lengths: one 64-key chunk
+                              at least per part); 0: the library's choice (the smaller
+                              estimated time) */
 } atn_tuning;
 /* Replaces the overrides (NULL: all zero) and drops cached plans.  Plans
  * that a forced setting makes impossible fall back to the library's
