@@ -304,14 +304,19 @@ hipError_t launch_pe_apply(int dtype, int out_dtype, int pek, const PeTensor* t,
 // K~ of the flash kernel, bf16 to fp16: one workgroup per tile of 64 keys
 // (the flash kernel's), NG groups of 4 dims per thread, all loads first.  The
 // tile's largest finite magnitude is known before anything is written, so
-// the values and units are those of the flash kernel's own staging.
+// the values and units are those of the flash kernel's own staging.  Bound by
+// the latency of those loads (bits, partners, two tables) on few workgroups a
+// CU: 512 threads with half the groups each keep twice the waves in flight as
+// 256: (4,8,1107,1107,128) rotate-half 11.5 -> 10.7 us, the calls
+// (4,16,300,1500,128) 57.4 -> 55.3, (2,32,900,900,96) 52.1 -> 50.5.
 namespace {
+constexpr int kKeyTileThreads = 512;
 template <int PEK, int NG>
-__global__ __launch_bounds__(256) void k_encode_key_tiles(const uint16_t* __restrict__ K,
-                                                          uint16_t* __restrict__ out,
-                                                          float* __restrict__ unit, int tiles,
-                                                          int Lk, int D, PeSide pe) {
-    __shared__ float slot[4];
+__global__ __launch_bounds__(kKeyTileThreads) void k_encode_key_tiles(
+    const uint16_t* __restrict__ K, uint16_t* __restrict__ out, float* __restrict__ unit, int tiles,
+    int Lk, int D, PeSide pe) {
+    constexpr int NT = kKeyTileThreads;
+    __shared__ float slot[NT / 64];
     const int tid = threadIdx.x, vpr = D >> 2;
     const int bh = blockIdx.x / tiles, k0 = (blockIdx.x % tiles) * 64;
     const int groups = min(64, Lk - k0) * vpr;  // the tile's rows are consecutive
@@ -322,7 +327,7 @@ __global__ __launch_bounds__(256) void k_encode_key_tiles(const uint16_t* __rest
     const uint16_t* row[NG];
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
-        const int g = min(tid + 256 * i, groups - 1), r = g / vpr;
+        const int g = min(tid + NT * i, groups - 1), r = g / vpr;
         d[i] = (g - r * vpr) * 4;
         pos[i] = k0 + r;
         row[i] = src + (size_t)r * D;
@@ -343,7 +348,8 @@ __global__ __launch_bounds__(256) void k_encode_key_tiles(const uint16_t* __rest
     m = wave_max(m);
     if ((tid & 63) == 0) slot[tid >> 6] = m;
     __syncthreads();
-    m = fmaxf(fmaxf(slot[0], slot[1]), fmaxf(slot[2], slot[3]));
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) m = fmaxf(m, slot[w]);
     const bool plain = m >= 0.125f && m < kF16Range;
     const float s = plain ? 1.f : pow2_scale(m);
     if (tid == 0) unit[blockIdx.x] = plain ? 1.f : pow2_unit(m);
@@ -351,8 +357,8 @@ __global__ __launch_bounds__(256) void k_encode_key_tiles(const uint16_t* __rest
     for (int i = 0; i < NG; ++i) {
         const f16x2 a = {(_Float16)(x[i].x * s), (_Float16)(x[i].y * s)};
         const f16x2 b = {(_Float16)(x[i].z * s), (_Float16)(x[i].w * s)};
-        if (tid + 256 * i < groups)
-            *reinterpret_cast<uint2*>(dst + 4 * (size_t)(tid + 256 * i)) =
+        if (tid + NT * i < groups)
+            *reinterpret_cast<uint2*>(dst + 4 * (size_t)(tid + NT * i)) =
                 make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
     }
 }
@@ -361,12 +367,12 @@ template <int PEK>
 void run_key_tiles(const uint16_t* K, uint16_t* out, float* unit, int BH, int Lk, int D,
                    const PeSide& pe, hipStream_t st) {
     const int tiles = (Lk + 63) / 64;
-    const dim3 grid((unsigned)(BH * tiles)), block(256);
+    const dim3 grid((unsigned)(BH * tiles)), block(kKeyTileThreads);
     if (D <= 64)
-        hipLaunchKernelGGL((k_encode_key_tiles<PEK, 4>), grid, block, 0, st, K, out, unit, tiles, Lk,
+        hipLaunchKernelGGL((k_encode_key_tiles<PEK, 2>), grid, block, 0, st, K, out, unit, tiles, Lk,
                            D, pe);
     else
-        hipLaunchKernelGGL((k_encode_key_tiles<PEK, 8>), grid, block, 0, st, K, out, unit, tiles, Lk,
+        hipLaunchKernelGGL((k_encode_key_tiles<PEK, 4>), grid, block, 0, st, K, out, unit, tiles, Lk,
                            D, pe);
 }
 }  // namespace
