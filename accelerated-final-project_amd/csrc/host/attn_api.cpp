@@ -946,6 +946,16 @@ size_t flash_bytes(const Shape& s, const FlashPlan& f) {
 // 169 -> 85; not worth its launch and traffic at (4,32,512,512,128) (39.4 us
 // against 42.7).  fp32 calls, whose products take three times as long beside
 // the same encoding, gained 3-5 % at most and lost up to 20 %.
+//
+// From about 100 MB of bf16 keys and values on, a call of few rows cannot end
+// before it has streamed them, at 5.6 TB/s whether a CU holds one workgroup or
+// two (a CU without one leaves its share unused); among the splits that reach
+// that the fewest are taken: (1,32,1,8192,128)
+// 8 splits 31.6 us, 16 splits 33.9; (4,16,1,4096,128) 4 splits 31.5, 8 splits
+// 33.4; from 200 MB on the two lie within 5 % either way.  Smaller calls are
+// bound by their tiles' latencies, and fp32 workgroups stream faster two to a
+// CU (55.5 us with 16 splits at (1,32,1,8192,128), 68.0 with 8): both as the
+// tile times say.
 FlashPlan flash_plan_uncached(int dtype, const Shape& s, const PePlan& plan, size_t cap) {
     // [fp32 plain, fp32 encoded, bf16 plain, bf16 encoded, bf16 K once][form][head_d class]
     static const double t[5][3][3] = {
@@ -959,6 +969,7 @@ FlashPlan flash_plan_uncached(int dtype, const Shape& s, const PePlan& plan, siz
     const int dc = s.D <= 64 ? 0 : (s.D <= 128 ? 1 : 2);
     const bool bf = dtype == ATN_DTYPE_BF16, enc = plan.pek != atn::kPeNone;
     const int chunks = (s.Lk + 63) / 64;
+    const double kv_us = bf ? 4.0 * (double)s.nk / 5.6e6 : 0.0;  // streaming K and V
     FlashPlan best;
     static const int forms[3] = {atn::kFlashForm4x16, atn::kFlashForm8x16, atn::kFlashForm8x32};
     const int forced = tn.flash_form;
@@ -997,6 +1008,7 @@ FlashPlan flash_plan_uncached(int dtype, const Shape& s, const PePlan& plan, siz
                 us += per * tile *
                       (two ? (double)(w / 512) * pair + (rem == 0 ? 0.0 : rem <= 256 ? 1.0 : pair)
                            : us);
+                if (kv_us > 18.0) us = std::max(us, kv_us / std::min(1.0, (double)w / 256.0));
                 if (ns > 1) us += 5.0 + (double)ns * s.BH * s.Lq * s.D * 4.0 * 0.5e-6;
                 if (once) us += 4.0 + (double)s.nk * 4.0 / 4.5e6;
                 if (best.form == 0 || us < best.us) {

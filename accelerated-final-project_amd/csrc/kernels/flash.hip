@@ -869,70 +869,66 @@ __global__ __launch_bounds__(256) void k_flash_combine(const float* __restrict__
                  make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv));
 }
 
-// The same for few rows of many splits (decoding), where a thread per group
-// would walk the splits one latency after another on a handful of CUs: each of
-// a workgroup's 4 waves takes every fourth split of 64 groups, up to 8 loads
-// at once, and the waves' sums meet in LDS, weighed by their own maxima.
+// The same, bit for bit, for few rows of many splits (decoding), where a thread
+// per group would walk the splits one latency after another on a handful of
+// CUs: each of a workgroup's 4 waves loads every fourth split of 64 groups, up
+// to 8 loads at once, weighs them by the maximum of all (exchanged through
+// LDS), and wave 0 adds them up in the splits' order.
+constexpr int kFewSplits = 32, kFewGroups = 1 << 15;
 template <typename T>
 __global__ __launch_bounds__(256) void k_flash_combine_few(const float* __restrict__ part,
                                                            const float4* __restrict__ stats,
                                                            T* __restrict__ Og, int Lq, int D,
-                                                           int nsplit, long groups) {
-    __shared__ float4 sum[4][64];
-    __shared__ float2 mw[4][64];  // a wave's maximum and weight sum
+                                                           int nsplit, unsigned groups) {
+    constexpr int PW = kFewSplits / 4;  // splits per wave
+    __shared__ float4 val[kFewSplits][64];
+    __shared__ float wt[kFewSplits][64];
+    __shared__ float mx[4][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const unsigned vpr = (unsigned)D >> 2;
-    const long g = min((long)blockIdx.x * 64 + lane, groups - 1);
-    const long row = g / vpr, bh = row / Lq;
+    const unsigned g = min(blockIdx.x * 64 + lane, groups - 1);  // (below kFewGroups)
+    const unsigned row = g / vpr, bh = row / (unsigned)Lq;
     const int d = 4 * (int)(g - row * vpr);
-    const size_t base = (size_t)bh * nsplit * Lq + (size_t)(row - bh * Lq);
-    float c0 = 0.f, m = -INFINITY, wsum = 0.f;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    // nsplit <= 32: at most 8 per wave
-    float4 st[8], v[8];
+    const size_t base = (size_t)bh * nsplit * Lq + (row - bh * (unsigned)Lq);
+    float M = -INFINITY;
+    float4 st[PW], v[PW];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < PW; ++i) {
         const int s = wave + 4 * i;
         const size_t pr = base + (size_t)(s < nsplit ? s : 0) * Lq;
         st[i] = stats[pr];
         v[i] = *reinterpret_cast<const float4*>(part + pr * D + d);
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-        if (wave + 4 * i < nsplit) m = fmaxf(m, st[i].x);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        if (wave + 4 * i >= nsplit) continue;
-        c0 = st[i].y;
-        const float w = __builtin_amdgcn_exp2f(fmaf(st[i].x - m, c0, st[i].z));
-        wsum += w;
-        acc.x = fmaf(w, v[i].x, acc.x);
-        acc.y = fmaf(w, v[i].y, acc.y);
-        acc.z = fmaf(w, v[i].z, acc.z);
-        acc.w = fmaf(w, v[i].w, acc.w);
-    }
-    sum[wave][lane] = acc;
-    mw[wave][lane] = make_float2(m, wsum);
+    for (int i = 0; i < PW; ++i)
+        if (wave + 4 * i < nsplit) M = fmaxf(M, st[i].x);
+    mx[wave][lane] = M;
     __syncthreads();
-    if (wave != 0 || (long)blockIdx.x * 64 + lane >= groups) return;
-    float M = m;  // (wave 0 always has a split; a wave without one weighs 2^-inf)
 #pragma unroll
-    for (int w = 1; w < 4; ++w) M = fmaxf(M, mw[w][lane].x);
-    float ws = 0.f;
-    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int w = 0; w < 4; ++w) M = fmaxf(M, mx[w][lane]);
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        if (w >= nsplit) continue;
-        const float f = __builtin_amdgcn_exp2f((mw[w][lane].x - M) * c0);
-        const float4 x = sum[w][lane];
-        ws = fmaf(f, mw[w][lane].y, ws);
-        o.x = fmaf(f, x.x, o.x);
-        o.y = fmaf(f, x.y, o.y);
-        o.z = fmaf(f, x.z, o.z);
-        o.w = fmaf(f, x.w, o.w);
+    for (int i = 0; i < PW; ++i) {
+        if (wave + 4 * i >= nsplit) continue;
+        wt[wave + 4 * i][lane] = __builtin_amdgcn_exp2f(fmaf(st[i].x - M, st[i].y, st[i].z));
+        val[wave + 4 * i][lane] = v[i];
     }
-    const float inv = 1.f / ws;
-    Elem<T>::st4(Og + (size_t)row * D, d, make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv));
+    __syncthreads();
+    if (wave != 0 || blockIdx.x * 64 + lane >= groups) return;
+    float wsum = 0.f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+    for (int s = 0; s < nsplit; ++s) {
+        const float w = wt[s][lane];
+        const float4 x = val[s][lane];
+        wsum += w;
+        acc.x = fmaf(w, x.x, acc.x);
+        acc.y = fmaf(w, x.y, acc.y);
+        acc.z = fmaf(w, x.z, acc.z);
+        acc.w = fmaf(w, x.w, acc.w);
+    }
+    const float inv = 1.f / wsum;
+    Elem<T>::st4(Og + (size_t)row * D, d,
+                 make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv));
 }
 
 // the arguments of one flash call (pointers typed by the launch)
@@ -968,10 +964,10 @@ hipError_t launch_t(const FlashArgs& a, hipStream_t st) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.nsplit == 1) return e;
     const long groups = (long)a.BH * a.Lq * (a.D / 4);
-    if (groups < (1 << 15) && a.nsplit >= 4 && a.nsplit <= 32) {
+    if (groups < kFewGroups && a.nsplit >= 4 && a.nsplit <= kFewSplits) {
         hipLaunchKernelGGL((k_flash_combine_few<T>), dim3((unsigned)((groups + 63) / 64)),
                            dim3(256), 0, st, a.part, a.stats, static_cast<T*>(a.O), a.Lq, a.D,
-                           a.nsplit, groups);
+                           a.nsplit, (unsigned)groups);
         return hipGetLastError();
     }
     hipLaunchKernelGGL((k_flash_combine<T>), dim3((unsigned)((groups + 255) / 256)), dim3(256), 0,

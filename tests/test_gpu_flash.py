@@ -741,3 +741,45 @@ def test_flash_three_quarter_heads(am, dev, tuner, dt, D, pe, form):
                                     nthreads=16)
     n, a, b = H.check_f32(out.numpy(), ref) if dt == "f32" else H.check_bf16(out.numpy(), ref)
     assert n == 0, (a, b)
+
+
+@pytest.mark.parametrize("shape,parts", [((1, 32, 1, 8192, 128), 8), ((4, 16, 1, 8192, 128), 4)], ids=str)
+def test_flash_decode_splits(am, dev, tuner, shape, parts):
+    """One bf16 query row against keys and values of over 100 MB: one workgroup
+    a CU streams them, so the call's splits are those of 256 workgroups (P is
+    rounded to bf16 against each part's own maxima, so other splits give other
+    bits)."""
+    import hip_rt
+    B, Hh, Lq, Lk, D = shape
+    print(f"[case] decode splits {shape}", flush=True)
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 760, "bf16")
+    out, same, more = (H.empty(Q.shape, "bf16") for _ in range(3))
+    am.attention_ex(q, k, v, out)
+    tuner.set(flash_split=parts)
+    am.attention_ex(q, k, v, same)
+    tuner.set(flash_split=2 * parts)
+    am.attention_ex(q, k, v, more)
+    hip_rt.synchronize()
+    assert np.array_equal(out.bits(), same.bits())
+    assert not np.array_equal(out.bits(), more.bits())
+    n, nrel, mabs = H.check_bf16(out.numpy(), oracle.attention(Q, K, V, nthreads=16))
+    assert n == 0, (nrel, mabs)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("parts", [4, 5])
+def test_flash_merges_agree(am, dev, tuner, dt, parts):
+    """The merge of few rows adds the parts in the order of the other one: a
+    head by itself and among 16 heads of 64 rows give the same bits."""
+    import hip_rt
+    B, Hh, Lq, Lk, D = 1, 16, 64, 320, 128  # 32768 groups of 4 dims: the merge of many rows
+    print(f"[case] merges agree {dt} {parts} parts", flush=True)
+    tuner.set(flash_split=parts)
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 770, dt)
+    many = H.empty(Q.shape, dt)
+    am.attention_ex(q, k, v, many)
+    q1, k1, v1 = (H.upload(x[:, :1], dt) for x in (Q, K, V))
+    one = H.empty((B, 1, Lq, D), dt)
+    am.attention_ex(q1, k1, v1, one)
+    hip_rt.synchronize()
+    assert np.array_equal(one.numpy(), many.numpy()[:, :1])
