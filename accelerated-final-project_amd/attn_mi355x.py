@@ -84,6 +84,13 @@ class FusedPlanInfo(ctypes.Structure):
         "rows", "dc", "nchunk", "gather1", "xcd", "workgroups", "lds")]
 
 
+class CallPlanInfo(ctypes.Structure):
+    """atn_call_plan_info."""
+    _fields_ = [(n, ctypes.c_int) for n in (
+        "path", "tiles", "flash_form", "flash_parts", "keys_once", "chunk_heads",
+        "chunk_rows")] + [("scratch", ctypes.c_size_t)]
+
+
 class AtnError(RuntimeError):
     def __init__(self, status: int, where: str):
         self.status = status
@@ -122,6 +129,8 @@ _SIGS = {
     "atn_get_tuning_ex": ([ctypes.POINTER(Tuning)], _i),
     "atn_fused_plan_ex": ([_i] * 6 + [ctypes.POINTER(PeDesc), ctypes.POINTER(FusedPlanInfo)],
                           _i),
+    "atn_call_plan_ex": ([_i] * 6 + [ctypes.POINTER(PeDesc), ctypes.c_size_t,
+                                     ctypes.POINTER(CallPlanInfo)], _i),
     "atn_rerun_count": ([_i], ctypes.c_long),
     "atn_retained_bytes_ex": ([], ctypes.c_size_t),
     "atn_release_ex": ([], _i),
@@ -238,6 +247,19 @@ def fused_plan(dtype_code: int, B, H, Lq, Lk, D, pe: PeDesc | None = None) -> di
     if r == 0:
         return None
     return {n: getattr(info, n) for n, _ in FusedPlanInfo._fields_}
+
+
+def call_plan(dtype_code: int, B, H, Lq, Lk, D, pe: PeDesc | None = None,
+              scratch_bytes: int = 0) -> dict:
+    """What a call of the shape runs as with this much scratch (0: the cap of
+    the library's own workspace)."""
+    info = CallPlanInfo()
+    st = lib().atn_call_plan_ex(dtype_code, B, H, Lq, Lk, D,
+                                ctypes.byref(pe) if pe is not None else None, scratch_bytes,
+                                ctypes.byref(info))
+    if st != ATN_OK:
+        raise AtnError(st, "atn_call_plan_ex")
+    return {n: getattr(info, n) for n, _ in CallPlanInfo._fields_}
 
 
 def rerun_count(reset: bool = False) -> int:

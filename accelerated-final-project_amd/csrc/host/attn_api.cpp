@@ -1053,25 +1053,54 @@ void plan_flash(int dtype, const Shape& s, PePlan& plan, size_t cap) {
     plan.dchunk = tp.dchunk;
 }
 
-// Scratch bytes of the path a call of shape s takes: fused (when planned and
-// vector-aligned), else GEMM (when planned and 16-byte aligned), else the
-// split-D pipeline.  vec / a16: the alignment of the call's pointers; pass
+// The kernels that a call (or chunk) of shape s runs on, and their scratch:
+// fused (when planned and vector-aligned), else flash, else GEMM (both 16-byte
+// aligned), else the split-D pipeline, on the tiles where tile_plan has one.
+struct Route {
+    int path = ATN_PATH_SPLIT_D;  // ATN_PATH_*
+    FusedPlan fused;
+    GemmPlan gemm;
+    TilePlan tile;
+    size_t need = 0;
+};
+
+Route route(int dtype, const Shape& s, const PePlan& plan, bool query_device, bool vec, bool a16) {
+    Route r;
+    if (!plan.no_fused && vec) r.fused = fused_plan(dtype, plan.pek, s, query_device);
+    if (r.fused.ok) {
+        r.path = ATN_PATH_FUSED_SMALL;
+        r.need = r.fused.bytes;
+        return r;
+    }
+    if (a16 && flash_ok(dtype, s, plan)) {  // only its key splits' parts and K~
+        r.path = ATN_PATH_FLASH;
+        r.need = kSyncBytes + flash_bytes(s, plan.flash);
+        return r;
+    }
+    r.tile = tile_plan(dtype, s, plan, a16);
+    if (a16 && !(plan.tiles && r.tile.ok)) r.gemm = gemm_plan(dtype, s, plan);
+    if (r.gemm.ok) {
+        r.path = ATN_PATH_GEMM;
+        r.need = r.gemm.bytes;
+        return r;
+    }
+    r.need = r.tile.ok ? r.tile.bytes : kSyncBytes + stream_plan(s).bytes;
+    return r;
+}
+
+// A route's scratch.  vec / a16: the alignment of the call's pointers; pass
 // -1 for "unknown" and get the largest of the candidate paths instead.
 size_t path_need(int dtype, const Shape& s, const PePlan& plan, bool query_device, int vec,
                  int a16) {
+    if (vec >= 0 && a16 >= 0) return route(dtype, s, plan, query_device, vec != 0, a16 != 0).need;
     const FusedPlan fp = plan.no_fused ? FusedPlan{} : fused_plan(dtype, plan.pek, s, query_device);
-    const GemmPlan gp = gemm_plan(dtype, s, plan);
     if (fp.ok && vec > 0) return fp.bytes;
-    if (a16 > 0 && vec >= 0 && flash_ok(dtype, s, plan))  // the flash kernel: only its key splits' parts
-        return kSyncBytes + flash_bytes(s, plan.flash);
+    const GemmPlan gp = gemm_plan(dtype, s, plan);
     const TilePlan tp = tile_plan(dtype, s, plan, a16 > 0);
     const size_t split = tp.ok ? tp.bytes : kSyncBytes + stream_plan(s).bytes;
-    if (vec < 0 || a16 < 0)
-        return std::max({fp.ok ? fp.bytes : (size_t)0, gp.ok ? gp.bytes : (size_t)0, split,
-                         flash_ok(dtype, s, plan) ? kSyncBytes + flash_bytes(s, plan.flash)
-                                                  : (size_t)0});
-    if (gp.ok && a16 && !(plan.tiles && tp.ok)) return gp.bytes;
-    return split;
+    return std::max({fp.ok ? fp.bytes : (size_t)0, gp.ok ? gp.bytes : (size_t)0, split,
+                     flash_ok(dtype, s, plan) ? kSyncBytes + flash_bytes(s, plan.flash)
+                                              : (size_t)0});
 }
 
 // How a call too large for its scratch is split: chunks of `heads`
@@ -1117,6 +1146,26 @@ Chunking plan_chunks(int dtype, const Shape& s, const PePlan& plan, size_t cap,
     return ch;
 }
 
+// Plans a call: fills plan's choices (tiles, flash, lean) and returns the
+// chunks it runs in with `cap` bytes of scratch (one of all heads and rows
+// where the whole call fits; heads == 0 where none does).  vec / a16: the
+// alignment of the call's tensors.  Chunk pointers keep it when a row is a
+// multiple of 16 bytes; otherwise the largest path is planned for.
+Chunking plan_call(int dtype, const Shape& s, PePlan& plan, size_t cap, bool query_device,
+                   int vec, int a16) {
+    if (!flash_ok(dtype, s, plan) &&
+        (plan.no_fused || !fused_plan(dtype, plan.pek, s, query_device).ok))
+        choose_tiles(dtype, s, plan);
+    if (flash_ok(dtype, s, plan)) plan_flash(dtype, s, plan, cap);
+    if ((s.D * elem_size(dtype)) % 16 != 0) vec = a16 = -1;
+    Chunking ch = plan_chunks(dtype, s, plan, cap, query_device, vec, a16);
+    if (ch.heads == 0) {  // not even a row beside the copies of K: without them
+        plan.lean = true;
+        ch = plan_chunks(dtype, s, plan, cap, query_device, vec, a16);
+    }
+    return ch;
+}
+
 // One call of the chosen path on (a chunk of) the job, tables already
 // bound; plan.q's tables start at the chunk's first query position.
 int attention_run(int dtype, const void* Q, const void* K, const void* V, void* out,
@@ -1124,27 +1173,16 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
                   size_t workspace_bytes, hipStream_t stream, bool no_alloc) {
     const int Lq = s.Lq, Lk = s.Lk, D = s.D;
     int st = ATN_OK;
-    const GemmPlan gp = gemm_plan(dtype, s, plan);
-    const StreamPlan sp = stream_plan(s);
-    // the device's own capacity decides between the single-launch kernel
-    // and the three-kernel pipeline
-    const FusedPlan fd = plan.no_fused ? FusedPlan{} : fused_plan(dtype, plan.pek, s, true);
     const size_t va = dtype == ATN_DTYPE_F32 ? 16 : 8;
     const int vec_qk = (D % 4 == 0) && aligned(Q, va) && aligned(K, va);
     const int vec_vo = (D % 4 == 0) && aligned(V, va) && aligned(out, va);
-    const bool use_fused = fd.ok && vec_qk && vec_vo;
     const bool a16 = aligned(Q, 16) && aligned(K, 16) && aligned(V, 16) && aligned(out, 16);
-    const bool use_flash = !use_fused && a16 && flash_ok(dtype, s, plan);
-    const bool use_gemm =
-        !use_fused && !use_flash && gp.ok && a16 && !(plan.tiles && !plan.lean);
-    const TilePlan tp = use_fused || use_flash || use_gemm ? TilePlan{}
-                                                           : tile_plan(dtype, s, plan, a16);
-    const bool use_tile = tp.ok;
-    const size_t need =
-        use_fused ? fd.bytes
-                  : (use_flash ? kSyncBytes + flash_bytes(s, plan.flash)
-                               : (use_gemm ? gp.bytes
-                                           : (use_tile ? tp.bytes : kSyncBytes + sp.bytes)));
+    // (the device's own capacity decides about the single-launch kernel)
+    const Route r = route(dtype, s, plan, true, vec_qk && vec_vo, a16);
+    const FusedPlan& fd = r.fused;
+    const GemmPlan& gp = r.gemm;
+    const TilePlan& tp = r.tile;
+    const size_t need = r.need;
     void* ws = workspace;
     if (no_alloc) {
         if (need > atn::kNoAllocScratchBytes) return ATN_ERR_SCRATCH_LIMIT;
@@ -1165,7 +1203,7 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
     const float scale = 1.0f / sqrtf((float)D);  // final/attention.cu:206
 
     float* scratch = reinterpret_cast<float*>((char*)ws + kSyncBytes);
-    if (use_gemm) {
+    if (r.path == ATN_PATH_GEMM) {
         char* w = static_cast<char*>(ws);
         const uint16_t* qe = static_cast<const uint16_t*>(Q);
         const uint16_t* ke = static_cast<const uint16_t*>(K);
@@ -1210,7 +1248,7 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
                                     static_cast<uint16_t*>(out), (int)s.BH, Lq, Lk, D, stream));
         return ATN_OK;
     }
-    if (use_fused) {
+    if (r.path == ATN_PATH_FUSED_SMALL) {
         unsigned* epochs = reinterpret_cast<unsigned*>((char*)ws + kSyncEpochOff);
         float* part = reinterpret_cast<float*>((char*)ws + kSyncBytes);
         float* red = reinterpret_cast<float*>((char*)ws + kSyncBytes + round256(fd.part_words * 4));
@@ -1231,7 +1269,7 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
                                         stream));
         return ATN_OK;
     }
-    if (use_flash) {
+    if (r.path == ATN_PATH_FLASH) {
         const void* kt = K;
         const float* kunit = nullptr;
         const FlashPlan& f = plan.flash;
@@ -1249,7 +1287,7 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
                                   stream));
         return ATN_OK;
     }
-    if (use_tile) {
+    if (tp.ok) {
         char* w = static_cast<char*>(ws);
         uint16_t* ph = reinterpret_cast<uint16_t*>(w + tp.ph_off);
         uint16_t* pl = reinterpret_cast<uint16_t*>(w + tp.pl_off);
@@ -1281,6 +1319,7 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
         ATN_HIP(atn::launch_pv_tile(dtype, tp.tile_pv, pa, stream));
         return ATN_OK;
     }
+    const StreamPlan sp = stream_plan(s);
     float* S = scratch;
     float* P = sp.nsplit > 1 ? S + sp.s_elems : S;
     ATN_HIP(atn::launch_qk_partial(dtype, plan.pek, Q, K, S, (int)s.BH, Lq, Lk, D, sp.dchunk,
@@ -1334,34 +1373,18 @@ int attention_core(int dtype, const void* Q, const void* K, const void* V, void*
     st = bind_tables(pe, plan, D, Lq > Lk ? Lq : Lk, stream, no_alloc);
     if (st != ATN_OK) return st;
 
-    if (!flash_ok(dtype, s, plan) &&
-        (plan.no_fused || !fused_plan(dtype, plan.pek, s, true).ok))
-        choose_tiles(dtype, s, plan);
-
     const size_t cap = no_alloc ? atn::kNoAllocScratchBytes
                                 : (workspace != nullptr ? workspace_bytes : library_cap());
-    if (flash_ok(dtype, s, plan)) plan_flash(dtype, s, plan, cap);
-    // chunk pointers keep the base alignment when a row is a multiple of 16
-    // bytes; otherwise plan for the largest path
     const size_t va = dtype == ATN_DTYPE_F32 ? 16 : 8;
-    const bool rows16 = ((size_t)D * es) % 16 == 0;
-    const int vec = rows16 ? ((D % 4 == 0) && aligned(Q, va) && aligned(K, va) &&
-                              aligned(V, va) && aligned(out, va))
-                           : -1;
-    const int a16 = rows16 ? (aligned(Q, 16) && aligned(K, 16) && aligned(V, 16) &&
-                              aligned(out, 16))
-                           : -1;
-    if (path_need(dtype, s, plan, true, vec, a16) <= cap)
+    bool vec = D % 4 == 0, a16 = true;
+    for (const void* p : {Q, K, V, (const void*)out}) {
+        vec = vec && aligned(p, va);
+        a16 = a16 && aligned(p, 16);
+    }
+    const Chunking ch = plan_call(dtype, s, plan, cap, true, vec, a16);
+    if (ch.heads == s.BH && ch.rows == Lq)
         return attention_run(dtype, Q, K, V, out, s, plan, dev, workspace, workspace_bytes,
                              stream, no_alloc);
-    Chunking ch = plan_chunks(dtype, s, plan, cap, true, vec, a16);
-    if (ch.heads == 0) {  // not even a row beside the copies of K: without them
-        plan.lean = true;
-        if (path_need(dtype, s, plan, true, vec, a16) <= cap)
-            return attention_run(dtype, Q, K, V, out, s, plan, dev, workspace, workspace_bytes,
-                                 stream, no_alloc);
-        ch = plan_chunks(dtype, s, plan, cap, true, vec, a16);
-    }
     if (ch.heads == 0) return no_alloc ? ATN_ERR_SCRATCH_LIMIT : ATN_ERR_WORKSPACE;
     const char* q8 = static_cast<const char*>(Q);
     const char* k8 = static_cast<const char*>(K);
@@ -1766,6 +1789,41 @@ int atn_attention_path_ex(int dtype, int batch, int heads, int len_q, int len_k,
     if (flash_ok(dtype, s, plan)) return ATN_PATH_FLASH;
     if (gemm_plan(dtype, s, plan).ok) return ATN_PATH_GEMM;
     return ATN_PATH_SPLIT_D;
+}
+
+int atn_call_plan_ex(int dtype, int batch, int heads, int len_q, int len_k, int head_d,
+                     const atn_pe_desc* pe, size_t scratch_bytes, atn_call_plan_info* info) {
+    if (!info) return ATN_ERR_NULL_POINTER;
+    if (dtype != ATN_DTYPE_F32 && dtype != ATN_DTYPE_BF16) return ATN_ERR_BAD_ARGUMENT;
+    Shape s;
+    int st = check_shape(batch, heads, len_q, len_k, head_d, &s);
+    if (st != ATN_OK) return st;
+    PePlan plan;
+    st = check_pe(pe, head_d, &plan);
+    if (st != ATN_OK) return st;
+    plan.no_fused = tune().no_fused != 0;
+    plan.no_flash = tune().no_flash != 0;
+    int n = 0;
+    const bool dev = hipGetDeviceCount(&n) == hipSuccess && n > 0;
+    const bool vec = head_d % 4 == 0;
+    *info = atn_call_plan_info{};
+    const Chunking ch = plan_call(dtype, s, plan, scratch_bytes ? scratch_bytes : library_cap(), dev,
+                                  vec, true);
+    if (ch.heads == 0) return ATN_ERR_WORKSPACE;
+    Shape c;
+    check_shape(1, ch.heads, ch.rows, len_k, head_d, &c);
+    const Route r = route(dtype, c, plan, dev, vec, true);
+    info->path = r.path;
+    info->tiles = r.path == ATN_PATH_SPLIT_D && r.tile.ok;
+    if (r.path == ATN_PATH_FLASH) {
+        info->flash_form = plan.flash.form;
+        info->flash_parts = plan.flash.nsplit;
+        info->keys_once = plan.flash.kpre;
+    }
+    info->chunk_heads = ch.heads;
+    info->chunk_rows = ch.rows;
+    info->scratch = r.need;
+    return ATN_OK;
 }
 
 int atn_sync_status_ex(void* workspace, int batch, int heads, void* stream) {

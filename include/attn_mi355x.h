@@ -286,11 +286,12 @@ int atn_sync_status_ex(void *workspace, int batch, int heads, void *stream);
  * path -- otherwise built on first use, which synchronizes. */
 int atn_prepare_pe_ex(const atn_pe_desc *pe, int head_d, int max_positions);
 
-/* Which kernels atn_attention_fwd_ex runs for this shape on the current
- * device (ATN_PATH_*), or a negative status for invalid arguments, assuming
+/* Which path atn_attention_fwd_ex takes for this shape on the current device
+ * (ATN_PATH_*), or a negative status for invalid arguments, assuming
  * vector-aligned tensors (16-byte fp32 / 8-byte bf16 bases; otherwise the
  * split-D pipeline runs).  Without a device the answer assumes 256 compute
- * units. */
+ * units.  Small grids of the FLASH and GEMM paths run the split-D kernels
+ * where those are faster: atn_call_plan_ex reports what runs. */
 #define ATN_PATH_FUSED_SMALL 1 /* one launch: split-D slices + device-side S all-reduce */
 #define ATN_PATH_SPLIT_D 2     /* partial QK^T over D-chunks, softmax, PV (before them a pass
                                   that encodes Q and K, or pads bf16 rows) */
@@ -372,6 +373,27 @@ typedef struct atn_fused_plan_info {
 } atn_fused_plan_info;
 int atn_fused_plan_ex(int dtype, int batch, int heads, int len_q, int len_k, int head_d,
                       const atn_pe_desc *pe, atn_fused_plan_info *info);
+
+/* What a call of this shape runs as on the current device (without one: the
+ * atn_tuning model), with `scratch_bytes` of scratch (0: the cap of the
+ * library's own workspace), for 16-byte aligned tensors.  Returns ATN_OK, or
+ * ATN_ERR_WORKSPACE where no chunk fits the scratch, or another negative
+ * status. */
+typedef struct atn_call_plan_info {
+    int path;        /* ATN_PATH_* of the kernels that run: SPLIT_D also for calls that
+                        atn_attention_path_ex reports as FLASH or GEMM and that run the
+                        split-D tiles */
+    int tiles;       /* path SPLIT_D: 1 the pipelined 16-bit tiles, 0 the kernels that need
+                        no copies */
+    int flash_form;  /* path FLASH: workgroup form (atn_tuning.flash_form) */
+    int flash_parts; /* ... key splits (1: none) */
+    int keys_once;   /* ... 1: K is encoded once into the scratch */
+    int chunk_heads; /* (batch, head) pairs and query rows of a chunk (batch * heads and */
+    int chunk_rows;  /*   len_q: the call is not split) */
+    size_t scratch;  /* scratch of one chunk in bytes */
+} atn_call_plan_info;
+int atn_call_plan_ex(int dtype, int batch, int heads, int len_q, int len_k, int head_d,
+                     const atn_pe_desc *pe, size_t scratch_bytes, atn_call_plan_info *info);
 
 /* Synchronous drop-in calls that were run a second time without the
  * single-launch kernel after its wait timed out (each such rerun also

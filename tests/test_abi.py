@@ -180,6 +180,31 @@ def test_path_selection_without_device(am, tuner):
     assert am.path(1, 4, 32, 512, 512, 128) == am.ATN_PATH_GEMM
 
 
+def test_call_plan_reports_what_runs(am, tuner):
+    """atn_call_plan_ex: the kernels of a call, also where a path's small
+    grids run on others, and its chunks."""
+    whole = lambda p, BH, Lq: (p["chunk_heads"], p["chunk_rows"]) == (BH, Lq)  # noqa: E731
+    p = am.call_plan(0, 1, 4, 64, 64, 2048)
+    assert p["path"] == am.ATN_PATH_FUSED_SMALL and whole(p, 4, 64)
+    p = am.call_plan(1, 1, 32, 1, 8192, 128)
+    assert (p["path"], p["flash_form"], p["flash_parts"], p["keys_once"]) == (am.ATN_PATH_FLASH, 1, 8, 0)
+    p = am.call_plan(1, 4, 8, 1107, 1107, 128, am.make_pe("rope"))
+    assert p["path"] == am.ATN_PATH_FLASH and p["keys_once"] == 1
+    for shape, path in [((1, 4, 417, 417, 256), am.ATN_PATH_FLASH), ((1, 2, 68, 68, 624), am.ATN_PATH_GEMM)]:
+        assert am.path(1, *shape) == path
+        p = am.call_plan(1, *shape)
+        assert (p["path"], p["tiles"]) == (am.ATN_PATH_SPLIT_D, 1) and whole(p, shape[1], shape[2])
+    p = am.call_plan(1, 8, 8, 1024, 1024, 4096, am.make_pe("rope", "half"))
+    assert p["path"] == am.ATN_PATH_GEMM
+    # little scratch: chunks of rows of one head, without copies; none at all
+    p = am.call_plan(0, 1, 2, 700, 400, 1024, am.make_pe("rope"), 1 << 20)
+    assert (p["path"], p["tiles"], p["chunk_heads"]) == (am.ATN_PATH_SPLIT_D, 0, 1)
+    assert p["chunk_rows"] < 700 and p["scratch"] <= 1 << 20
+    with pytest.raises(am.AtnError) as e:
+        am.call_plan(0, 1, 2, 700, 400000, 1024, None, 1 << 20)
+    assert e.value.status == am.ATN_ERR_WORKSPACE
+
+
 def test_no_device_path(am, L):
     if am.device_count() > 0:
         pytest.skip("a HIP device is visible; the no-device path is exercised on the CPU host")
