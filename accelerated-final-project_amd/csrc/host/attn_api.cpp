@@ -867,8 +867,11 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
 // and win there: (1,2,68,68,624) 37.3 -> 10.6 us, (2,4,82,82,2392) 72.5 ->
 // 16.3, (1,4,512,512,2048) 62.5 -> 31, (1,8,64,4096,2048) 195 -> 91; from
 // about 128 GEMM tiles on the GEMMs lead ((4,8,444,444,1008) 66 against 93
-// us, (4,16,508,508,1888) 201 against 315).
-void choose_tiles(int dtype, const Shape& s, PePlan& plan) {
+// us, (4,16,508,508,1888) 201 against 315).  Only where the whole call's scratch
+// fits: the tiles need fp32 copies of encoded Q and K, and in chunks of a head
+// or fewer each they lose to the one GEMM call ((1,8,64,4096,2048) rotate-half
+// in 64 MiB 715 us, the GEMMs 225).
+void choose_tiles(int dtype, const Shape& s, PePlan& plan, size_t cap) {
     const TilePlan tp = tile_plan(dtype, s, plan, true);
     if (!tp.ok) return;
     plan.dchunk = tp.dchunk;
@@ -882,7 +885,7 @@ void choose_tiles(int dtype, const Shape& s, PePlan& plan) {
                 std::ceil(wgs(s.Lq, s.D)) * ((s.Lk + 63) / 64) * 2.2;
     if (gp.encoded) us += 4.0 + (double)s.nq * 4.0 / 4.5e6;
     if (gp.encoded && gp.benc == 0) us += 4.0 + (double)s.nk * 4.0 / 4.5e6;
-    plan.tiles = tp.us < 0.95 * us;
+    plan.tiles = tp.bytes <= cap && tp.us < 0.95 * us;
 }
 
 // ---------------------------------------------------------------- core
@@ -1155,7 +1158,7 @@ Chunking plan_call(int dtype, const Shape& s, PePlan& plan, size_t cap, bool que
                    int vec, int a16) {
     if (!flash_ok(dtype, s, plan) &&
         (plan.no_fused || !fused_plan(dtype, plan.pek, s, query_device).ok))
-        choose_tiles(dtype, s, plan);
+        choose_tiles(dtype, s, plan, cap);
     if (flash_ok(dtype, s, plan)) plan_flash(dtype, s, plan, cap);
     if ((s.D * elem_size(dtype)) % 16 != 0) vec = a16 = -1;
     Chunking ch = plan_chunks(dtype, s, plan, cap, query_device, vec, a16);
@@ -1752,7 +1755,7 @@ size_t atn_attention_workspace_bytes(int dtype, int batch, int heads, int len_q,
     if (check_shape(batch, heads, len_q, len_k, head_d, &s) != ATN_OK) return 0;
     PePlan plan;
     if (check_pe(pe, head_d, &plan) != ATN_OK) return 0;
-    choose_tiles(dtype, s, plan);
+    choose_tiles(dtype, s, plan, library_cap());
     if (flash_ok(dtype, s, plan)) plan_flash(dtype, s, plan, library_cap());
     // the largest workspace of every plan the call could take, or, when that
     // exceeds the library's cap, of the chunks the call then runs in
