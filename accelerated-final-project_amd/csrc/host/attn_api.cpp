@@ -840,6 +840,8 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
     // and 4 written per element of Q and K; 4 and 4 for fp32)
     p.us = best + std::min(pv64, pv128) + 9.0 + (double)s.BH * s.Lq * p.ldS * 4.0 / 5.5e6;
     if (plan.pek != atn::kPeNone) p.us += 3.0 + (double)(s.nq + s.nk) * (bf ? 6.0 : 8.0) / 4.5e6;
+    // (the padding pass: V, and Q and K where no encoding pass writes them)
+    if (p.Dp) p.us += 3.0 + (double)(s.nk + (plan.pek == atn::kPeNone ? s.nq + s.nk : 0)) * 4.0 / 4.5e6;
     size_t off = kSyncBytes;
     auto take = [&](size_t b) { size_t o = off; off += round256(b); return o; };
     take((size_t)p.nsplit * s.BH * s.Lq * p.ldS * 4);
@@ -1162,11 +1164,33 @@ Chunking plan_call(int dtype, const Shape& s, PePlan& plan, size_t cap, bool que
     if (flash_ok(dtype, s, plan)) plan_flash(dtype, s, plan, cap);
     if ((s.D * elem_size(dtype)) % 16 != 0) vec = a16 = -1;
     Chunking ch = plan_chunks(dtype, s, plan, cap, query_device, vec, a16);
-    if (ch.heads == 0) {  // not even a row beside the copies of K: without them
-        plan.lean = true;
-        ch = plan_chunks(dtype, s, plan, cap, query_device, vec, a16);
+    if (ch.heads == s.BH && ch.rows == s.Lq) return ch;
+    // Not the whole call: without copies of K (and V) a chunk holds more heads
+    // or rows, and where the copies leave room for a few rows only, each such
+    // chunk writes them again: fp32 RoPE (1,1,4096,4000,4096) in 64 MiB, which
+    // K~ fills up to 1.4, ran in 256 chunks of 16 rows, 31.1 ms, whole without
+    // copies 3.4 ms; at 80 MiB the tiles' chunks lead again (2.25 ms).  By
+    // estimate: the kernels without copies take 2.2 to 4.2 times the tiles'
+    // time (1010 us against 240 at bf16 (1,1,2000,4000,3004), 135 against 62 at
+    // RoPE (1,4,512,512,2048)).
+    PePlan lean = plan;
+    lean.lean = true;
+    const Chunking lc = plan_chunks(dtype, s, lean, cap, query_device, vec, a16);
+    if (lc.heads == 0) return ch;
+    if (ch.heads != 0) {
+        auto us = [&](const Chunking& c) {
+            Shape x;
+            check_shape(1, c.heads, c.rows, s.Lk, s.D, &x);
+            return (double)((s.BH + c.heads - 1) / c.heads) * ((s.Lq + c.rows - 1) / c.rows) *
+                   tile_plan(dtype, x, plan, a16 > 0).us;
+        };
+        Shape x;
+        check_shape(1, ch.heads, ch.rows, s.Lk, s.D, &x);
+        if (!route(dtype, x, plan, query_device, vec > 0, a16 > 0).tile.ok || us(ch) <= 3.5 * us(lc))
+            return ch;
     }
-    return ch;
+    plan.lean = true;
+    return lc;
 }
 
 // One call of the chosen path on (a chunk of) the job, tables already

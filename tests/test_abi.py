@@ -217,6 +217,21 @@ def test_tiles_only_where_the_whole_call_fits(am):
     assert p["tiles"] == 1 and p["chunk_heads"] == 2
 
 
+@pytest.mark.parametrize("dtype,shape,pe,mib", [
+    (0, (1, 1, 4096, 4000, 4096), "rope", (64, 96)),   # K~ 62.5 MiB of the scratch
+    (1, (1, 1, 2000, 4000, 3004), "none", (48, 64)),   # padded K and V 45.9 MiB
+], ids=str)
+def test_no_chunks_of_a_few_rows_beside_copies(am, dtype, shape, pe, mib):
+    """Scratch just above what the copies of K (and V) take: the kernels
+    without copies, instead of many chunks of a few rows that each write them
+    again; with room for more rows, the tiles."""
+    desc = am.make_pe(pe) if pe != "none" else None
+    tight, room = (am.call_plan(dtype, *shape, desc, m << 20) for m in mib)
+    assert tight["path"] == am.ATN_PATH_SPLIT_D and tight["tiles"] == 0
+    assert tight["chunk_rows"] * 4 >= shape[2]
+    assert room["tiles"] == 1 and room["chunk_rows"] * 16 >= shape[2]
+
+
 def test_no_device_path(am, L):
     if am.device_count() > 0:
         pytest.skip("a HIP device is visible; the no-device path is exercised on the CPU host")

@@ -107,6 +107,24 @@ def test_scratch_without_encoded_copies(am, dev, tuner, pe):
     _check(out.numpy(), Q, K, V, pe)
 
 
+@pytest.mark.parametrize("dt,D,pe,kib", [("f32", 1024, "rope", 1160), ("bf16", 1004, "none", 1200)], ids=str)
+def test_scratch_that_copies_nearly_fill(am, dev, dt, D, pe, kib):
+    """K's copy (and V's) would leave the scratch a few rows a chunk: the
+    kernels without copies."""
+    import hip_rt
+    B, Hh, Lq, Lk = 1, 1, 300, 260
+    print(f"[case] copies nearly fill the scratch {dt} {D} {pe}", flush=True)
+    desc, code = _desc(am, pe), {"f32": 0, "bf16": 1}[dt]
+    assert am.call_plan(code, B, Hh, Lq, Lk, D, desc, kib << 10)["tiles"] == 0
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 975, dt)
+    ws = hip_rt.DeviceArray(((kib << 10) // 4,), "f32", fill=0)
+    out = H.empty(Q.shape, dt)
+    am.attention_ex(q, k, v, out, pe=desc, workspace=ws)
+    hip_rt.synchronize()
+    n, a, b = (H.check_f32 if dt == "f32" else H.check_bf16)(out.numpy(), _ref(pe, Q, K, V))
+    assert n == 0, (a, b)
+
+
 @pytest.mark.parametrize("tile", [0, 64, 128])
 @pytest.mark.parametrize("shape,pe", [
     ((1, 2, 68, 68, 624), "none"),       # a small grid of the GEMM path's
