@@ -999,8 +999,10 @@ FlashPlan flash_plan_uncached(int dtype, const Shape& s, const PePlan& plan, siz
             const bool two = fi == 0 || (bf && !enc && fi == 1 && dc < 2);
             const double pair = fi == 0 ? 1.5 : 1.78;
             int last = 0;
-            for (int n = 1; n <= std::min(chunks, 32); ++n) {
-                if (tn.flash_split >= 1 && n != std::min(tn.flash_split, chunks)) continue;
+            // (a forced count, which may exceed the 32 that the choice considers)
+            const int lo = tn.flash_split >= 1 ? std::min(tn.flash_split, chunks) : 1;
+            const int hi = tn.flash_split >= 1 ? lo : std::min(chunks, 32);
+            for (int n = lo; n <= hi; ++n) {
                 const int per = (chunks + n - 1) / n, ns = (chunks + per - 1) / per;
                 if (ns == last) continue;
                 last = ns;

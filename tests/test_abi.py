@@ -217,6 +217,17 @@ def test_tiles_only_where_the_whole_call_fits(am):
     assert p["tiles"] == 1 and p["chunk_heads"] == 2
 
 
+@pytest.mark.parametrize("parts,Lk,got", [(2, 2112, 2), (32, 2112, 17), (33, 2112, 33), (40, 5000, 40),
+                                          (100, 2112, 33), (1, 5000, 1)])
+def test_forced_key_splits(am, tuner, parts, Lk, got):
+    """Any forced count of key splits gives a plan: whole 64-key chunks per
+    part, one at least."""
+    tuner.set(flash_split=parts)
+    p = am.call_plan(0, 1, 3, 70, Lk, 64)
+    assert p["path"] == am.ATN_PATH_FLASH and p["flash_form"] != 0
+    assert p["flash_parts"] == got
+
+
 @pytest.mark.parametrize("dtype,shape,pe,mib", [
     (0, (1, 1, 4096, 4000, 4096), "rope", (64, 96)),   # K~ 62.5 MiB of the scratch
     (1, (1, 1, 2000, 4000, 3004), "none", (48, 64)),   # padded K and V 45.9 MiB

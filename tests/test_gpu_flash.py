@@ -702,7 +702,7 @@ def test_flash_keys_encoded_once(am, dev, tuner, shape, scale, pe):
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
-@pytest.mark.parametrize("parts", [3, 4, 5, 8, 9, 31, 32])
+@pytest.mark.parametrize("parts", [3, 4, 5, 8, 9, 31, 32, 33])
 @pytest.mark.parametrize("Lq", [3, 700], ids=str)
 def test_flash_merge_forms(am, dev, tuner, dt, parts, Lq):
     """Both merge kernels (few rows of 4 to 32 parts; the rest), with parts
