@@ -1164,9 +1164,10 @@ Chunking plan_call(int dtype, const Shape& s, PePlan& plan, size_t cap, bool que
         (plan.no_fused || !fused_plan(dtype, plan.pek, s, query_device).ok))
         choose_tiles(dtype, s, plan, cap);
     if (flash_ok(dtype, s, plan)) plan_flash(dtype, s, plan, cap);
+    const size_t need = route(dtype, s, plan, query_device, vec != 0, a16 != 0).need;
+    if (need <= cap) return Chunking{(int)s.BH, s.Lq, need};
     if ((s.D * elem_size(dtype)) % 16 != 0) vec = a16 = -1;
-    Chunking ch = plan_chunks(dtype, s, plan, cap, query_device, vec, a16);
-    if (ch.heads == s.BH && ch.rows == s.Lq) return ch;
+    const Chunking ch = plan_chunks(dtype, s, plan, cap, query_device, vec, a16);
     // Not the whole call: without copies of K (and V) a chunk holds more heads
     // or rows, and where the copies leave room for a few rows only, each such
     // chunk writes them again: fp32 RoPE (1,1,4096,4000,4096) in 64 MiB, which
@@ -1781,19 +1782,16 @@ size_t atn_attention_workspace_bytes(int dtype, int batch, int heads, int len_q,
     if (check_shape(batch, heads, len_q, len_k, head_d, &s) != ATN_OK) return 0;
     PePlan plan;
     if (check_pe(pe, head_d, &plan) != ATN_OK) return 0;
-    choose_tiles(dtype, s, plan, library_cap());
-    if (flash_ok(dtype, s, plan)) plan_flash(dtype, s, plan, library_cap());
-    // the largest workspace of every plan the call could take, or, when that
-    // exceeds the library's cap, of the chunks the call then runs in
-    const size_t full = path_need(dtype, s, plan, false, -1, -1);
-    if (full <= library_cap()) return full;
-    Chunking ch = plan_chunks(dtype, s, plan, library_cap(), false, -1, -1);
-    if (ch.heads > 0) return ch.need;
+    // what the call takes with aligned tensors, and for others the largest of
+    // every path that needs no copies (copies are made where the scratch holds
+    // them); each in the chunks that the library's cap would cut it into
+    const size_t cap = library_cap();
+    const size_t planned = plan_call(dtype, s, plan, cap, false, head_d % 4 == 0, true).need;
     plan.lean = true;
-    const size_t lean = path_need(dtype, s, plan, false, -1, -1);
-    if (lean <= library_cap()) return lean;
-    ch = plan_chunks(dtype, s, plan, library_cap(), false, -1, -1);
-    return ch.heads > 0 ? ch.need : lean;
+    const size_t full = path_need(dtype, s, plan, false, -1, -1);
+    if (full <= cap) return std::max(full, planned);
+    const Chunking ch = plan_chunks(dtype, s, plan, cap, false, -1, -1);
+    return std::max(ch.heads > 0 ? ch.need : full, planned);
 }
 
 int atn_pe_apply_ex(int dtype, const void* in, void* out, long n_rows, int seq_len, int head_d,

@@ -265,7 +265,9 @@ int atn_attention_fwd_noalloc_ex(int dtype, const void *Q, const void *K, const 
  * in chunks of consecutive (batch, head) pairs, or of query rows of one head,
  * that fit, and this query then reports the largest chunk's need.  Only a
  * shape whose single query row of one head exceeds the cap reports its full
- * need, above the cap: such a call fails with ATN_ERR_WORKSPACE. */
+ * need, above the cap: such a call fails with ATN_ERR_WORKSPACE.  It is what
+ * the call takes with 16-byte aligned tensors, and enough for any others
+ * (which run without aligned copies where those do not fit). */
 size_t atn_attention_workspace_bytes(int dtype, int batch, int heads, int len_q, int len_k,
                                      int head_d, const atn_pe_desc *pe);
 

@@ -143,6 +143,38 @@ def test_workspace_bytes_bound_every_plan(am, tuner, dtype, shape):
         assert am.workspace_bytes(dtype, *shape) == base, (rows, dc, x)
 
 
+@pytest.mark.parametrize("dtype,shape,pe,mb", [
+    (1, (1, 32, 1, 8192, 128), "none", 1.2),        # decoding: partial scores, no copy of the cache
+    (1, (4, 32, 1, 16384, 128), "none", 9),
+    (1, (1, 32, 1, 8192, 100), "none", 1.2),        # rows of 200 bytes
+    (1, (4, 16, 256, 2048, 1024), "sinusoidal", 135),
+    (1, (8, 8, 1024, 1024, 4096), "rope", 675),
+    (0, (4, 32, 512, 512, 128), "none", 135),
+    (1, (4, 8, 1107, 1107, 128), "rope", 157),
+], ids=str)
+def test_workspace_bytes_without_copies_for_other_alignments(am, dtype, shape, pe, mb):
+    """The query covers misaligned tensors by the path that needs no copies of
+    them, not by padded copies of Q, K and V that an aligned call never makes."""
+    desc = am.make_pe(pe, "half" if pe == "rope" else "interleaved") if pe != "none" else None
+    assert am.workspace_bytes(dtype, *shape, desc) <= mb * 1e6
+
+
+def test_workspace_bytes_hold_the_planned_call(am):
+    """A workspace of the reported size runs the call as the library's own
+    scratch does."""
+    rng = np.random.default_rng(5)
+    kinds = [None, am.make_pe("rope"), am.make_pe("rope", "half"), am.make_pe("sinusoidal")]
+    for _ in range(400):
+        shape = (int(rng.integers(1, 5)), int(rng.integers(1, 17)), *(int(2 ** rng.uniform(0, 12)) for _ in range(2)),
+                 2 * int(2 ** rng.uniform(1, 11)) + int(rng.random() < 0.2))
+        dtype, pe = int(rng.integers(0, 2)), kinds[int(rng.integers(0, 4))]
+        if shape[-1] % 2 and pe is not None and pe.kind == am.ATN_PE_ROPE:
+            pe = None
+        free = am.call_plan(dtype, *shape, pe)
+        held = am.call_plan(dtype, *shape, pe, am.workspace_bytes(dtype, *shape, pe))
+        assert held == free, (dtype, shape)
+
+
 def test_path_selection_without_device(am, tuner):
     """Short sequences take the single-launch kernel, long ones the pipeline."""
     assert am.path(0, 1, 4, 64, 64, 2048) == am.ATN_PATH_FUSED_SMALL       # config 2

@@ -175,6 +175,29 @@ def test_misaligned_bases_bf16(am, dev, D):
     assert n == 0, (nrel, mabs)
 
 
+@pytest.mark.parametrize("dt,D", [("bf16", 264), ("bf16", 40), ("bf16", 267), ("f32", 264), ("f32", 64)], ids=str)
+def test_misaligned_bases_in_the_reported_workspace(am, dev, dt, D):
+    """atn_attention_workspace_bytes covers tensors off a 16-byte boundary."""
+    import hip_rt
+    B, Hh, Lq, Lk = 1, 2, 100, 140
+    code, es = (1, 2) if dt == "bf16" else (0, 4)
+    print(f"[case] misaligned in the reported workspace {dt} {D}", flush=True)
+    (Q, K, V) = H.rng_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), seed=963)
+    if dt == "bf16":
+        Q, K, V = (oracle.bf16_bits_to_f32(oracle.f32_to_bf16_bits(x)) for x in (Q, K, V))
+    dev_t = [H.upload(np.concatenate([[0.0], x.ravel()]).astype(np.float32), dt) for x in (Q, K, V)]
+    out = H.empty((Q.size + 1,), dt)
+    nb = am.workspace_bytes(code, B, Hh, Lq, Lk, D)
+    ws = hip_rt.DeviceArray((nb // 4,), "f32", fill=0)
+    st = am.lib().atn_attention_fwd_ex(code, *[t.ptr + es for t in dev_t], out.ptr + es, B, Hh, Lq, Lk, D,
+                                       None, ws.ptr, nb // 4 * 4, None)
+    assert st == 0
+    hip_rt.synchronize()
+    n, a, b = (H.check_f32 if dt == "f32" else H.check_bf16)(out.numpy()[1:].reshape(Q.shape),
+                                                             _ref("none", Q, K, V))
+    assert n == 0, (a, b)
+
+
 @pytest.mark.parametrize("scale", [2.0 ** 40, 2.0 ** -40], ids=str)
 def test_bf16_range(am, dev, scale):
     """bf16 keeps fp32's exponents: V far outside fp16's range."""
