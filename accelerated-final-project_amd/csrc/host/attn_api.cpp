@@ -473,6 +473,14 @@ int ensure_workspace(size_t bytes, hipStream_t stream, void** ws) {
     return ATN_OK;
 }
 
+// Bytes of the stream's library workspace as it stands.
+size_t library_bytes(int dev, hipStream_t stream) {
+    std::lock_guard<std::mutex> lk(g_mu);
+    const auto& m = g_dev[dev].ws;
+    const auto it = m.find(stream);
+    return it == m.end() ? 0 : it->second.bytes;
+}
+
 // ---------------------------------------------------------------- fused plan
 // Workspace layout (every path): a fixed 40 KiB sync region -- [0, 4) the
 // status word, [256, 8448) one epoch word per row group of the
@@ -1411,7 +1419,27 @@ int attention_core(int dtype, const void* Q, const void* K, const void* V, void*
         vec = vec && aligned(p, va);
         a16 = a16 && aligned(p, 16);
     }
-    const Chunking ch = plan_call(dtype, s, plan, cap, true, vec, a16);
+    const PePlan fresh = plan;
+    Chunking ch = plan_call(dtype, s, plan, cap, true, vec, a16);
+    if (workspace == nullptr && !no_alloc && ch.heads != 0) {
+        // The stream's workspace cannot grow while captured.  Where the plan
+        // needs more, the whole call with what there is (another flash plan,
+        // the GEMMs), or the plan without copies; else ATN_ERR_CAPTURE.
+        const size_t have = library_bytes(dev, stream);
+        if (ch.need > have && is_capturing(stream)) {
+            PePlan p = fresh;
+            Chunking c{};
+            if (have >= kSyncBytes) c = plan_call(dtype, s, p, have, true, vec, a16);
+            if (c.heads != s.BH || c.rows != Lq) {
+                p = plan;
+                p.lean = true;
+                c = plan_chunks(dtype, s, p, cap, true, vec, a16);
+            }
+            if (c.heads == 0 || c.need > have) return ATN_ERR_CAPTURE;
+            plan = p;
+            ch = c;
+        }
+    }
     if (ch.heads == s.BH && ch.rows == Lq)
         return attention_run(dtype, Q, K, V, out, s, plan, dev, workspace, workspace_bytes,
                              stream, no_alloc);

@@ -10,6 +10,8 @@ runs here too, as in test_gpu_parity.py.
 fp32 bar: the reference's (abs and rel above 1e-4).  bf16 bar: within rel
 2e-2 of the fp32 oracle run on the bf16-rounded inputs (helpers.check_bf16).
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -783,3 +785,50 @@ def test_flash_merges_agree(am, dev, tuner, dt, parts):
     am.attention_ex(q1, k1, v1, one)
     hip_rt.synchronize()
     assert np.array_equal(one.numpy(), many.numpy()[:, :1])
+
+
+def test_capture_in_a_smaller_workspace(am, dev):
+    """A call whose plan needs more than its stream's workspace is captured on
+    the plan that fits (K encoded in the kernel); one that no plan fits is
+    refused."""
+    import hip_rt
+    B, Hh, Lq, Lk, D = 4, 8, 1107, 1107, 128
+    print("[case] capture in a smaller workspace", flush=True)
+    pe = am.make_pe("rope")
+    assert am.call_plan(1, B, Hh, Lq, Lk, D, pe)["keys_once"] == 1
+    small = am.call_plan(1, B, Hh, Lq, Lk, D, pe, 40960)
+    assert (small["keys_once"], small["scratch"]) == (0, 40960)
+    assert am.lib().atn_prepare_pe_ex(ctypes.byref(pe), D, Lk) == 0
+    st = hip_rt.Stream()
+    (q1, k1, v1), _ = H.device_inputs((1, 1, 70, 64), (1, 1, 200, 64), 780, "bf16")
+    out1 = am.attention_ex(q1, k1, v1, stream=st)  # the stream's workspace: 40 KiB
+    st.synchronize()
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 781, "bf16")
+    ws = hip_rt.DeviceArray((40960 // 4,), "f32", fill=0)
+    eager, out = H.empty(Q.shape, "bf16"), H.empty(Q.shape, "bf16")
+    am.attention_ex(q, k, v, eager, pe=pe, workspace=ws)
+    hip_rt.synchronize()
+    g = hip_rt.Graph(st, lambda: am.attention_ex(q, k, v, out, pe=pe, stream=st))
+    for _ in range(3):
+        out.fill_nan()
+        hip_rt.synchronize()
+        g.launch()
+        st.synchronize()
+        assert np.array_equal(out.bits(), eager.bits())
+        am.attention_ex(q, k, v, eager, pe=pe, workspace=ws)
+        hip_rt.synchronize()
+    g.destroy()
+    # split-D needs its scores at least
+    (q2, k2, v2), _ = H.device_inputs((1, 1, 300, 512), (1, 1, 300, 512), 782)
+    out2, status = H.empty(q2.shape), []
+
+    def refused():
+        try:
+            am.attention_ex(q2, k2, v2, out2, stream=st)
+        except am.AtnError as e:
+            status.append(e.status)
+        am.attention_ex(q1, k1, v1, out1, stream=st)
+
+    hip_rt.Graph(st, refused).destroy()
+    assert status == [am.ATN_ERR_CAPTURE]
+    st.destroy()
