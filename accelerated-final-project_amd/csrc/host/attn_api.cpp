@@ -763,7 +763,7 @@ GemmPlan gemm_plan(int dtype, const Shape& s, const PePlan& plan) {
 
 // ---------------------------------------------------------------- tile plan
 // The split-D pipeline on pipelined 16-bit tiles (tile16.hip).  Workspace
-// after the sync region: partial scores [nsplit][BH][Lq][ldS] (fp32), P's two
+// after the sync region: partial scores [nsplit][BH][Lq][ldS] (fp32), P's
 // 16-bit parts [BH][Lq][ldP] each, and, with a positional encoding, the
 // encoded Q and K (fp32): encoding them once in a pass of its own costs a
 // read and a write of each, encoding them inside the QK^T tiles a table read
@@ -774,9 +774,10 @@ struct TilePlan {
     bool ok = false;
     int tile_qk = 0, tile_pv = 0, nsplit = 0, dchunk = 0, ldS = 0, ldP = 0;
     int Dp = 0;              // bf16: row stride of the copies (0: none)
-    bool qk_f32 = false;     // Q K^T on fp32 (encoded or fp32 inputs)
+    int qk = 0, pv = 0;      // the products' kinds (atn::kTile*)
+    int pparts = 2;          // parts of P
     double us = 0;           // estimated time of the call
-    size_t ph_off = 0, pl_off = 0, q_off = 0, k_off = 0, v_off = 0, bytes = 0;
+    size_t p_off[3] = {0, 0, 0}, q_off = 0, k_off = 0, v_off = 0, bytes = 0;
 };
 
 // Estimated time (us) of a tile kernel: wgs workgroups of `stages` stages on
@@ -787,12 +788,13 @@ struct TilePlan {
 // 128 x 128 does four times the work of 64 x 64 in two to three times the
 // time, so it is the faster wherever its grid fills the chip.  Stages: fp32
 // (and Q K^T of encoded bf16) 32 deep, bf16 Q K^T 64 deep, bf16 P V 32 keys.
-enum { kTileF32 = 0, kTileQkBf16 = 1, kTilePvBf16 = 2 };
-double tile_us(int kind, int tile, int64_t wgs, int64_t stages) {
-    static const double c[3][2][4] = {{{0.36, 0.09, 0.45, 0.28}, {0.58, 0.36, 1.50, 0.75}},
+double tile_us(int kind, bool pv, int tile, int64_t wgs, int64_t stages) {
+    // fp32, bf16 Q K^T, exact fp32, bf16 P V
+    static const double c[4][2][4] = {{{0.36, 0.09, 0.45, 0.28}, {0.58, 0.36, 1.50, 0.75}},
                                       {{0.30, 0.08, 0.40, 0.23}, {0.58, 0.17, 1.30, 0.60}},
+                                      {{0.42, 0.42, 1.03, 0.54}, {1.20, 0.55, 3.10, 1.80}},
                                       {{0.30, 0.10, 0.42, 0.26}, {0.45, 0.42, 1.50, 0.68}}};
-    const double* k = c[kind][tile == 128];
+    const double* k = c[pv && kind == atn::kTileBF16 ? 3 : kind][tile == 128];
     const double w = (double)wgs / 256.0;
     return (w <= 1.0 ? k[0] + k[1] * w : std::max(k[2], k[3] * w)) * (double)stages;
 }
@@ -803,13 +805,18 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
     p.ldS = (int)((s.Lk + 3) / 4 * 4);
     p.ldP = (int)((s.Lk + 7) / 8 * 8);
     const bool bf = dtype == ATN_DTYPE_BF16;
-    p.qk_f32 = !bf || plan.pek != atn::kPeNone;
+    // fp32 rows that no 16-byte load takes (head_d % 4 != 0, misaligned bases)
+    // keep all 24 bits at any magnitude, as on fp32 MFMA
+    const bool exact = !bf && (s.D % 4 != 0 || !a16);
+    p.qk = bf && plan.pek == atn::kPeNone ? atn::kTileBF16 : exact ? atn::kTileF32Exact : atn::kTileF32;
+    p.pv = bf ? atn::kTileBF16 : exact ? atn::kTileF32Exact : atn::kTileF32;
+    p.pparts = p.pv == atn::kTileF32Exact ? 3 : 2;
     if (bf && (s.D % 8 != 0 || !a16)) p.Dp = (s.D + 7) / 8 * 8;
-    const int64_t es = p.qk_f32 ? 4 : 2, lim = atn::kTileMaxBytes, W = std::max(s.D, p.Dp);
+    const int64_t es = p.qk == atn::kTileBF16 ? 2 : 4, lim = atn::kTileMaxBytes, W = std::max(s.D, p.Dp);
     if ((int64_t)s.Lq * W * es >= lim || (int64_t)s.Lk * W * es >= lim ||
         (int64_t)s.Lq * p.ldP * 2 >= lim)
         return p;
-    const int depth = p.qk_f32 ? 32 : 64;  // of a Q K^T stage
+    const int depth = p.qk == atn::kTileBF16 ? 64 : 32;  // of a Q K^T stage
     auto tiles = [](int64_t a, int64_t b, int t) { return ((a + t - 1) / t) * ((b + t - 1) / t); };
     // a forced tile (atn_tuning.splitd_tile): 128 only where both sides reach it
     const int force = tune().splitd_tile;
@@ -820,7 +827,6 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
     // D-chunks: each more is one more partial of every score, written at
     // 3.7 TB/s and read back at 6.  A chunked call keeps the whole call's.
     double best = 0;
-    const int kq = p.qk_f32 ? kTileF32 : kTileQkBf16, kv = bf ? kTilePvBf16 : kTileF32;
     const double part = (double)s.BH * s.Lq * p.ldS * 4.0 * (1 / 3.7e6 + 1 / 6.0e6);
     const int maxs = std::max(1, std::min(s.D / 64, 32));
     for (int t : {128, 64}) {
@@ -831,7 +837,7 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
             const int dchunk = fixed ? plan.dchunk : ((s.D + want - 1) / want + 31) / 32 * 32;
             const int ns = (s.D + dchunk - 1) / dchunk;
             if (ns != want) continue;
-            const double us = tile_us(kq, t, n * ns, (dchunk + depth - 1) / depth) + part * ns;
+            const double us = tile_us(p.qk, false, t, n * ns, (dchunk + depth - 1) / depth) + part * ns;
             if (p.nsplit == 0 || us < best) {
                 best = us;
                 p.tile_qk = t;
@@ -841,8 +847,8 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
         }
     }
     const int kst = (s.Lk + 31) / 32;
-    const double pv64 = tile_us(kv, 64, s.BH * tiles(s.Lq, s.D, 64), kst),
-                 pv128 = tile_us(kv, 128, s.BH * tiles(s.Lq, s.D, 128), kst);
+    const double pv64 = tile_us(p.pv, true, 64, s.BH * tiles(s.Lq, s.D, 64), kst),
+                 pv128 = tile_us(p.pv, true, 128, s.BH * tiles(s.Lq, s.D, 128), kst);
     p.tile_pv = !allowed(64, s.Lq, s.D) || (allowed(128, s.Lq, s.D) && pv128 < pv64) ? 128 : 64;
     // + launches, the softmax's own traffic, the encoding pass (2 bytes read
     // and 4 written per element of Q and K; 4 and 4 for fp32)
@@ -853,8 +859,7 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
     size_t off = kSyncBytes;
     auto take = [&](size_t b) { size_t o = off; off += round256(b); return o; };
     take((size_t)p.nsplit * s.BH * s.Lq * p.ldS * 4);
-    p.ph_off = take((size_t)s.BH * s.Lq * p.ldP * 2);
-    p.pl_off = take((size_t)s.BH * s.Lq * p.ldP * 2);
+    for (int i = 0; i < p.pparts; ++i) p.p_off[i] = take((size_t)s.BH * s.Lq * p.ldP * 2);
     if (plan.pek != atn::kPeNone) {
         if (plan.q.on || bf) p.q_off = take((size_t)s.nq * 4);
         if (plan.k.on || bf) p.k_off = take((size_t)s.nk * 4);
@@ -1327,8 +1332,8 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
     }
     if (tp.ok) {
         char* w = static_cast<char*>(ws);
-        uint16_t* ph = reinterpret_cast<uint16_t*>(w + tp.ph_off);
-        uint16_t* pl = reinterpret_cast<uint16_t*>(w + tp.pl_off);
+        uint16_t* p[3] = {};
+        for (int i = 0; i < tp.pparts; ++i) p[i] = reinterpret_cast<uint16_t*>(w + tp.p_off[i]);
         const void *qt = tp.q_off ? w + tp.q_off : Q, *kt = tp.k_off ? w + tp.k_off : K;
         const void* vt = tp.v_off ? w + tp.v_off : V;
         const long nq = (long)(s.BH * Lq), nk = (long)(s.BH * Lk);
@@ -1349,12 +1354,12 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
             ATN_HIP(atn::launch_pad_rows(t, plan.pek == atn::kPeNone ? 3 : 1, D, tp.Dp, stream));
         }
         const atn::QkTileArgs qa{qt, kt, scratch, (int)s.BH, Lq, Lk, Dqk, tp.dchunk, tp.nsplit, tp.ldS, 0, 0};
-        ATN_HIP(atn::launch_qk_tile(tp.qk_f32 ? ATN_DTYPE_F32 : ATN_DTYPE_BF16, tp.tile_qk, qa, stream));
-        ATN_HIP(atn::launch_softmax_split(dtype, scratch, ph, pl, nq, Lk, tp.ldS, tp.ldP, tp.nsplit,
-                                          (size_t)s.BH * Lq * tp.ldS, scale, stream));
-        const atn::PvTileArgs pa{ph, pl, vt, out, (int)s.BH, Lq, Lk, tp.Dp ? tp.Dp : D, D, tp.ldP,
+        ATN_HIP(atn::launch_qk_tile(tp.qk, tp.tile_qk, qa, stream));
+        ATN_HIP(atn::launch_softmax_split(tp.pv, tp.pparts, scratch, p, nq, Lk, tp.ldS, tp.ldP,
+                                          tp.nsplit, (size_t)s.BH * Lq * tp.ldS, scale, stream));
+        const atn::PvTileArgs pa{{p[0], p[1], p[2]}, vt, out, (int)s.BH, Lq, Lk, tp.Dp ? tp.Dp : D, D, tp.ldP,
                                  aligned(out, dtype == ATN_DTYPE_F32 ? 16 : 8), 0, 0};
-        ATN_HIP(atn::launch_pv_tile(dtype, tp.tile_pv, pa, stream));
+        ATN_HIP(atn::launch_pv_tile(tp.pv, tp.pparts, tp.tile_pv, pa, stream));
         return ATN_OK;
     }
     const StreamPlan sp = stream_plan(s);

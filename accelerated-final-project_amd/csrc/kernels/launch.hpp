@@ -45,9 +45,15 @@ hipError_t launch_pv_s16(const float* P, const float* V, float* O, int BH, int L
                          hipStream_t st);
 // The same three steps on pipelined 16-bit MFMA tiles (tile16.hip): output
 // tiles of tile x tile (64 or 128), rows of S ldS (a multiple of 4) and of
-// P's two 16-bit parts ldP (a multiple of 8) elements apart.  fp32 takes any
-// head_d and element-aligned bases, bf16 head_d % 8 == 0 and 16-byte aligned
-// Q, K and V; every head's tensors and P parts under kTileMaxBytes.
+// P's 16-bit parts ldP (a multiple of 8) elements apart.  A kind says how the
+// operands enter the products: fp32 as two fp16 parts (22 bits; a tile with
+// values beyond fp16's range scales its stages), fp32 as three bf16 parts
+// (all 24 bits at any magnitude), or bf16 as it is.  P has two fp16 parts for
+// the first, three bf16 parts for the second, pparts bf16 parts for bf16 V.
+// fp32 takes any head_d and element-aligned bases, bf16 head_d % 8 == 0 and
+// 16-byte aligned Q, K and V; every head's tensors and P parts under
+// kTileMaxBytes.
+constexpr int kTileF32 = 0, kTileBF16 = 1, kTileF32Exact = 2;
 constexpr long kTileMaxBytes = (1L << 31) - 65536;
 struct QkTileArgs {
     const void* Q;
@@ -57,8 +63,7 @@ struct QkTileArgs {
     int tiles_q, tiles_k;  // (filled by the launcher)
 };
 struct PvTileArgs {
-    const uint16_t* ph;  // 2^15 P, hi and lo parts [BH][Lq][ldP]
-    const uint16_t* pl;
+    const uint16_t* p[3];  // P's parts [BH][Lq][ldP]
     const void* V;
     void* O;
     int BH, Lq, Lk;
@@ -68,11 +73,12 @@ struct PvTileArgs {
     int o_align;  // O may be stored 4 elements at a time
     int tiles_q, tiles_d;  // (filled by the launcher)
 };
-hipError_t launch_qk_tile(int dtype, int tile, QkTileArgs a, hipStream_t st);
-hipError_t launch_softmax_split(int dtype, float* S, uint16_t* ph, uint16_t* pl, long rows, int Lk,
-                                int ldS, int ldP, int nsplit, size_t split_stride, float scale,
-                                hipStream_t st);
-hipError_t launch_pv_tile(int dtype, int tile, PvTileArgs a, hipStream_t st);
+hipError_t launch_qk_tile(int kind, int tile, QkTileArgs a, hipStream_t st);
+// kind and pparts: those of the product with V
+hipError_t launch_softmax_split(int kind, int pparts, float* S, uint16_t* const p[3], long rows,
+                                int Lk, int ldS, int ldP, int nsplit, size_t split_stride,
+                                float scale, hipStream_t st);
+hipError_t launch_pv_tile(int kind, int pparts, int tile, PvTileArgs a, hipStream_t st);
 
 // Single-launch split-D kernel for len_q <= 64, len_k <= 128 (fused_small.hip):
 // row groups of MB query rows, D slices of dc dims; gather1 selects the

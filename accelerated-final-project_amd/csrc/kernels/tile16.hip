@@ -1,11 +1,23 @@
 // The split-D pipeline on pipelined 16-bit MFMA tiles (gfx950): k_qk_tile
 // (partial scores over a D-chunk), k_softmax_split (exact row softmax, P as
-// two 16-bit parts) and k_pv_tile (O = P V).
+// 16-bit parts) and k_pv_tile (O = P V).
 //
 // Operands (KIND): fp32 as hi + lo fp16 parts (split16.hpp, three exact
-// products per product), or raw bf16 (one exact product; P as hi + lo bf16
-// parts).  P leaves the softmax already split (times 2^15, so that small
-// probabilities keep their bits), so the PV kernel converts V alone.
+// products per product), fp32 as three bf16 parts (X: all 24 bits at any
+// magnitude, six products), or raw bf16 (one exact product).  P leaves the
+// softmax already split, so the PV kernel converts V alone.
+//
+// X serves fp32 rows at any alignment (head_d % 4 != 0, misaligned bases), which
+// ran on fp32 MFMA before and keep its accuracy at any magnitude.  Two fp16
+// parts keep 22 bits, an absolute 2^-25 below 2^-3: V of 2^-20 loses half of
+// them, and one large element takes them from its whole stage.  Six products
+// and 11 instead of 4 instructions to split a value pair make the tiles 1.25 to
+// 1.5 times as long, still half of what fp32 MFMA takes, and the error against
+// 64 bits halves, for the parts lose nothing: (2,2,422,422,2361) 189 us on
+// fp32 MFMA, 67 on two parts, 94 on three (5.7e-7, 4.3e-7, 2.2e-7 normwise);
+// (1,4,1453,1453,1025) 797, 199, 305 us.  An infinity's later parts are NaN,
+// and its product with a part that is zero: a tile that holds one (or a value
+// that rounds to one) is computed again on fp32 MFMA.
 //
 // What bounds these kernels is VALU issue (the fp16 split: 4 instructions per
 // value pair) beside the MFMAs where the grid fills the chip, and the latency
@@ -13,7 +25,7 @@
 // go out one stage (128 x 128 tiles) or two (64 x 64: two register sets)
 // before their LDS writes, LDS is double-buffered with one barrier per stage,
 // and two stages run through one MFMA chain before their sum is added to the
-// tile's (half the additions of a sum per stage; the rounding against exact
+// sum (half the additions of a sum per stage; the rounding against exact
 // 64-bit results stays below that of a sum per stage and of one chain: 4.3e-7
 // normwise at (1,4,512,512,2048), 6.7e-7 with one chain).  Register use stays
 // clear of spills: a spill's reload waits (vmcnt) for the loads in flight.  A
@@ -31,7 +43,8 @@
 // us against 136.9).  LDS rows of 32 elements (64 bytes) per part, their
 // 16-byte chunks permuted by tile_swz(row) so that fragment reads hit
 // distinct banks unpadded (SQ_LDS_BANK_CONFLICT 0): 64 KiB for both stages of
-// a 128 x 128 tile, two workgroups per CU.  Rows of S and P are padded to
+// a 128 x 128 tile, two workgroups per CU (X: 96 KiB, one, always of 8 waves).
+// Rows of S and P are padded to
 // whole vectors, so ragged key counts store and load 16 bytes as well; rows
 // of O whose D is odd are stored 4 elements at a time at any alignment
 // ((2,8,400,400,1501) P V of bf16 56 -> 33 us).
@@ -54,19 +67,21 @@ namespace atn {
 namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef short bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
 
-constexpr int kKindF32 = 0, kKindBF16 = 1;
+constexpr int kKindF32 = kTileF32, kKindBF16 = kTileBF16, kKindX = kTileF32Exact;
 
 // Depth of a QK stage: 128 bytes of a row either way (fp32: 32 elements as
-// two parts; bf16: 64 elements, the two 32-deep halves in the parts' places).
+// PARTS parts; bf16: 64 elements, the two 32-deep halves in the parts' places).
 template <int KIND>
 struct Tile {
-    using T = typename std::conditional<KIND == kKindF32, float, uint16_t>::type;
-    static constexpr int ES = KIND == kKindF32 ? 4 : 2;
+    using T = typename std::conditional<KIND == kKindBF16, uint16_t, float>::type;
+    static constexpr int ES = KIND == kKindBF16 ? 2 : 4;
     static constexpr int DEPTH = 128 / ES;
     static constexpr int PER16 = 16 / ES;  // elements per 16-byte load
+    static constexpr int PARTS = KIND == kKindX ? 3 : 2;
 };
 
 __device__ __forceinline__ int tile_swz(int row) { return ((row >> 1) & 3) ^ ((row >> 3) & 1); }
@@ -104,6 +119,58 @@ __device__ __forceinline__ void split4_scaled(const uint4& u, float s, uint2& hi
     split2_f16(v.z * s, v.w * s, hi.y, lo.y);
 }
 
+// two values as bf16, rounded to nearest even (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
+    const v2f v = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2bf));
+}
+// a and b as N bf16 parts each, every part the nearest to what the ones before
+// it leave; three hold an fp32 value exactly (8 + 8 + 8 bits)
+template <int N>
+__device__ __forceinline__ void split_bf16(float a, float b, uint32_t (&w)[N]) {
+#pragma unroll
+    for (int p = 0; p < N; ++p) {
+        w[p] = pk_bf16(a, b);
+        a -= __uint_as_float(w[p] << 16);
+        b -= __uint_as_float(w[p] & 0xffff0000u);
+    }
+}
+// Magnitudes from here on round to an infinite first part.
+constexpr float kBf16Range = 0x1.ffp127f;
+
+// The parts of 4 values (16 bytes) of kind F32 (one = 1) or X
+template <int KIND>
+__device__ __forceinline__ void split_parts(const uint4& u, float one, uint2 (&p)[Tile<KIND>::PARTS]) {
+    if constexpr (KIND == kKindF32) {
+        split4(u, one, p[0], p[1]);
+    } else {
+        const float4 v = as_f4(u);
+        uint32_t a[3], b[3];
+        split_bf16(v.x, v.y, a);
+        split_bf16(v.z, v.w, b);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) p[k] = make_uint2(a[k], b[k]);
+    }
+}
+
+// One 32 x 32 x 16 product of split operands added to c: the parts' products
+// down to 2^-22 (two fp16 parts) or 2^-25 (three bf16 parts) of the leading
+// one, the smallest first.
+template <int KIND, int N>
+__device__ __forceinline__ v16f mfma_parts(const uint4 (&a)[N], const uint4 (&b)[N], v16f c) {
+    if constexpr (KIND == kKindX) {
+        c = mfma32<KIND>(a[2], b[0], c);
+        c = mfma32<KIND>(a[0], b[2], c);
+        c = mfma32<KIND>(a[1], b[1], c);
+    }
+    c = mfma32<KIND>(a[1], b[0], c);
+    c = mfma32<KIND>(a[0], b[1], c);
+    return mfma32<KIND>(a[0], b[0], c);
+}
+__device__ __forceinline__ v16f mfma_f32(float a, float b, const v16f& c) {
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+
 // Consecutive tiles on one XCD: workgroup ids are dealt to the 8 XCDs in
 // turn, each XCD takes a contiguous share of the n tiles.
 __device__ __forceinline__ unsigned xcd_tile(unsigned id, unsigned n) {
@@ -136,16 +203,26 @@ __device__ __forceinline__ float max4abs(float m, const uint4& u) {
     return vmax3abs(vmax3abs(m, v.x, v.y), v.z, v.w);
 }
 
-// Whether any thread of the workgroup saw a value outside fp16's range
+// Whether any thread of the workgroup saw a magnitude of `range` or more
 template <int NW>
-__device__ __forceinline__ bool wg_over(float big, int* flag) {
-    const bool over = __ballot(!(big < kF16Range)) != 0;
+__device__ __forceinline__ bool wg_over(float big, float range, int* flag) {
+    const bool over = __ballot(!(big < range)) != 0;
     if ((threadIdx.x & 63) == 0) flag[threadIdx.x >> 6] = over;
     __syncthreads();
     int any = flag[0];
 #pragma unroll
     for (int w = 1; w < NW; ++w) any |= flag[w];
     return any != 0;
+}
+
+// 4 consecutive elements to an address of element alignment only: one store
+// (the device runs in unaligned-access mode)
+__device__ __forceinline__ void st4_any(float* p, float4 v) { __builtin_memcpy(p, &v, 16); }
+__device__ __forceinline__ void st4_any(uint16_t* p, float4 v) {
+    uint2 w;
+    w.x = (uint32_t)f32_to_bf16_bits(v.x) | ((uint32_t)f32_to_bf16_bits(v.y) << 16);
+    w.y = (uint32_t)f32_to_bf16_bits(v.z) | ((uint32_t)f32_to_bf16_bits(v.w) << 16);
+    __builtin_memcpy(p, &w, 8);
 }
 
 // Partial scores S_split[bh][i][j] = sum over the chunk's dims of q_id k_jd
@@ -162,8 +239,9 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
     constexpr int NK = TL / WK / 32, NQ = TL / 64;      // 32 x 32 MFMA tiles per wave
     constexpr int PART = TL * 32;       // elements of one part of one operand
     constexpr int AHEAD = TL == 64 || NW == 8 ? 2 : 1;  // stages a load is issued before its LDS write
-    __shared__ __align__(16) uint16_t sq[2][2 * PART];  // [stage][part][row][32]
-    __shared__ __align__(16) uint16_t sk[2][2 * PART];
+    constexpr int NP = G::PARTS;
+    __shared__ __align__(16) uint16_t sq[2][NP * PART];  // [stage][part][row][32]
+    __shared__ __align__(16) uint16_t sk[2][NP * PART];
     __shared__ float slot[2 * NW];
     __shared__ int flag[NW];
 
@@ -225,25 +303,25 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
     };
     float big = 0.f;
     const float one = unit_opaque();
-    // LDS place of this thread's 16 bytes: fp32 half a chunk of both parts,
+    // LDS place of this thread's 16 bytes: fp32 half a chunk of every part,
     // bf16 a chunk of one part
     auto place = [&](int i) {
         const int row = lrow + LROWS * i;
-        return KIND == kKindF32 ? tile_at(row, lc >> 1) + 4 * (lc & 1)
+        return KIND != kKindBF16 ? tile_at(row, lc >> 1) + 4 * (lc & 1)
                                 : (lc >> 2) * PART + tile_at(row, lc & 3);
     };
     auto store = [&](const Regs& r, uint16_t* q, uint16_t* k) {
 #pragma unroll
         for (int i = 0; i < ROUNDS; ++i) {
             const int o = place(i);
-            if constexpr (KIND == kKindF32) {
-                uint2 hi, lo;
-                split4(r.q[i], one, hi, lo);
-                *reinterpret_cast<uint2*>(q + o) = hi;
-                *reinterpret_cast<uint2*>(q + PART + o) = lo;
-                split4(r.k[i], one, hi, lo);
-                *reinterpret_cast<uint2*>(k + o) = hi;
-                *reinterpret_cast<uint2*>(k + PART + o) = lo;
+            if constexpr (KIND != kKindBF16) {
+                uint2 w[NP];
+                split_parts<KIND>(r.q[i], one, w);
+#pragma unroll
+                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint2*>(q + p * PART + o) = w[p];
+                split_parts<KIND>(r.k[i], one, w);
+#pragma unroll
+                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint2*>(k + p * PART + o) = w[p];
                 big = max4abs(max4abs(big, r.q[i]), r.k[i]);
             } else {
                 *reinterpret_cast<uint4*>(q + o) = r.q[i];
@@ -267,16 +345,16 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
     auto compute = [&](const uint16_t* q, const uint16_t* k, auto fresh) {
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            uint4 ka[2][NK], qa[2][NQ];
+            uint4 ka[NK][NP], qa[NQ][NP];
 #pragma unroll
-            for (int p = 0; p < 2; ++p) {
+            for (int p = 0; p < NP; ++p) {
 #pragma unroll
                 for (int i = 0; i < NK; ++i)
-                    ka[p][i] = *reinterpret_cast<const uint4*>(
+                    ka[i][p] = *reinterpret_cast<const uint4*>(
                         k + p * PART + tile_at(wk + 32 * i + fr, 2 * ks + fc));
 #pragma unroll
                 for (int j = 0; j < NQ; ++j)
-                    qa[p][j] = *reinterpret_cast<const uint4*>(
+                    qa[j][p] = *reinterpret_cast<const uint4*>(
                         q + p * PART + tile_at(wq + 32 * j + fr, 2 * ks + fc));
             }
 #pragma unroll
@@ -284,13 +362,11 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
 #pragma unroll
                 for (int j = 0; j < NQ; ++j) {
                     v16f c = decltype(fresh)::value && ks == 0 ? v16f{} : acc[i][j];
-                    if constexpr (KIND == kKindF32) {
-                        c = mfma32<KIND>(ka[1][i], qa[0][j], c);
-                        c = mfma32<KIND>(ka[0][i], qa[1][j], c);
-                        c = mfma32<KIND>(ka[0][i], qa[0][j], c);
+                    if constexpr (KIND != kKindBF16) {
+                        c = mfma_parts<KIND>(ka[i], qa[j], c);
                     } else {
-                        c = mfma32<KIND>(ka[0][i], qa[0][j], c);
-                        c = mfma32<KIND>(ka[1][i], qa[1][j], c);
+                        c = mfma32<KIND>(ka[i][0], qa[j][0], c);
+                        c = mfma32<KIND>(ka[i][1], qa[j][1], c);
                     }
                     acc[i][j] = c;
                 }
@@ -322,7 +398,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
         flush();
     }
     if constexpr (KIND == kKindF32) {
-        if (wg_over<NW>(big, flag)) {
+        if (wg_over<NW>(big, kF16Range, flag)) {
             zero();
             for (int d0 = dbeg; d0 < dend; d0 += G::DEPTH) {
                 issue(r0, d0);
@@ -354,6 +430,34 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
         }
     }
 
+    if constexpr (KIND == kKindX) {
+        if (wg_over<NW>(big, kBf16Range, flag)) {
+            // on fp32 MFMA, from rows of fp32 (33 apart) in the parts' places
+            constexpr int R = 33;
+            float* fq = reinterpret_cast<float*>(sq);
+            float* fk = reinterpret_cast<float*>(sk);
+            zero();
+            for (int d0 = dbeg; d0 < dend; d0 += G::DEPTH) {
+                issue(r0, d0);
+                __syncthreads();  // the last stage's reads are done
+#pragma unroll
+                for (int i = 0; i < ROUNDS; ++i) {
+                    const int o = (lrow + LROWS * i) * R + 4 * lc;
+                    st4_any(fq + o, as_f4(r0.q[i]));
+                    st4_any(fk + o, as_f4(r0.k[i]));
+                }
+                __syncthreads();
+                for (int d = fc; d < G::DEPTH; d += 2)
+#pragma unroll
+                    for (int i = 0; i < NK; ++i)
+#pragma unroll
+                        for (int j = 0; j < NQ; ++j)
+                            sum[i][j] = mfma_f32(fk[(wk + 32 * i + fr) * R + d],
+                                                 fq[(wq + 32 * j + fr) * R + d], sum[i][j]);
+            }
+        }
+    }
+
     // register r of a tile: key 8 (r / 4) + 4 (lane / 32) + r % 4 of query lane % 32
 #pragma unroll
     for (int j = 0; j < NQ; ++j) {
@@ -372,34 +476,38 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
     }
 }
 
-// 2^15 p as hi + lo parts: fp16 (fp32 calls) or bf16
-template <int KIND>
-__device__ __forceinline__ void split_p(float4 p, uint2& hi, uint2& lo) {
+// P as its 16-bit parts, 4 values at column c of its row: two fp16 parts of
+// 2^15 p (so that small probabilities keep their bits), or NP bf16 parts of p
+// (fp32's exponents: nothing to scale, and no V whose products then overflow).
+struct PParts {
+    uint16_t* p[3];
+};
+template <int KIND, int NP>
+__device__ __forceinline__ void store_p4(const PParts& out, size_t at, float4 v) {
+    uint2 w[3];
     if constexpr (KIND == kKindF32) {
-        split2_f16(p.x, p.y, hi.x, lo.x);
-        split2_f16(p.z, p.w, hi.y, lo.y);
+        split2_f16(v.x, v.y, w[0].x, w[1].x);
+        split2_f16(v.z, v.w, w[0].y, w[1].y);
     } else {
-        const float v[4] = {p.x, p.y, p.z, p.w};
-        uint32_t h[4], l[4];
+        uint32_t a[NP], b[NP];
+        split_bf16(v.x, v.y, a);
+        split_bf16(v.z, v.w, b);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            h[c] = f32_to_bf16_bits(v[c]);
-            l[c] = f32_to_bf16_bits(v[c] - bf16_bits_to_f32(h[c]));
-        }
-        hi = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-        lo = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+        for (int k = 0; k < NP; ++k) w[k] = make_uint2(a[k], b[k]);
     }
+#pragma unroll
+    for (int k = 0; k < NP; ++k) *reinterpret_cast<uint2*>(out.p[k] + at) = w[k];
 }
+template <int KIND>
+constexpr float kPScale = KIND == kKindF32 ? 32768.0f : 1.0f;
 
 // Row softmax of the summed partial scores, exact (max, exp, sum, divide),
-// written as two 16-bit parts of 2^15 P (rows ldP apart, zeros from Lk on).
+// written as 16-bit parts (rows ldP apart, zeros from Lk on).
 // TPR threads per row hold it in registers (thread t the 4 keys from
 // 4 (t + TPR u) on), so S is read once; every partial's load is independent.
-template <int KIND, int TPR, int NV>
-__global__ __launch_bounds__(256) void k_softmax_split(const float* __restrict__ S,
-                                                       uint16_t* __restrict__ ph,
-                                                       uint16_t* __restrict__ pl, long rows,
-                                                       int Lk, int ldS, int ldP, int nsplit,
+template <int KIND, int NP, int TPR, int NV>
+__global__ __launch_bounds__(256) void k_softmax_split(const float* __restrict__ S, PParts out,
+                                                       long rows, int Lk, int ldS, int ldP, int nsplit,
                                                        size_t split_stride, float scale) {
     __shared__ float red[8];
     const int tid = threadIdx.x, t = tid % TPR;
@@ -460,24 +568,21 @@ __global__ __launch_bounds__(256) void k_softmax_split(const float* __restrict__
         __syncthreads();
         l = (red[4] + red[5]) + (red[6] + red[7]);
     }
-    l *= 1.0f / 32768.0f;  // P written times 2^15 (exact)
+    l *= 1.0f / kPScale<KIND>;  // (exact)
 #pragma unroll
     for (int u = 0; u < NV; ++u) {
         const int c = 4 * (t + TPR * u);
         if (c < ldP) {
-            uint2 hi, lo;
-            split_p<KIND>(make_float4(v[u].x / l, v[u].y / l, v[u].z / l, v[u].w / l), hi, lo);
-            *reinterpret_cast<uint2*>(ph + (size_t)row * ldP + c) = hi;
-            *reinterpret_cast<uint2*>(pl + (size_t)row * ldP + c) = lo;
+            store_p4<KIND, NP>(out, (size_t)row * ldP + c,
+                               make_float4(v[u].x / l, v[u].y / l, v[u].z / l, v[u].w / l));
         }
     }
 }
 
 // Rows longer than the registers hold: the sums go back to the first
 // partial's place, and the row is read three times.
-template <int KIND>
-__global__ __launch_bounds__(256) void k_softmax_long(float* S, uint16_t* __restrict__ ph,
-                                                      uint16_t* __restrict__ pl, long rows, int Lk,
+template <int KIND, int NP>
+__global__ __launch_bounds__(256) void k_softmax_long(float* S, PParts out, long rows, int Lk,
                                                       int ldS, int ldP, int nsplit,
                                                       size_t split_stride, float scale) {
     __shared__ float red[8];
@@ -505,28 +610,15 @@ __global__ __launch_bounds__(256) void k_softmax_long(float* S, uint16_t* __rest
         l = wave_sum(l);
         if ((tid & 63) == 0) red[4 + (tid >> 6)] = l;
         __syncthreads();
-        l = ((red[4] + red[5]) + (red[6] + red[7])) * (1.0f / 32768.0f);
+        l = ((red[4] + red[5]) + (red[6] + red[7])) * (1.0f / kPScale<KIND>);
         for (int c = 4 * tid; c < ldP; c += 1024) {
             float p[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) p[k] = c + k < Lk ? s[c + k] / l : 0.f;
-            uint2 hi, lo;
-            split_p<KIND>(make_float4(p[0], p[1], p[2], p[3]), hi, lo);
-            *reinterpret_cast<uint2*>(ph + (size_t)row * ldP + c) = hi;
-            *reinterpret_cast<uint2*>(pl + (size_t)row * ldP + c) = lo;
+            store_p4<KIND, NP>(out, (size_t)row * ldP + c, make_float4(p[0], p[1], p[2], p[3]));
         }
         __syncthreads();  // red reused by the next row
     }
-}
-
-// 4 consecutive elements to an address of element alignment only: one store
-// (the device runs in unaligned-access mode)
-__device__ __forceinline__ void st4_any(float* p, float4 v) { __builtin_memcpy(p, &v, 16); }
-__device__ __forceinline__ void st4_any(uint16_t* p, float4 v) {
-    uint2 w;
-    w.x = (uint32_t)f32_to_bf16_bits(v.x) | ((uint32_t)f32_to_bf16_bits(v.y) << 16);
-    w.y = (uint32_t)f32_to_bf16_bits(v.z) | ((uint32_t)f32_to_bf16_bits(v.w) << 16);
-    __builtin_memcpy(p, &w, 8);
 }
 
 // O[bh][i][d] = sum_j P_ij V_jd for one tile of TL queries x TL dims, 32 keys
@@ -534,17 +626,18 @@ __device__ __forceinline__ void st4_any(uint16_t* p, float4 v) {
 // holds 4 consecutive dims of one query.  P rows go to LDS as they are; V
 // stays [key][dim] there and reaches the MFMA by the transposing LDS read
 // (rows of TL + 32 elements: the four rows of a read on distinct banks).
-template <int KIND, int TL, int NW, bool RAG>
+template <int KIND, int PP, int TL, int NW, bool RAG>
 __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_pv_tile(PvTileArgs a) {
     using G = Tile<KIND>;
     constexpr int PART = TL * 32, WD = NW / 2;          // waves along the dims (2 along the queries)
     constexpr int ND = TL / WD / 32, NQ = TL / 64;      // 32 x 32 MFMA tiles per wave
     constexpr int AHEAD = TL == 64 || NW == 8 ? 2 : 1;
-    constexpr int VSTR = TL + 32, VPARTS = KIND == kKindF32 ? 2 : 1, VPART = 32 * VSTR;
+    constexpr int VSTR = TL + 32, VPARTS = KIND == kKindBF16 ? 1 : G::PARTS, VPART = 32 * VSTR;
     constexpr int VL = TL / G::PER16;             // V loader: lanes per row
     constexpr int VROWS = 64 * NW / VL, VROUNDS = 32 / VROWS > 0 ? 32 / VROWS : 1;
+    static_assert(KIND == kKindBF16 || PP == VPARTS, "parts of P");
     static_assert(VROWS <= 32, "a round of V rows within a stage");
-    __shared__ __align__(16) uint16_t sp[2][2 * PART];
+    __shared__ __align__(16) uint16_t sp[2][PP * PART];
     __shared__ __align__(16) uint16_t sv[2][VPARTS * VPART];
     __shared__ float slot[2 * NW];
     __shared__ int flag[NW];
@@ -557,11 +650,10 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_pv_tile(PvTileArgs
     const int td = (int)(t % a.tiles_d), bh = (int)(t / a.tiles_d);
     const int q0 = tq * TL, d0 = td * TL;
 
-    const char* ph = reinterpret_cast<const char*>(a.ph + (size_t)bh * a.Lq * a.ldP);
-    const char* pl = reinterpret_cast<const char*>(a.pl + (size_t)bh * a.Lq * a.ldP);
+    const size_t pbase = (size_t)bh * a.Lq * a.ldP;
     const int pbytes = a.Lq * a.ldP * 2, vbytes = a.Lk * a.D * G::ES;
     const char* Vh = static_cast<const char*>(a.V) + (size_t)bh * a.Lk * a.D * G::ES;
-    // P loader: row lrow + PROWS i, chunk lc of both parts
+    // P loader: row lrow + PROWS i, chunk lc of every part
     constexpr int PROWS = 16 * NW, PR = TL / PROWS;
     const int lrow = tid >> 2, lc = tid & 3;
     unsigned poff[PR];
@@ -578,23 +670,22 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_pv_tile(PvTileArgs
                       ? (unsigned)(((vrow + VROWS * i) * a.D + d0 + vcol) * G::ES)
                       : (unsigned)kBufOob;
     struct Regs {
-        uint4 h[PR], l[PR], v[VROUNDS];
+        uint4 p[PP][PR], v[VROUNDS];
     };
     auto issue = [&](Regs& r, int kk) {
-const int psh = min(kk, a.ldP) * 2;
-        const __amdgpu_buffer_rsrc_t rh = buf_rsrc(ph + psh, pbytes - psh);
-        const __amdgpu_buffer_rsrc_t rl = buf_rsrc(pl + psh, pbytes - psh);
+        const int psh = min(kk, a.ldP);
 #pragma unroll
-        for (int i = 0; i < PR; ++i) {
-            const unsigned o = kk + 8 * lc < a.ldP ? poff[i] : (unsigned)kBufOob;
-            r.h[i] = ld_buf_u4(rh, o);
-            r.l[i] = ld_buf_u4(rl, o);
+        for (int w = 0; w < PP; ++w) {
+            const __amdgpu_buffer_rsrc_t rp = buf_rsrc(a.p[w] + pbase + psh, pbytes - 2 * psh);
+#pragma unroll
+            for (int i = 0; i < PR; ++i)
+                r.p[w][i] = ld_buf_u4(rp, kk + 8 * lc < a.ldP ? poff[i] : (unsigned)kBufOob);
         }
         const size_t vsh = (size_t)min(kk, a.Lk) * a.D * G::ES;
         const __amdgpu_buffer_rsrc_t rv = buf_rsrc(Vh + vsh, vbytes - (int)vsh);
 #pragma unroll
         for (int i = 0; i < VROUNDS; ++i) {
-            if (RAG && KIND == kKindF32 && d0 + TL > a.D) {
+            if (RAG && KIND != kKindBF16 && d0 + TL > a.D) {
                 uint32_t w[4];
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
@@ -612,8 +703,8 @@ const int psh = min(kk, a.ldP) * 2;
 #pragma unroll
         for (int i = 0; i < PR; ++i) {
             const int o = tile_at(lrow + PROWS * i, lc);
-            *reinterpret_cast<uint4*>(p + o) = r.h[i];
-            *reinterpret_cast<uint4*>(p + PART + o) = r.l[i];
+#pragma unroll
+            for (int w = 0; w < PP; ++w) *reinterpret_cast<uint4*>(p + w * PART + o) = r.p[w][i];
         }
     };
     auto store = [&](const Regs& r, uint16_t* p, uint16_t* v) {
@@ -621,11 +712,11 @@ const int psh = min(kk, a.ldP) * 2;
 #pragma unroll
         for (int i = 0; i < VROUNDS; ++i) {
             const int o = (vrow + VROWS * i) * VSTR + vcol;
-            if constexpr (KIND == kKindF32) {
-                uint2 hi, lo;
-                split4(r.v[i], one, hi, lo);
-                *reinterpret_cast<uint2*>(v + o) = hi;
-                *reinterpret_cast<uint2*>(v + VPART + o) = lo;
+            if constexpr (KIND != kKindBF16) {
+                uint2 w[VPARTS];
+                split_parts<KIND>(r.v[i], one, w);
+#pragma unroll
+                for (int p = 0; p < VPARTS; ++p) *reinterpret_cast<uint2*>(v + p * VPART + o) = w[p];
                 big = max4abs(big, r.v[i]);
             } else {
                 *reinterpret_cast<uint4*>(v + o) = r.v[i];
@@ -650,30 +741,32 @@ const int psh = min(kk, a.ldP) * 2;
     auto compute = [&](const uint16_t* p, const uint16_t* v, auto fresh) {
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            uint4 pa[2][NQ], vv[VPARTS][ND];
+            uint4 pa[NQ][PP], vv[ND][VPARTS];
 #pragma unroll
             for (int i = 0; i < ND; ++i)
 #pragma unroll
                 for (int w = 0; w < VPARTS; ++w) {
                     const uint16_t* at = v + w * VPART + va + 16 * ks * VSTR + 32 * i;
                     const uint2 x = lds_tr16(at), y = lds_tr16(at + 4 * VSTR);
-                    vv[w][i] = make_uint4(x.x, x.y, y.x, y.y);
+                    vv[i][w] = make_uint4(x.x, x.y, y.x, y.y);
                 }
 #pragma unroll
             for (int j = 0; j < NQ; ++j)
 #pragma unroll
-                for (int w = 0; w < 2; ++w)
-                    pa[w][j] = *reinterpret_cast<const uint4*>(
+                for (int w = 0; w < PP; ++w)
+                    pa[j][w] = *reinterpret_cast<const uint4*>(
                         p + w * PART + tile_at(wq + 32 * j + fr, 2 * ks + fc));
 #pragma unroll
             for (int i = 0; i < ND; ++i)
 #pragma unroll
                 for (int j = 0; j < NQ; ++j) {
                     v16f c = decltype(fresh)::value && ks == 0 ? v16f{} : acc[i][j];
-                    if constexpr (KIND == kKindF32)
-                        c = mfma32<KIND>(vv[VPARTS - 1][i], pa[0][j], c);
-                    c = mfma32<KIND>(vv[0][i], pa[1][j], c);
-                    c = mfma32<KIND>(vv[0][i], pa[0][j], c);
+                    if constexpr (KIND != kKindBF16) {
+                        c = mfma_parts<KIND>(vv[i], pa[j], c);
+                    } else {
+#pragma unroll
+                        for (int w = PP - 1; w >= 0; --w) c = mfma32<KIND>(vv[i][0], pa[j][w], c);
+                    }
                     acc[i][j] = c;
                 }
         }
@@ -704,7 +797,7 @@ const int psh = min(kk, a.ldP) * 2;
         flush();
     }
     if constexpr (KIND == kKindF32) {
-        if (wg_over<NW>(big, flag)) {
+        if (wg_over<NW>(big, kF16Range, flag)) {
             zero();
             for (int kk = 0; kk < a.Lk; kk += 32) {
                 issue(r0, kk);
@@ -730,7 +823,46 @@ const int psh = min(kk, a.ldP) * 2;
         }
     }
 
-    constexpr float kPInv = 1.0f / 32768.0f;  // P's 2^15
+    if constexpr (KIND == kKindX) {
+        if (wg_over<NW>(big, kBf16Range, flag)) {
+            // on fp32 MFMA: P put together again (rows 33 apart), V as it is
+            constexpr int R = 33;
+            float* fp = reinterpret_cast<float*>(sp);
+            float* fv = reinterpret_cast<float*>(sv);
+            zero();
+            for (int kk = 0; kk < a.Lk; kk += 32) {
+                issue(r0, kk);
+                __syncthreads();  // the last stage's reads are done
+#pragma unroll
+                for (int i = 0; i < PR; ++i) {
+                    float* o = fp + (lrow + PROWS * i) * R + 8 * lc;
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) {
+                        float x = 0.f;
+#pragma unroll
+                        for (int w = 0; w < PP; ++w) {
+                            const uint32_t u = (&r0.p[w][i].x)[c >> 1];
+                            x += __uint_as_float(c & 1 ? u & 0xffff0000u : u << 16);
+                        }
+                        o[c] = x;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < VROUNDS; ++i)
+                    *reinterpret_cast<uint4*>(fv + (vrow + VROWS * i) * TL + vcol) = r0.v[i];
+                __syncthreads();
+                for (int k = fc; k < 32; k += 2)
+#pragma unroll
+                    for (int i = 0; i < ND; ++i)
+#pragma unroll
+                        for (int j = 0; j < NQ; ++j)
+                            sum[i][j] = mfma_f32(fv[k * TL + wd + 32 * i + fr],
+                                                 fp[(wq + 32 * j + fr) * R + k], sum[i][j]);
+            }
+        }
+    }
+
+    constexpr float kPInv = 1.0f / kPScale<KIND>;
     using T = typename G::T;
     T* Oh = static_cast<T*>(a.O) + (size_t)bh * a.Lq * a.ldO;
 #pragma unroll
@@ -772,8 +904,8 @@ constexpr unsigned kOnePerCu = 256;
 
 template <int KIND, int TL, int NW>
 void run_qk(const QkTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
-    if (KIND == kKindF32 && rag)
-        hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, KIND == kKindF32>), dim3(grid), dim3(64 * NW), 0,
+    if (KIND != kKindBF16 && rag)
+        hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, KIND != kKindBF16>), dim3(grid), dim3(64 * NW), 0,
                            st, a);
     else
         hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, false>), dim3(grid), dim3(64 * NW), 0, st, a);
@@ -782,42 +914,42 @@ template <int KIND>
 void run_qk_tile(int tile, const QkTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
     if (tile == 64)
         run_qk<KIND, 64, 4>(a, rag, grid, st);
-    else if (grid <= kOnePerCu)
+    else if (KIND == kKindX || grid <= kOnePerCu)
         run_qk<KIND, 128, 8>(a, rag, grid, st);
-    else
+    else if constexpr (KIND != kKindX)
         run_qk<KIND, 128, 4>(a, rag, grid, st);
 }
 
-template <int KIND, int TL, int NW>
+template <int KIND, int PP, int TL, int NW>
 void run_pv(const PvTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
     if (rag)
-        hipLaunchKernelGGL((k_pv_tile<KIND, TL, NW, true>), dim3(grid), dim3(64 * NW), 0, st, a);
+        hipLaunchKernelGGL((k_pv_tile<KIND, PP, TL, NW, true>), dim3(grid), dim3(64 * NW), 0, st, a);
     else
-        hipLaunchKernelGGL((k_pv_tile<KIND, TL, NW, false>), dim3(grid), dim3(64 * NW), 0, st, a);
+        hipLaunchKernelGGL((k_pv_tile<KIND, PP, TL, NW, false>), dim3(grid), dim3(64 * NW), 0, st, a);
 }
-template <int KIND>
+template <int KIND, int PP>
 void run_pv_tile(int tile, const PvTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
     if (tile == 64)
-        run_pv<KIND, 64, 4>(a, rag, grid, st);
-    else if (grid <= kOnePerCu)
-        run_pv<KIND, 128, 8>(a, rag, grid, st);
-    else
-        run_pv<KIND, 128, 4>(a, rag, grid, st);
+        run_pv<KIND, PP, 64, 4>(a, rag, grid, st);
+    else if (KIND == kKindX || grid <= kOnePerCu)
+        run_pv<KIND, PP, 128, 8>(a, rag, grid, st);
+    else if constexpr (KIND != kKindX)
+        run_pv<KIND, PP, 128, 4>(a, rag, grid, st);
 }
 
-template <int KIND>
-hipError_t softmax_k(float* S, uint16_t* ph, uint16_t* pl, long rows, int Lk, int ldS, int ldP,
-                     int nsplit, size_t stride, float scale, hipStream_t st) {
+template <int KIND, int NP>
+hipError_t softmax_k(float* S, const PParts& out, long rows, int Lk, int ldS, int ldP, int nsplit,
+                     size_t stride, float scale, hipStream_t st) {
     // a wave per row while that gives every CU several waves; a workgroup
     // per row for few rows and for rows longer than a wave's registers hold
     const bool wave = Lk <= 2048 && (rows >= 4096 || Lk <= 256);
 #define ATN_SOFTMAX(TPR, NV)                                                                    \
-    hipLaunchKernelGGL((k_softmax_split<KIND, TPR, NV>),                                        \
+    hipLaunchKernelGGL((k_softmax_split<KIND, NP, TPR, NV>),                                    \
                        dim3((unsigned)((rows + 256 / TPR - 1) / (256 / TPR))), dim3(256), 0, st, \
-                       S, ph, pl, rows, Lk, ldS, ldP, nsplit, stride, scale)
+                       S, out, rows, Lk, ldS, ldP, nsplit, stride, scale)
     if (Lk > 8192 || rows > INT32_MAX)
-        hipLaunchKernelGGL(k_softmax_long<KIND>, dim3((unsigned)std::min<long>(rows, 65536)),
-                           dim3(256), 0, st, S, ph, pl, rows, Lk, ldS, ldP, nsplit, stride, scale);
+        hipLaunchKernelGGL((k_softmax_long<KIND, NP>), dim3((unsigned)std::min<long>(rows, 65536)),
+                           dim3(256), 0, st, S, out, rows, Lk, ldS, ldP, nsplit, stride, scale);
     else if (wave && Lk <= 256)
         ATN_SOFTMAX(64, 1);
     else if (wave && Lk <= 512)
@@ -840,35 +972,44 @@ hipError_t softmax_k(float* S, uint16_t* ph, uint16_t* pl, long rows, int Lk, in
 
 }  // namespace
 
-hipError_t launch_qk_tile(int dtype, int tile, QkTileArgs a, hipStream_t st) {
+hipError_t launch_qk_tile(int kind, int tile, QkTileArgs a, hipStream_t st) {
     a.tiles_q = (a.Lq + tile - 1) / tile;
     a.tiles_k = (a.Lk + tile - 1) / tile;
     const unsigned grid = (unsigned)((long)a.BH * a.tiles_q * a.tiles_k * a.nsplit);
     const bool rag = a.D % 4 != 0;
-    if (dtype == kDtypeF32)
+    if (kind == kTileF32)
         run_qk_tile<kKindF32>(tile, a, rag, grid, st);
-    else
+    else if (kind == kTileBF16)
         run_qk_tile<kKindBF16>(tile, a, false, grid, st);
+    else
+        run_qk_tile<kKindX>(tile, a, rag, grid, st);
     return hipGetLastError();
 }
 
-hipError_t launch_softmax_split(int dtype, float* S, uint16_t* ph, uint16_t* pl, long rows, int Lk,
-                                int ldS, int ldP, int nsplit, size_t split_stride, float scale,
-                                hipStream_t st) {
-    return dtype == kDtypeF32
-               ? softmax_k<kKindF32>(S, ph, pl, rows, Lk, ldS, ldP, nsplit, split_stride, scale, st)
-               : softmax_k<kKindBF16>(S, ph, pl, rows, Lk, ldS, ldP, nsplit, split_stride, scale, st);
+hipError_t launch_softmax_split(int kind, int pparts, float* S, uint16_t* const p[3], long rows,
+                                int Lk, int ldS, int ldP, int nsplit, size_t split_stride,
+                                float scale, hipStream_t st) {
+    const PParts out{{p[0], p[1], p[2]}};
+    if (kind == kTileF32)
+        return softmax_k<kKindF32, 2>(S, out, rows, Lk, ldS, ldP, nsplit, split_stride, scale, st);
+    return pparts == 2
+               ? softmax_k<kKindX, 2>(S, out, rows, Lk, ldS, ldP, nsplit, split_stride, scale, st)
+               : softmax_k<kKindX, 3>(S, out, rows, Lk, ldS, ldP, nsplit, split_stride, scale, st);
 }
 
-hipError_t launch_pv_tile(int dtype, int tile, PvTileArgs a, hipStream_t st) {
+hipError_t launch_pv_tile(int kind, int pparts, int tile, PvTileArgs a, hipStream_t st) {
     a.tiles_q = (a.Lq + tile - 1) / tile;
     a.tiles_d = (a.D + tile - 1) / tile;
     const unsigned grid = (unsigned)((long)a.BH * a.tiles_q * a.tiles_d);
     const bool rag = a.ldO % 4 != 0 || a.o_align == 0;
-    if (dtype == kDtypeF32)
-        run_pv_tile<kKindF32>(tile, a, rag, grid, st);
+    if (kind == kTileF32)
+        run_pv_tile<kKindF32, 2>(tile, a, rag, grid, st);
+    else if (kind == kTileF32Exact)
+        run_pv_tile<kKindX, 3>(tile, a, rag, grid, st);
+    else if (pparts == 2)
+        run_pv_tile<kKindBF16, 2>(tile, a, rag, grid, st);
     else
-        run_pv_tile<kKindBF16>(tile, a, rag, grid, st);
+        run_pv_tile<kKindBF16, 3>(tile, a, rag, grid, st);
     return hipGetLastError();
 }
 

@@ -799,10 +799,18 @@ def test_capture_in_a_smaller_workspace(am, dev):
     small = am.call_plan(1, B, Hh, Lq, Lk, D, pe, 40960)
     assert (small["keys_once"], small["scratch"]) == (0, 40960)
     assert am.lib().atn_prepare_pe_ex(ctypes.byref(pe), D, Lk) == 0
-    st = hip_rt.Stream()
     (q1, k1, v1), _ = H.device_inputs((1, 1, 70, 64), (1, 1, 200, 64), 780, "bf16")
-    out1 = am.attention_ex(q1, k1, v1, stream=st)  # the stream's workspace: 40 KiB
-    st.synchronize()
+    out1, streams = H.empty(q1.shape, "bf16"), []
+    for _ in range(32):  # (a stream may have the handle, and the workspace, of one destroyed before)
+        st = hip_rt.Stream()
+        streams.append(st)
+        held = am.retained_bytes()
+        am.attention_ex(q1, k1, v1, out1, stream=st)
+        st.synchronize()
+        if am.retained_bytes() - held == 40960:  # its workspace, allocated now
+            break
+    else:
+        pytest.fail("no stream without a workspace")
     (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 781, "bf16")
     ws = hip_rt.DeviceArray((40960 // 4,), "f32", fill=0)
     eager, out = H.empty(Q.shape, "bf16"), H.empty(Q.shape, "bf16")
@@ -831,4 +839,5 @@ def test_capture_in_a_smaller_workspace(am, dev):
 
     hip_rt.Graph(st, refused).destroy()
     assert status == [am.ATN_ERR_CAPTURE]
-    st.destroy()
+    for x in streams:
+        x.destroy()

@@ -89,6 +89,90 @@ def test_misaligned_bases(am, dev, D):
     _check(out.numpy()[1:].reshape(Q.shape), Q, K, V, "none")
 
 
+# Inputs far from magnitude 1 (exponents of 2 on Q, K and V), and one large
+# element among ordinary ones.
+RANGES = {"v-20": (0, 0, -20), "v-30": (0, 0, -30), "v-90": (0, 0, -90), "v+60": (0, 0, 60), "v+120": (0, 0, 120),
+          "q-13": (-13, 13, 0), "q+13": (13, -13, 0), "q-60": (-60, 60, 0), "outliers": (0, 0, 0)}
+
+
+def _ranged(rng_case, dims, seed):
+    B, Hh, Lq, Lk, D = dims
+    Q, K, V = H.rng_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), seed=seed)
+    eq, ek, ev = RANGES[rng_case]
+    Q, K, V = (np.ldexp(x, e).astype(np.float32) for x, e in ((Q, eq), (K, ek), (V, ev)))
+    if rng_case == "outliers":
+        V[:, :, Lk // 2, 5] = 1e9     # one column; the others keep their bits
+        Q[:, :, 7] *= np.float32(1e-6)
+        K[:, :, 3] *= np.float32(1e-6)
+        K[:, :, 40, 11] = 1e6         # a key that some rows see alone
+    return Q, K, V
+
+
+def _offset_call(am, Q, K, V, es=4):
+    """The call on tensors `es` bytes off a 16-byte boundary."""
+    import hip_rt
+    B, Hh, Lq, D = Q.shape
+    dev_t = [H.upload(np.concatenate([[0.0], x.ravel()]).astype(np.float32)) for x in (Q, K, V)]
+    out = H.empty((Q.size + 1,))
+    st = am.lib().atn_attention_fwd_ex(0, *[t.ptr + es for t in dev_t], out.ptr + es, B, Hh, Lq, K.shape[2], D,
+                                       None, None, 0, None)
+    assert st == 0
+    hip_rt.synchronize()
+    return out.numpy()[1:].reshape(Q.shape)
+
+
+def _check64(got, Q, K, V, skip=()):
+    """Normwise against float64, column by column of the output (an outlier's
+    column says nothing about the others).  fp32 sums keep 2^-24 of their
+    terms; with the exponential's and the softmax's roundings the worst column
+    of these sizes shows 1e-6, the bar is 4e-6."""
+    ref = H.sdpa64(Q, K, V)
+    keep = [d for d in range(Q.shape[-1]) if d not in skip]
+    g, r = (x[..., keep].reshape(-1, len(keep)).astype(np.float64) for x in (got, ref))
+    assert np.isfinite(g).all()
+    err = np.linalg.norm(g - r, axis=0) / np.linalg.norm(r, axis=0)
+    assert err.max() < 4e-6, (float(err.max()), int(err.argmax()))
+
+
+@pytest.mark.parametrize("rng_case", list(RANGES))
+@pytest.mark.parametrize("D,off", [(258, 0), (261, 0), (263, 0), (264, 4), (1030, 0)], ids=str)
+def test_fp32_magnitudes_of_odd_rows(am, dev, D, off, rng_case):
+    """fp32 with head_d % 4 != 0 or misaligned bases keeps fp32's accuracy
+    wherever the values lie."""
+    print(f"[case] magnitudes {D} +{off} {rng_case}", flush=True)
+    Q, K, V = _ranged(rng_case, (1, 2, 150, 140, D), 980 + D)
+    if off:
+        got = _offset_call(am, Q, K, V, off)
+    else:
+        import hip_rt
+        out = H.empty(Q.shape)
+        am.attention_ex(*(H.upload(x) for x in (Q, K, V)), out)
+        hip_rt.synchronize()
+        got = out.numpy()
+    _check64(got, Q, K, V)
+
+
+@pytest.mark.parametrize("tile", [64, 128])
+def test_fp32_infinities_of_odd_rows(am, dev, tuner, tile):
+    """Infinite operands: a key whose scores are -inf weighs nothing, an
+    infinite value stays in its column, as the same products in float64."""
+    import hip_rt
+    tuner.set(splitd_tile=tile)
+    B, Hh, Lq, Lk, D = 1, 1, 140, 150, 261
+    print(f"[case] infinities, tile {tile}", flush=True)
+    Q, K, V = H.rng_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), seed=991)
+    K[0, 0, 20, 9] = -np.inf
+    Q[..., 9] = np.abs(Q[..., 9])      # every score of key 20 is -inf
+    V[0, 0, 77, 130] = np.inf
+    V[0, 0, 78, 200] = np.float32(3.4e38)
+    out = H.empty(Q.shape)
+    am.attention_ex(*(H.upload(x) for x in (Q, K, V)), out)
+    hip_rt.synchronize()
+    got = out.numpy()
+    assert np.isposinf(got[..., 130]).all()
+    _check64(got, Q, K, V, skip=(130,))
+
+
 @pytest.mark.parametrize("pe", ["rope", "half", "sin"])
 def test_scratch_without_encoded_copies(am, dev, tuner, pe):
     """K's encoded copy alone exceeds the scratch: encoded in the QK^T kernel."""
