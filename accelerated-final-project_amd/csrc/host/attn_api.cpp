@@ -806,8 +806,9 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
     p.ldP = (int)((s.Lk + 7) / 8 * 8);
     const bool bf = dtype == ATN_DTYPE_BF16;
     // fp32 rows that no 16-byte load takes (head_d % 4 != 0, misaligned bases)
-    // keep all 24 bits at any magnitude, as on fp32 MFMA
-    const bool exact = !bf && (s.D % 4 != 0 || !a16);
+    // keep all 24 bits at any magnitude, as on fp32 MFMA, and so do the flash
+    // kernel's calls (plan.tiles), which scales Q and K tile by tile
+    const bool exact = !bf && (s.D % 4 != 0 || !a16 || plan.tiles);
     p.qk = bf && plan.pek == atn::kPeNone ? atn::kTileBF16 : exact ? atn::kTileF32Exact : atn::kTileF32;
     p.pv = bf ? atn::kTileBF16 : exact ? atn::kTileF32Exact : atn::kTileF32;
     p.pparts = p.pv == atn::kTileF32Exact ? 3 : 2;
@@ -1058,17 +1059,24 @@ FlashPlan flash_plan(int dtype, const Shape& s, const PePlan& plan, size_t cap) 
 // those are the faster: head_d 129-256 on a grid so small that the flash
 // kernel's workgroups, which hold 256 dims of output each and take about 7 us
 // beside their tiles (first loads, last stores), leave CUs idle and its key
-// splits need a merge.  (1,4,417,417,256) fp32 27.4 -> 21.0 us, bf16 22.8 ->
-// 17.2; (2,16,142,142,256) fp32 25.4 -> 18.7; (1,8,130,130,200) 17.6 -> 12.4 and
-// 14.9 -> 11.2.  Of 42 calls timed both ways the line at 0.8 takes 10 over,
-// each faster, and leaves 6 that would gain 6-12 %; (1,8,600,600,256) is past
-// it (34.7 us against 36.2, bf16 29.2 against 34.2).  At head_d <= 128 the
+// splits need a merge.  bf16 (1,4,417,417,256) 22.8 -> 17.2 us, (1,8,130,130,200)
+// 14.9 -> 11.2.  fp32 runs there as three bf16 parts, since the flash kernel
+// scales Q and K into fp16's range and the two fp16 parts of other tiles do
+// not: (1,16,100,100,256) 21.8 -> 15.5, (1,4,300,300,256) 24.0 -> 20.4,
+// (1,8,300,300,256) 27.1 -> 25.1, (2,16,142,142,256) 26.1 -> 25.4.  The line at
+// 0.8 leaves calls that would gain 6-12 %; fp32 past 192 dims, where the two
+// estimates agree to a few per cent, has it at 0.93 (at 136 and 132 dims the
+// flash kernel leads by 15 and 7 % at ratios of 0.82).  (1,8,600,600,256) is
+// past it (36.9 us against 49.1, bf16 29.2 against 34.2).  At head_d <= 128 the
 // flash kernel led at 50 of 52.  Only where the whole call's scratch fits.
 void plan_flash(int dtype, const Shape& s, PePlan& plan, size_t cap) {
     plan.flash = flash_plan(dtype, s, plan, cap);
     if (s.D <= 128 || tune().flash_form != 0 || tune().flash_split != 0) return;
-    const TilePlan tp = tile_plan(dtype, s, plan, true);
-    if (!tp.ok || tp.Dp != 0 || tp.bytes > cap || tp.us >= 0.8 * (plan.flash.us + 7.0)) return;
+    PePlan t = plan;
+    t.tiles = true;
+    const TilePlan tp = tile_plan(dtype, s, t, true);
+    const double line = dtype == ATN_DTYPE_F32 && s.D > 192 ? 0.93 : 0.8;
+    if (!tp.ok || tp.Dp != 0 || tp.bytes > cap || tp.us >= line * (plan.flash.us + 7.0)) return;
     plan.tiles = true;
     plan.dchunk = tp.dchunk;
 }

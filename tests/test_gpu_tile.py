@@ -315,9 +315,10 @@ def test_chunked_tiles(am, dev):
     assert n == 0, (nrel, mabs)
 
 
-@pytest.mark.parametrize("dt", ["f32", "bf16"])
-@pytest.mark.parametrize("shape", [(1, 4, 417, 417, 256), (1, 8, 130, 130, 200), (1, 1, 300, 290, 136),
-                                   (2, 3, 65, 129, 248)], ids=str)
+@pytest.mark.parametrize("dt,shape", [
+    ("f32", (1, 4, 300, 300, 256)), ("f32", (1, 8, 130, 130, 200)), ("f32", (1, 16, 100, 100, 256)),
+    ("f32", (2, 3, 65, 129, 248)), ("bf16", (1, 4, 417, 417, 256)), ("bf16", (1, 8, 130, 130, 200)),
+    ("bf16", (2, 3, 65, 129, 248))], ids=str)
 def test_small_grids_of_the_flash_kernel(am, dev, tuner, dt, shape):
     """head_d 129-256 on small grids runs on the tiles, and on the flash kernel
     where the scratch is too small for them: both against the oracle, and a
@@ -327,6 +328,8 @@ def test_small_grids_of_the_flash_kernel(am, dev, tuner, dt, shape):
     code = {"f32": 0, "bf16": 1}[dt]
     print(f"[case] flash or tiles {dt} {shape}", flush=True)
     assert am.path(code, B, Hh, Lq, Lk, D) == am.ATN_PATH_FLASH
+    assert am.call_plan(code, B, Hh, Lq, Lk, D)["tiles"] == 1
+    assert am.call_plan(code, B, Hh, Lq, Lk, D, None, 64 << 10)["path"] == am.ATN_PATH_FLASH
     (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 820 + Lq, dt)
     out, small, flash = (H.empty(Q.shape, dt) for _ in range(3))
     am.attention_ex(q, k, v, out)
@@ -341,3 +344,18 @@ def test_small_grids_of_the_flash_kernel(am, dev, tuner, dt, shape):
         assert n == 0, (nrel, mabs)
     assert np.array_equal(small.numpy(), flash.numpy())
     assert not np.array_equal(out.numpy(), flash.numpy())  # the tiles' sums
+
+
+@pytest.mark.parametrize("rng_case", list(RANGES))
+def test_fp32_magnitudes_of_small_flash_grids(am, dev, rng_case):
+    """fp32 of head_d 129-256 moved to the tiles keeps its accuracy wherever
+    the values lie."""
+    import hip_rt
+    dims = (1, 2, 150, 140, 256)
+    print(f"[case] magnitudes, small flash grid {rng_case}", flush=True)
+    assert am.call_plan(0, *dims)["tiles"] == 1
+    Q, K, V = _ranged(rng_case, dims, 985)
+    out = H.empty(Q.shape)
+    am.attention_ex(*(H.upload(x) for x in (Q, K, V)), out)
+    hip_rt.synchronize()
+    _check64(out.numpy(), Q, K, V)
