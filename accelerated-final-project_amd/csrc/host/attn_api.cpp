@@ -789,12 +789,13 @@ struct TilePlan {
 // time, so it is the faster wherever its grid fills the chip.  Stages: fp32
 // (and Q K^T of encoded bf16) 32 deep, bf16 Q K^T 64 deep, bf16 P V 32 keys.
 double tile_us(int kind, bool pv, int tile, int64_t wgs, int64_t stages) {
-    // fp32, bf16 Q K^T, exact fp32, bf16 P V
-    static const double c[4][2][4] = {{{0.36, 0.09, 0.45, 0.28}, {0.58, 0.36, 1.50, 0.75}},
+    // fp32, bf16 Q K^T, exact fp32, fp32 as two bf16 parts, bf16 P V
+    static const double c[5][2][4] = {{{0.36, 0.09, 0.45, 0.28}, {0.58, 0.36, 1.50, 0.75}},
                                       {{0.30, 0.08, 0.40, 0.23}, {0.58, 0.17, 1.30, 0.60}},
                                       {{0.42, 0.42, 1.03, 0.54}, {1.20, 0.55, 3.10, 1.80}},
+                                      {{0.36, 0.12, 0.48, 0.32}, {0.60, 0.50, 1.70, 0.84}},
                                       {{0.30, 0.10, 0.42, 0.26}, {0.45, 0.42, 1.50, 0.68}}};
-    const double* k = c[pv && kind == atn::kTileBF16 ? 3 : kind][tile == 128];
+    const double* k = c[pv && kind == atn::kTileBF16 ? 4 : kind][tile == 128];
     const double w = (double)wgs / 256.0;
     return (w <= 1.0 ? k[0] + k[1] * w : std::max(k[2], k[3] * w)) * (double)stages;
 }
@@ -809,10 +810,17 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
     // keep all 24 bits at any magnitude, as on fp32 MFMA, and so do the flash
     // kernel's calls (plan.tiles), which scales Q and K tile by tile
     const bool exact = !bf && (s.D % 4 != 0 || !a16 || plan.tiles);
-    p.qk = bf && plan.pek == atn::kPeNone ? atn::kTileBF16 : exact ? atn::kTileF32Exact : atn::kTileF32;
+    p.qk = exact ? atn::kTileF32Exact : atn::kTileF32;
+    // bf16 with an encoding: the GEMM path holds encoded rows in 11 bits at any
+    // magnitude (fp16 and a scale per row), its small grids here in 16; calls
+    // that it does not take ran on fp32 MFMA
+    const bool odd = s.D % 8 != 0 || !a16;
+    if (bf)
+        p.qk = plan.pek == atn::kPeNone ? atn::kTileBF16
+                                        : (odd ? atn::kTileF32Exact : atn::kTileF32Bf16x2);
     p.pv = bf ? atn::kTileBF16 : exact ? atn::kTileF32Exact : atn::kTileF32;
     p.pparts = p.pv == atn::kTileF32Exact ? 3 : 2;
-    if (bf && (s.D % 8 != 0 || !a16)) p.Dp = (s.D + 7) / 8 * 8;
+    if (bf && odd) p.Dp = (s.D + 7) / 8 * 8;
     const int64_t es = p.qk == atn::kTileBF16 ? 2 : 4, lim = atn::kTileMaxBytes, W = std::max(s.D, p.Dp);
     if ((int64_t)s.Lq * W * es >= lim || (int64_t)s.Lk * W * es >= lim ||
         (int64_t)s.Lq * p.ldP * 2 >= lim)
@@ -881,12 +889,13 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
 // workgroups (wall times of 29 shapes; K's encoding inside the GEMM makes a
 // step 2.2 us, an encoding pass costs its traffic).  The tiles cut D as well
 // and win there: (1,2,68,68,624) 37.3 -> 10.6 us, (2,4,82,82,2392) 72.5 ->
-// 16.3, (1,4,512,512,2048) 62.5 -> 31, (1,8,64,4096,2048) 195 -> 91; from
-// about 128 GEMM tiles on the GEMMs lead ((4,8,444,444,1008) 66 against 93
-// us, (4,16,508,508,1888) 201 against 315).  Only where the whole call's scratch
-// fits: the tiles need fp32 copies of encoded Q and K, and in chunks of a head
-// or fewer each they lose to the one GEMM call ((1,8,64,4096,2048) rotate-half
-// in 64 MiB 715 us, the GEMMs 225).
+// 16.3, (1,4,512,512,2048) 62.5 -> 31, (1,8,64,4096,2048) 195 -> 91, rotate-half
+// (2,8,300,300,1024) 70 -> 59; from about 128 GEMM tiles on the GEMMs lead
+// ((4,8,444,444,1008) 66 against 93 us, (4,16,508,508,1888) 201 against 315).
+// At 0.85 of the GEMMs' estimate and below: rotate-half (1,8,64,4096,2048), at
+// 0.87, takes 224 us either way and 289 MB of scratch for encoded copies
+// against 25.  Only where the whole call's scratch fits: in chunks of a head or
+// fewer each the tiles lose to the one GEMM call (that one in 64 MiB 715 us).
 void choose_tiles(int dtype, const Shape& s, PePlan& plan, size_t cap) {
     const TilePlan tp = tile_plan(dtype, s, plan, true);
     if (!tp.ok) return;
@@ -901,7 +910,7 @@ void choose_tiles(int dtype, const Shape& s, PePlan& plan, size_t cap) {
                 std::ceil(wgs(s.Lq, s.D)) * ((s.Lk + 63) / 64) * 2.2;
     if (gp.encoded) us += 4.0 + (double)s.nq * 4.0 / 4.5e6;
     if (gp.encoded && gp.benc == 0) us += 4.0 + (double)s.nk * 4.0 / 4.5e6;
-    plan.tiles = tp.bytes <= cap && tp.us < 0.95 * us;
+    plan.tiles = tp.bytes <= cap && tp.us < 0.85 * us;
 }
 
 // ---------------------------------------------------------------- core

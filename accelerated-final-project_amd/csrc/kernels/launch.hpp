@@ -48,12 +48,13 @@ hipError_t launch_pv_s16(const float* P, const float* V, float* O, int BH, int L
 // P's 16-bit parts ldP (a multiple of 8) elements apart.  A kind says how the
 // operands enter the products: fp32 as two fp16 parts (22 bits; a tile with
 // values beyond fp16's range scales its stages), fp32 as three bf16 parts
-// (all 24 bits at any magnitude), or bf16 as it is.  P has two fp16 parts for
-// the first, three bf16 parts for the second, pparts bf16 parts for bf16 V.
+// (all 24 bits at any magnitude) or, Q K^T alone, as two (16 bits), or bf16 as
+// it is.  P has two fp16 parts for the first, three bf16 parts for the second,
+// pparts bf16 parts for bf16 V.
 // fp32 takes any head_d and element-aligned bases, bf16 head_d % 8 == 0 and
 // 16-byte aligned Q, K and V; every head's tensors and P parts under
 // kTileMaxBytes.
-constexpr int kTileF32 = 0, kTileBF16 = 1, kTileF32Exact = 2;
+constexpr int kTileF32 = 0, kTileBF16 = 1, kTileF32Exact = 2, kTileF32Bf16x2 = 3;
 constexpr long kTileMaxBytes = (1L << 31) - 65536;
 struct QkTileArgs {
     const void* Q;

@@ -4,8 +4,9 @@
 //
 // Operands (KIND): fp32 as hi + lo fp16 parts (split16.hpp, three exact
 // products per product), fp32 as three bf16 parts (X: all 24 bits at any
-// magnitude, six products), or raw bf16 (one exact product).  P leaves the
-// softmax already split, so the PV kernel converts V alone.
+// magnitude, six products) or two (B2: 16 bits, three products), or raw bf16
+// (one exact product).  P leaves the softmax already split, so the PV kernel
+// converts V alone.
 //
 // X serves fp32 rows at any alignment (head_d % 4 != 0, misaligned bases), which
 // ran on fp32 MFMA before and keep its accuracy at any magnitude.  Two fp16
@@ -71,7 +72,7 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 
-constexpr int kKindF32 = kTileF32, kKindBF16 = kTileBF16, kKindX = kTileF32Exact;
+constexpr int kKindF32 = kTileF32, kKindBF16 = kTileBF16, kKindX = kTileF32Exact, kKindB2 = kTileF32Bf16x2;
 
 // Depth of a QK stage: 128 bytes of a row either way (fp32: 32 elements as
 // PARTS parts; bf16: 64 elements, the two 32-deep halves in the parts' places).
@@ -138,24 +139,25 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t (&w)[N]) {
 // Magnitudes from here on round to an infinite first part.
 constexpr float kBf16Range = 0x1.ffp127f;
 
-// The parts of 4 values (16 bytes) of kind F32 (one = 1) or X
+// The parts of 4 values (16 bytes) of kind F32 (one = 1), X or B2
 template <int KIND>
 __device__ __forceinline__ void split_parts(const uint4& u, float one, uint2 (&p)[Tile<KIND>::PARTS]) {
     if constexpr (KIND == kKindF32) {
         split4(u, one, p[0], p[1]);
     } else {
+        constexpr int N = Tile<KIND>::PARTS;
         const float4 v = as_f4(u);
-        uint32_t a[3], b[3];
+        uint32_t a[N], b[N];
         split_bf16(v.x, v.y, a);
         split_bf16(v.z, v.w, b);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) p[k] = make_uint2(a[k], b[k]);
+        for (int k = 0; k < N; ++k) p[k] = make_uint2(a[k], b[k]);
     }
 }
 
 // One 32 x 32 x 16 product of split operands added to c: the parts' products
-// down to 2^-22 (two fp16 parts) or 2^-25 (three bf16 parts) of the leading
-// one, the smallest first.
+// down to 2^-22 (two fp16 parts), 2^-25 (three bf16 parts) or 2^-17 (two) of the
+// leading one, the smallest first.
 template <int KIND, int N>
 __device__ __forceinline__ v16f mfma_parts(const uint4 (&a)[N], const uint4 (&b)[N], v16f c) {
     if constexpr (KIND == kKindX) {
@@ -430,7 +432,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
         }
     }
 
-    if constexpr (KIND == kKindX) {
+    if constexpr (KIND == kKindX || KIND == kKindB2) {
         if (wg_over<NW>(big, kBf16Range, flag)) {
             // on fp32 MFMA, from rows of fp32 (33 apart) in the parts' places
             constexpr int R = 33;
@@ -981,6 +983,8 @@ hipError_t launch_qk_tile(int kind, int tile, QkTileArgs a, hipStream_t st) {
         run_qk_tile<kKindF32>(tile, a, rag, grid, st);
     else if (kind == kTileBF16)
         run_qk_tile<kKindBF16>(tile, a, false, grid, st);
+    else if (kind == kTileF32Bf16x2)
+        run_qk_tile<kKindB2>(tile, a, rag, grid, st);
     else
         run_qk_tile<kKindX>(tile, a, rag, grid, st);
     return hipGetLastError();

@@ -240,6 +240,25 @@ def test_tile_edges_bf16(am, dev, tuner, tile, shape, pe):
     assert nrel < 2.0 ** -9
 
 
+@pytest.mark.parametrize("eq,ek", [(-60, 60), (60, -60), (-14, 14), (18, -18)], ids=str)
+@pytest.mark.parametrize("D,pe", [(272, "half"), (262, "rope"), (272, "half_k")], ids=str)
+def test_bf16_encoded_magnitudes(am, dev, D, pe, eq, ek):
+    """Encoded bf16 Q and K at any magnitude (16 bits of them, 24 where head_d
+    % 8 != 0): the output's own rounding is the error."""
+    import hip_rt
+    B, Hh, Lq, Lk = 1, 2, 130, 140
+    print(f"[case] bf16 encoded magnitudes {D} {pe} {eq} {ek}", flush=True)
+    assert am.call_plan(1, B, Hh, Lq, Lk, D, _desc(am, pe))["tiles"] == 1
+    (_, _, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 815, "bf16")
+    q, k = H.upload(np.ldexp(Q, eq), "bf16"), H.upload(np.ldexp(K, ek), "bf16")
+    out = H.empty(Q.shape, "bf16")
+    am.attention_ex(q, k, v, out, pe=_desc(am, pe))
+    hip_rt.synchronize()
+    n, nrel, mabs = H.check_bf16(out.numpy(), _ref(pe, Q, K, V))
+    assert n == 0, (nrel, mabs)
+    assert nrel < 2.0 ** -9
+
+
 @pytest.mark.parametrize("D", [264, 267, 40], ids=str)
 def test_misaligned_bases_bf16(am, dev, D):
     """bf16 tensors 2 bytes off: copied into aligned rows first."""
