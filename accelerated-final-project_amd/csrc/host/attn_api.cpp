@@ -806,21 +806,25 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
     p.ldS = (int)((s.Lk + 3) / 4 * 4);
     p.ldP = (int)((s.Lk + 7) / 8 * 8);
     const bool bf = dtype == ATN_DTYPE_BF16;
-    // fp32 rows that no 16-byte load takes (head_d % 4 != 0, misaligned bases)
-    // keep all 24 bits at any magnitude, as on fp32 MFMA, and so do the flash
-    // kernel's calls (plan.tiles), which scales Q and K tile by tile
+    // No call holds its operands in fewer bits than on the path it comes from:
+    // - fp32 rows that no 16-byte load takes (head_d % 4 != 0, misaligned
+    //   bases) ran on fp32 MFMA, the flash kernel's calls (plan.tiles) with
+    //   scales per tile: all 24 bits at any magnitude;
+    // - bf16 that the GEMM path does not take (head_d % 8 != 0, misaligned)
+    //   ran on fp32 MFMA: encoded Q and K and P keep 24 bits;
+    // - bf16 of the GEMM path, which holds encoded rows and P in 11 bits
+    //   (fp16, a scale per row): 16.
     const bool exact = !bf && (s.D % 4 != 0 || !a16 || plan.tiles);
-    p.qk = exact ? atn::kTileF32Exact : atn::kTileF32;
-    // bf16 with an encoding: the GEMM path holds encoded rows in 11 bits at any
-    // magnitude (fp16 and a scale per row), its small grids here in 16; calls
-    // that it does not take ran on fp32 MFMA
-    const bool odd = s.D % 8 != 0 || !a16;
-    if (bf)
+    const bool odd = bf && (s.D % 8 != 0 || !a16);
+    if (!bf)
+        p.qk = p.pv = exact ? atn::kTileF32Exact : atn::kTileF32;
+    else {
+        p.pv = atn::kTileBF16;
         p.qk = plan.pek == atn::kPeNone ? atn::kTileBF16
                                         : (odd ? atn::kTileF32Exact : atn::kTileF32Bf16x2);
-    p.pv = bf ? atn::kTileBF16 : exact ? atn::kTileF32Exact : atn::kTileF32;
-    p.pparts = p.pv == atn::kTileF32Exact ? 3 : 2;
-    if (bf && odd) p.Dp = (s.D + 7) / 8 * 8;
+    }
+    p.pparts = exact || odd ? 3 : 2;
+    if (odd) p.Dp = (s.D + 7) / 8 * 8;
     const int64_t es = p.qk == atn::kTileBF16 ? 2 : 4, lim = atn::kTileMaxBytes, W = std::max(s.D, p.Dp);
     if ((int64_t)s.Lq * W * es >= lim || (int64_t)s.Lk * W * es >= lim ||
         (int64_t)s.Lq * p.ldP * 2 >= lim)
