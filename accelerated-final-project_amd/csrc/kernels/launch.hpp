@@ -51,8 +51,9 @@ hipError_t launch_pv_s16(const float* P, const float* V, float* O, int BH, int L
 // (all 24 bits at any magnitude) or, Q K^T alone, as two (16 bits), or bf16 as
 // it is.  P has two fp16 parts for the first, three bf16 parts for the second,
 // pparts bf16 parts for bf16 V.
-// fp32 takes any head_d and element-aligned bases, bf16 head_d % 8 == 0 and
-// 16-byte aligned Q, K and V; every head's tensors and P parts under
+// kTileF32Exact takes any head_d and element-aligned bases, kTileF32 head_d % 4
+// == 0 and aligned output rows, bf16 head_d % 8 == 0 and 16-byte aligned Q, K and
+// V; every head's tensors and P parts under
 // kTileMaxBytes.
 constexpr int kTileF32 = 0, kTileBF16 = 1, kTileF32Exact = 2, kTileF32Bf16x2 = 3;
 constexpr long kTileMaxBytes = (1L << 31) - 65536;

@@ -32,7 +32,10 @@
 // clear of spills: a spill's reload waits (vmcnt) for the loads in flight.  A
 // value beyond fp16's range is found in passing (one v_max3 per pair); its
 // workgroup then computes the tile again, every stage scaled by powers of two
-// from its largest finite magnitudes.
+// from its largest finite magnitudes, the next stage's loads in flight.  Where
+// the first stage already holds one, the pass before is left out: K of 2^20
+// at (1,4,512,512,2048) 92 -> 75 us, with V of 2^20 115 -> 82 (a look at every
+// pair of stages instead made ordinary calls 6-8 % longer).
 //
 // Tiles of 128 x 128 or 64 x 64 (4 waves) on 32 x 32 x 16 MFMA.  A grid of at
 // most one 128 x 128 workgroup a CU runs it as 8 waves of 64 x 32, two to a
@@ -205,16 +208,18 @@ __device__ __forceinline__ float max4abs(float m, const uint4& u) {
     return vmax3abs(vmax3abs(m, v.x, v.y), v.z, v.w);
 }
 
-// Whether any thread of the workgroup saw a magnitude of `range` or more
-template <int NW>
-__device__ __forceinline__ bool wg_over(float big, float range, int* flag) {
+// Whether any thread of the workgroup saw a magnitude of `range` or more:
+// told before a barrier, asked behind it (of words that nothing overwrites)
+__device__ __forceinline__ void tell_over(float big, float range, int* flag) {
     const bool over = __ballot(!(big < range)) != 0;
     if ((threadIdx.x & 63) == 0) flag[threadIdx.x >> 6] = over;
-    __syncthreads();
+}
+template <int NW>
+__device__ __forceinline__ bool any_over(const int* flag) {
     int any = flag[0];
 #pragma unroll
     for (int w = 1; w < NW; ++w) any |= flag[w];
-    return any != 0;
+    return __builtin_amdgcn_readfirstlane(any) != 0;
 }
 
 // 4 consecutive elements to an address of element alignment only: one store
@@ -245,7 +250,9 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
     __shared__ __align__(16) uint16_t sq[2][NP * PART];  // [stage][part][row][32]
     __shared__ __align__(16) uint16_t sk[2][NP * PART];
     __shared__ float slot[2 * NW];
-    __shared__ int flag[NW];
+    __shared__ int flag[2][NW];
+    constexpr bool kRanged = KIND != kKindBF16;
+    constexpr float kRange = KIND == kKindF32 ? kF16Range : kBf16Range;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -381,29 +388,39 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
     if (AHEAD == 2) issue(r1, dbeg + G::DEPTH);
     zero();
     store(r0, sq[0], sk[0]);
+    if (kRanged) tell_over(big, kRange, flag[0]);
     issue(r0, dbeg + AHEAD * G::DEPTH);
     __syncthreads();
-    const int stages = (dend - dbeg + G::DEPTH - 1) / G::DEPTH;
-    for (int n = 0, d0 = dbeg; n < stages >> 1; ++n, d0 += 2 * G::DEPTH) {
-        compute(sq[0], sk[0], std::true_type{});
-        store(rb, sq[1], sk[1]);
-        issue(rb, d0 + (AHEAD + 1) * G::DEPTH);
-        __syncthreads();
-        compute(sq[1], sk[1], std::false_type{});
-        flush();
-        store(r0, sq[0], sk[0]);
-        issue(r0, d0 + (AHEAD + 2) * G::DEPTH);
-        __syncthreads();
-    }
-    if (stages & 1) {
-        compute(sq[0], sk[0], std::true_type{});
-        flush();
+    // a tensor far from 1 shows in the first stage: no pass in vain then
+    bool redo = kRanged && any_over<NW>(flag[0]);
+    if (!redo) {
+        const int stages = (dend - dbeg + G::DEPTH - 1) / G::DEPTH;
+        for (int n = 0, d0 = dbeg; n < stages >> 1; ++n, d0 += 2 * G::DEPTH) {
+            compute(sq[0], sk[0], std::true_type{});
+            store(rb, sq[1], sk[1]);
+            issue(rb, d0 + G::DEPTH * (AHEAD + 1));
+            __syncthreads();
+            compute(sq[1], sk[1], std::false_type{});
+            flush();
+            store(r0, sq[0], sk[0]);
+            issue(r0, d0 + G::DEPTH * (AHEAD + 2));
+            __syncthreads();
+        }
+        if (stages & 1) {
+            compute(sq[0], sk[0], std::true_type{});
+            flush();
+        }
+        if (kRanged) {
+            tell_over(big, kRange, flag[1]);
+            __syncthreads();
+            redo = any_over<NW>(flag[1]);
+            if (redo) zero();
+        }
     }
     if constexpr (KIND == kKindF32) {
-        if (wg_over<NW>(big, kF16Range, flag)) {
-            zero();
+        if (redo) {  // every stage scaled by its largest magnitudes
+            issue(r0, dbeg);
             for (int d0 = dbeg; d0 < dend; d0 += G::DEPTH) {
-                issue(r0, d0);
                 float mq = 0.f, mk = 0.f;
 #pragma unroll
                 for (int i = 0; i < ROUNDS; ++i) {
@@ -424,6 +441,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
                     *reinterpret_cast<uint2*>(sk[0] + o) = hi;
                     *reinterpret_cast<uint2*>(sk[0] + PART + o) = lo;
                 }
+                issue(r0, d0 + G::DEPTH);
                 __syncthreads();
                 const float u = pow2_unit(mq) * pow2_unit(mk);
                 compute(sq[0], sk[0], std::true_type{});
@@ -433,12 +451,11 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
     }
 
     if constexpr (KIND == kKindX || KIND == kKindB2) {
-        if (wg_over<NW>(big, kBf16Range, flag)) {
+        if (redo) {
             // on fp32 MFMA, from rows of fp32 (33 apart) in the parts' places
             constexpr int R = 33;
             float* fq = reinterpret_cast<float*>(sq);
             float* fk = reinterpret_cast<float*>(sk);
-            zero();
             for (int d0 = dbeg; d0 < dend; d0 += G::DEPTH) {
                 issue(r0, d0);
                 __syncthreads();  // the last stage's reads are done
@@ -642,7 +659,9 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_pv_tile(PvTileArgs
     __shared__ __align__(16) uint16_t sp[2][PP * PART];
     __shared__ __align__(16) uint16_t sv[2][VPARTS * VPART];
     __shared__ float slot[2 * NW];
-    __shared__ int flag[NW];
+    __shared__ int flag[2][NW];
+    constexpr bool kRanged = KIND != kKindBF16;
+    constexpr float kRange = KIND == kKindF32 ? kF16Range : kBf16Range;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -780,29 +799,39 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_pv_tile(PvTileArgs
     if (AHEAD == 2) issue(r1, 32);
     zero();
     store(r0, sp[0], sv[0]);
+    if (kRanged) tell_over(big, kRange, flag[0]);
     issue(r0, 32 * AHEAD);
     __syncthreads();
-    const int stages = (a.Lk + 31) / 32;
-    for (int n = 0, kk = 0; n < stages >> 1; ++n, kk += 64) {
-        compute(sp[0], sv[0], std::true_type{});
-        store(rb, sp[1], sv[1]);
-        issue(rb, kk + 32 * (AHEAD + 1));
-        __syncthreads();
-        compute(sp[1], sv[1], std::false_type{});
-        flush();
-        store(r0, sp[0], sv[0]);
-        issue(r0, kk + 32 * (AHEAD + 2));
-        __syncthreads();
-    }
-    if (stages & 1) {
-        compute(sp[0], sv[0], std::true_type{});
-        flush();
+    // a tensor far from 1 shows in the first stage: no pass in vain then
+    bool redo = kRanged && any_over<NW>(flag[0]);
+    if (!redo) {
+        const int stages = (a.Lk + 31) / 32;
+        for (int n = 0, kk = 0; n < stages >> 1; ++n, kk += 64) {
+            compute(sp[0], sv[0], std::true_type{});
+            store(rb, sp[1], sv[1]);
+            issue(rb, kk + 32 * (AHEAD + 1));
+            __syncthreads();
+            compute(sp[1], sv[1], std::false_type{});
+            flush();
+            store(r0, sp[0], sv[0]);
+            issue(r0, kk + 32 * (AHEAD + 2));
+            __syncthreads();
+        }
+        if (stages & 1) {
+            compute(sp[0], sv[0], std::true_type{});
+            flush();
+        }
+        if (kRanged) {
+            tell_over(big, kRange, flag[1]);
+            __syncthreads();
+            redo = any_over<NW>(flag[1]);
+            if (redo) zero();
+        }
     }
     if constexpr (KIND == kKindF32) {
-        if (wg_over<NW>(big, kF16Range, flag)) {
-            zero();
+        if (redo) {  // V's stages scaled by their largest magnitudes
+            issue(r0, 0);
             for (int kk = 0; kk < a.Lk; kk += 32) {
-                issue(r0, kk);
                 float mv = 0.f, none = 0.f;
 #pragma unroll
                 for (int i = 0; i < VROUNDS; ++i) mv = max_finite4(mv, as_f4(r0.v[i]));
@@ -818,6 +847,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_pv_tile(PvTileArgs
                     *reinterpret_cast<uint2*>(sv[0] + o) = hi;
                     *reinterpret_cast<uint2*>(sv[0] + (VPARTS - 1) * VPART + o) = lo;
                 }
+                issue(r0, kk + 32);
                 __syncthreads();
                 compute(sp[0], sv[0], std::true_type{});
                 each([u](v16f& x, v16f& y) { y += x * u; });
@@ -826,12 +856,11 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_pv_tile(PvTileArgs
     }
 
     if constexpr (KIND == kKindX) {
-        if (wg_over<NW>(big, kBf16Range, flag)) {
+        if (redo) {
             // on fp32 MFMA: P put together again (rows 33 apart), V as it is
             constexpr int R = 33;
             float* fp = reinterpret_cast<float*>(sp);
             float* fv = reinterpret_cast<float*>(sv);
-            zero();
             for (int kk = 0; kk < a.Lk; kk += 32) {
                 issue(r0, kk);
                 __syncthreads();  // the last stage's reads are done
@@ -906,8 +935,9 @@ constexpr unsigned kOnePerCu = 256;
 
 template <int KIND, int TL, int NW>
 void run_qk(const QkTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
-    if (KIND != kKindBF16 && rag)
-        hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, KIND != kKindBF16>), dim3(grid), dim3(64 * NW), 0,
+    // (the other kinds' rows are whole 16-byte vectors)
+    if (KIND == kKindX && rag)
+        hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, KIND == kKindX>), dim3(grid), dim3(64 * NW), 0,
                            st, a);
     else
         hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, false>), dim3(grid), dim3(64 * NW), 0, st, a);
@@ -924,8 +954,9 @@ void run_qk_tile(int tile, const QkTileArgs& a, bool rag, unsigned grid, hipStre
 
 template <int KIND, int PP, int TL, int NW>
 void run_pv(const PvTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
-    if (rag)
-        hipLaunchKernelGGL((k_pv_tile<KIND, PP, TL, NW, true>), dim3(grid), dim3(64 * NW), 0, st, a);
+    if (KIND != kKindF32 && rag)
+        hipLaunchKernelGGL((k_pv_tile<KIND, PP, TL, NW, KIND != kKindF32>), dim3(grid), dim3(64 * NW),
+                           0, st, a);
     else
         hipLaunchKernelGGL((k_pv_tile<KIND, PP, TL, NW, false>), dim3(grid), dim3(64 * NW), 0, st, a);
 }
@@ -975,6 +1006,7 @@ hipError_t softmax_k(float* S, const PParts& out, long rows, int Lk, int ldS, in
 }  // namespace
 
 hipError_t launch_qk_tile(int kind, int tile, QkTileArgs a, hipStream_t st) {
+    if (a.D % 4 != 0 && kind != kTileF32Exact) return hipErrorInvalidValue;
     a.tiles_q = (a.Lq + tile - 1) / tile;
     a.tiles_k = (a.Lk + tile - 1) / tile;
     const unsigned grid = (unsigned)((long)a.BH * a.tiles_q * a.tiles_k * a.nsplit);
@@ -1006,6 +1038,7 @@ hipError_t launch_pv_tile(int kind, int pparts, int tile, PvTileArgs a, hipStrea
     a.tiles_d = (a.D + tile - 1) / tile;
     const unsigned grid = (unsigned)((long)a.BH * a.tiles_q * a.tiles_d);
     const bool rag = a.ldO % 4 != 0 || a.o_align == 0;
+    if (rag && kind == kTileF32) return hipErrorInvalidValue;
     if (kind == kTileF32)
         run_pv_tile<kKindF32, 2>(tile, a, rag, grid, st);
     else if (kind == kTileF32Exact)

@@ -173,6 +173,32 @@ def test_fp32_infinities_of_odd_rows(am, dev, tuner, tile):
     _check64(got, Q, K, V, skip=(130,))
 
 
+@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("D,Lk", [(260, 150), (288, 31), (320, 129)], ids=str)  # odd, one and even stage counts
+@pytest.mark.parametrize("where", ["first", "late", "all"])
+def test_values_beyond_fp16_range(am, dev, tuner, tile, D, Lk, where):
+    """fp32 values of 65504 and more, in the first stage of Q K^T and P V (seen
+    before the pass), in the last (after it) and everywhere."""
+    import hip_rt
+    tuner.set(splitd_tile=tile)
+    B, Hh, Lq = 1, 2, 140
+    print(f"[case] beyond fp16 {tile} {D} {Lk} {where}", flush=True)
+    Q, K, V = H.rng_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), seed=992)
+    if where == "all":
+        Q, K, V = np.ldexp(Q, -20), np.ldexp(K, 20), np.ldexp(V, 18)
+    else:
+        d, j = (3, 2) if where == "first" else (D - 2, Lk - 1)
+        Q[:, :, :, d] *= np.float32(2.0 ** -17)
+        K[:, :, :, d] *= np.float32(2.0 ** 17)
+        V[:, :, j, 7] = 1e6
+    out = H.empty(Q.shape)
+    am.attention_ex(*(H.upload(x) for x in (Q, K, V)), out)
+    hip_rt.synchronize()
+    scale = np.float32(2.0 ** 18 if where == "all" else 1.0)
+    n, mabs, _ = H.check_f32(out.numpy() / scale, _ref("none", Q, K, V) / scale)
+    assert n == 0, mabs
+
+
 @pytest.mark.parametrize("pe", ["rope", "half", "sin"])
 def test_scratch_without_encoded_copies(am, dev, tuner, pe):
     """K's encoded copy alone exceeds the scratch: encoded in the QK^T kernel."""
