@@ -800,7 +800,10 @@ double tile_us(int kind, bool pv, int tile, int64_t wgs, int64_t stages) {
     return (w <= 1.0 ? k[0] + k[1] * w : std::max(k[2], k[3] * w)) * (double)stages;
 }
 
-TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
+// 16-byte alignment of a call's tensors
+enum { kA16None = 0, kA16Inputs = 1, kA16All = 2 };
+
+TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, int a16) {
     TilePlan p;
     if (plan.lean) return p;
     p.ldS = (int)((s.Lk + 3) / 4 * 4);
@@ -814,8 +817,8 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
     //   ran on fp32 MFMA: encoded Q and K and P keep 24 bits;
     // - bf16 of the GEMM path, which holds encoded rows and P in 11 bits
     //   (fp16, a scale per row): 16.
-    const bool exact = !bf && (s.D % 4 != 0 || !a16 || plan.tiles);
-    const bool odd = bf && (s.D % 8 != 0 || !a16);
+    const bool exact = !bf && (s.D % 4 != 0 || a16 != kA16All || plan.tiles);
+    const bool odd = bf && (s.D % 8 != 0 || a16 != kA16All);
     if (!bf)
         p.qk = p.pv = exact ? atn::kTileF32Exact : atn::kTileF32;
     else {
@@ -824,7 +827,8 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
                                         : (odd ? atn::kTileF32Exact : atn::kTileF32Bf16x2);
     }
     p.pparts = exact || odd ? 3 : 2;
-    if (odd) p.Dp = (s.D + 7) / 8 * 8;
+    // (the output takes stores at any alignment: no copies for it)
+    if (bf && (s.D % 8 != 0 || a16 == kA16None)) p.Dp = (s.D + 7) / 8 * 8;
     const int64_t es = p.qk == atn::kTileBF16 ? 2 : 4, lim = atn::kTileMaxBytes, W = std::max(s.D, p.Dp);
     if ((int64_t)s.Lq * W * es >= lim || (int64_t)s.Lk * W * es >= lim ||
         (int64_t)s.Lq * p.ldP * 2 >= lim)
@@ -901,7 +905,7 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, bool a16) {
 // against 25.  Only where the whole call's scratch fits: in chunks of a head or
 // fewer each the tiles lose to the one GEMM call (that one in 64 MiB 715 us).
 void choose_tiles(int dtype, const Shape& s, PePlan& plan, size_t cap) {
-    const TilePlan tp = tile_plan(dtype, s, plan, true);
+    const TilePlan tp = tile_plan(dtype, s, plan, kA16All);
     if (!tp.ok) return;
     plan.dchunk = tp.dchunk;
     if (dtype != ATN_DTYPE_BF16 || plan.no_flash || tune().gemm_fused_k != 0) return;
@@ -1087,7 +1091,7 @@ void plan_flash(int dtype, const Shape& s, PePlan& plan, size_t cap) {
     if (s.D <= 128 || tune().flash_form != 0 || tune().flash_split != 0) return;
     PePlan t = plan;
     t.tiles = true;
-    const TilePlan tp = tile_plan(dtype, s, t, true);
+    const TilePlan tp = tile_plan(dtype, s, t, kA16All);
     const double line = dtype == ATN_DTYPE_F32 && s.D > 192 ? 0.93 : 0.8;
     if (!tp.ok || tp.Dp != 0 || tp.bytes > cap || tp.us >= line * (plan.flash.us + 7.0)) return;
     plan.tiles = true;
@@ -1105,7 +1109,7 @@ struct Route {
     size_t need = 0;
 };
 
-Route route(int dtype, const Shape& s, const PePlan& plan, bool query_device, bool vec, bool a16) {
+Route route(int dtype, const Shape& s, const PePlan& plan, bool query_device, bool vec, int a16) {
     Route r;
     if (!plan.no_fused && vec) r.fused = fused_plan(dtype, plan.pek, s, query_device);
     if (r.fused.ok) {
@@ -1113,13 +1117,13 @@ Route route(int dtype, const Shape& s, const PePlan& plan, bool query_device, bo
         r.need = r.fused.bytes;
         return r;
     }
-    if (a16 && flash_ok(dtype, s, plan)) {  // only its key splits' parts and K~
+    if (a16 == kA16All && flash_ok(dtype, s, plan)) {  // only its key splits' parts and K~
         r.path = ATN_PATH_FLASH;
         r.need = kSyncBytes + flash_bytes(s, plan.flash);
         return r;
     }
     r.tile = tile_plan(dtype, s, plan, a16);
-    if (a16 && !(plan.tiles && r.tile.ok)) r.gemm = gemm_plan(dtype, s, plan);
+    if (a16 == kA16All && !(plan.tiles && r.tile.ok)) r.gemm = gemm_plan(dtype, s, plan);
     if (r.gemm.ok) {
         r.path = ATN_PATH_GEMM;
         r.need = r.gemm.bytes;
@@ -1129,19 +1133,24 @@ Route route(int dtype, const Shape& s, const PePlan& plan, bool query_device, bo
     return r;
 }
 
-// A route's scratch.  vec / a16: the alignment of the call's pointers; pass
-// -1 for "unknown" and get the largest of the candidate paths instead.
+// A route's scratch.  vec / a16 (kA16*): the alignment of the call's pointers;
+// pass -1 for "unknown" and get the largest of the candidate paths instead.
 size_t path_need(int dtype, const Shape& s, const PePlan& plan, bool query_device, int vec,
                  int a16) {
-    if (vec >= 0 && a16 >= 0) return route(dtype, s, plan, query_device, vec != 0, a16 != 0).need;
+    if (vec >= 0 && a16 >= 0) return route(dtype, s, plan, query_device, vec != 0, a16).need;
     const FusedPlan fp = plan.no_fused ? FusedPlan{} : fused_plan(dtype, plan.pek, s, query_device);
     if (fp.ok && vec > 0) return fp.bytes;
     const GemmPlan gp = gemm_plan(dtype, s, plan);
-    const TilePlan tp = tile_plan(dtype, s, plan, a16 > 0);
+    const TilePlan tp = tile_plan(dtype, s, plan, kA16None);
     const size_t split = tp.ok ? tp.bytes : kSyncBytes + stream_plan(s).bytes;
     return std::max({fp.ok ? fp.bytes : (size_t)0, gp.ok ? gp.bytes : (size_t)0, split,
                      flash_ok(dtype, s, plan) ? kSyncBytes + flash_bytes(s, plan.flash)
                                               : (size_t)0});
+}
+
+int alignment16(const void* Q, const void* K, const void* V, const void* out) {
+    if (!aligned(Q, 16) || !aligned(K, 16) || !aligned(V, 16)) return kA16None;
+    return aligned(out, 16) ? kA16All : kA16Inputs;
 }
 
 // How a call too large for its scratch is split: chunks of `heads`
@@ -1198,7 +1207,7 @@ Chunking plan_call(int dtype, const Shape& s, PePlan& plan, size_t cap, bool que
         (plan.no_fused || !fused_plan(dtype, plan.pek, s, query_device).ok))
         choose_tiles(dtype, s, plan, cap);
     if (flash_ok(dtype, s, plan)) plan_flash(dtype, s, plan, cap);
-    const size_t need = route(dtype, s, plan, query_device, vec != 0, a16 != 0).need;
+    const size_t need = route(dtype, s, plan, query_device, vec != 0, a16).need;
     if (need <= cap) return Chunking{(int)s.BH, s.Lq, need};
     if ((s.D * elem_size(dtype)) % 16 != 0) vec = a16 = -1;
     const Chunking ch = plan_chunks(dtype, s, plan, cap, query_device, vec, a16);
@@ -1219,11 +1228,11 @@ Chunking plan_call(int dtype, const Shape& s, PePlan& plan, size_t cap, bool que
             Shape x;
             check_shape(1, c.heads, c.rows, s.Lk, s.D, &x);
             return (double)((s.BH + c.heads - 1) / c.heads) * ((s.Lq + c.rows - 1) / c.rows) *
-                   tile_plan(dtype, x, plan, a16 > 0).us;
+                   tile_plan(dtype, x, plan, std::max(a16, 0)).us;
         };
         Shape x;
         check_shape(1, ch.heads, ch.rows, s.Lk, s.D, &x);
-        if (!route(dtype, x, plan, query_device, vec > 0, a16 > 0).tile.ok || us(ch) <= 3.5 * us(lc))
+        if (!route(dtype, x, plan, query_device, vec > 0, std::max(a16, 0)).tile.ok || us(ch) <= 3.5 * us(lc))
             return ch;
     }
     plan.lean = true;
@@ -1240,7 +1249,7 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
     const size_t va = dtype == ATN_DTYPE_F32 ? 16 : 8;
     const int vec_qk = (D % 4 == 0) && aligned(Q, va) && aligned(K, va);
     const int vec_vo = (D % 4 == 0) && aligned(V, va) && aligned(out, va);
-    const bool a16 = aligned(Q, 16) && aligned(K, 16) && aligned(V, 16) && aligned(out, 16);
+    const int a16 = alignment16(Q, K, V, out);
     // (the device's own capacity decides about the single-launch kernel)
     const Route r = route(dtype, s, plan, true, vec_qk && vec_vo, a16);
     const FusedPlan& fd = r.fused;
@@ -1440,11 +1449,9 @@ int attention_core(int dtype, const void* Q, const void* K, const void* V, void*
     const size_t cap = no_alloc ? atn::kNoAllocScratchBytes
                                 : (workspace != nullptr ? workspace_bytes : library_cap());
     const size_t va = dtype == ATN_DTYPE_F32 ? 16 : 8;
-    bool vec = D % 4 == 0, a16 = true;
-    for (const void* p : {Q, K, V, (const void*)out}) {
-        vec = vec && aligned(p, va);
-        a16 = a16 && aligned(p, 16);
-    }
+    bool vec = D % 4 == 0;
+    for (const void* p : {Q, K, V, (const void*)out}) vec = vec && aligned(p, va);
+    const int a16 = alignment16(Q, K, V, out);
     const PePlan fresh = plan;
     Chunking ch = plan_call(dtype, s, plan, cap, true, vec, a16);
     if (workspace == nullptr && !no_alloc && ch.heads != 0) {
@@ -1840,7 +1847,7 @@ size_t atn_attention_workspace_bytes(int dtype, int batch, int heads, int len_q,
     // every path that needs no copies (copies are made where the scratch holds
     // them); each in the chunks that the library's cap would cut it into
     const size_t cap = library_cap();
-    const size_t planned = plan_call(dtype, s, plan, cap, false, head_d % 4 == 0, true).need;
+    const size_t planned = plan_call(dtype, s, plan, cap, false, head_d % 4 == 0, kA16All).need;
     plan.lean = true;
     const size_t full = path_need(dtype, s, plan, false, -1, -1);
     if (full <= cap) return std::max(full, planned);
@@ -1889,11 +1896,11 @@ int atn_call_plan_ex(int dtype, int batch, int heads, int len_q, int len_k, int 
     const bool vec = head_d % 4 == 0;
     *info = atn_call_plan_info{};
     const Chunking ch = plan_call(dtype, s, plan, scratch_bytes ? scratch_bytes : library_cap(), dev,
-                                  vec, true);
+                                  vec, kA16All);
     if (ch.heads == 0) return ATN_ERR_WORKSPACE;
     Shape c;
     check_shape(1, ch.heads, ch.rows, len_k, head_d, &c);
-    const Route r = route(dtype, c, plan, dev, vec, true);
+    const Route r = route(dtype, c, plan, dev, vec, kA16All);
     info->path = r.path;
     info->tiles = r.path == ATN_PATH_SPLIT_D && r.tile.ok;
     if (r.path == ATN_PATH_FLASH) {

@@ -2,6 +2,8 @@
 sizes, odd and even stage counts, head sizes that are no whole number of
 vectors, misaligned bases, encodings per side, every softmax row form, and the
 in-kernel encoding that remains where the scratch holds no encoded copies."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -74,8 +76,6 @@ def test_softmax_row_forms(am, dev, Lq, Lk):
 @pytest.mark.parametrize("D", [264, 267], ids=str)
 def test_misaligned_bases(am, dev, D):
     """Tensors 4 bytes off a 16-byte boundary."""
-    import ctypes
-
     import hip_rt
     B, Hh, Lq, Lk = 1, 2, 100, 140
     print(f"[case] misaligned {D}", flush=True)
@@ -302,6 +302,26 @@ def test_misaligned_bases_bf16(am, dev, D):
     hip_rt.synchronize()
     n, nrel, mabs = H.check_bf16(out.numpy()[1:].reshape(Q.shape), _ref("none", Q, K, V))
     assert n == 0, (nrel, mabs)
+
+
+@pytest.mark.parametrize("dt,D,pe", [("bf16", 264, "none"), ("bf16", 264, "half"), ("bf16", 40, "none"),
+                                     ("f32", 264, "none"), ("f32", 40, "none")], ids=str)
+def test_misaligned_output(am, dev, dt, D, pe):
+    """The output alone off a 16-byte boundary."""
+    import hip_rt
+    B, Hh, Lq, Lk = 1, 2, 100, 140
+    code, es = (1, 2) if dt == "bf16" else (0, 4)
+    print(f"[case] misaligned output {dt} {D} {pe}", flush=True)
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 964, dt)
+    out = H.empty((Q.size + 1,), dt)
+    desc = _desc(am, pe)
+    st = am.lib().atn_attention_fwd_ex(code, q.ptr, k.ptr, v.ptr, out.ptr + es, B, Hh, Lq, Lk, D,
+                                       ctypes.byref(desc) if desc else None, None, 0, None)
+    assert st == 0
+    hip_rt.synchronize()
+    n, a, b = (H.check_f32 if dt == "f32" else H.check_bf16)(out.numpy()[1:].reshape(Q.shape),
+                                                             _ref(pe, Q, K, V))
+    assert n == 0, (a, b)
 
 
 @pytest.mark.parametrize("dt,D", [("bf16", 264), ("bf16", 40), ("bf16", 267), ("f32", 264), ("f32", 64)], ids=str)
