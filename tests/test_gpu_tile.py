@@ -199,22 +199,54 @@ def test_values_beyond_fp16_range(am, dev, tuner, tile, D, Lk, where):
     assert n == 0, mabs
 
 
-@pytest.mark.parametrize("pe", ["rope", "half", "sin"])
-def test_scratch_without_encoded_copies(am, dev, tuner, pe):
-    """K's encoded copy alone exceeds the scratch: encoded in the QK^T kernel."""
+@pytest.mark.parametrize("dt,D,pe,off", [
+    ("f32", 1024, "rope", 0), ("f32", 1024, "half", 0), ("f32", 1024, "sin", 0), ("f32", 1024, "half_k", 0),
+    ("f32", 1026, "rope", 0), ("f32", 1026, "half", 0), ("f32", 1025, "sin", 0), ("f32", 1024, "half", 1),
+    ("bf16", 1004, "none", 0), ("bf16", 1004, "rope", 0), ("bf16", 1002, "half", 0), ("bf16", 1001, "sin", 0),
+    ("bf16", 1001, "none", 0), ("bf16", 1008, "none", 1), ("bf16", 1008, "rope", 1)], ids=str)
+def test_scratch_without_copies(am, dev, dt, D, pe, off):
+    """What K's encoded copy, or K's and V's padded ones, would need exceeds the
+    scratch: the kernels that need none, in chunks of rows (positions and
+    pointers at an offset), for every row alignment; `off`: tensors one element
+    off a 16-byte boundary."""
     import hip_rt
-    B, Hh, Lq, Lk, D = 1, 1, 70, 400, 1024  # 1.6 MB of encoded K
-    print(f"[case] lean {pe}", flush=True)
-    desc = _desc(am, pe)
-    tuner.set(workspace_cap_mib=1)
-    assert am.workspace_bytes(0, B, Hh, Lq, Lk, D, desc) <= 1 << 20
+    B, Hh, Lq, Lk = 1, 2, 70, 400  # 1.6 MB of copies
+    print(f"[case] lean {dt} {D} {pe} +{off}", flush=True)
+    desc, (code, es) = _desc(am, pe), {"f32": (0, 4), "bf16": (1, 2)}[dt]
+    if not off:
+        plan = am.call_plan(code, B, Hh, Lq, Lk, D, desc, 1 << 20)
+        assert (plan["path"], plan["tiles"]) == (am.ATN_PATH_SPLIT_D, 0) and plan["chunk_rows"] < Lq
     sigma = 0.5 if pe == "sin" else 1.0
-    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 970, "f32", sigma)
+    Q, K, V = H.rng_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 970, sigma)
+    if dt == "bf16":
+        Q, K, V = (oracle.bf16_bits_to_f32(oracle.f32_to_bf16_bits(x)) for x in (Q, K, V))
+    dev_t = [H.upload(np.concatenate([[0.0] * off, x.ravel()]).astype(np.float32), dt) for x in (Q, K, V)]
     ws = hip_rt.DeviceArray(((1 << 20) // 4,), "f32", fill=0)
-    out = H.empty(Q.shape)
-    am.attention_ex(q, k, v, out, pe=desc, workspace=ws)
+    out = H.empty((Q.size + off,), dt)
+    st = am.lib().atn_attention_fwd_ex(code, *[t.ptr + off * es for t in dev_t], out.ptr + off * es, B, Hh, Lq,
+                                       Lk, D, ctypes.byref(desc) if desc else None, ws.ptr, 1 << 20, None)
+    assert st == 0
     hip_rt.synchronize()
-    _check(out.numpy(), Q, K, V, pe)
+    got = out.numpy()[off:].reshape(Q.shape)
+    n, a, b = (H.check_f32 if dt == "f32" else H.check_bf16)(got, _ref(pe, Q, K, V))
+    assert n == 0, (a, b)
+
+
+@pytest.mark.parametrize("D", [264, 263], ids=str)
+def test_scratch_for_scores_alone(am, dev, D):
+    """fp32 without an encoding needs no copies: a scratch that holds one row of
+    scores but not P beside them."""
+    import hip_rt
+    B, Hh, Lq, Lk = 1, 1, 3, 90001
+    nb = 40960 + 256 + 4 * Lk + 4096
+    print(f"[case] scores alone {D}", flush=True)
+    plan = am.call_plan(0, B, Hh, Lq, Lk, D, None, nb)
+    assert (plan["tiles"], plan["chunk_rows"]) == (0, 1)
+    (q, k, v), (Q, K, V) = H.device_inputs((B, Hh, Lq, D), (B, Hh, Lk, D), 971)
+    ws, out = hip_rt.DeviceArray((nb // 4,), "f32", fill=0), H.empty(Q.shape)
+    am.attention_ex(q, k, v, out, workspace=ws)
+    hip_rt.synchronize()
+    _check(out.numpy(), Q, K, V, "none")
 
 
 @pytest.mark.parametrize("dt,D,pe,kib", [("f32", 1024, "rope", 1160), ("bf16", 1004, "none", 1200)], ids=str)
