@@ -1383,7 +1383,8 @@ int attention_run(int dtype, const void* Q, const void* K, const void* V, void* 
             atn::PadTensor t[3] = {{V, w + tp.v_off, nk}, {Q, w + tp.q_off, nq}, {K, w + tp.k_off, nk}};
             ATN_HIP(atn::launch_pad_rows(t, plan.pek == atn::kPeNone ? 3 : 1, D, tp.Dp, stream));
         }
-        const atn::QkTileArgs qa{qt, kt, scratch, (int)s.BH, Lq, Lk, Dqk, tp.dchunk, tp.nsplit, tp.ldS, 0, 0};
+        const atn::QkTileArgs qa{qt, kt, scratch, (int)s.BH, Lq, Lk, Dqk, tp.dchunk,
+                                tp.nsplit, tp.ldS, plan.pek != atn::kPeNone, 0, 0};
         ATN_HIP(atn::launch_qk_tile(tp.qk, tp.tile_qk, qa, stream));
         ATN_HIP(atn::launch_softmax_split(tp.pv, tp.pparts, scratch, p, nq, Lk, tp.ldS, tp.ldP,
                                           tp.nsplit, (size_t)s.BH * Lq * tp.ldS, scale, stream));

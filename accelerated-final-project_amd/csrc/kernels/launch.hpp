@@ -62,6 +62,7 @@ struct QkTileArgs {
     const void* K;
     float* S;  // [nsplit][BH][Lq][ldS]
     int BH, Lq, Lk, D, dchunk, nsplit, ldS;
+    int comp;              // kTileF32: compensated sums
     int tiles_q, tiles_k;  // (filled by the launcher)
 };
 struct PvTileArgs {

@@ -237,8 +237,13 @@ __device__ __forceinline__ void st4_any(uint16_t* p, float4 v) {
 // queries: a lane holds 4 consecutive keys of one query per 16-byte store
 // (rows of S are ldS, a multiple of 4, apart).  RAG: head_d is no multiple of
 // 4 (fp32; rows then start at 4-byte boundaries and the last group of a row
-// is read element by element).
-template <int KIND, int TL, int NW, bool RAG>
+// is read element by element).  COMP: compensated sums.  Encoded rows make long
+// sums of one sign (sinusoidal), whose additions' roundings grow with the
+// D-chunk, and chunks are longer here than on the kernels without copies:
+// (4,4,567,279,904) sinusoidal 6.8e-7 there, 7.6e-7 with plain sums, 5.6e-7 with
+// compensated ones (at 2048 dims 8.0, 8.5, 6.9), for 4 % of the call; sums
+// without an encoding are no further off than there as they are.
+template <int KIND, int TL, int NW, bool RAG, bool COMP>
 __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs a) {
     using G = Tile<KIND>;
     constexpr int LROWS = 8 * NW, ROUNDS = TL / LROWS;  // loader: rows per round, rounds
@@ -348,9 +353,20 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
 #pragma unroll
             for (int j = 0; j < NQ; ++j) f(acc[i][j], sum[i][j]);
     };
-    auto zero = [&]() { each([](v16f&, v16f& y) { y = v16f{}; }); };
-    // the pair of stages just summed, into the tile's sum
-    auto flush = [&]() { each([](v16f& x, v16f& y) { y += x; }); };
+    auto zero = [&]() { each([](v16f& x, v16f& y) { x = y = v16f{}; }); };
+    // the pair of stages just summed, into the tile's sum; COMP: what the
+    // addition rounds off starts the next chain
+    auto flush = [&]() {
+        each([](v16f& x, v16f& y) {
+            if constexpr (COMP) {
+                const v16f t = y + x;
+                x -= t - y;
+                y = t;
+            } else {
+                y += x;
+            }
+        });
+    };
     auto compute = [&](const uint16_t* q, const uint16_t* k, auto fresh) {
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
@@ -370,7 +386,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
             for (int i = 0; i < NK; ++i)
 #pragma unroll
                 for (int j = 0; j < NQ; ++j) {
-                    v16f c = decltype(fresh)::value && ks == 0 ? v16f{} : acc[i][j];
+                    v16f c = decltype(fresh)::value && ks == 0 && !COMP ? v16f{} : acc[i][j];
                     if constexpr (KIND != kKindBF16) {
                         c = mfma_parts<KIND>(ka[i], qa[j], c);
                     } else {
@@ -406,10 +422,8 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
             issue(r0, d0 + G::DEPTH * (AHEAD + 2));
             __syncthreads();
         }
-        if (stages & 1) {
-            compute(sq[0], sk[0], std::true_type{});
-            flush();
-        }
+        if (stages & 1) compute(sq[0], sk[0], std::true_type{});
+        if (COMP || (stages & 1)) flush();
         if (kRanged) {
             tell_over(big, kRange, flag[1]);
             __syncthreads();
@@ -444,6 +458,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
                 issue(r0, d0 + G::DEPTH);
                 __syncthreads();
                 const float u = pow2_unit(mq) * pow2_unit(mk);
+                each([](v16f& x, v16f&) { x = v16f{}; });
                 compute(sq[0], sk[0], std::true_type{});
                 each([u](v16f& x, v16f& y) { y += x * u; });
             }
@@ -937,10 +952,14 @@ template <int KIND, int TL, int NW>
 void run_qk(const QkTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
     // (the other kinds' rows are whole 16-byte vectors)
     if (KIND == kKindX && rag)
-        hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, KIND == kKindX>), dim3(grid), dim3(64 * NW), 0,
-                           st, a);
+        hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, KIND == kKindX, false>), dim3(grid),
+                           dim3(64 * NW), 0, st, a);
+    else if (KIND == kKindF32 && a.comp)
+        hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, false, KIND == kKindF32>), dim3(grid),
+                           dim3(64 * NW), 0, st, a);
     else
-        hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, false>), dim3(grid), dim3(64 * NW), 0, st, a);
+        hipLaunchKernelGGL((k_qk_tile<KIND, TL, NW, false, false>), dim3(grid), dim3(64 * NW), 0, st,
+                           a);
 }
 template <int KIND>
 void run_qk_tile(int tile, const QkTileArgs& a, bool rag, unsigned grid, hipStream_t st) {
