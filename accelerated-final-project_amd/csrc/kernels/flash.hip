@@ -884,7 +884,7 @@ __global__ __launch_bounds__(256) void k_flash_combine_few(const float* __restri
     __shared__ float4 val[kFewSplits][64];
     __shared__ float wt[kFewSplits][64];
     __shared__ float mx[4][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned vpr = (unsigned)D >> 2;
     const unsigned g = min(blockIdx.x * 64 + lane, groups - 1);  // (below kFewGroups)
     const unsigned row = g / vpr, bh = row / (unsigned)Lq;
@@ -894,8 +894,8 @@ __global__ __launch_bounds__(256) void k_flash_combine_few(const float* __restri
     float4 st[PW], v[PW];
 #pragma unroll
     for (int i = 0; i < PW; ++i) {
-        const int s = wave + 4 * i;
-        const size_t pr = base + (size_t)(s < nsplit ? s : 0) * Lq;
+        if (wave + 4 * i >= nsplit) break;
+        const size_t pr = base + (size_t)(wave + 4 * i) * Lq;
         st[i] = stats[pr];
         v[i] = *reinterpret_cast<const float4*>(part + pr * D + d);
     }
