@@ -900,7 +900,8 @@ TilePlan tile_plan(int dtype, const Shape& s, const PePlan& plan, int a16) {
 // 16.3, (1,4,512,512,2048) 62.5 -> 31, (1,8,64,4096,2048) 195 -> 91, rotate-half
 // (2,8,300,300,1024) 70 -> 59; from about 128 GEMM tiles on the GEMMs lead
 // ((4,8,444,444,1008) 66 against 93 us, (4,16,508,508,1888) 201 against 315).
-// At 0.85 of the GEMMs' estimate and below: rotate-half (1,8,64,4096,2048), at
+// At 0.95 of the GEMMs' estimate and below ((2,4,603,603,1016), at 0.9: 48.7 us
+// against 62.8), with an encoding at 0.85: rotate-half (1,8,64,4096,2048), at
 // 0.87, takes 224 us either way and 289 MB of scratch for encoded copies
 // against 25.  Only where the whole call's scratch fits: in chunks of a head or
 // fewer each the tiles lose to the one GEMM call (that one in 64 MiB 715 us).
@@ -918,7 +919,7 @@ void choose_tiles(int dtype, const Shape& s, PePlan& plan, size_t cap) {
                 std::ceil(wgs(s.Lq, s.D)) * ((s.Lk + 63) / 64) * 2.2;
     if (gp.encoded) us += 4.0 + (double)s.nq * 4.0 / 4.5e6;
     if (gp.encoded && gp.benc == 0) us += 4.0 + (double)s.nk * 4.0 / 4.5e6;
-    plan.tiles = tp.bytes <= cap && tp.us < 0.85 * us;
+    plan.tiles = tp.bytes <= cap && tp.us < (gp.encoded ? 0.85 : 0.95) * us;
 }
 
 // ---------------------------------------------------------------- core
