@@ -433,8 +433,12 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
     }
     if constexpr (KIND == kKindF32) {
         if (redo) {  // every stage scaled by its largest magnitudes
-            issue(r0, dbeg);
+            // (4 waves of 128 x 128 without loads ahead: with them the
+            // compiler's schedule of the ordinary loop above is 3 % longer)
+            constexpr bool kLoadAhead = TL == 64 || NW == 8 || COMP;
+            if (kLoadAhead) issue(r0, dbeg);
             for (int d0 = dbeg; d0 < dend; d0 += G::DEPTH) {
+                if (!kLoadAhead) issue(r0, d0);
                 float mq = 0.f, mk = 0.f;
 #pragma unroll
                 for (int i = 0; i < ROUNDS; ++i) {
@@ -455,7 +459,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void k_qk_tile(QkTileArgs
                     *reinterpret_cast<uint2*>(sk[0] + o) = hi;
                     *reinterpret_cast<uint2*>(sk[0] + PART + o) = lo;
                 }
-                issue(r0, d0 + G::DEPTH);
+                if (kLoadAhead) issue(r0, d0 + G::DEPTH);
                 __syncthreads();
                 const float u = pow2_unit(mq) * pow2_unit(mk);
                 each([](v16f& x, v16f&) { x = v16f{}; });
