@@ -25,7 +25,7 @@
 //
 // What comes here: calls whose scratch cannot hold what the pipelined tiles
 // need beside the scores (tile16.hip: encoded or padded copies of Q, K and V,
-// P in two parts), and heads of 2 GiB and more.  Encodings are applied at
+// P in its 16-bit parts), and heads of 2 GiB and more.  Encodings are applied at
 // load, so the only scratch is the scores'.  Of those calls fp32 with head_d
 // % 4 == 0 and 16-byte aligned bases runs stages 1 and 3 on 16-bit MFMA
 // (stream16.hip), the rest on the kernels below.
