@@ -197,8 +197,9 @@ __device__ __forceinline__ uint32_t pk_bf16_rne(float a, float b) {
 // bf16 -- without an encoding ("raw") the loaded bits go to LDS as they are
 // and the products run on the bf16 MFMA (exact products, fp32's exponent
 // range: no scales, no tile maxima), P as bf16; with an encoding the
-// encoded values are fp32, staged as one fp16 part each (a power-of-two
-// scale per tile brings K and V into fp16's normal range), P as fp16.
+// encoded values of Q and K are fp32, staged as one fp16 part each (a
+// power-of-two scale per tile brings K into fp16's normal range), V and P as
+// without one.
 // waves per SIMD the register allocation leaves room for: 4 (two 8-wave
 // workgroups per CU) for the raw bf16 form of 8 waves of 16 rows at head_d
 // <= 128, which needs few registers; else what the form itself brings
